@@ -24,8 +24,11 @@ __device__ __forceinline__ bf16_bits f32_to_bf16(float f) {
   return __builtin_bit_cast(bf16_bits, h);
 }
 
+// Two of them in one word: one v_cvt_pk_bf16_f32 (as two conversions and an or it took four instructions).
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
+  typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+  const f32x2_t f = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2_v));
 }
 
 // fp32 -> float16, round to nearest even (v_cvt_f16_f32), and two of them in one word
@@ -67,8 +70,22 @@ __device__ __forceinline__ uint32_t fp8e4m3_to_bf16(uint32_t b) {
 
 __device__ __forceinline__ float bf16_to_f32(bf16_bits b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
 
-__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
-__device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
+// A vector at any address of global memory (the hardware takes accesses of up to 16 bytes at any alignment).
+template <class V>
+__device__ __forceinline__ V load_any(const void* p) {
+  typedef const __attribute__((address_space(1))) unsigned char* global_bytes;
+  typedef V unaligned_t __attribute__((aligned(1)));
+  return *reinterpret_cast<const __attribute__((address_space(1))) unaligned_t*>((global_bytes)p);
+}
+template <class V>
+__device__ __forceinline__ void store_any(void* p, V v) {
+  typedef __attribute__((address_space(1))) unsigned char* global_bytes;
+  typedef V unaligned_t __attribute__((aligned(1)));
+  *reinterpret_cast<__attribute__((address_space(1))) unaligned_t*>((global_bytes)p) = v;
+}
+
+__host__ __device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
+__host__ __device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
 
 // Work-groups are dealt to the 8 XCDs round-robin by launch index.  Remap the launch index so that each XCD
 // (own 4 MB L2) walks one contiguous range of logical tile ids.  Returns -1 for the padding of the last range.

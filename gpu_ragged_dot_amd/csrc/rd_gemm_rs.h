@@ -1,0 +1,426 @@
+// Four-wave GEMM core for operands that cannot be loaded straight into LDS: row pitches that are no multiple of 16 bytes
+// (bf16 and float16), and float32 arrays that are rounded to bf16 on the way (compute_dtype = bfloat16).  A 256 x 256 tile
+// held by a 2 x 2 grid of waves, 128 x 128 per wave, as in rd_gemm_w4.h; HBM -> registers -> LDS as in rd_gemm_w4r.h,
+// for any of the four operand layouts.
+//
+// What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
+// element per instruction where the pitch is odd, one slab in flight where the source is float32 - at 40-85 and 300-430
+// TFLOP/s (bf16 8191 x 2047 x 4095 in 16 groups, fwd / dlhs / drhs: 2300 / 3080 / 1620 us; float32 8192 x 4096 x 4096 in
+// 8: 683 / 668 / 899).  Here: 244 / 270 / 337 and 412 / 424 / 473 us; aligned bf16 16384 x 4096 x 4096 in 8 groups 574 us
+// (960 TFLOP/s).  Left over: the latency of the first slabs and of the epilogue, which nothing else on the compute unit
+// hides under a 256 x 256 tile, and pieces that straddle cache lines (20-50 % against the same sizes aligned).  How:
+//  * a load is always 16 bytes per lane (a "piece"), at whatever address the element has: global memory takes 16-byte
+//    accesses at any alignment.  Every 8 lanes (K-major) or every 32 / 64 (MN-major) read consecutive memory;
+//  * a slab is 128 bytes of every K-major row (64 bf16 or 32 float32 contraction indices), 16 pieces per lane for both
+//    operands, and two slabs are in flight in registers beside the two in LDS (bf16: 2 x 64 KB, float32 rounded: 2 x 32 KB);
+//  * the pieces are converted and written to LDS, and their registers refilled, spread evenly over the gaps between the
+//    matrix-core instructions of a slab.
+// No predicate sits in the steady loop: a slab that holds the last contraction index, or lies behind it, is loaded by
+// fetch_tail(), which never touches memory outside the operand's rows and fills with zeros.
+#pragma once
+#include <type_traits>
+#include "rd_gemm_dlds.h"
+
+namespace rd {
+
+// Src: bf16_bits, f16_t, or float (rounded to bf16; float32 out).  VEC: k and n are multiples of 8, so that no piece crosses
+// the end of a row and the last slab needs no shifting.
+template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, typename Src, bool VEC_>
+struct RsCfg {
+  typedef Src Elem;
+  static constexpr bool F32 = false, RS = true, HALF = std::is_same<Src, f16_t>::value;
+  static constexpr int BM = BM_, BN = BN_, BK = 128 / (int)sizeof(Src), WAVES_M = 2, WAVES_N = 2, STAGES = 2;
+  static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, VEC = VEC_, DLDS = false, PINGPONG = false, MIXED = false,
+                        SPLITK = true;
+  static constexpr int NW = 4, NT = 256;
+  static constexpr int WM = BM / 2, WN = BN / 2;
+  static constexpr int TM = WM / 32, TN = WN / 32;
+  static constexpr int KSTEPS = BK / 16;
+  static constexpr int WAVES_PER_EU = BM * BN > 128 * 128 ? 1 : 2;  // work-groups per compute unit
+  static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2;  // one slab in LDS, 16 bits per element
+  static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;
+  static constexpr int EPI_PITCH = WN * 2 + 16;
+  static constexpr int EPI_BYTES = sizeof(Src) == 2 ? NW * WM * EPI_PITCH : 0;
+  static constexpr int RING_BYTES = 2 * SLOT_BYTES;
+  static constexpr int LDS_BYTES = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
+  static_assert(BM % 128 == 0 && BN % 128 == 0, "tile shape");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
+};
+
+template <class C, class = void>
+struct IsRs { static constexpr bool value = false; };
+template <class C>
+struct IsRs<C, decltype((void)C::RS)> { static constexpr bool value = true; };
+
+// The 128-bit value v shifted down by `bytes` (0 .. 16, whole elements), zeros from above.
+__device__ __forceinline__ u32x4_t shift_down(u32x4_t v, int bytes) {
+  uint64_t lo = (uint64_t)v[0] | ((uint64_t)v[1] << 32), hi = (uint64_t)v[2] | ((uint64_t)v[3] << 32);
+  if (bytes >= 8) { lo = hi; hi = 0; bytes -= 8; }
+  if (bytes >= 8) { lo = 0; bytes = 0; }
+  const int b = bytes * 8;
+  lo = (lo >> b) | (b ? hi << (64 - b) : 0);
+  hi >>= b;
+  return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
+// One operand's slab, [T rows][BK] (K-major) or [BK][T columns] (MN-major), in pieces of 16 bytes: which memory each lane
+// reads for each of its pieces, and where the piece goes in LDS (the layout DldsFragReader reads).
+template <int T, int BK, int NW, bool KMAJOR, typename Src, bool VEC>
+struct RsLoader {
+  static constexpr int EPP = 16 / (int)sizeof(Src);              // elements per piece
+  static constexpr int PPR = (KMAJOR ? BK : T) / EPP;            // pieces per slab row
+  static constexpr int RPI = 64 / PPR;                           // slab rows per wave-wide load
+  static constexpr int PER = (KMAJOR ? T : BK) / RPI / NW;       // pieces per lane
+  static constexpr int LDS_ROW = (KMAJOR ? BK : T) * 2;          // bytes of a slab row in LDS
+  static constexpr int LDS_STEP = NW * RPI * LDS_ROW;            // from one of a lane's pieces to its next
+  static_assert(PPR <= 64 && 64 % PPR == 0 && (KMAJOR ? T : BK) % (RPI * NW) == 0, "slab does not split evenly");
+  // the chunk permutation of DldsFragReader repeats from one of a lane's pieces to the next
+  static_assert(KMAJOR ? (NW * RPI) % 16 == 0 : (NW * RPI) % 4 == 0, "chunk permutation");
+
+  const Src* base;   // first element of the current slab
+  long long step;    // elements from one slab to the next
+  uint32_t off0;     // byte offset of piece 0 from base; piece j lies j * row_step further, but no further than off_last
+  uint32_t row_step, off_last;
+  int ld, lim, klen;
+  int lds;           // byte of piece 0 in the operand's region of a slot
+
+  static __host__ __device__ __forceinline__ int slab_row(int wave, int lane, int j) { return wave * RPI + lane / PPR + j * NW * RPI; }
+
+  __host__ __device__ __forceinline__ void init(const Src* p, int ld_, int lim_, int klen_, int wave, int lane) {
+    base = p; ld = ld_; lim = lim_; klen = klen_;
+    step = KMAJOR ? BK : (long long)BK * ld;
+    const int row0 = slab_row(wave, lane, 0), piece = lane % PPR;
+    // rows past the tile's limit re-read its last row, columns past it the last piece that holds one of the tile's:
+    // what they hold never reaches a stored element
+    const int e = KMAJOR ? piece * EPP : imin(piece * EPP, (lim - 1) / EPP * EPP);
+    off_last = KMAJOR ? ((uint32_t)(lim - 1) * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src) : ~0u;
+    off0 = ((uint32_t)row0 * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src);
+    row_step = (uint32_t)(NW * RPI * sizeof(Src)) * (uint32_t)ld;
+    const int chunk = sizeof(Src) == 2 ? piece : piece >> 1;  // 16-byte chunk of the LDS row; a float32 piece fills half of one
+    const int c = KMAJOR ? (BK == 64 ? chunk ^ ((row0 >> 1) & 7) : chunk ^ ((row0 >> 2) & 3)) : chunk ^ ((row0 & 3) << 2);
+    lds = row0 * LDS_ROW + (c << 4) + (sizeof(Src) == 2 ? 0 : (piece & 1) * 8);
+  }
+
+  __host__ __device__ __forceinline__ uint32_t offset(int j) const {
+    const uint32_t o = off0 + (uint32_t)j * row_step;
+    return KMAJOR && o > off_last ? off_last : o;
+  }
+  // Piece j of the slab at base; the slab holds contraction indices below klen - 1 only.  (An MN-major piece may run past
+  // the end of its row, at most into the row behind it, which exists.)
+  __device__ __forceinline__ u32x4_t fetch(int j) const { return load_any<u32x4_t>(reinterpret_cast<const unsigned char*>(base) + offset(j)); }
+  // The same for any slab, its first contraction index being k0: element `at` of slab row `row` (counted from base; `at` may
+  // be negative).  Once there the piece is shifted down by `shift` elements (EPP or more: all zeros), which takes out what
+  // is not the operand's and zeroes what lies past the contraction length.  Slabs that fetch() serves come from where
+  // fetch() reads them, unshifted.
+  __host__ __device__ __forceinline__ void tail_source(int wave, int lane, int j, int k0, int* row, int* at, int* shift) const {
+    const int r = slab_row(wave, lane, j), e = lane % PPR * EPP;
+    if (KMAJOR) {
+      *row = imin(r, lim - 1);
+      *at = imin(e, klen - EPP - k0);
+      *shift = e - *at;
+    } else {
+      const bool whole = k0 + BK < klen;
+      *row = imin(r, klen - 1 - k0);
+      *at = imin(e, whole ? (lim - 1) / EPP * EPP : lim - EPP);
+      *shift = r != *row ? EPP : whole ? 0 : e - *at;
+    }
+  }
+  __device__ __forceinline__ u32x4_t fetch_tail(int wave, int lane, int j, int k0) const {
+    int row, at, shift;
+    tail_source(wave, lane, j, k0, &row, &at, &shift);
+    return load_any<u32x4_t>(base + ((long long)row * ld + at));
+  }
+  __device__ __forceinline__ u32x4_t shift_tail(int wave, int lane, int j, int k0, u32x4_t v) const {
+    int row, at, shift;
+    tail_source(wave, lane, j, k0, &row, &at, &shift);
+    if constexpr (VEC) return shift == 0 ? v : u32x4_t{0, 0, 0, 0};
+    else return shift_down(v, imin(shift, EPP) * (int)sizeof(Src));
+  }
+  __device__ __forceinline__ void commit(unsigned char* region, int j, u32x4_t v) const {
+    unsigned char* d = region + lds + j * LDS_STEP;
+    if constexpr (sizeof(Src) == 2) {
+      *reinterpret_cast<u32x4_t*>(d) = v;
+    } else {
+      const f32x4_t f = __builtin_bit_cast(f32x4_t, v);
+      *reinterpret_cast<u32x2_t*>(d) = u32x2_t{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
+    }
+  }
+  // The new base and the lane's offset are opaque to the compiler: it would otherwise carry an address per piece through
+  // the loop, and there are no registers for those.
+  __device__ __forceinline__ void advance() {
+    const uint64_t b = reinterpret_cast<uint64_t>(base + step);
+    base = reinterpret_cast<const Src*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b) |
+                                        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32));
+    asm volatile("" : "+v"(off0));
+  }
+};
+
+namespace rs_detail {
+template <int V>
+struct Int { static constexpr int value = V; };
+// how a slab's pieces are loaded: it ends before the last contraction index, or it may hold that index or lie behind it
+constexpr int kWhole = 0, kTail = 1;
+}  // namespace rs_detail
+
+// Slab t lives in LDS slot t & 1 and, before that, in register set t & 1.  The pieces of slab t + 1 are written to LDS
+// during the substeps of slab t (16 contraction indices each, fragments read one substep ahead), except that the last
+// substep, which follows the slab's barrier, already writes the first pieces of slab t + 2 into the slot slab t has left.
+// Each write is followed by the load of the same piece two slabs further on.  float32 slabs have half as many substeps
+// for as many pieces, so a gap there carries a write and a load where a 16-bit slab alternates them.
+template <class C, bool LIVE>
+__device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap, int lda, int a_lim,
+                                         const typename C::Elem* __restrict__ Bp, int ldb, int b_lim, int klen,
+                                         unsigned char* smem, int wave, int lane, f32x16_t (&acc)[C::TM][C::TN]) {
+  typedef typename C::Elem E;
+  const int wm = wave >> 1, wn = wave & 1;
+  typedef RsLoader<C::BM, C::BK, C::NW, C::A_KMAJOR, E, C::VEC> LdA;
+  typedef RsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR, E, C::VEC> LdB;
+  LdA la; LdB lb;
+  la.init(Ap, lda, a_lim, klen, wave, lane);
+  lb.init(Bp, ldb, b_lim, klen, wave, lane);
+  DldsFragReader<C::BM, C::BK, C::TM, C::A_KMAJOR> fra;
+  DldsFragReader<C::BN, C::BK, C::TN, C::B_KMAJOR> frb;
+  fra.init(wm * C::WM, lane);
+  frb.init(wn * C::WN, lane);
+
+  const int nk = (klen + C::BK - 1) / C::BK;  // the last slab, nk - 1, holds the last contraction index
+  constexpr int PA = LdA::PER, PB = LdB::PER, P = PA + PB;
+  constexpr int MF = C::TM * C::TN, R0 = C::TM + C::TN;
+  constexpr int HEAD = P / C::KSTEPS;       // pieces moved per substep
+  // What the gaps between a substep's matrix-core instructions carry.  Large patches: one fragment read each in the first
+  // ones, then the pieces, spread out (a write and the load that refills its registers in one gap or in two).  Small
+  // patches have fewer gaps than reads and pieces: every gap carries its share of both.
+  constexpr bool ROOMY = MF - R0 >= HEAD;
+  constexpr int GAP = MF - R0 >= 2 * HEAD ? 2 : 1;
+  static_assert(P % C::KSTEPS == 0 && (ROOMY || HEAD % MF == 0 || MF % HEAD == 0), "every substep has room for its pieces");
+
+  u32x4_t regs[2][P];
+  auto fetch_one = [&](auto set_tag, int step, int q, auto mode_tag) {
+    constexpr int SET = decltype(set_tag)::value, MODE = decltype(mode_tag)::value;
+    if constexpr (MODE == rs_detail::kWhole) regs[SET][q] = q < PA ? la.fetch(q) : lb.fetch(q - PA);
+    else
+      regs[SET][q] = q < PA ? la.fetch_tail(wave, lane, q, step * C::BK) : lb.fetch_tail(wave, lane, q - PA, step * C::BK);
+  };
+  // (a piece is shifted here and not where it is fetched, or every load would be waited for at once)
+  auto commit_one = [&](auto set_tag, int slot_off, int step, int q, auto mode_tag) {
+    constexpr int SET = decltype(set_tag)::value, MODE = decltype(mode_tag)::value;
+    u32x4_t v = regs[SET][q];
+    if constexpr (MODE == rs_detail::kTail)
+      v = q < PA ? la.shift_tail(wave, lane, q, step * C::BK, v) : lb.shift_tail(wave, lane, q - PA, step * C::BK, v);
+    if (q < PA) la.commit(smem + slot_off, q, v);
+    else lb.commit(smem + slot_off + C::A_BYTES, q - PA, v);
+  };
+  auto advance = [&]() { la.advance(); lb.advance(); };
+
+  // slab 0 through the registers into LDS, slab 1 in registers with its first pieces written, slab 2 requested
+  auto prologue = [&](auto mode_tag) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, 0, q, mode_tag);
+    advance();
+#pragma unroll
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<1>{}, 1, q, mode_tag);
+    advance();
+#pragma unroll
+    for (int q = 0; q < P; ++q) commit_one(rs_detail::Int<0>{}, 0, 0, q, mode_tag);
+#pragma unroll
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, 2, q, mode_tag);
+    advance();
+#pragma unroll
+    for (int q = 0; q < HEAD; ++q) commit_one(rs_detail::Int<1>{}, C::SLOT_BYTES, 1, q, mode_tag);
+#pragma unroll
+    for (int q = 0; q < HEAD; ++q) fetch_one(rs_detail::Int<1>{}, 3, q, mode_tag);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): slab 0 is written
+    __builtin_amdgcn_s_barrier();
+  };
+
+  bf16x8_t fa[2][C::TM], fb[2][C::TN];
+  auto first_fragments = [&]() {
+    if (LIVE) {
+#pragma unroll
+      for (int i = 0; i < C::TM; ++i) fa[0][i] = fra.read(smem, i, 0);
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j) fb[0][j] = frb.read(smem + C::A_BYTES, j, 0);
+    }
+  };
+
+  // mode: how the pieces of slabs t + 3 and t + 4 are loaded
+  auto slab = [&](int t, auto next_tag, auto mode_tag) {
+    constexpr int NEXT = decltype(next_tag)::value;  // (t + 1) & 1
+    const int cur_off = (1 - NEXT) * C::SLOT_BYTES, next_off = NEXT * C::SLOT_BYTES;
+#pragma unroll
+    for (int u = 0; u < C::KSTEPS; ++u) {
+      const bool last = u == C::KSTEPS - 1;
+      if (last) {  // own reads of slab t returned, own pieces of slab t + 1 written; behind the barrier slab t + 1 is complete
+        advance();
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const unsigned char* ra = smem + (last ? next_off : cur_off);  // fragments of the next substep
+      const unsigned char* rb = ra + C::A_BYTES;
+      const int us = last ? 0 : u + 1;
+#pragma unroll
+      for (int m = 0; m < MF; ++m) {
+        const int i = m / C::TN, j = m % C::TN;
+        if (LIVE && ROOMY) {
+          if (m < C::TM) fa[(u + 1) & 1][m] = fra.read(ra, m, us);
+          else if (m < R0) fb[(u + 1) & 1][m - C::TM] = frb.read(rb, m - C::TM, us);
+        } else if (LIVE) {
+#pragma unroll
+          for (int r = m * R0 / MF; r < (m + 1) * R0 / MF; ++r) {
+            if (r < C::TM) fa[(u + 1) & 1][r] = fra.read(ra, r, us);
+            else fb[(u + 1) & 1][r - C::TM] = frb.read(rb, r - C::TM, us);
+          }
+        }
+        auto write = [&](int p) {
+          if (last) commit_one(rs_detail::Int<1 - NEXT>{}, cur_off, t + 2, p, mode_tag);
+          else commit_one(next_tag, next_off, t + 1, (u + 1) * HEAD + p, mode_tag);
+        };
+        auto load = [&](int p) {
+          if (last) fetch_one(rs_detail::Int<1 - NEXT>{}, t + 4, p, mode_tag);
+          else fetch_one(next_tag, t + 3, (u + 1) * HEAD + p, mode_tag);
+        };
+        if constexpr (ROOMY) {
+          const int p = (m - R0) / GAP;
+          if (m >= R0 && p < HEAD) {
+            if ((m - R0) % GAP == 0) write(p);
+            if ((m - R0) % GAP == GAP - 1) load(p);
+          }
+        } else {
+#pragma unroll
+          for (int p = m * HEAD / MF; p < (m + 1) * HEAD / MF; ++p) { write(p); load(p); }
+        }
+        if (LIVE) {
+          // float32 results leave straight from the accumulators, a register holding 32 consecutive columns of a row;
+          // 16-bit results go through LDS and want four consecutive columns per lane (operands swapped)
+          if constexpr (sizeof(E) == 2) acc[i][j] = mfma_32x32x16<C::HALF>(fb[u & 1][j], fa[u & 1][i], acc[i][j]);
+          else acc[i][j] = mfma_32x32x16<false>(fa[u & 1][i], fb[u & 1][j], acc[i][j]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  // Slabs t < n_steady load slabs up to t + 4, which are whole.  An even count, entered straight from the prologue of whole
+  // slabs: the compiler counts the loads outstanding at each register's use along every path into the loop.  The slabs
+  // behind it run one loop of the same shape with all loads as tails (what lies past the contraction length comes as zeros):
+  // with a condition around the loads, or the last slabs written out one by one, the registers no longer suffice.
+  constexpr rs_detail::Int<rs_detail::kWhole> whole{};
+  constexpr rs_detail::Int<rs_detail::kTail> tail{};
+  const int n_steady = (nk - 5) & ~1;
+  int t = 0;
+  if (n_steady > 0) {
+    prologue(whole);
+    first_fragments();
+    for (; t < n_steady; t += 2) {
+      slab(t, rs_detail::Int<1>{}, whole);
+      slab(t + 1, rs_detail::Int<0>{}, whole);
+    }
+  } else {
+    prologue(tail);
+    first_fragments();
+  }
+  for (; t < nk; t += 2) {  // (an odd nk multiplies one slab of zeros)
+    slab(t, rs_detail::Int<1>{}, tail);
+    slab(t + 1, rs_detail::Int<0>{}, tail);
+  }
+
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();  // the slots are no longer read by any wave
+}
+
+// 16-bit results: each wave turns its patch through LDS into rows and stores 16 bytes per lane at whatever address the
+// row has; the piece that crosses the tile's last column goes element by element.
+template <class C>
+__device__ __forceinline__ void rs_store16(const f32x16_t (&acc)[C::TM][C::TN], int wm, int wn, int wave, int lane, int a_lim,
+                                           int b_lim, typename C::Elem* __restrict__ Op, int ldo, unsigned char* smem) {
+  unsigned char* st = smem + wave * (C::WM * C::EPI_PITCH);
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int row = i * 32 + (lane & 31), col = j * 32 + 8 * g + 4 * (lane >> 5);
+        u32x2_t w;
+        w[0] = pack_out_x2<C::HALF>(acc[i][j][4 * g + 0], acc[i][j][4 * g + 1]);
+        w[1] = pack_out_x2<C::HALF>(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+        *reinterpret_cast<u32x2_t*>(st + row * C::EPI_PITCH + col * 2) = w;
+      }
+  constexpr int CPR = C::WN / 8, ROWS_PER = 64 / CPR, NIT = C::WM / ROWS_PER, BATCH = NIT < 8 ? NIT : 8;
+  static_assert(NIT % BATCH == 0, "whole batches");
+  const int chunk = lane % CPR, r0 = lane / CPR;
+  const int gcol = wn * C::WN + chunk * 8, live = b_lim - gcol;  // live: the lane's columns inside the tile
+#pragma unroll
+  for (int t0 = 0; t0 < NIT; t0 += BATCH) {
+    u32x4_t v[BATCH];
+#pragma unroll
+    for (int b = 0; b < BATCH; ++b)
+      v[b] = *reinterpret_cast<const u32x4_t*>(st + ((t0 + b) * ROWS_PER + r0) * C::EPI_PITCH + chunk * 16);
+#pragma unroll
+    for (int b = 0; b < BATCH; ++b) {
+      const int grow = wm * C::WM + (t0 + b) * ROWS_PER + r0;
+      if (grow >= a_lim || live <= 0) continue;
+      unsigned char* d = reinterpret_cast<unsigned char*>(Op + (size_t)grow * ldo + gcol);
+      if (live >= 8) store_any(d, v[b]);
+      else
+#pragma unroll
+        for (int e = 0; e < 7; ++e)
+          if (e < live) reinterpret_cast<uint16_t*>(d)[e] = (uint16_t)(v[b][e >> 1] >> ((e & 1) * 16));
+    }
+  }
+}
+
+// float32 results: register v of a 32 x 32 block is 32 consecutive columns of row 8 (v >> 2) + 4 (lane >> 5) + (v & 3) - a
+// whole 128-byte line per half wave.  Rows and columns past the tile's limits get an offset outside the output's window,
+// which the hardware drops.
+template <class C>
+__device__ __forceinline__ void rs_store32(const f32x16_t (&acc)[C::TM][C::TN], int wm, int wn, int lane, int a_lim, int b_lim,
+                                           float* __restrict__ Op, int ldo) {
+  const int bytes = ((a_lim - 1) * ldo + b_lim) * 4;  // below 2 GiB: checked on the host
+  __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc((void*)Op, 0, __builtin_amdgcn_readfirstlane(bytes), kBufferFlags);
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+      const int col = wn * C::WN + j * 32 + (lane & 31);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = wm * C::WM + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+        const int off = row < a_lim && col < b_lim ? (row * ldo + col) * 4 : kOobOffset;
+        const float f = acc[i][j][v];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), orsrc, off, 0, kCachePolicyStream);
+      }
+    }
+}
+
+// Same contract as gemm_tile(), and: the rows the operands are read along hold at least 8 elements (16-bit) or 4
+// (float32) up to and including the tile's last one - k >= 8 and n >= 8.
+template <class C>
+__device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict__ Ap, int lda, int a_lim,
+                                             const typename C::Elem* __restrict__ Bp, int ldb, int b_lim, int klen,
+                                             typename C::Elem* __restrict__ Op, int ldo, unsigned char* smem,
+                                             const SplitK& sk = SplitK()) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const bool patch_live = wm * C::WM < a_lim && wn * C::WN < b_lim;
+
+  f32x16_t acc[C::TM][C::TN];
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  if (patch_live) rs_kloop<C, true>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
+  else rs_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
+
+  if (!splitk_combine<C>(acc, sk, tid, smem)) return;
+  if constexpr (sizeof(typename C::Elem) == 2) rs_store16<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
+  else rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
+}
+
+}  // namespace rd

@@ -7,6 +7,7 @@
 #include "rd_gemm_w4.h"
 #include "rd_gemm_w4r.h"
 #include "rd_gemm_pp.h"
+#include "rd_gemm_rs.h"
 #include "rd_gemm_tile.h"
 #include "rd_sched.h"
 
@@ -79,6 +80,7 @@ __device__ __forceinline__ void run_tile(const typename C::Elem* Ap, int lda, in
                                          int ldb, int b_lim, int klen, typename OutOf<C>::type* Op, int ldo,
                                          typename C::Elem* smem, const SplitK& sk = SplitK()) {
   if constexpr (C::F32) gemm_tile_f32<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem);
+  else if constexpr (IsRs<C>::value) gemm_tile_rs<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, reinterpret_cast<unsigned char*>(smem), sk);
   else if constexpr (IsF8Direct<C>::value) {
     if constexpr (C::PINGPONG) gemm_tile_f8_pingpong<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
     else gemm_tile_f8<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
@@ -357,6 +359,7 @@ struct TileVariant {
   int dtype;   // RD_DTYPE_* of the operands and the output this shape is compiled for
   int dlds;    // 1: direct-to-LDS core (byte extents of one tile's operand window must stay below 2 GiB)
   int stages;  // LDS ring depth
+  int any_pitch_core;  // 1: the register-staged core of rd_gemm_rs.h (k >= 8, n >= 8, 32-bit offsets within 256 rows)
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product
   tgmm_launch_fn tgmm;

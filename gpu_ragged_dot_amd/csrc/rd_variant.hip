@@ -1,5 +1,5 @@
 // One compiled tile shape.  Built once per entry of the variant list in the Makefile, with
-//   -DRD_BM= -DRD_BN= -DRD_BK= -DRD_WAVES_M= -DRD_WAVES_N= -DRD_VEC= -DRD_NAME= [-DRD_DLDS=1|2|3 -DRD_STAGES= -DRD_PINGPONG=1
+//   -DRD_BM= -DRD_BN= -DRD_BK= -DRD_WAVES_M= -DRD_WAVES_N= -DRD_VEC= -DRD_NAME= [-DRD_DLDS=1|2|3|4 -DRD_STAGES= -DRD_PINGPONG=1
 //   -DRD_F32=1|2|3|4]
 // and exports a getter rd_variant_<name>() for its TileVariant record that the C-ABI file collects.
 #include "rd_kernels.h"
@@ -23,8 +23,28 @@
 #define RD_F32 0
 #endif
 
+#if RD_DLDS == 4
+#define RD_ANY_PITCH 1
+#undef RD_DLDS
+#define RD_DLDS 0
+#else
+#define RD_ANY_PITCH 0
+#endif
+
 namespace rd {
-#if RD_F32 == 4 && RD_DLDS == 3
+#if RD_ANY_PITCH
+// 16-byte pieces at any address through registers (rd_gemm_rs.h): bf16, float16, or float32 rounded to bf16
+#if RD_F32 == 2
+typedef float RsElem;
+#elif RD_F32 == 4
+typedef f16_t RsElem;
+#else
+typedef bf16_bits RsElem;
+#endif
+typedef RsCfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RsElem, RD_VEC != 0> CfgNN;
+typedef RsCfg<RD_BM, RD_BN, true, true, RsElem, RD_VEC != 0> CfgNT;
+typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0> CfgTN;
+#elif RD_F32 == 4 && RD_DLDS == 3
 // float16 arrays on the four-wave direct-to-LDS core: the bf16 core's data movement with the float16 instruction
 typedef W4Cfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, true> CfgNN;
 typedef W4RCfg<RD_BM, RD_BN, true> CfgNT;
@@ -84,7 +104,7 @@ typedef TileCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, false, false, RD_VE
 extern "C" const rd::TileVariant* RD_CAT(rd_variant_, RD_NAME)() {
   static const rd::TileVariant v = {
       RD_STR(RD_NAME), RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, RD_VEC, /*dtype: RD_DTYPE_* */ RD_F32, RD_DLDS != 0, RD_STAGES,
-      /*splitk*/ RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4),
+      RD_ANY_PITCH, /*splitk*/ RD_ANY_PITCH || (RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4)),
 #ifdef RD_NO_TGMM
       &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr};
 #else

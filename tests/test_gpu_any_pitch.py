@@ -1,0 +1,71 @@
+"""The any-pitch core (register-staged 256 x 256 and 128 x 128 tiles for odd row pitches and for float32 rounded to bf16)
+and the 64 x 64 tiles that share its unaligned loads, against the oracle.
+
+Sizes where it can go wrong: contractions of less than one slab, of one element more and less than a whole number of slabs
+around the point where the pipelined loop takes over, rows of one piece only, tile edges, groups of 0, 1 and one more than
+a tile's rows.  One group's operands are NaN: pieces that run past a row or a group must not carry them into the others.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_ragged_dot_amd import _capi, ops
+from oracle import ragged_dot_oracle as oracle
+from tests import util
+
+pytestmark = pytest.mark.gpu
+
+HP = dict(block_m=64, block_k=64, block_n=64, interpret=False, acc_dtype=torch.float32, chunk_m=512)
+KINDS = {_capi.RD_DTYPE_BF16: ("bfloat16", torch.bfloat16, None), _capi.RD_DTYPE_F16: ("float16", torch.float16, None),
+         _capi.RD_DTYPE_F32_BF16: ("bfloat16", torch.float32, torch.bfloat16)}
+VARIANTS = [(v.id, v.name.decode(), v.dtype) for v in _capi.variants()
+            if v.name.decode().startswith(("r", "hr", "cr", "cs", "s64", "h64x64", "c64"))]
+# (k, n): slabs of 64 (16-bit) or 32 (float32); the pipelined loop takes over from seven slabs on
+SHAPES = [(8, 8), (57, 77), (63, 129), (65, 257), (191, 9), (225, 131), (385, 255), (449, 250), (577, 264)]
+
+
+@pytest.mark.parametrize("vid,vname,dtype", VARIANTS, ids=[v[1] for v in VARIANTS])
+@pytest.mark.parametrize("k,n", SHAPES, ids=[f"k{k}n{n}" for k, n in SHAPES])
+def test_any_pitch_edges(vid, vname, dtype, k, n):
+    if vname.startswith("cr") and (k % 8 or n % 8):
+        k, n = (k + 7) // 8 * 8, (n + 7) // 8 * 8
+    print(f"variant {vname} k {k} n {n}", flush=True)
+    rounding, storage, compute = KINDS[dtype]
+    gs = np.array([257, 0, 1, 63, 40, 129, 7], np.int32)
+    poisoned, tail = 4, 5
+    g, m, total = len(gs), int(gs.sum()) + tail, int(gs.sum())
+    rng = np.random.default_rng(k * 1000 + n)
+    r = lambda a: oracle.round_to(a, rounding)
+    x, A, dy = r(rng.normal(size=(m, k))), r(rng.normal(size=(g, k, n)) / np.sqrt(k)), r(rng.normal(size=(m, n)))
+    first = int(gs[:poisoned].sum())
+    hit = slice(first, first + int(gs[poisoned]))
+    clean = np.ones(m, bool)
+    clean[hit] = False
+    x_in, A_in, dy_in = x.copy(), A.copy(), dy.copy()
+    x_in[hit], A_in[poisoned], dy_in[hit] = np.nan, np.nan, np.nan
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda().to(storage)
+    gs_t, plan = torch.from_numpy(gs).cuda(), _capi.Plan(vid)
+    y = util.to_np(ops._gmm_fwd(dev(x_in), dev(A_in), gs_t, trans_rhs=False, compute_dtype=compute, plan=plan, **HP))
+    yt = util.to_np(ops._gmm_fwd(dev(x_in), dev(np.swapaxes(A_in, 1, 2)), gs_t, trans_rhs=True, compute_dtype=compute, plan=plan, **HP))
+    dA = util.to_np(ops._tgmm_fwd(dev(x_in), dev(dy_in), gs_t, compute_dtype=compute, plan=plan, **HP))
+    f64 = dict(out_dtype="float32", acc=np.float64)
+    y_ref, dA_ref = oracle.gmm(x, A, gs, **f64), oracle.tgmm(x, dy, gs, **f64)
+    # 16-bit results: one rounding to a significand of 8 or 11 bits (at most 2^-8 or 2^-11 of the value) on top of fp32 sums
+    # of at most 577 products (577 x 2^-24 = 3.5e-5); float32 results: the sums alone
+    eps = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11}[rounding] if storage != torch.float32 else 0.0
+    eps += 577 * 2.0 ** -24
+    for name, got in (("y", y), ("y (trans_rhs)", yt)):
+        assert np.all(np.isnan(got[hit])), f"{name}: the poisoned group's rows"
+        live = clean & (np.arange(m) < total)
+        err = np.linalg.norm(got[live] - y_ref[live], axis=1) / np.linalg.norm(y_ref[live], axis=1)
+        assert err.max() < eps, f"{name}: {err.max()} >= {eps}"
+        assert not np.any(got[total:]), f"{name}: tail rows"
+    for i in range(g):
+        if i == poisoned:
+            continue
+        if gs[i] == 0:
+            assert not np.any(dA[i])
+        else:
+            err = np.linalg.norm(dA[i] - dA_ref[i]) / np.linalg.norm(dA_ref[i])
+            assert err < eps, f"dA[{i}]: {err} >= {eps}"
