@@ -1,18 +1,19 @@
 """``ragged_dot`` / ``trans_ragged_dot`` with the reference's Python signature, running on HIP kernels.
 
 Mirrors gpu_ragged_dot.py:345-454 (``gmm``, ``tgmm``, their aliases and the custom VJP).  Arrays are
-``torch.Tensor`` on a ROCm device: torch supplies device memory and the stream, nothing else - every product is
-computed by ``csrc/libragged_dot_hip.so`` through its C ABI.
+``torch.Tensor`` on a ROCm device: torch supplies device memory, the stream and the autograd engine, nothing else - every
+product is computed by ``csrc/libragged_dot_hip.so`` through its C ABI.  What a call does on the host - checks, plan,
+allocation, the autograd node - is native code (``csrc/rd_torch.cpp``); this module maps the reference's keywords onto it.
 """
 
 from __future__ import annotations
 
-import ctypes
 from typing import Optional
 
 import torch
 
 from . import _capi, planner
+from ._native import lib as _native
 from .planner import CHUNK_M, DEFAULT_BLOCK_K, DEFAULT_BLOCK_M, DEFAULT_BLOCK_N
 
 __all__ = ["gmm", "tgmm", "ragged_dot", "trans_ragged_dot", "ragged_dot_vjp", "make_group_metadata"]
@@ -21,10 +22,10 @@ _DTYPES = {torch.bfloat16: _capi.RD_DTYPE_BF16, torch.float32: _capi.RD_DTYPE_F3
            torch.float8_e4m3fn: _capi.RD_DTYPE_F8E4M3_BF16, torch.float16: _capi.RD_DTYPE_F16}
 
 
-def _out_dtype(t: torch.Tensor) -> torch.dtype:
-    """The output has the operands' element type (gpu_ragged_dot.py:210,324); float8 operands, which the reference does
-    not have, give bfloat16 (jax.lax.ragged_dot with preferred_element_type=bfloat16)."""
-    return torch.bfloat16 if t.dtype == torch.float8_e4m3fn else t.dtype
+# (storage dtype, compute_dtype) of the usual calls; _dtype_code() explains the rest
+_CODES = {(t, None): code for t, code in _DTYPES.items()}
+_CODES.update({(t, t): code for t, code in _DTYPES.items()})
+_CODES[torch.float32, torch.bfloat16] = _capi.RD_DTYPE_F32_BF16
 
 
 def _dtype_code(t: torch.Tensor, compute_dtype, acc_dtype) -> int:
@@ -50,25 +51,6 @@ def _dtype_code(t: torch.Tensor, compute_dtype, acc_dtype) -> int:
     raise NotImplementedError(f"no kernel for compute_dtype={compute_dtype} on {t.dtype} operands")
 
 
-def _aligned16(*tensors: torch.Tensor) -> bool:
-    """The fast tile shapes move 16 bytes at a time: every buffer must start on a 16-byte boundary (a view at an odd
-    element offset does not, however contiguous it is)."""
-    return all(t.data_ptr() % 16 == 0 for t in tensors)
-
-
-def _check_device(*tensors: torch.Tensor) -> torch.device:
-    dev = tensors[0].device
-    if dev.type != "cuda":
-        raise RuntimeError(
-            "ragged_dot runs on a ROCm device only (tensors must be on 'cuda'); there is no CPU path. "
-            "interpret=True of the reference (the Pallas interpreter) has no counterpart here."
-        )
-    for t in tensors:
-        if t.device != dev:
-            raise RuntimeError("all operands must live on the same device")
-    return dev
-
-
 def _group_sizes_i32(group_sizes, dev: torch.device) -> torch.Tensor:
     gs = torch.as_tensor(group_sizes)
     if gs.dtype != torch.int32:
@@ -78,10 +60,6 @@ def _group_sizes_i32(group_sizes, dev: torch.device) -> torch.Tensor:
 
 def _stream_ptr(dev: torch.device) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
-
-
-def _plan_ref(plan: Optional[_capi.Plan]):
-    return ctypes.byref(plan) if plan is not None else None
 
 
 def _group_offset(group_offset) -> int:
@@ -94,135 +72,103 @@ def _group_offset(group_offset) -> int:
     return int(group_offset)
 
 
-def _gmm_fwd(x, A, group_sizes, block_m, block_k, block_n, trans_rhs, interpret, compute_dtype, acc_dtype, chunk_m,
-             plan: Optional[_capi.Plan] = None, group_offset=None) -> torch.Tensor:
-    """gpu_ragged_dot.py:171-228 (_gpu_gmm_fwd): checks, planning, one call across the C ABI.
+def _aligned16(*tensors: torch.Tensor) -> bool:
+    """The fast tile shapes move 16 bytes at a time: every buffer must start on a 16-byte boundary (a view at an odd
+    element offset does not, however contiguous it is)."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _fields(plan: _capi.Plan) -> tuple:
+    return (plan.variant, plan.group_m, plan.group_n, plan.decode_nb, plan.split_k)
+
+
+def _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset):
+    """What both products need from the reference's keywords: the element-type code, group_sizes as a tensor, and the first
+    group as a host integer (-1: no group_offset given)."""
+    if interpret:
+        raise NotImplementedError("interpret=True (Pallas interpreter) has no counterpart; kernels run on the GPU only")
+    code = _CODES.get((x.dtype, compute_dtype)) if acc_dtype is torch.float32 else None
+    if code is None:
+        code = _dtype_code(x, compute_dtype, acc_dtype)
+    if type(group_sizes) is not torch.Tensor:
+        group_sizes = torch.as_tensor(group_sizes)
+    return code, group_sizes, -1 if group_offset is None else _group_offset(group_offset)
+
+
+def _default_blocks(block_m, block_k, block_n) -> bool:
+    return block_m == DEFAULT_BLOCK_M and block_k == DEFAULT_BLOCK_K and block_n == DEFAULT_BLOCK_N
+
+
+def _gmm_plans(x, A, trans_rhs, g, code, block_m, block_k, block_n):
+    """Plans of the product and of its two gradients for explicit block sizes (gpu_ragged_dot.py:194-197)."""
+    (m, k), n = x.shape, A.shape[-2 if trans_rhs else -1]
+    planner.normalize_gmm_blocks(block_m, block_k, block_n, m, k, n)  # validates the request
+    blocks = dict(block_m=block_m, block_k=block_k, block_n=block_n, dtype=code)
+    fwd, bwd = (_capi.OP_GMM_TRANS, _capi.OP_GMM) if trans_rhs else (_capi.OP_GMM, _capi.OP_GMM_TRANS)
+    weights = (n, k) if trans_rhs else (k, n)
+    return tuple(_fields(p) for p in (
+        planner.select_plan(fwd, m, k, n, g, aligned=_aligned16(x, A), **blocks),
+        planner.select_plan(bwd, m, n, k, g, **blocks),
+        planner.select_plan(_capi.OP_TGMM, m, *weights, g, **blocks)))
+
+
+def _tgmm_plans(x, y, g, code, block_m, block_k, block_n):
+    """The same for tgmm (gpu_ragged_dot.py:308-314)."""
+    (m, k), n = x.shape, y.shape[-1]
+    planner.normalize_tgmm_blocks(block_m, block_k, block_n, m, k, n)
+    blocks = dict(block_m=block_m, block_k=block_k, block_n=block_n, dtype=code)
+    return tuple(_fields(p) for p in (
+        planner.select_plan(_capi.OP_TGMM, m, k, n, g, aligned=_aligned16(x, y), **blocks),
+        planner.select_plan(_capi.OP_GMM_TRANS, m, n, k, g, **blocks),
+        planner.select_plan(_capi.OP_GMM, m, k, n, g, **blocks)))
+
+
+def _gmm(x, A, group_sizes, block_m, block_k, block_n, trans_rhs, interpret, compute_dtype, acc_dtype, chunk_m,
+         plan: Optional[_capi.Plan] = None, group_offset=None) -> torch.Tensor:
+    """gpu_ragged_dot.py:171-228 (_gpu_gmm_fwd), as an autograd node where an operand asks for it.
 
     ``group_offset`` (jax.lax.ragged_dot's parameter; not in the reference): A holds the groups
     [group_offset, group_offset + A.shape[0]) of the ones group_sizes describes; rows of the others come out zero."""
-    if interpret:
-        raise NotImplementedError("interpret=True (Pallas interpreter) has no counterpart; kernels run on the GPU only")
+    code, gs, g_first = _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset)
     assert A.ndim == 3 and x.ndim == 2, f"but {A.ndim=} {x.ndim=}"  # :188
-    gs_host_shape = tuple(torch.as_tensor(group_sizes).shape)
-    g_first = _group_offset(group_offset)
-    if group_offset is None:
-        assert tuple(A.shape[:1]) == gs_host_shape, f"{A.shape[:1]=} != {gs_host_shape=}"  # :189
-    else:
-        assert len(gs_host_shape) == 1 and 0 <= g_first and g_first + A.shape[0] <= gs_host_shape[0], \
-            f"groups [{g_first}, {g_first}+{A.shape[0]}) are not within {gs_host_shape=}"
-    m, k = x.shape
-    g_local, g = A.shape[0], gs_host_shape[0]
-    n = A.shape[-1] if not trans_rhs else A.shape[-2]  # :190
-    k_rhs = A.shape[-2] if not trans_rhs else A.shape[-1]
-    assert k_rhs == k, f"contraction mismatch: x has k={k}, A has {k_rhs}"
-    assert chunk_m >= 1
-    planner.normalize_gmm_blocks(block_m, block_k, block_n, m, k, n)  # validates the request like :194-197
-    dev = _check_device(x, A)
-    code = _dtype_code(x, compute_dtype, acc_dtype)
-    if A.dtype != x.dtype:
-        raise TypeError(f"x is {x.dtype} but A is {A.dtype}")
-    x, A = x.contiguous(), A.contiguous()
-    gs = _group_sizes_i32(group_sizes, dev)
-    y = torch.empty((m, n), dtype=_out_dtype(x), device=dev)  # :210
-    if plan is None:
-        plan = planner.select_plan(_capi.OP_GMM_TRANS if trans_rhs else _capi.OP_GMM, m, k, n, g, block_m, block_k, block_n,
-                                   dtype=code, aligned=_aligned16(x, A, y))
-    if (g_first, g_local) != (0, g) and plan.decode_nb:
-        plan = _capi.Plan(plan.variant, plan.group_m, 0, plan.group_n, plan.split_k)  # streaming kernels: all groups only
-    ws_bytes = _capi.lib.rd_gmm_workspace_bytes(m, g, _plan_ref(plan))
-    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
-        _capi.check(
-            _capi.lib.rd_gmm_sharded(_stream_ptr(dev), x.data_ptr(), A.data_ptr(), gs.data_ptr(), y.data_ptr(), m, k, n,
-                                     g, g_first, g_local, int(bool(trans_rhs)), code, _plan_ref(plan), ws.data_ptr(),
-                                     ws.numel())
-        )
-    return y
+    assert chunk_m >= 1 and (group_offset is None or g_first >= 0)
+    plans = None
+    if plan is not None:
+        plans = (_fields(plan),)
+    elif not _default_blocks(block_m, block_k, block_n):
+        plans = _gmm_plans(x, A, trans_rhs, gs.numel(), code, block_m, block_k, block_n)
+    return _native.gmm(x, A, gs, bool(trans_rhs), code, g_first, plans)
 
 
-def _tgmm_fwd(x, y, group_sizes, block_m, block_k, block_n, interpret, compute_dtype, acc_dtype, chunk_m,
-              plan: Optional[_capi.Plan] = None, group_offset=None, num_actual_groups=None) -> torch.Tensor:
+def _tgmm(x, y, group_sizes, block_m, block_k, block_n, interpret, compute_dtype, acc_dtype, chunk_m,
+          plan: Optional[_capi.Plan] = None, group_offset=None, num_actual_groups=None) -> torch.Tensor:
     """gpu_ragged_dot.py:287-342 (_gpu_tgmm_fwd).  With ``group_offset`` / ``num_actual_groups`` only the slices of the
     groups [group_offset, group_offset + num_actual_groups) are computed: out[i] belongs to group group_offset + i."""
     del chunk_m  # :303
-    if interpret:
-        raise NotImplementedError("interpret=True (Pallas interpreter) has no counterpart; kernels run on the GPU only")
+    code, gs, g_first = _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset)
     assert y.ndim == 2 and x.ndim == 2 and x.shape[0] == y.shape[0]  # :304
-    (m, k), n = x.shape, y.shape[-1]
-    gs_t = torch.as_tensor(group_sizes)
-    g = gs_t.numel()
-    planner.normalize_tgmm_blocks(block_m, block_k, block_n, m, k, n)  # :308-314
-    dev = _check_device(x, y)
-    code = _dtype_code(x, compute_dtype, acc_dtype)
-    if y.dtype != x.dtype:
-        raise TypeError(f"x is {x.dtype} but y is {y.dtype}")
-    x, y = x.contiguous(), y.contiguous()
-    gs = _group_sizes_i32(gs_t, dev)
-    g_first = _group_offset(group_offset)
-    g_local = g - g_first if num_actual_groups is None else int(num_actual_groups)
-    assert 0 <= g_first and g_local >= 1 and g_first + g_local <= g, f"groups [{g_first}, {g_first}+{g_local}) are not within {g}"
-    out = torch.empty((g_local, k, n), dtype=_out_dtype(x), device=dev)  # :324
-    if plan is None:
-        plan = planner.select_plan(_capi.OP_TGMM, m, k, n, g, block_m, block_k, block_n, dtype=code,
-                                   aligned=_aligned16(x, y, out))
-    ws_bytes = _capi.lib.rd_tgmm_workspace_bytes(m, g, _plan_ref(plan))
-    ws = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
-        _capi.check(
-            _capi.lib.rd_tgmm_sharded(_stream_ptr(dev), x.data_ptr(), y.data_ptr(), gs.data_ptr(), out.data_ptr(), m, k, n,
-                                      g, g_first, g_local, code, _plan_ref(plan), ws.data_ptr(), ws.numel())
-        )
-    return out
+    assert group_offset is None or g_first >= 0
+    plans = None
+    if plan is not None:
+        plans = (_fields(plan),)
+    elif not _default_blocks(block_m, block_k, block_n):
+        plans = _tgmm_plans(x, y, gs.numel(), code, block_m, block_k, block_n)
+    g_local = -1
+    if num_actual_groups is not None:
+        g_local = int(num_actual_groups)
+        assert g_local >= 1
+    return _native.tgmm(x, y, gs, code, g_first, g_local, plans)
 
 
-class _GmmFn(torch.autograd.Function):
-    """The custom VJP of gpu_ragged_dot.py:360-405, as a torch autograd node."""
-
-    @staticmethod
-    def forward(ctx, x, A, group_sizes, hp):
-        ctx.hp = hp
-        ctx.save_for_backward(x, A, group_sizes)  # residuals (x, A, group_sizes), :227
-        return _gmm_fwd(x, A, group_sizes, **hp)
-
-    @staticmethod
-    def backward(ctx, do):
-        x, A, group_sizes = ctx.saved_tensors
-        hp = dict(ctx.hp)
-        trans_rhs = hp.pop("trans_rhs")
-        hp.pop("plan", None)
-        do = do.contiguous()
-        dx = dA = None
-        if ctx.needs_input_grad[0]:
-            dx = _gmm_fwd(do, A, group_sizes, **hp, trans_rhs=not trans_rhs)  # :400 (rows of groups outside A's slice: zero)
-        if ctx.needs_input_grad[1]:
-            thp = {k_: v for k_, v in hp.items()}
-            thp["num_actual_groups"] = A.shape[0]
-            dA = _tgmm_fwd(x, do, group_sizes, **thp) if not trans_rhs else _tgmm_fwd(do, x, group_sizes, **thp)  # :401
-        return dx, dA, None, None  # group_sizes gets no cotangent, :402
+def _gmm_fwd(*args, **kw) -> torch.Tensor:
+    """The product alone."""
+    with torch.no_grad():
+        return _gmm(*args, **kw)
 
 
-class _TgmmFn(torch.autograd.Function):
-    """tgmm with the VJP gpu_ragged_dot.py:431-450 intends: dx = gmm(y, do, trans_rhs=True), dy = gmm(x, do)."""
-
-    @staticmethod
-    def forward(ctx, x, y, group_sizes, hp):
-        ctx.hp = hp
-        ctx.save_for_backward(x, y, group_sizes)
-        return _tgmm_fwd(x, y, group_sizes, **hp)
-
-    @staticmethod
-    def backward(ctx, do):
-        x, y, group_sizes = ctx.saved_tensors
-        hp = dict(ctx.hp)
-        hp.pop("plan", None)
-        hp.pop("num_actual_groups", None)  # do has that many slices; group_offset says which groups they are
-        do = do.contiguous()
-        dx = dy = None
-        if ctx.needs_input_grad[0]:
-            dx = _gmm_fwd(y, do, group_sizes, **hp, trans_rhs=True)
-        if ctx.needs_input_grad[1]:
-            dy = _gmm_fwd(x, do, group_sizes, **hp, trans_rhs=False)
-        return dx, dy, None, None
+def _tgmm_fwd(*args, **kw) -> torch.Tensor:
+    with torch.no_grad():
+        return _tgmm(*args, **kw)
 
 
 def gmm(
@@ -249,16 +195,10 @@ def gmm(
     of those in group_sizes - an expert-parallel rank's slice; rows of the other groups are zero.
     """
     del num_warps, num_stages
-    hp = dict(block_m=block_m, block_k=block_k, block_n=block_n, trans_rhs=trans_rhs, interpret=interpret,
-              compute_dtype=compute_dtype, acc_dtype=acc_dtype, chunk_m=chunk_m)
-    if group_offset is not None:
-        hp["group_offset"] = _group_offset(group_offset)
-    if torch.is_grad_enabled() and (x.requires_grad or A.requires_grad):
-        if x.dtype == torch.float8_e4m3fn:
-            raise NotImplementedError("float8 operands are forward only: their cotangents are bfloat16, differentiate a bfloat16 copy")
-        gs = _group_sizes_i32(group_sizes, x.device)
-        return _GmmFn.apply(x, A, gs, hp)
-    return _gmm_fwd(x, A, group_sizes, **hp)
+    if x.dtype == torch.float8_e4m3fn and torch.is_grad_enabled() and (x.requires_grad or A.requires_grad):
+        raise NotImplementedError("float8 operands are forward only: their cotangents are bfloat16, differentiate a bfloat16 copy")
+    return _gmm(x, A, group_sizes, block_m, block_k, block_n, trans_rhs, interpret, compute_dtype, acc_dtype, chunk_m,
+                group_offset=group_offset)
 
 
 def tgmm(
@@ -280,15 +220,8 @@ def tgmm(
     """Transposed ragged dot: (m, k) x (m, n) -> (g, k, n).  gpu_ragged_dot.py:411-428.  With ``group_offset`` /
     ``num_actual_groups`` only the slices of the groups [group_offset, group_offset + num_actual_groups) are computed."""
     del num_warps, num_stages
-    hp = dict(block_m=block_m, block_k=block_k, block_n=block_n, interpret=interpret, compute_dtype=compute_dtype,
-              acc_dtype=acc_dtype, chunk_m=chunk_m)
-    if group_offset is not None or num_actual_groups is not None:
-        hp["group_offset"] = _group_offset(group_offset)
-        hp["num_actual_groups"] = num_actual_groups
-    if torch.is_grad_enabled() and (x.requires_grad or y.requires_grad):
-        gs = _group_sizes_i32(group_sizes, x.device)
-        return _TgmmFn.apply(x, y, gs, hp)
-    return _tgmm_fwd(x, y, group_sizes, **hp)
+    return _tgmm(x, y, group_sizes, block_m, block_k, block_n, interpret, compute_dtype, acc_dtype, chunk_m,
+                 group_offset=group_offset, num_actual_groups=num_actual_groups)
 
 
 ragged_dot = gmm  # gpu_ragged_dot.py:406

@@ -76,6 +76,22 @@ def tuned_plans() -> dict:
     return _TUNED
 
 
+def _tuned_plan(entry: dict) -> _capi.Plan:
+    return _capi.Plan(variant_id(entry["variant"]), int(entry.get("group_m", 0)), int(entry.get("decode_nb", 0)),
+                      int(entry.get("group_n", 0)))
+
+
+def tuned_plan_fields() -> list:
+    """The tuned table as [((op, m, k, n, g), plan fields in the order of rd_plan), ...]."""
+    ops = {"gmm": _capi.OP_GMM, "gmm_t": _capi.OP_GMM_TRANS, "tgmm": _capi.OP_TGMM}
+    out = []
+    for key, entry in tuned_plans().items():
+        op, *sizes = key.split(":")
+        p = _tuned_plan(entry)
+        out.append(((ops[op], *(int(v[1:]) for v in sizes)), (p.variant, p.group_m, p.group_n, p.decode_nb, p.split_k)))
+    return out
+
+
 def plan_key(op: int, m: int, k: int, n: int, g: int) -> str:
     return f"{('gmm', 'gmm_t', 'tgmm')[op]}:m{m}:k{k}:n{n}:g{g}"
 
@@ -104,8 +120,7 @@ def select_plan(
     explicit = (block_m, block_k, block_n) != (DEFAULT_BLOCK_M, DEFAULT_BLOCK_K, DEFAULT_BLOCK_N)
     entry = tuned_plans().get(plan_key(op, m, k, n, g))
     if entry is not None and vec and not explicit:
-        return _capi.Plan(variant_id(entry["variant"]), int(entry.get("group_m", 0)), int(entry.get("decode_nb", 0)),
-                          int(entry.get("group_n", 0)))
+        return _tuned_plan(entry)
     plan = _capi.default_plan(op, m, k, n, g)
     if explicit and not plan.decode_nb:
         # explicit request: nearest compiled shape.  For tgmm the output tile is (block_k, block_n).
