@@ -9,6 +9,7 @@
 #include "rd_gemm_pp.h"
 #include "rd_gemm_rs.h"
 #include "rd_gemm_tile.h"
+#include "rd_lookup.h"
 #include "rd_sched.h"
 
 namespace rd {
@@ -23,7 +24,7 @@ struct GmmArgs {
   const int32_t* tile2group;     // [U]   scheduling map built with chunk = tile height
   const int32_t* tile2it;        // [U]
   const int32_t* tile2band;      // [U]   band of row tiles each row tile belongs to (see rd_sched.h)
-  const int32_t* total_tiles;    // [1]
+  const int32_t* total_tiles;    // [1]   null: no map was built, every work-group looks its tile up itself (rd_lookup.h)
   int m, k, n, g;  // g: all groups of group_sizes
   int g_first, g_local;  // A holds the g_local groups [g_first, g_first + g_local); rows of the others are zero
   int U;        // static bound on row tiles: ceil(m / BM) + g
@@ -47,7 +48,7 @@ struct TgmmArgs {
   const void* dy;
   void* dA;
   const int32_t* group_sizes;
-  const int32_t* group_offsets;
+  const int32_t* group_offsets;  // null: every work-group adds up the sizes before its group itself
   int m, k, n, g;  // g: groups of dA (the slices computed)
   int g_first;     // dA[i] belongs to group g_first + i of group_sizes / group_offsets
   int k_tiles, n_tiles;  // ceil(k / BM), ceil(n / BN)
@@ -179,7 +180,10 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   // what one XCD runs at a time, so the block's operand slabs are fetched into that XCD's L2 once - and the blocks are
   // dealt to the 8 XCDs (launch index mod 8) round-robin.  No block spans two groups' weights except where a band ends.
   // Everything read through the map is the same for the whole work-group: pin it to scalar registers.
-  const int total = imin(uniform(*p.total_tiles), p.U);
+  const bool mapped = p.total_tiles != nullptr;
+  GroupScan<C::BM> scan;
+  if (!mapped) scan.init(p.group_sizes, p.g);
+  const int total = imin(mapped ? uniform(*p.total_tiles) : scan.total_tiles, p.U);
   const int live = total * p.n_tiles;
   SplitPlan sp{live, 1, 0};
   if constexpr (C::SPLITK) sp = split_plan(live, p.k, sizeof(E) == 1 ? p.k >> 1 : p.k, p.split_slots, p.num_cus, p.max_parts);
@@ -234,9 +238,21 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
     sk.parts = sp.parts;
     sk.part = part;
   }
-  const int band = uniform(p.tile2band[t / p.n_tiles]);
-  const bool deferred = (band & kBandDeferred) != 0;  // a short last row tile the map has moved behind all other tiles
-  const int band_row0 = (band & ~kBandDeferred) >> kBandShift, band_rows = band & kBandMaxRows;
+  const int walk_row = t / p.n_tiles;
+  bool deferred = false;  // a short last row tile the map has moved behind all other tiles
+  int band_row0 = walk_row, band_rows = 1;
+  int gi = 0, first_row = 0, group_rows = 0, first_tile = 0;  // of the tile's group, where there is no map
+  if (mapped) {
+    const int band = uniform(p.tile2band[walk_row]);
+    deferred = (band & kBandDeferred) != 0;
+    band_row0 = (band & ~kBandDeferred) >> kBandShift;
+    band_rows = band & kBandMaxRows;
+  } else if (walk_row < total) {
+    scan.find(walk_row, &gi, &group_rows, &first_row, &first_tile);
+    int first;
+    band_of((group_rows + C::BM - 1) / C::BM, p.group_m, walk_row - first_tile, &first, &band_rows);
+    band_row0 = first_tile + first;
+  }
   const int w = t - band_row0 * p.n_tiles;
   const int nj = w / band_rows;
   const int mi = band_row0 + (w - nj * band_rows);
@@ -244,10 +260,15 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   const int cols = imin(C::BN, p.n - col0);
 
   if (mi < total) {
-    const int gi = uniform(p.tile2group[mi]);
-    const int it = uniform(p.tile2it[mi]);
-    const int row0 = uniform(p.group_offsets[gi]) + it * C::BM;
-    int rows = imin(C::BM, uniform(p.group_sizes[gi]) - it * C::BM);
+    int it = mi - first_tile;
+    if (mapped) {
+      gi = uniform(p.tile2group[mi]);
+      it = uniform(p.tile2it[mi]);
+      first_row = uniform(p.group_offsets[gi]);
+      group_rows = uniform(p.group_sizes[gi]);
+    }
+    const int row0 = first_row + it * C::BM;
+    int rows = imin(C::BM, group_rows - it * C::BM);
     rows = imin(rows, p.m - row0);  // group_sizes summing past m: never touch rows >= m
     if (rows <= 0 || row0 < 0) return;
     O* Op = py + (size_t)row0 * p.n + col0;
@@ -294,7 +315,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   } else {
     // Rows past sum(group_sizes) are defined to be zero.  The map never uses more than
     // U - ceil(tail / BM) entries, so the unused tile slots cover the tail.
-    long long s = (long long)uniform(p.group_offsets[p.g - 1]) + uniform(p.group_sizes[p.g - 1]);
+    long long s = mapped ? (long long)uniform(p.group_offsets[p.g - 1]) + uniform(p.group_sizes[p.g - 1]) : scan.total_rows;
     if (s < 0) s = 0;
     const long long r0 = s + (long long)(mi - total) * C::BM;
     if (r0 >= p.m) return;
@@ -324,7 +345,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p
     const int32_t* rec = p.group_order + 4 * (size_t)slot;
     gi = uniform(rec[0]); row0 = uniform(rec[1]); rows = uniform(rec[2]);
   } else {
-    row0 = uniform(p.group_offsets[slot + p.g_first]);
+    row0 = p.group_offsets ? uniform(p.group_offsets[slot + p.g_first]) : rows_before_group(p.group_sizes, slot + p.g_first);
     rows = uniform(p.group_sizes[slot + p.g_first]);
   }
   const int t = ((xcd + slot) & 7) * quota + (pos - slot * quota);

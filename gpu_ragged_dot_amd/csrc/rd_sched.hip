@@ -2,6 +2,7 @@
 // kernel.  Produces exactly the five arrays of the reference's GMMGroupLookupMetadata
 // (gpu_ragged_dot.py:60-90) in int32, every output element written once.
 #include "rd_common.h"
+#include "rd_lookup.h"
 #include "rd_sched.h"
 
 namespace rd {
@@ -126,14 +127,8 @@ __global__ __launch_bounds__(kSchedThreads) void sched_map_kernel(const int32_t*
       tile2group[t] = base + l;
       tile2it[t] = t - start;
       if (tile2band) {
-        // The group's R row tiles are cut into ceil(R / band_rows) bands of nearly equal height (the first R % bands of
-        // them one taller), so that no band spans two groups; the entry says where this tile's band starts and how tall
-        // it is.
-        const int32_t R = incl[l] - start, it = t - start;
-        const int32_t nb = (R + band_rows - 1) / band_rows, r = R / nb, rem = R - r * nb;
         int32_t row0, rb;
-        if (it < rem * (r + 1)) { rb = r + 1; row0 = (it / rb) * rb; }
-        else { rb = r; row0 = rem * (r + 1) + ((it - rem * (r + 1)) / rb) * rb; }
+        band_of(incl[l] - start, band_rows, t - start, &row0, &rb);  // no band spans two groups
         tile2band[t] = ((start + row0) << kBandShift) | rb;
       }
     }
