@@ -115,6 +115,106 @@ __global__ __launch_bounds__(64) void moe_rank_kernel(const int32_t* __restrict_
   }
 }
 
+// Routing in one or two launches, for up to kRouteBlocks x 1024 slots.  What bounds it is not the 128-256 KB it moves but the
+// chain of launches and round trips: three kernels took 12.4 us for 2048 slots and 16.9 us for 32768 of 128 experts, this 4.1
+// and 7.9.  Here a work-group
+// of 16 waves ranks 1024 slots, one per thread, in a single pass (one ballot per id bit finds a lane's equals), and gets
+// the counts of the slots before and behind its own either from a histogram kernel's [blocks][g] table (BLOCK_HIST) or, for
+// few slots, by counting them all itself (a launch less).
+constexpr int kRouteSlots = 1024;   // per work-group
+constexpr int kRouteBlocks = 64;    // beyond that the per-expert sums over the blocks are a kernel of their own again
+constexpr int kRouteAlone = 16;     // up to that many blocks every work-group counts all slots
+constexpr int kRouteGroups = 512;   // LDS: 16 waves' counts, and two tables of counts
+
+__global__ __launch_bounds__(kRouteSlots) void moe_block_hist_kernel(const int32_t* __restrict__ ids, int S, int g,
+                                                                      int32_t* __restrict__ hist) {
+  __shared__ int32_t cnt[kRouteGroups];
+  for (int e = threadIdx.x; e < g; e += kRouteSlots) cnt[e] = 0;
+  __syncthreads();
+  const int s = blockIdx.x * kRouteSlots + threadIdx.x;
+  const int e = s < S ? ids[s] : -1;
+  if (e >= 0 && e < g) atomicAdd(&cnt[e], 1);
+  __syncthreads();
+  for (int i = threadIdx.x; i < g; i += kRouteSlots) hist[(size_t)blockIdx.x * g + i] = cnt[i];
+}
+
+template <bool BLOCK_HIST>
+__global__ __launch_bounds__(kRouteSlots) void moe_route_kernel(const int32_t* __restrict__ ids, int S, int g, int id_bits,
+                                                                const int32_t* __restrict__ hist,
+                                                                int32_t* __restrict__ group_sizes,
+                                                                int32_t* __restrict__ row_of_slot,
+                                                                int32_t* __restrict__ slot_of_row) {
+  constexpr int W = kRouteSlots / 64;
+  __shared__ int32_t own[W][kRouteGroups];    // slots of this block per wave and expert; then their first rows
+  __shared__ int32_t before[kRouteGroups], behind[kRouteGroups];  // slots of the other blocks
+  __shared__ int32_t wave_sum[W];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b = blockIdx.x;
+  for (int i = tid; i < W * g; i += kRouteSlots) own[i / g][i % g] = 0;
+  for (int i = tid; i < g; i += kRouteSlots) { before[i] = 0; behind[i] = 0; }
+  __syncthreads();
+
+  // this wave's 64 slots: a lane's equals, its place among them, and - by the first of them - their number
+  const int s = b * kRouteSlots + tid;
+  const int e = s < S ? ids[s] : -1;
+  const bool keep = e >= 0 && e < g;
+  unsigned long long same = __ballot(keep);
+  for (int bit = 0; bit < id_bits; ++bit) {
+    const bool one = (e >> bit) & 1;
+    const unsigned long long ones = __ballot(keep && one);
+    same &= one ? ones : ~ones;
+  }
+  const int place = __popcll(same & ((1ull << lane) - 1ull));
+  if (keep && place == 0) own[wave][e] = __popcll(same);
+  if constexpr (!BLOCK_HIST) {
+    for (int o = tid; o < S; o += kRouteSlots) {
+      if ((o - tid) == b * kRouteSlots) continue;  // (blocks are whole strides)
+      const int oe = ids[o];
+      if (oe >= 0 && oe < g) atomicAdd(o < b * kRouteSlots ? &before[oe] : &behind[oe], 1);
+    }
+  }
+  __syncthreads();
+
+  // per expert (one thread each): its rows, and where this block's waves' rows start among them
+  int total = 0, at = 0;
+  if (tid < g) {
+    if constexpr (BLOCK_HIST) {
+      const int nb = gridDim.x;
+      for (int b0 = 0; b0 < nb; b0 += 8) {
+        int32_t c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = b0 + u < nb ? hist[(size_t)(b0 + u) * g + tid] : 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { total += c[u]; at += b0 + u < b ? c[u] : 0; }
+      }
+      for (int w = 0; w < W; ++w) { const int c = own[w][tid]; own[w][tid] = at; at += c; }
+    } else {
+      at = before[tid];
+      for (int w = 0; w < W; ++w) { const int c = own[w][tid]; own[w][tid] = at; at += c; }
+      total = at + behind[tid];
+    }
+    if (b == 0) group_sizes[tid] = total;
+  }
+  int incl = total;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();
+  int rows_before = 0, rows_all = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) { rows_before += w < wave ? wave_sum[w] : 0; rows_all += wave_sum[w]; }
+  if (tid < g) before[tid] = rows_before + incl - total;  // the expert's first row
+  __syncthreads();
+
+  const int row = keep ? before[e] + own[wave][e] + place : -1;
+  if (s < S) row_of_slot[s] = row;
+  if (keep) slot_of_row[row] = s;
+  // rows past the last kept slot; every block takes its share
+  for (int r = rows_all + b * kRouteSlots + tid; r < S; r += gridDim.x * kRouteSlots) slot_of_row[r] = -1;
+}
+
 // ---- rows ------------------------------------------------------------------------------------------------------------
 
 template <class T> __device__ __forceinline__ float to_f32(T v);
@@ -127,6 +227,16 @@ template <> __device__ __forceinline__ float from_f32<float>(float v) { return v
 template <> __device__ __forceinline__ f16_t from_f32<f16_t>(float v) { return (f16_t)v; }
 
 constexpr int kRowThreads = 256;
+
+// A piece of a row that the launch reads once.  STREAM: past the caches - for matrices larger than the 256 MB last-level
+// cache, which cannot be in it (4096 tokens x 8 rows of 7168 bf16, 470 MB, combine: 112 -> 98 us).  Smaller ones have
+// just been written and are left where they are (8192 x 2 rows of 4096, 134 MB: 30 us so, 37 us streamed).
+constexpr long long kStreamBytes = 256ll << 20;
+template <bool STREAM>
+__device__ __forceinline__ u32x4_t load_row_piece(const u32x4_t* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  else return *p;
+}
 
 // x[row_of_slot[t, s]] = h[t] * scale[t, s] for every kept slot of token t: the token's row is read once and written
 // top_k times.  The rows past sum(group_sizes) (slot_of_row = -1) are zeroed by the work-group that owns their index
@@ -193,7 +303,7 @@ __global__ __launch_bounds__(kRowThreads) void moe_dispatch_kernel(const T* __re
 }
 
 // out[t] = sum_s weights[t, s] * y[row_of_slot[t, s]], fp32, slots in order.
-template <class T, bool VEC>
+template <class T, bool VEC, bool STREAM>
 __global__ __launch_bounds__(kRowThreads) void moe_combine_kernel(const T* __restrict__ y,
                                                                   const int32_t* __restrict__ row_of_slot,
                                                                   const float* __restrict__ weights, T* __restrict__ out,
@@ -216,7 +326,7 @@ __global__ __launch_bounds__(kRowThreads) void moe_combine_kernel(const T* __res
       for (int s = 0; s < top_k; ++s) {
         if (rows[s] < 0) continue;
         alignas(16) T v[PER];
-        *reinterpret_cast<u32x4_t*>(v) = reinterpret_cast<const u32x4_t*>(y + (size_t)rows[s] * d)[c];
+        *reinterpret_cast<u32x4_t*>(v) = load_row_piece<STREAM>(reinterpret_cast<const u32x4_t*>(y + (size_t)rows[s] * d) + c);
 #pragma unroll
         for (int e = 0; e < PER; ++e) acc[e] = __builtin_fmaf(ws[s], to_f32<T>(v[e]), acc[e]);
       }
@@ -235,28 +345,57 @@ __global__ __launch_bounds__(kRowThreads) void moe_combine_kernel(const T* __res
   }
 }
 
-// dw[t, s] = <y[row_of_slot[t, s]], dout[t]>, fp32.
-template <class T>
+// dw[t, s] = <y[row_of_slot[t, s]], dout[t]>, fp32.  A wave takes slots wave, wave + 4, ... of the token, four at a time: a
+// 16-byte piece of dout is multiplied with the same piece of four rows, so that four row loads are in flight per piece and
+// dout comes from L1.  (One slot at a time with the whole work-group, by element, with two barriers each: 51 us on 4096
+// tokens x 8 rows of 2048 bf16, 3.0 TB/s, and 236 us on rows of 7168; so 25 and 79 us, 6.0 and 6.7 TB/s.)
+constexpr int kWgradSlots = 4;
+template <class T, bool VEC, bool STREAM>
 __global__ __launch_bounds__(kRowThreads) void moe_combine_wgrad_kernel(const T* __restrict__ y,
                                                                         const T* __restrict__ dout,
                                                                         const int32_t* __restrict__ row_of_slot,
                                                                         float* __restrict__ dw, int top_k, int d) {
-  __shared__ float part[kRowThreads / 64];
-  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int W = kRowThreads / 64, PER = VEC ? 16 / sizeof(T) : 1;
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const T* g = dout + (size_t)t * d;
-  for (int s = 0; s < top_k; ++s) {
-    const int row = __builtin_amdgcn_readfirstlane(row_of_slot[(size_t)t * top_k + s]);
-    float acc = 0.f;
-    if (row >= 0) {
-      const T* yr = y + (size_t)row * d;
-      for (int c = tid; c < d; c += kRowThreads) acc = __builtin_fmaf(to_f32<T>(yr[c]), to_f32<T>(g[c]), acc);
+  for (int s0 = wave; s0 < top_k; s0 += W * kWgradSlots) {
+    const T* rows[kWgradSlots];
+    bool live[kWgradSlots];
+    float acc[kWgradSlots];
+#pragma unroll
+    for (int i = 0; i < kWgradSlots; ++i) {
+      const int s = s0 + i * W;
+      const int row = __builtin_amdgcn_readfirstlane(s < top_k ? row_of_slot[(size_t)t * top_k + s] : -1);
+      live[i] = row >= 0;
+      rows[i] = y + (size_t)imax(row, 0) * d;
+      acc[i] = 0.f;
+    }
+    for (int c = lane; c < d / PER; c += 64) {
+      alignas(16) T gv[PER], yv[kWgradSlots][PER];
+      if constexpr (VEC) {
+        *reinterpret_cast<u32x4_t*>(gv) = reinterpret_cast<const u32x4_t*>(g)[c];
+#pragma unroll
+        for (int i = 0; i < kWgradSlots; ++i)
+          if (live[i]) *reinterpret_cast<u32x4_t*>(yv[i]) = load_row_piece<STREAM>(reinterpret_cast<const u32x4_t*>(rows[i]) + c);
+      } else {
+        gv[0] = g[c];
+#pragma unroll
+        for (int i = 0; i < kWgradSlots; ++i)
+          if (live[i]) yv[i][0] = rows[i][c];
+      }
+#pragma unroll
+      for (int i = 0; i < kWgradSlots; ++i)
+        if (live[i])
+#pragma unroll
+          for (int e = 0; e < PER; ++e) acc[i] = __builtin_fmaf(to_f32<T>(yv[i][e]), to_f32<T>(gv[e]), acc[i]);
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    __syncthreads();  // previous slot's partials consumed
-    if (lane == 0) part[wave] = acc;
-    __syncthreads();
-    if (tid == 0) dw[(size_t)t * top_k + s] = part[0] + part[1] + part[2] + part[3];
+    for (int i = 0; i < kWgradSlots; ++i) {
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) acc[i] += __shfl_xor(acc[i], o, 64);
+      const int s = s0 + i * W;
+      if (lane == 0 && s < top_k) dw[(size_t)t * top_k + s] = live[i] ? acc[i] : 0.f;
+    }
   }
 }
 
@@ -280,12 +419,24 @@ size_t moe_route_workspace_bytes(long long slots, int g) {
 
 int launch_moe_route(hipStream_t s, const int32_t* ids, int slots, int g, int32_t* group_sizes, int32_t* row_of_slot,
                      int32_t* slot_of_row, int32_t* workspace) {
+  int id_bits = 0;
+  while ((1 << id_bits) < g) ++id_bits;
+  const int blocks = (slots + kRouteSlots - 1) / kRouteSlots;
+  if (blocks >= 1 && blocks <= kRouteBlocks && g <= kRouteGroups) {
+    if (blocks <= kRouteAlone) {
+      hipLaunchKernelGGL(moe_route_kernel<false>, dim3(blocks), dim3(kRouteSlots), 0, s, ids, slots, g, id_bits, nullptr,
+                         group_sizes, row_of_slot, slot_of_row);
+    } else {
+      hipLaunchKernelGGL(moe_block_hist_kernel, dim3(blocks), dim3(kRouteSlots), 0, s, ids, slots, g, workspace);
+      hipLaunchKernelGGL(moe_route_kernel<true>, dim3(blocks), dim3(kRouteSlots), 0, s, ids, slots, g, id_bits, workspace,
+                         group_sizes, row_of_slot, slot_of_row);
+    }
+    return (int)hipGetLastError();
+  }
   const int chunk = route_chunk(slots, g);
   const int nb = (slots + chunk - 1) / chunk;
   int32_t* hist = workspace;
   int32_t* group_first = workspace + (size_t)nb * g;
-  int id_bits = 0;
-  while ((1 << id_bits) < g) ++id_bits;
   const size_t lds = (size_t)g * sizeof(int32_t);
   if (nb > 0) hipLaunchKernelGGL(moe_hist_kernel, dim3(nb), dim3(64), lds, s, ids, slots, g, chunk, hist);
   hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, hist, nb, g, slots, group_sizes, group_first,
@@ -317,8 +468,10 @@ template <class T>
 static int combine_t(hipStream_t s, const void* y, const int32_t* row_of_slot, const float* weights, void* out,
                      int tokens, int top_k, int d) {
   const bool vec = (d * sizeof(T)) % 16 == 0 && aligned16(y) && aligned16(out);
-  if (vec) hipLaunchKernelGGL((moe_combine_kernel<T, true>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, row_of_slot, weights, (T*)out, top_k, d);
-  else hipLaunchKernelGGL((moe_combine_kernel<T, false>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, row_of_slot, weights, (T*)out, top_k, d);
+  const bool stream = (long long)tokens * top_k * d * (long long)sizeof(T) > kStreamBytes;
+  if (vec && stream) hipLaunchKernelGGL((moe_combine_kernel<T, true, true>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, row_of_slot, weights, (T*)out, top_k, d);
+  else if (vec) hipLaunchKernelGGL((moe_combine_kernel<T, true, false>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, row_of_slot, weights, (T*)out, top_k, d);
+  else hipLaunchKernelGGL((moe_combine_kernel<T, false, false>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, row_of_slot, weights, (T*)out, top_k, d);
   return (int)hipGetLastError();
 }
 
@@ -330,13 +483,23 @@ int launch_moe_combine(hipStream_t s, const void* y, const int32_t* row_of_slot,
                    : combine_t<bf16_bits>(s, y, row_of_slot, weights, out, tokens, top_k, d);
 }
 
+template <class T>
+static int wgrad_t(hipStream_t s, const void* y, const void* dout, const int32_t* row_of_slot, float* dw, int tokens, int top_k,
+                   int d) {
+  const bool vec = (d * sizeof(T)) % 16 == 0 && aligned16(y) && aligned16(dout);
+  const bool stream = (long long)tokens * top_k * d * (long long)sizeof(T) > kStreamBytes;
+  if (vec && stream) hipLaunchKernelGGL((moe_combine_wgrad_kernel<T, true, true>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, (const T*)dout, row_of_slot, dw, top_k, d);
+  else if (vec) hipLaunchKernelGGL((moe_combine_wgrad_kernel<T, true, false>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, (const T*)dout, row_of_slot, dw, top_k, d);
+  else hipLaunchKernelGGL((moe_combine_wgrad_kernel<T, false, false>), dim3(tokens), dim3(kRowThreads), 0, s, (const T*)y, (const T*)dout, row_of_slot, dw, top_k, d);
+  return (int)hipGetLastError();
+}
+
 int launch_moe_combine_wgrad(hipStream_t s, const void* y, const void* dout, const int32_t* row_of_slot, float* dw,
                              int tokens, int top_k, int d, int elem) {
   if (tokens <= 0 || top_k <= 0) return hipSuccess;
-  if (elem == 2) hipLaunchKernelGGL(moe_combine_wgrad_kernel<f16_t>, dim3(tokens), dim3(kRowThreads), 0, s, (const f16_t*)y, (const f16_t*)dout, row_of_slot, dw, top_k, d);
-  else if (elem == 1) hipLaunchKernelGGL(moe_combine_wgrad_kernel<float>, dim3(tokens), dim3(kRowThreads), 0, s, (const float*)y, (const float*)dout, row_of_slot, dw, top_k, d);
-  else hipLaunchKernelGGL(moe_combine_wgrad_kernel<bf16_bits>, dim3(tokens), dim3(kRowThreads), 0, s, (const bf16_bits*)y, (const bf16_bits*)dout, row_of_slot, dw, top_k, d);
-  return (int)hipGetLastError();
+  return elem == 1 ? wgrad_t<float>(s, y, dout, row_of_slot, dw, tokens, top_k, d)
+       : elem == 2 ? wgrad_t<f16_t>(s, y, dout, row_of_slot, dw, tokens, top_k, d)
+                   : wgrad_t<bf16_bits>(s, y, dout, row_of_slot, dw, tokens, top_k, d);
 }
 
 }  // namespace rd
