@@ -1,6 +1,7 @@
 // fp32 operands: one BM x BN tile of C = sum_kk Aop(i,kk)*Bop(j,kk) on v_mfma_f32_32x32x2_f32 (fp32 in, fp32 accumulate),
 // so that float32 inputs - which the reference accepts - give float32-accurate results.
 //
+// Used where the any-pitch core (rd_gemm_rs.h) is not: rows of fewer than 8 elements, and tgmm over groups of few rows.
 // Any shape is taken.  Four waves in a 2 x 2 grid, each holding (BM/2) x (BN/2) of the tile in 32 x 32 blocks; the
 // contraction runs in slabs of 16 through two LDS buffers: the loads of slab s+1 are issued into registers before the
 // MFMAs of slab s and written to the other buffer after them, one barrier per slab.  LDS holds a slab as [kk][row]

@@ -1,7 +1,8 @@
 // Four-wave GEMM core for operands that cannot be loaded straight into LDS: row pitches that are no multiple of 16 bytes
-// (bf16 and float16), and float32 arrays that are rounded to bf16 on the way (compute_dtype = bfloat16).  A 256 x 256 tile
-// held by a 2 x 2 grid of waves, 128 x 128 per wave, as in rd_gemm_w4.h; HBM -> registers -> LDS as in rd_gemm_w4r.h,
-// for any of the four operand layouts.
+// (bf16 and float16), float32 arrays that are rounded to bf16 on the way (compute_dtype = bfloat16), and float32 arrays of
+// any pitch multiplied as they are.  A 256 x 256 tile held by a 2 x 2 grid of waves, 128 x 128 per wave, as in
+// rd_gemm_w4.h (or a smaller tile, several work-groups to a compute unit); HBM -> registers -> LDS as in rd_gemm_w4r.h, for
+// any of the four operand layouts.
 //
 // What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
 // element per instruction where the pitch is odd, one slab in flight where the source is float32 - at 40-85 and 300-430
@@ -15,6 +16,9 @@
 //    operands, and two slabs are in flight in registers beside the two in LDS (bf16: 2 x 64 KB, float32 rounded: 2 x 32 KB);
 //  * the pieces are converted and written to LDS, and their registers refilled, spread evenly over the gaps between the
 //    matrix-core instructions of a slab.
+// float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most: the plain tile of
+// rd_gemm_f32.h, one slab of 16 ahead with element-wise LDS traffic, kept it busy 72-78 % of the time (4096 x 4096 x 3072:
+// 946 / 870 / 883 us), this core 86-92 % (766 / 733 / 713 us).
 // No predicate sits in the steady loop: a slab that holds the last contraction index, or lies behind it, is loaded by
 // fetch_tail(), which never touches memory outside the operand's rows and fills with zeros.
 #pragma once
@@ -23,9 +27,10 @@
 
 namespace rd {
 
-// Src: bf16_bits, f16_t, or float (rounded to bf16; float32 out).  VEC: k and n are multiples of 8, so that no piece crosses
-// the end of a row and the last slab needs no shifting.
-template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, typename Src, bool VEC_>
+// Src: bf16_bits, f16_t, or float (float32 out).  FULL: float32 stays float32 on its way through LDS and is multiplied by
+// v_mfma_f32_32x32x2_f32; otherwise it is rounded to bf16.  VEC: k and n are multiples of 8 (FULL: of 4), so that no piece
+// crosses the end of a row and the last slab needs no shifting.
+template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, typename Src, bool VEC_, bool FULL_ = false>
 struct RsCfg {
   typedef Src Elem;
   static constexpr bool F32 = false, RS = true, HALF = std::is_same<Src, f16_t>::value;
@@ -35,15 +40,19 @@ struct RsCfg {
   static constexpr int NW = 4, NT = 256;
   static constexpr int WM = BM / 2, WN = BN / 2;
   static constexpr int TM = WM / 32, TN = WN / 32;
-  static constexpr int KSTEPS = BK / 16;
-  static constexpr int WAVES_PER_EU = BM * BN > 128 * 128 ? 1 : 2;  // work-groups per compute unit
-  static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2;  // one slab in LDS, 16 bits per element
+  static constexpr bool FULL = FULL_;
+  static constexpr int LB = FULL ? 4 : 2;                  // bytes of an element in LDS
+  static constexpr int KMF = FULL ? 4 : 1;                 // matrix-core instructions per block and substep
+  static constexpr int KSTEPS = FULL ? BK / 8 : BK / 16;   // substeps per slab
+  static constexpr int WAVES_PER_EU = BM * BN > 128 * 128 ? 1 : BM * BN < 128 * 128 ? 3 : 2;  // work-groups per compute unit
+  static constexpr int A_BYTES = BM * BK * LB, B_BYTES = BN * BK * LB;  // one slab in LDS
   static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;
   static constexpr int EPI_PITCH = WN * 2 + 16;
   static constexpr int EPI_BYTES = sizeof(Src) == 2 ? NW * WM * EPI_PITCH : 0;
   static constexpr int RING_BYTES = 2 * SLOT_BYTES;
   static constexpr int LDS_BYTES = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
-  static_assert(BM % 128 == 0 && BN % 128 == 0, "tile shape");
+  static_assert(FULL ? BM % 64 == 0 && BN % 64 == 0 : BM % 128 == 0 && BN % 128 == 0, "tile shape");
+  static_assert(!FULL || std::is_same<Src, float>::value, "float32 only");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
@@ -65,17 +74,17 @@ __device__ __forceinline__ u32x4_t shift_down(u32x4_t v, int bytes) {
 
 // One operand's slab, [T rows][BK] (K-major) or [BK][T columns] (MN-major), in pieces of 16 bytes: which memory each lane
 // reads for each of its pieces, and where the piece goes in LDS (the layout DldsFragReader reads).
-template <int T, int BK, int NW, bool KMAJOR, typename Src, bool VEC>
+template <int T, int BK, int NW, bool KMAJOR, typename Src, bool VEC, int LB = 2>
 struct RsLoader {
   static constexpr int EPP = 16 / (int)sizeof(Src);              // elements per piece
   static constexpr int PPR = (KMAJOR ? BK : T) / EPP;            // pieces per slab row
   static constexpr int RPI = 64 / PPR;                           // slab rows per wave-wide load
   static constexpr int PER = (KMAJOR ? T : BK) / RPI / NW;       // pieces per lane
-  static constexpr int LDS_ROW = (KMAJOR ? BK : T) * 2;          // bytes of a slab row in LDS
+  static constexpr int LDS_ROW = (KMAJOR ? BK : T) * LB;         // bytes of a slab row in LDS
   static constexpr int LDS_STEP = NW * RPI * LDS_ROW;            // from one of a lane's pieces to its next
   static_assert(PPR <= 64 && 64 % PPR == 0 && (KMAJOR ? T : BK) % (RPI * NW) == 0, "slab does not split evenly");
   // the chunk permutation of DldsFragReader repeats from one of a lane's pieces to the next
-  static_assert(KMAJOR ? (NW * RPI) % 16 == 0 : (NW * RPI) % 4 == 0, "chunk permutation");
+  static_assert(KMAJOR ? (NW * RPI) % 16 == 0 : (NW * RPI) % (LB == 4 ? 8 : 4) == 0, "chunk permutation");
 
   const Src* base;   // first element of the current slab
   long long step;    // elements from one slab to the next
@@ -96,9 +105,10 @@ struct RsLoader {
     off_last = KMAJOR ? ((uint32_t)(lim - 1) * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src) : ~0u;
     off0 = ((uint32_t)row0 * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src);
     row_step = (uint32_t)(NW * RPI * sizeof(Src)) * (uint32_t)ld;
-    const int chunk = sizeof(Src) == 2 ? piece : piece >> 1;  // 16-byte chunk of the LDS row; a float32 piece fills half of one
-    const int c = KMAJOR ? (BK == 64 ? chunk ^ ((row0 >> 1) & 7) : chunk ^ ((row0 >> 2) & 3)) : chunk ^ ((row0 & 3) << 2);
-    lds = row0 * LDS_ROW + (c << 4) + (sizeof(Src) == 2 ? 0 : (piece & 1) * 8);
+    const int chunk = sizeof(Src) == LB ? piece : piece >> 1;  // 16-byte chunk of the LDS row; a rounded float32 piece fills half of one
+    const int c = KMAJOR ? (LDS_ROW == 128 ? chunk ^ ((row0 >> 1) & 7) : chunk ^ ((row0 >> 2) & 3))
+                : LB == 4 ? chunk ^ (((row0 >> 2) & 1) << 3) : chunk ^ ((row0 & 3) << 2);
+    lds = row0 * LDS_ROW + (c << 4) + (sizeof(Src) == LB ? 0 : (piece & 1) * 8);
   }
 
   __host__ __device__ __forceinline__ uint32_t offset(int j) const {
@@ -138,7 +148,7 @@ struct RsLoader {
   }
   __device__ __forceinline__ void commit(unsigned char* region, int j, u32x4_t v) const {
     unsigned char* d = region + lds + j * LDS_STEP;
-    if constexpr (sizeof(Src) == 2) {
+    if constexpr (sizeof(Src) == LB) {
       *reinterpret_cast<u32x4_t*>(d) = v;
     } else {
       const f32x4_t f = __builtin_bit_cast(f32x4_t, v);
@@ -153,6 +163,42 @@ struct RsLoader {
                                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32));
     asm volatile("" : "+v"(off0));
   }
+};
+
+// Fragments of float32 slabs (FULL), 8 contraction indices at a time: lane l feeds row / column (l & 31) of a block with the
+// four indices 4 (l >> 5) .. + 3, one per matrix-core instruction - that instruction multiplies two indices, one per half
+// wave, and since both operands name the same two it does not matter that they are not neighbours.  K-major rows give the
+// four in one 16-byte read, MN-major slabs in four reads of 32 consecutive columns.
+template <int T, int TILES, bool KMAJOR>
+struct RsFullFrag {
+  int addr[KMAJOR ? 4 : 1];
+  __device__ __forceinline__ void init(int idx0, int lane) {
+    const int h = lane >> 5;
+    if (KMAJOR) {
+      const int r = lane & 31;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) addr[ks] = (idx0 + r) * 128 + (((2 * ks + h) ^ ((r >> 1) & 7)) << 4);
+    } else {
+      // rows 8 ks + 4 h + e have bit 2 equal to h: their 32-column halves of 64 are exchanged where it is set
+      addr[0] = 4 * h * T * 4 + (((idx0 + (lane & 31)) * 4) ^ (h << 7));
+    }
+  }
+  __device__ __forceinline__ f32x4_t read(const unsigned char* region, int tile, int ks) const {
+    if (KMAJOR) {
+      return *reinterpret_cast<const f32x4_t*>(region + addr[ks] + tile * 32 * 128);
+    } else {
+      // a block's 32 columns are one half of an aligned 64: the next block is the other half
+      const unsigned char* p = region + (addr[0] ^ ((tile & 1) << 7)) + (tile >> 1) * 256 + ks * 8 * T * 4;
+      f32x4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = *reinterpret_cast<const float*>(p + e * T * 4);
+      return v;
+    }
+  }
+};
+template <class C, int T, int TILES, bool KMAJOR>
+struct RsFrag {
+  typedef typename std::conditional<C::FULL, RsFullFrag<T, TILES, KMAJOR>, DldsFragReader<T, C::BK, TILES, KMAJOR>>::type type;
 };
 
 namespace rs_detail {
@@ -173,26 +219,29 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
                                          unsigned char* smem, int wave, int lane, f32x16_t (&acc)[C::TM][C::TN]) {
   typedef typename C::Elem E;
   const int wm = wave >> 1, wn = wave & 1;
-  typedef RsLoader<C::BM, C::BK, C::NW, C::A_KMAJOR, E, C::VEC> LdA;
-  typedef RsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR, E, C::VEC> LdB;
+  typedef RsLoader<C::BM, C::BK, C::NW, C::A_KMAJOR, E, C::VEC, C::LB> LdA;
+  typedef RsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR, E, C::VEC, C::LB> LdB;
   LdA la; LdB lb;
   la.init(Ap, lda, a_lim, klen, wave, lane);
   lb.init(Bp, ldb, b_lim, klen, wave, lane);
-  DldsFragReader<C::BM, C::BK, C::TM, C::A_KMAJOR> fra;
-  DldsFragReader<C::BN, C::BK, C::TN, C::B_KMAJOR> frb;
+  typename RsFrag<C, C::BM, C::TM, C::A_KMAJOR>::type fra;
+  typename RsFrag<C, C::BN, C::TN, C::B_KMAJOR>::type frb;
   fra.init(wm * C::WM, lane);
   frb.init(wn * C::WN, lane);
 
   const int nk = (klen + C::BK - 1) / C::BK;  // the last slab, nk - 1, holds the last contraction index
   constexpr int PA = LdA::PER, PB = LdB::PER, P = PA + PB;
-  constexpr int MF = C::TM * C::TN, R0 = C::TM + C::TN;
-  constexpr int HEAD = P / C::KSTEPS;       // pieces moved per substep
+  constexpr int MF = C::TM * C::TN * C::KMF, R0 = C::TM + C::TN;
+  // pieces moved per substep: the last one, which follows the slab's barrier, takes pieces 0 .. HEAD - 1 (of the slab after
+  // next), substep u of the others pieces part(u + 1) .. part(u + 2) - 1
+  constexpr auto part = [](int u) constexpr { return u * P / C::KSTEPS; };
+  constexpr int HEAD = part(1), MOST = (P + C::KSTEPS - 1) / C::KSTEPS;
   // What the gaps between a substep's matrix-core instructions carry.  Large patches: one fragment read each in the first
   // ones, then the pieces, spread out (a write and the load that refills its registers in one gap or in two).  Small
   // patches have fewer gaps than reads and pieces: every gap carries its share of both.
-  constexpr bool ROOMY = MF - R0 >= HEAD;
-  constexpr int GAP = MF - R0 >= 2 * HEAD ? 2 : 1;
-  static_assert(P % C::KSTEPS == 0 && (ROOMY || HEAD % MF == 0 || MF % HEAD == 0), "every substep has room for its pieces");
+  constexpr bool ROOMY = MF - R0 >= MOST;
+  constexpr int GAP = MF - R0 >= 2 * MOST ? 2 : 1;
+  static_assert(HEAD >= 1, "every substep moves a piece");
 
   u32x4_t regs[2][P];
   auto fetch_one = [&](auto set_tag, int step, int q, auto mode_tag) {
@@ -233,7 +282,8 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
     __builtin_amdgcn_s_barrier();
   };
 
-  bf16x8_t fa[2][C::TM], fb[2][C::TN];
+  typedef typename std::conditional<C::FULL, f32x4_t, bf16x8_t>::type frag_t;
+  frag_t fa[2][C::TM], fb[2][C::TN];
   auto first_fragments = [&]() {
     if (LIVE) {
 #pragma unroll
@@ -260,9 +310,10 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
       const unsigned char* ra = smem + (last ? next_off : cur_off);  // fragments of the next substep
       const unsigned char* rb = ra + C::A_BYTES;
       const int us = last ? 0 : u + 1;
+      const int first = last ? 0 : part(u + 1), count = last ? HEAD : part(u + 2) - part(u + 1);
 #pragma unroll
       for (int m = 0; m < MF; ++m) {
-        const int i = m / C::TN, j = m % C::TN;
+        const int i = m % (C::TM * C::TN) / C::TN, j = m % C::TN, ke = m / (C::TM * C::TN);
         if (LIVE && ROOMY) {
           if (m < C::TM) fa[(u + 1) & 1][m] = fra.read(ra, m, us);
           else if (m < R0) fb[(u + 1) & 1][m - C::TM] = frb.read(rb, m - C::TM, us);
@@ -275,26 +326,27 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
         }
         auto write = [&](int p) {
           if (last) commit_one(rs_detail::Int<1 - NEXT>{}, cur_off, t + 2, p, mode_tag);
-          else commit_one(next_tag, next_off, t + 1, (u + 1) * HEAD + p, mode_tag);
+          else commit_one(next_tag, next_off, t + 1, first + p, mode_tag);
         };
         auto load = [&](int p) {
           if (last) fetch_one(rs_detail::Int<1 - NEXT>{}, t + 4, p, mode_tag);
-          else fetch_one(next_tag, t + 3, (u + 1) * HEAD + p, mode_tag);
+          else fetch_one(next_tag, t + 3, first + p, mode_tag);
         };
         if constexpr (ROOMY) {
           const int p = (m - R0) / GAP;
-          if (m >= R0 && p < HEAD) {
+          if (m >= R0 && p < count) {
             if ((m - R0) % GAP == 0) write(p);
             if ((m - R0) % GAP == GAP - 1) load(p);
           }
         } else {
 #pragma unroll
-          for (int p = m * HEAD / MF; p < (m + 1) * HEAD / MF; ++p) { write(p); load(p); }
+          for (int p = m * count / MF; p < (m + 1) * count / MF; ++p) { write(p); load(p); }
         }
         if (LIVE) {
           // float32 results leave straight from the accumulators, a register holding 32 consecutive columns of a row;
           // 16-bit results go through LDS and want four consecutive columns per lane (operands swapped)
-          if constexpr (sizeof(E) == 2) acc[i][j] = mfma_32x32x16<C::HALF>(fb[u & 1][j], fa[u & 1][i], acc[i][j]);
+          if constexpr (C::FULL) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u & 1][i][ke], fb[u & 1][j][ke], acc[i][j], 0, 0, 0);
+          else if constexpr (sizeof(E) == 2) acc[i][j] = mfma_32x32x16<C::HALF>(fb[u & 1][j], fa[u & 1][i], acc[i][j]);
           else acc[i][j] = mfma_32x32x16<false>(fa[u & 1][i], fb[u & 1][j], acc[i][j]);
         }
         __builtin_amdgcn_sched_barrier(0);

@@ -34,16 +34,16 @@
 namespace rd {
 #if RD_ANY_PITCH
 // 16-byte pieces at any address through registers (rd_gemm_rs.h): bf16, float16, or float32 rounded to bf16
-#if RD_F32 == 2
+#if RD_F32 == 2 || RD_F32 == 1
 typedef float RsElem;
 #elif RD_F32 == 4
 typedef f16_t RsElem;
 #else
 typedef bf16_bits RsElem;
 #endif
-typedef RsCfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RsElem, RD_VEC != 0> CfgNN;
-typedef RsCfg<RD_BM, RD_BN, true, true, RsElem, RD_VEC != 0> CfgNT;
-typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0> CfgTN;
+typedef RsCfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RsElem, RD_VEC != 0, RD_F32 == 1> CfgNN;
+typedef RsCfg<RD_BM, RD_BN, true, true, RsElem, RD_VEC != 0, RD_F32 == 1> CfgNT;
+typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0, RD_F32 == 1> CfgTN;
 #elif RD_F32 == 4 && RD_DLDS == 3
 // float16 arrays on the four-wave direct-to-LDS core: the bf16 core's data movement with the float16 instruction
 typedef W4Cfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, true> CfgNN;

@@ -18,9 +18,9 @@ pytestmark = pytest.mark.gpu
 
 HP = dict(block_m=64, block_k=64, block_n=64, interpret=False, acc_dtype=torch.float32, chunk_m=512)
 KINDS = {_capi.RD_DTYPE_BF16: ("bfloat16", torch.bfloat16, None), _capi.RD_DTYPE_F16: ("float16", torch.float16, None),
-         _capi.RD_DTYPE_F32_BF16: ("bfloat16", torch.float32, torch.bfloat16)}
+         _capi.RD_DTYPE_F32_BF16: ("bfloat16", torch.float32, torch.bfloat16), _capi.RD_DTYPE_F32: ("float32", torch.float32, None)}
 VARIANTS = [(v.id, v.name.decode(), v.dtype) for v in _capi.variants()
-            if v.name.decode().startswith(("r", "hr", "cr", "cs", "s64", "h64x64", "c64"))]
+            if v.name.decode().startswith(("r", "hr", "cr", "cs", "fr", "s64", "h64x64", "c64"))]
 # (k, n): slabs of 64 (16-bit) or 32 (float32); the pipelined loop takes over from seven slabs on
 SHAPES = [(8, 8), (57, 77), (63, 129), (65, 257), (191, 9), (225, 131), (385, 255), (449, 250), (577, 264)]
 
@@ -53,7 +53,7 @@ def test_any_pitch_edges(vid, vname, dtype, k, n):
     y_ref, dA_ref = oracle.gmm(x, A, gs, **f64), oracle.tgmm(x, dy, gs, **f64)
     # 16-bit results: one rounding to a significand of 8 or 11 bits (at most 2^-8 or 2^-11 of the value) on top of fp32 sums
     # of at most 577 products (577 x 2^-24 = 3.5e-5); float32 results: the sums alone
-    eps = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11}[rounding] if storage != torch.float32 else 0.0
+    eps = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11, "float32": 0.0}[rounding] if storage != torch.float32 else 0.0
     eps += 577 * 2.0 ** -24
     for name, got in (("y", y), ("y (trans_rhs)", yt)):
         assert np.all(np.isnan(got[hit])), f"{name}: the poisoned group's rows"
