@@ -217,7 +217,8 @@ Tensor gmm(const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int c
 Tensor tgmm(const Tensor& x, const Tensor& y, const Tensor& gs, int code, int64_t g_first, int64_t g_local, const py::object& plans) {
   if (x.scalar_type() != y.scalar_type()) throw py::type_error("x and y have different element types");
   Call c;
-  c.code = code; c.g_first = g_first; c.g_local = g_local; c.plans = plans_from(plans);
+  // a number of groups without a first one means the first ones (the gradients' A then holds those only)
+  c.code = code; c.g_first = g_first < 0 && g_local >= 0 ? 0 : g_first; c.g_local = g_local; c.plans = plans_from(plans);
   if (!wants_grad(x, y)) return tgmm_forward(x, y, gs, c, 0, g_local);
   check_devices(x, y);
   return TgmmNode::apply(x, y, gs, c);

@@ -167,6 +167,20 @@ def test_tgmm_vjp_empty_group_and_tail():
     assert torch.equal(dx2, dx) and torch.equal(dy2, dy)
 
 
+def test_tgmm_vjp_of_the_first_groups_only():
+    """num_actual_groups without group_offset: the slices of the first groups, and their gradients."""
+    m, k, n, g, first = 96, 32, 48, 5, 3
+    lhs, _, dout2d, _, _ = util.make_case(32, m, k, n, g, 1.0, True)
+    gs = np.array([20, 0, 30, 26, 20], np.int32)
+    x_t, y_t = util.bf16_dev(lhs).requires_grad_(True), util.bf16_dev(dout2d).requires_grad_(True)
+    sizes = torch.from_numpy(gs)
+    out = rd.tgmm(x_t, y_t, sizes, num_actual_groups=first)
+    do = torch.randn_like(out)
+    got = torch.autograd.grad(out, (x_t, y_t), do)
+    want = torch.autograd.grad(rd.tgmm(x_t, y_t, sizes, group_offset=0, num_actual_groups=first), (x_t, y_t), do)
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and got[0][:20].any() and not got[0][50:].any()
+
+
 # ---------------------------------------------------------------------------------------------------------------------
 # compute_dtype (gpu_ragged_dot.py:116-119, 145, 248, 270)
 # ---------------------------------------------------------------------------------------------------------------------
