@@ -86,6 +86,11 @@ void check_devices(const Tensor& a, const Tensor& b) {
   if (b.device() != a.device()) throw std::runtime_error("all operands must live on the same device");
 }
 
+// (also in the gradients: a cotangent need not have its operand's type - float8 products come out as bfloat16)
+void same_type(const Tensor& a, const Tensor& b) {
+  TORCH_CHECK_TYPE(a.scalar_type() == b.scalar_type(), "the operands are ", a.scalar_type(), " and ", b.scalar_type());
+}
+
 Tensor sizes_on(const Tensor& gs, const at::Device& dev) {
   Tensor t = gs.scalar_type() == at::kInt ? gs : gs.to(at::kInt);
   if (t.device() != dev) t = t.to(dev);
@@ -112,6 +117,7 @@ struct Call {
 // gpu_ragged_dot.py:171-228 (_gpu_gmm_fwd)
 Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const Call& c, int which, bool trans) {
   expect(A_.dim() == 3 && x_.dim() == 2, "x must be [m, k] and A [g, k, n]");  // :188
+  same_type(x_, A_);
   expect(gs_.dim() == 1, "group_sizes must have one dimension");
   const int64_t g_local = A_.size(0), g = gs_.numel(), g_first = c.g_first < 0 ? 0 : c.g_first;
   expect(c.g_first < 0 ? g_local == g : g_first + g_local <= g, "A does not hold the groups that group_sizes describes");  // :189
@@ -136,6 +142,7 @@ Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const 
 // gpu_ragged_dot.py:287-342 (_gpu_tgmm_fwd)
 Tensor tgmm_forward(const Tensor& x_, const Tensor& y_, const Tensor& gs_, const Call& c, int which, int64_t g_local) {
   expect(y_.dim() == 2 && x_.dim() == 2 && x_.size(0) == y_.size(0), "x must be [m, k] and y [m, n]");  // :304
+  same_type(x_, y_);
   const int64_t m = x_.size(0), k = x_.size(1), n = y_.size(1), g = gs_.numel(), g_first = c.g_first < 0 ? 0 : c.g_first;
   if (g_local < 0) g_local = g - g_first;
   expect(g_local >= 1 && g_first + g_local <= g, "the groups asked for are not within group_sizes");

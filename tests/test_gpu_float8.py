@@ -310,3 +310,16 @@ def test_float8_is_forward_only_and_rejects_mixed_operands():
     bf16 = [v.id for v in _capi.variants() if v.dtype == _capi.RD_DTYPE_BF16][0]
     with pytest.raises(_capi.RaggedDotError):
         ops._gmm_fwd(x, A, gs_t, **HP, trans_rhs=False, plan=_capi.Plan(bf16))
+
+
+def test_float8_tgmm_refuses_its_bfloat16_cotangent():
+    """tgmm takes float8 arrays that ask for gradients, but no kernel multiplies its bfloat16 cotangent with them."""
+    x8, _, dy8, gs, _ = _case(1, 128, 64, 64, 2)
+    x, dy = _f8_dev(x8), _f8_dev(dy8)
+    try:
+        x.requires_grad_(True)
+    except RuntimeError:
+        return  # this torch does not let a float8 tensor require a gradient at all
+    out = rd.tgmm(x, dy, torch.from_numpy(gs))
+    with pytest.raises(TypeError):
+        torch.autograd.grad(out, x, torch.ones_like(out))
