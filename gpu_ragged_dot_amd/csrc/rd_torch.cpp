@@ -295,36 +295,37 @@ Tensor combine_wgrad(const Tensor& y_, const Tensor& dout_, const Routing& r) {
   return dw;
 }
 
-Routing routing_of(AutogradContext* ctx, const Tensor& row_of_slot, const Tensor& slot_of_row) {
-  return Routing{row_of_slot, slot_of_row, ctx->saved_data["tokens"].toInt(), ctx->saved_data["top_k"].toInt()};
-}
+// A node keeps its routing aside from its saved tensors: a dispatch saves none, so that gradients can be taken through it
+// any number of times without retain_graph.
+struct RoutingHolder : torch::CustomClassHolder {
+  Routing r;
+  explicit RoutingHolder(const Routing& routing) : r(routing) {}
+};
+Routing routing_of(AutogradContext* ctx) { return static_cast<RoutingHolder*>(ctx->saved_data["routing"].toCapsule().get())->r; }
 void keep_routing(AutogradContext* ctx, const Routing& r) {
-  ctx->saved_data["tokens"] = r.tokens;
-  ctx->saved_data["top_k"] = r.top_k;
+  ctx->saved_data["routing"] = c10::IValue::make_capsule(c10::make_intrusive<RoutingHolder>(r));
 }
 
 struct DispatchNode : torch::autograd::Function<DispatchNode> {
   static Tensor forward(AutogradContext* ctx, const Tensor& h, const Routing& r) {
-    ctx->save_for_backward({r.row_of_slot, r.slot_of_row});
     keep_routing(ctx, r);
     return dispatch_rows(h, r, Tensor());
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto s = ctx->get_saved_variables();
-    return {combine_rows(grads[0], routing_of(ctx, s[0], s[1]), Tensor()), Tensor()};  // each token collects the gradients of its rows
+    return {combine_rows(grads[0], routing_of(ctx), Tensor()), Tensor()};  // each token collects the gradients of its rows
   }
 };
 
 struct CombineNode : torch::autograd::Function<CombineNode> {
   static Tensor forward(AutogradContext* ctx, const Tensor& y, const std::optional<Tensor>& weights, const Routing& r) {
     const Tensor w = weights.value_or(Tensor());
-    ctx->save_for_backward({y, w, r.row_of_slot, r.slot_of_row});
+    ctx->save_for_backward({y, w});
     keep_routing(ctx, r);
     return combine_rows(y, r, w);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
-    const Routing r = routing_of(ctx, s[2], s[3]);
+    const Routing r = routing_of(ctx);
     const Tensor &y = s[0], &w = s[1], &dout = grads[0];
     Tensor dy, dw;
     if (ctx->needs_input_grad(0)) dy = dispatch_rows(dout, r, w);  // dy[row] = weight of the row's slot * dout[token]

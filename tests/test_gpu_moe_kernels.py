@@ -52,3 +52,14 @@ def test_combine_and_weight_gradient(top_k, d, dtype):
     ref, mag = np.einsum("tsd,ts->td", picked, wv), np.einsum("tsd,ts->td", np.abs(picked), wv)
     got = out.detach().double().cpu().numpy()
     assert np.all(np.abs(got - ref) <= half_ulp * np.abs(ref) + (top_k + 1) * 2.0 ** -24 * mag + 2.0 ** -24)
+
+
+def test_dispatch_gradient_twice():
+    """A dispatch keeps no operand for its gradient, so asking for it twice needs no retain_graph."""
+    ids = torch.tensor([[0, 1], [2, 0], [1, 1]], device="cuda")
+    r = moe.route(ids, 3)
+    h = torch.randn(3, 16, device="cuda").requires_grad_()
+    x = moe.dispatch(h, r)
+    dx = torch.randn_like(x)
+    first, again = (torch.autograd.grad(x, h, dx)[0] for _ in range(2))
+    assert torch.equal(first, again)
