@@ -7,9 +7,10 @@
 // What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
 // element per instruction where the pitch is odd, one slab in flight where the source is float32 - at 40-85 and 300-430
 // TFLOP/s (bf16 8191 x 2047 x 4095 in 16 groups, fwd / dlhs / drhs: 2300 / 3080 / 1620 us; float32 8192 x 4096 x 4096 in
-// 8: 683 / 668 / 899).  Here: 244 / 270 / 337 and 412 / 424 / 473 us; aligned bf16 16384 x 4096 x 4096 in 8 groups 574 us
+// 8: 683 / 668 / 899).  Here: 221 / 270 / 337 and 402 / 412 / 371 us; aligned bf16 16384 x 4096 x 4096 in 8 groups 574 us
 // (960 TFLOP/s).  Left over: the latency of the first slabs and of the epilogue, which nothing else on the compute unit
-// hides under a 256 x 256 tile, and pieces that straddle cache lines (20-50 % against the same sizes aligned).  How:
+// hides under a 256 x 256 tile (one round of them, 4096^3 float32: 146 us, 940 TFLOP/s), the last, partly filled round, and
+// pieces that straddle cache lines (20-50 % against the same sizes aligned).  How:
 //  * a load is always 16 bytes per lane (a "piece"), at whatever address the element has: global memory takes 16-byte
 //    accesses at any alignment.  Every 8 lanes (K-major) or every 32 / 64 (MN-major) read consecutive memory;
 //  * a slab is 128 bytes of every K-major row (64 bf16 or 32 float32 contraction indices), 16 pieces per lane for both
@@ -19,8 +20,11 @@
 // float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most: the plain tile of
 // rd_gemm_f32.h, one slab of 16 ahead with element-wise LDS traffic, kept it busy 72-78 % of the time (4096 x 4096 x 3072:
 // 946 / 870 / 883 us), this core 86-92 % (766 / 733 / 713 us).
-// No predicate sits in the steady loop: a slab that holds the last contraction index, or lies behind it, is loaded by
-// fetch_tail(), which never touches memory outside the operand's rows and fills with zeros.
+// One loop serves all slabs.  Where a load goes is a clamped offset from a base; on the slab that holds the last contraction
+// index the base, the offset and its limit change (enter_last), so that no load touches memory outside the operand's rows,
+// and from there on what is not the operand's is cut off on the way into LDS (trim).  A second loop for those slabs, with
+// loads of their own, had the compiler spill 300 registers under two MN-major operands (float32 tgmm, 8192 x 4096 x 4096 in 8
+// groups: 499 us so, 371 without; 16384 x 2048 x 2048 in 32: 408 and 266).
 #pragma once
 #include <type_traits>
 #include "rd_gemm_dlds.h"
@@ -86,11 +90,12 @@ struct RsLoader {
   // the chunk permutation of DldsFragReader repeats from one of a lane's pieces to the next
   static_assert(KMAJOR ? (NW * RPI) % 16 == 0 : (NW * RPI) % (LB == 4 ? 8 : 4) == 0, "chunk permutation");
 
-  const Src* base;   // first element of the current slab
+  const Src* base;   // first element of the current slab (one piece before it once the slab holds the last contraction index)
   long long step;    // elements from one slab to the next
   uint32_t off0;     // byte offset of piece 0 from base; piece j lies j * row_step further, but no further than off_last
   uint32_t row_step, off_last;
   int ld, lim, klen;
+  int slab, last;    // index of the current slab; of the slab that holds the last contraction index
   int lds;           // byte of piece 0 in the operand's region of a slot
 
   static __host__ __device__ __forceinline__ int slab_row(int wave, int lane, int j) { return wave * RPI + lane / PPR + j * NW * RPI; }
@@ -98,9 +103,11 @@ struct RsLoader {
   __host__ __device__ __forceinline__ void init(const Src* p, int ld_, int lim_, int klen_, int wave, int lane) {
     base = p; ld = ld_; lim = lim_; klen = klen_;
     step = KMAJOR ? BK : (long long)BK * ld;
+    slab = 0; last = (klen - 1) / BK;
     const int row0 = slab_row(wave, lane, 0), piece = lane % PPR;
     // rows past the tile's limit re-read its last row, columns past it the last piece that holds one of the tile's:
-    // what they hold never reaches a stored element
+    // what they hold never reaches a stored element.  (An MN-major piece may run past the end of its row, at most into the
+    // row behind it, which exists: the slab ends before the last contraction index.)
     const int e = KMAJOR ? piece * EPP : imin(piece * EPP, (lim - 1) / EPP * EPP);
     off_last = KMAJOR ? ((uint32_t)(lim - 1) * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src) : ~0u;
     off0 = ((uint32_t)row0 * (uint32_t)ld + (uint32_t)e) * (uint32_t)sizeof(Src);
@@ -109,40 +116,42 @@ struct RsLoader {
     const int c = KMAJOR ? (LDS_ROW == 128 ? chunk ^ ((row0 >> 1) & 7) : chunk ^ ((row0 >> 2) & 3))
                 : LB == 4 ? chunk ^ (((row0 >> 2) & 1) << 3) : chunk ^ ((row0 & 3) << 2);
     lds = row0 * LDS_ROW + (c << 4) + (sizeof(Src) == LB ? 0 : (piece & 1) * 8);
+    if (last == 0) enter_last(wave, lane);
   }
 
+  // The slab that holds the last contraction index.  A piece that would run past the contraction length (K-major) or past
+  // the tile's columns (MN-major) is read from before them instead, rows past the contraction length re-read its last one;
+  // trim() takes out what is not the operand's.  The place may lie before the slab's first element (the row it is read
+  // along holds a whole piece up to there): offsets count from one piece before it.
+  __host__ __device__ __forceinline__ int last_at(int lane) const {
+    const int e = lane % PPR * EPP;
+    return KMAJOR ? imin(e, klen - EPP - last * BK) : imin(e, lim - EPP);
+  }
+  __host__ __device__ __forceinline__ void enter_last(int wave, int lane) {
+    const uint32_t at = (uint32_t)(last_at(lane) + EPP);
+    const int rows = KMAJOR ? lim : klen - last * BK;
+    base -= EPP;
+    off0 = ((uint32_t)slab_row(wave, lane, 0) * (uint32_t)ld + at) * (uint32_t)sizeof(Src);
+    off_last = ((uint32_t)(rows - 1) * (uint32_t)ld + at) * (uint32_t)sizeof(Src);
+  }
+  // On to the next slab; behind the last one the loads stay where they are (and trim() leaves only zeros).
+  __host__ __device__ __forceinline__ void next(int wave, int lane) {
+    ++slab;
+    if (slab <= last) base += step;
+    if (slab == last) enter_last(wave, lane);
+  }
   __host__ __device__ __forceinline__ uint32_t offset(int j) const {
     const uint32_t o = off0 + (uint32_t)j * row_step;
-    return KMAJOR && o > off_last ? off_last : o;
+    return o > off_last ? off_last : o;
   }
-  // Piece j of the slab at base; the slab holds contraction indices below klen - 1 only.  (An MN-major piece may run past
-  // the end of its row, at most into the row behind it, which exists.)
   __device__ __forceinline__ u32x4_t fetch(int j) const { return load_any<u32x4_t>(reinterpret_cast<const unsigned char*>(base) + offset(j)); }
-  // The same for any slab, its first contraction index being k0: element `at` of slab row `row` (counted from base; `at` may
-  // be negative).  Once there the piece is shifted down by `shift` elements (EPP or more: all zeros), which takes out what
-  // is not the operand's and zeroes what lies past the contraction length.  Slabs that fetch() serves come from where
-  // fetch() reads them, unshifted.
-  __host__ __device__ __forceinline__ void tail_source(int wave, int lane, int j, int k0, int* row, int* at, int* shift) const {
-    const int r = slab_row(wave, lane, j), e = lane % PPR * EPP;
-    if (KMAJOR) {
-      *row = imin(r, lim - 1);
-      *at = imin(e, klen - EPP - k0);
-      *shift = e - *at;
-    } else {
-      const bool whole = k0 + BK < klen;
-      *row = imin(r, klen - 1 - k0);
-      *at = imin(e, whole ? (lim - 1) / EPP * EPP : lim - EPP);
-      *shift = r != *row ? EPP : whole ? 0 : e - *at;
-    }
+  // By how many elements piece j of slab `at_slab` (the last one or behind it) has to come down; EPP or more: all zeros.
+  __host__ __device__ __forceinline__ int surplus(int wave, int lane, int j, int at_slab) const {
+    const bool gone = at_slab > last || (!KMAJOR && slab_row(wave, lane, j) >= klen - last * BK);
+    return gone ? EPP : lane % PPR * EPP - last_at(lane);
   }
-  __device__ __forceinline__ u32x4_t fetch_tail(int wave, int lane, int j, int k0) const {
-    int row, at, shift;
-    tail_source(wave, lane, j, k0, &row, &at, &shift);
-    return load_any<u32x4_t>(base + ((long long)row * ld + at));
-  }
-  __device__ __forceinline__ u32x4_t shift_tail(int wave, int lane, int j, int k0, u32x4_t v) const {
-    int row, at, shift;
-    tail_source(wave, lane, j, k0, &row, &at, &shift);
+  __device__ __forceinline__ u32x4_t trim(int wave, int lane, int j, int at_slab, u32x4_t v) const {
+    const int shift = surplus(wave, lane, j, at_slab);
     if constexpr (VEC) return shift == 0 ? v : u32x4_t{0, 0, 0, 0};
     else return shift_down(v, imin(shift, EPP) * (int)sizeof(Src));
   }
@@ -157,8 +166,9 @@ struct RsLoader {
   }
   // The new base and the lane's offset are opaque to the compiler: it would otherwise carry an address per piece through
   // the loop, and there are no registers for those.
-  __device__ __forceinline__ void advance() {
-    const uint64_t b = reinterpret_cast<uint64_t>(base + step);
+  __device__ __forceinline__ void advance(int wave, int lane) {
+    next(wave, lane);
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
     base = reinterpret_cast<const Src*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b) |
                                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32));
     asm volatile("" : "+v"(off0));
@@ -204,8 +214,6 @@ struct RsFrag {
 namespace rs_detail {
 template <int V>
 struct Int { static constexpr int value = V; };
-// how a slab's pieces are loaded: it ends before the last contraction index, or it may hold that index or lie behind it
-constexpr int kWhole = 0, kTail = 1;
 }  // namespace rs_detail
 
 // Slab t lives in LDS slot t & 1 and, before that, in register set t & 1.  The pieces of slab t + 1 are written to LDS
@@ -244,40 +252,46 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
   static_assert(HEAD >= 1, "every substep moves a piece");
 
   u32x4_t regs[2][P];
-  auto fetch_one = [&](auto set_tag, int step, int q, auto mode_tag) {
-    constexpr int SET = decltype(set_tag)::value, MODE = decltype(mode_tag)::value;
-    if constexpr (MODE == rs_detail::kWhole) regs[SET][q] = q < PA ? la.fetch(q) : lb.fetch(q - PA);
-    else
-      regs[SET][q] = q < PA ? la.fetch_tail(wave, lane, q, step * C::BK) : lb.fetch_tail(wave, lane, q - PA, step * C::BK);
+  auto fetch_one = [&](auto set_tag, int q) {
+    constexpr int SET = decltype(set_tag)::value;
+    regs[SET][q] = q < PA ? la.fetch(q) : lb.fetch(q - PA);
   };
-  // (a piece is shifted here and not where it is fetched, or every load would be waited for at once)
-  auto commit_one = [&](auto set_tag, int slot_off, int step, int q, auto mode_tag) {
-    constexpr int SET = decltype(set_tag)::value, MODE = decltype(mode_tag)::value;
-    u32x4_t v = regs[SET][q];
-    if constexpr (MODE == rs_detail::kTail)
-      v = q < PA ? la.shift_tail(wave, lane, q, step * C::BK, v) : lb.shift_tail(wave, lane, q - PA, step * C::BK, v);
-    if (q < PA) la.commit(smem + slot_off, q, v);
-    else lb.commit(smem + slot_off + C::A_BYTES, q - PA, v);
+  auto commit_one = [&](auto set_tag, int slot_off, int q) {
+    constexpr int SET = decltype(set_tag)::value;
+    if (q < PA) la.commit(smem + slot_off, q, regs[SET][q]);
+    else lb.commit(smem + slot_off + C::A_BYTES, q - PA, regs[SET][q]);
   };
-  auto advance = [&]() { la.advance(); lb.advance(); };
+  // Before pieces first .. first + count - 1 of slab `step` are written: where that slab holds the last contraction index or
+  // lies behind it, take out what is not the operand's.
+  auto trim_some = [&](auto set_tag, int step, int first, int count) {
+    constexpr int SET = decltype(set_tag)::value;
+    if (step >= nk - 1) {
+#pragma unroll
+      for (int q = first; q < first + count; ++q)
+        regs[SET][q] = q < PA ? la.trim(wave, lane, q, step, regs[SET][q]) : lb.trim(wave, lane, q - PA, step, regs[SET][q]);
+    }
+  };
+  auto advance = [&]() { la.advance(wave, lane); lb.advance(wave, lane); };
 
   // slab 0 through the registers into LDS, slab 1 in registers with its first pieces written, slab 2 requested
-  auto prologue = [&](auto mode_tag) {
+  auto prologue = [&]() {
 #pragma unroll
-    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, 0, q, mode_tag);
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, q);
     advance();
 #pragma unroll
-    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<1>{}, 1, q, mode_tag);
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<1>{}, q);
     advance();
+    trim_some(rs_detail::Int<0>{}, 0, 0, P);
 #pragma unroll
-    for (int q = 0; q < P; ++q) commit_one(rs_detail::Int<0>{}, 0, 0, q, mode_tag);
+    for (int q = 0; q < P; ++q) commit_one(rs_detail::Int<0>{}, 0, q);
 #pragma unroll
-    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, 2, q, mode_tag);
+    for (int q = 0; q < P; ++q) fetch_one(rs_detail::Int<0>{}, q);
     advance();
+    trim_some(rs_detail::Int<1>{}, 1, 0, HEAD);
 #pragma unroll
-    for (int q = 0; q < HEAD; ++q) commit_one(rs_detail::Int<1>{}, C::SLOT_BYTES, 1, q, mode_tag);
+    for (int q = 0; q < HEAD; ++q) commit_one(rs_detail::Int<1>{}, C::SLOT_BYTES, q);
 #pragma unroll
-    for (int q = 0; q < HEAD; ++q) fetch_one(rs_detail::Int<1>{}, 3, q, mode_tag);
+    for (int q = 0; q < HEAD; ++q) fetch_one(rs_detail::Int<1>{}, q);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): slab 0 is written
     __builtin_amdgcn_s_barrier();
   };
@@ -293,8 +307,7 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
     }
   };
 
-  // mode: how the pieces of slabs t + 3 and t + 4 are loaded
-  auto slab = [&](int t, auto next_tag, auto mode_tag) {
+  auto slab = [&](int t, auto next_tag) {
     constexpr int NEXT = decltype(next_tag)::value;  // (t + 1) & 1
     const int cur_off = (1 - NEXT) * C::SLOT_BYTES, next_off = NEXT * C::SLOT_BYTES;
 #pragma unroll
@@ -311,6 +324,8 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
       const unsigned char* rb = ra + C::A_BYTES;
       const int us = last ? 0 : u + 1;
       const int first = last ? 0 : part(u + 1), count = last ? HEAD : part(u + 2) - part(u + 1);
+      if (last) trim_some(rs_detail::Int<1 - NEXT>{}, t + 2, first, count);
+      else trim_some(next_tag, t + 1, first, count);
 #pragma unroll
       for (int m = 0; m < MF; ++m) {
         const int i = m % (C::TM * C::TN) / C::TN, j = m % C::TN, ke = m / (C::TM * C::TN);
@@ -325,12 +340,12 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
           }
         }
         auto write = [&](int p) {
-          if (last) commit_one(rs_detail::Int<1 - NEXT>{}, cur_off, t + 2, p, mode_tag);
-          else commit_one(next_tag, next_off, t + 1, first + p, mode_tag);
+          if (last) commit_one(rs_detail::Int<1 - NEXT>{}, cur_off, p);  // of slab t + 2
+          else commit_one(next_tag, next_off, first + p);                // of slab t + 1
         };
         auto load = [&](int p) {
-          if (last) fetch_one(rs_detail::Int<1 - NEXT>{}, t + 4, p, mode_tag);
-          else fetch_one(next_tag, t + 3, first + p, mode_tag);
+          if (last) fetch_one(rs_detail::Int<1 - NEXT>{}, p);  // of slab t + 4
+          else fetch_one(next_tag, first + p);                 // of slab t + 3
         };
         if constexpr (ROOMY) {
           const int p = (m - R0) / GAP;
@@ -354,28 +369,11 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
     }
   };
 
-  // Slabs t < n_steady load slabs up to t + 4, which are whole.  An even count, entered straight from the prologue of whole
-  // slabs: the compiler counts the loads outstanding at each register's use along every path into the loop.  The slabs
-  // behind it run one loop of the same shape with all loads as tails (what lies past the contraction length comes as zeros):
-  // with a condition around the loads, or the last slabs written out one by one, the registers no longer suffice.
-  constexpr rs_detail::Int<rs_detail::kWhole> whole{};
-  constexpr rs_detail::Int<rs_detail::kTail> tail{};
-  const int n_steady = (nk - 5) & ~1;
-  int t = 0;
-  if (n_steady > 0) {
-    prologue(whole);
-    first_fragments();
-    for (; t < n_steady; t += 2) {
-      slab(t, rs_detail::Int<1>{}, whole);
-      slab(t + 1, rs_detail::Int<0>{}, whole);
-    }
-  } else {
-    prologue(tail);
-    first_fragments();
-  }
-  for (; t < nk; t += 2) {  // (an odd nk multiplies one slab of zeros)
-    slab(t, rs_detail::Int<1>{}, tail);
-    slab(t + 1, rs_detail::Int<0>{}, tail);
+  prologue();
+  first_fragments();
+  for (int t = 0; t < nk; t += 2) {  // (an odd nk multiplies one slab of zeros)
+    slab(t, rs_detail::Int<1>{});
+    slab(t + 1, rs_detail::Int<0>{});
   }
 
   __builtin_amdgcn_s_waitcnt(0xc07f);

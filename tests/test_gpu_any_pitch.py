@@ -21,8 +21,8 @@ KINDS = {_capi.RD_DTYPE_BF16: ("bfloat16", torch.bfloat16, None), _capi.RD_DTYPE
          _capi.RD_DTYPE_F32_BF16: ("bfloat16", torch.float32, torch.bfloat16), _capi.RD_DTYPE_F32: ("float32", torch.float32, None)}
 VARIANTS = [(v.id, v.name.decode(), v.dtype) for v in _capi.variants()
             if v.name.decode().startswith(("r", "hr", "cr", "cs", "fr", "s64", "h64x64", "c64"))]
-# (k, n): slabs of 64 (16-bit) or 32 (float32); the pipelined loop takes over from seven slabs on
-SHAPES = [(8, 8), (57, 77), (63, 129), (65, 257), (191, 9), (225, 131), (385, 255), (449, 250), (577, 264)]
+# (k, n): slabs of 64 (16-bit) or 32 (float32), two of them in LDS and two in registers
+SHAPES = [(8, 8), (57, 77), (63, 129), (65, 257), (191, 9), (225, 131), (257, 64), (321, 72), (385, 255), (449, 250), (577, 264)]
 
 
 @pytest.mark.parametrize("vid,vname,dtype", VARIANTS, ids=[v[1] for v in VARIANTS])
