@@ -7,7 +7,7 @@
 // What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
 // element per instruction where the pitch is odd, one slab in flight where the source is float32 - at 40-85 and 300-430
 // TFLOP/s (bf16 8191 x 2047 x 4095 in 16 groups, fwd / dlhs / drhs: 2300 / 3080 / 1620 us; float32 8192 x 4096 x 4096 in
-// 8: 683 / 668 / 899).  Here: 221 / 270 / 337 and 402 / 412 / 371 us; aligned bf16 16384 x 4096 x 4096 in 8 groups 574 us
+// 8: 683 / 668 / 899).  Here: 218 / 271 / 337 and 387 / 397 / 371 us; aligned bf16 16384 x 4096 x 4096 in 8 groups 574 us
 // (960 TFLOP/s).  Left over: the latency of the first slabs and of the epilogue, which nothing else on the compute unit
 // hides under a 256 x 256 tile (one round of them, 4096^3 float32: 146 us, 940 TFLOP/s), the last, partly filled round, and
 // pieces that straddle cache lines (20-50 % against the same sizes aligned).  How:
@@ -55,7 +55,7 @@ struct RsCfg {
   static constexpr int EPI_BYTES = sizeof(Src) == 2 ? NW * WM * EPI_PITCH : 0;
   static constexpr int RING_BYTES = 2 * SLOT_BYTES;
   static constexpr int LDS_BYTES = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
-  static_assert(FULL ? BM % 64 == 0 && BN % 64 == 0 : BM % 128 == 0 && BN % 128 == 0, "tile shape");
+  static_assert(FULL ? BM % 64 == 0 && BN % 64 == 0 : BM % (A_KMAJOR ? 64 : 128) == 0 && BN % 128 == 0, "tile shape");
   static_assert(!FULL || std::is_same<Src, float>::value, "float32 only");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
@@ -471,6 +471,23 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
   if constexpr (sizeof(typename C::Elem) == 2) rs_store16<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
   else rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
+}
+
+// A row tile of a gmm launch with fewer rows than its height: the same routine on the least multiple of 64 that holds them,
+// with as many fewer loads, LDS traffic and matrix-core instructions.  False: the tile is to be computed whole.
+template <class C, int ROWS = 64>
+__device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict__ Ap, int lda, int rows,
+                                              const typename C::Elem* __restrict__ Bp, int ldb, int cols, int klen,
+                                              typename C::Elem* __restrict__ Op, int ldo, void* smem, const SplitK& sk) {
+  if constexpr (ROWS >= C::BM || C::FULL) {
+    return false;
+  } else {
+    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC> S;
+    static_assert(C::A_KMAJOR && S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "runs in the tall tile's launch");
+    if (rows > ROWS) return rs_short_tile<C, ROWS + 64>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, smem, sk);
+    gemm_tile_rs<S>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, static_cast<unsigned char*>(smem), sk);
+    return true;
+  }
 }
 
 }  // namespace rd

@@ -311,6 +311,13 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
         }
       }
     }
+    if constexpr (IsRs<C>::value) {
+      // A group's only row tile, and a few rows behind whole ones (8192 x 4096 x 4096 in 8 groups of about 1024 rows, float32
+      // in bf16, half of them a few rows over: 403 -> 387 us, 417 -> 398 with trans_rhs).  Taller last tiles stay on the
+      // whole routine: out of step with their neighbours they cost more in shared operand slabs than they save (4096 x
+      // 4096 x 4096 in 16: 323 us, 337 with every height cut).
+      if ((it == 0 || rows <= 64) && rs_short_tile<C>(Ap, p.k, rows, Bp, TRANS_RHS ? p.k : p.n, cols, klen, Op, p.n, smem, sk)) return;
+    }
     run_tile<C>(Ap, p.k, rows, Bp, TRANS_RHS ? p.k : p.n, cols, klen, Op, p.n, smem, sk);
   } else {
     // Rows past sum(group_sizes) are defined to be zero.  The map never uses more than

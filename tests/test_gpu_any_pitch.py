@@ -69,3 +69,28 @@ def test_any_pitch_edges(vid, vname, dtype, k, n):
         else:
             err = np.linalg.norm(dA[i] - dA_ref[i]) / np.linalg.norm(dA_ref[i])
             assert err < eps, f"dA[{i}]: {err} >= {eps}"
+
+
+@pytest.mark.parametrize("vid,vname,dtype", [v for v in VARIANTS if "256x256" in v[1] or "128x128" in v[1]],
+                         ids=[v[1] for v in VARIANTS if "256x256" in v[1] or "128x128" in v[1]])
+@pytest.mark.parametrize("trans_rhs", [False, True])
+def test_row_tiles_shorter_than_the_tile(vid, vname, dtype, trans_rhs):
+    """A gmm launch computes a row tile of few rows at a multiple of 64: every height and one row to either side of it, as a
+    group's only tile and behind a whole one; the rows behind a group belong to the next and must stay its own."""
+    print(f"short row tiles, variant {vname} trans_rhs {trans_rhs}", flush=True)
+    rounding, storage, compute = KINDS[dtype]
+    gs = np.array([1, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 256 + 1, 256 + 64, 256 + 65, 0, 2 * 256 + 130], np.int32)
+    g, m, k, n = len(gs), int(gs.sum()) + 3, 200, 264
+    rng = np.random.default_rng(vid)
+    r = lambda a: oracle.round_to(a, rounding)
+    x, A = r(rng.normal(size=(m, k))), r(rng.normal(size=(g, k, n)) / np.sqrt(k))
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda().to(storage)
+    y = util.to_np(ops._gmm_fwd(dev(x), dev(np.swapaxes(A, 1, 2) if trans_rhs else A), torch.from_numpy(gs).cuda(), trans_rhs=trans_rhs,
+                                compute_dtype=compute, plan=_capi.Plan(vid), **HP))
+    ref = oracle.gmm(x, A, gs, out_dtype="float32", acc=np.float64)
+    # the bound of the test above, for 200 products
+    eps = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11, "float32": 0.0}[rounding] if storage != torch.float32 else 0.0
+    eps += 200 * 2.0 ** -24
+    err = np.linalg.norm(y[:m - 3] - ref[:m - 3], axis=1) / np.linalg.norm(ref[:m - 3], axis=1)
+    assert err.max() < eps, f"{err.max()} >= {eps} in row {err.argmax()}"
+    assert not np.any(y[m - 3:])
