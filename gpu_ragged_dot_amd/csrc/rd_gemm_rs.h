@@ -482,7 +482,7 @@ __device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict
   if constexpr (ROWS >= C::BM || C::FULL) {
     return false;
   } else {
-    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC> S;
+    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC, C::FULL> S;
     static_assert(C::A_KMAJOR && S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "runs in the tall tile's launch");
     if (rows > ROWS) return rs_short_tile<C, ROWS + 64>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, smem, sk);
     gemm_tile_rs<S>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, static_cast<unsigned char*>(smem), sk);

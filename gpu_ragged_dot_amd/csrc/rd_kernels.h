@@ -126,10 +126,23 @@ struct SplitPlan {
   int tiles;       // live - first_tile
 };
 constexpr int kMaxSplitParts = 8;
-constexpr int kMinSplitK = 512;  // contraction elements a piece must keep
 
-// k_cost: the contraction length in units of what a bf16 K loop spends per element (float8 operands: k / 2).
-__device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int slots, int num_cus, int max_parts) {
+// What a cut is worth depends on the core: its K loop per contraction index and how much a piece's partial sums are.
+// QUARTERS: the former over the latter, in quarters of the 256 x 256 bf16 cores' (float8: twice the rate; float32
+// multiplied as it is: 16 times the time per multiplication, so twice per tile of a quarter of the size).  MIN_K: contraction indices a piece must keep.  float32 without
+// and with the cut, forward product: 256 x 16384 x 256 in 2 groups 291 -> 52 us, 2048 x 8192 x 1024 in 4 372 -> 283,
+// 512 x 4096 x 4096 in 3 202 -> 166, 8192 x 2048 x 2048 in 8 549 -> 506, 4096 x 4096 x 4096 in 4 1073 -> 992; level where the
+// last round is full or more than half full.  float32 rounded to bf16 stays at the bf16 cores' limit (cut from k = 3700 on, 8192 x
+// 4096 x 4096 in 8 groups went from 377 to 429 us: its 256 x 256 pieces cost what a bf16 core's do).
+template <class C, class = void>
+struct SplitCost { static constexpr int QUARTERS = sizeof(typename C::Elem) == 1 ? 2 : 4, MIN_K = 512; };
+template <class C>
+struct SplitCost<C, typename std::enable_if<IsRs<C>::value>::type> {
+  static constexpr int QUARTERS = C::FULL ? 32 : 4, MIN_K = C::FULL ? 256 : 512;
+};
+
+// k_cost: k in units of what a bf16 K loop spends per element.
+__device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int min_k, int slots, int num_cus, int max_parts) {
   SplitPlan sp{live, 1, 0};
   if (slots <= 0 || live <= 0) return sp;
   const int first = (live / num_cus) * num_cus;
@@ -139,7 +152,7 @@ __device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int
   // 25 GB/s: ~10 us per piece), so the gain of a finer cut, T/parts for a K loop of T us, is soon eaten: parts ~
   // sqrt(T / 10 us), with T ~ k / 32 x 0.77 us, i.e. sqrt(k) / 20 - and below k = 6400 (4 pieces) cutting was measured
   // to gain nothing.  max_parts > 0 is the caller's own choice and is taken as it is.
-  int parts = imin(imin(slots / tiles, kMaxSplitParts), k / kMinSplitK);
+  int parts = imin(imin(slots / tiles, kMaxSplitParts), k / min_k);
   if (max_parts > 0) {
     parts = imin(parts, max_parts);
   } else {
@@ -186,7 +199,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   const int total = imin(mapped ? uniform(*p.total_tiles) : scan.total_tiles, p.U);
   const int live = total * p.n_tiles;
   SplitPlan sp{live, 1, 0};
-  if constexpr (C::SPLITK) sp = split_plan(live, p.k, sizeof(E) == 1 ? p.k >> 1 : p.k, p.split_slots, p.num_cus, p.max_parts);
+  if constexpr (C::SPLITK) sp = split_plan(live, p.k, (int)((long long)p.k * SplitCost<C>::QUARTERS / 4), SplitCost<C>::MIN_K, p.split_slots, p.num_cus, p.max_parts);
 
   int t;
   SplitK sk;
@@ -389,6 +402,7 @@ struct TileVariant {
   int stages;  // LDS ring depth
   int any_pitch_core;  // 1: the register-staged core of rd_gemm_rs.h (k >= 8, n >= 8, 32-bit offsets within 256 rows)
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
+  int split_quarters, split_min_k;  // SplitCost of the gmm kernels
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product
   tgmm_launch_fn tgmm;
 };

@@ -94,3 +94,27 @@ def test_row_tiles_shorter_than_the_tile(vid, vname, dtype, trans_rhs):
     err = np.linalg.norm(y[:m - 3] - ref[:m - 3], axis=1) / np.linalg.norm(ref[:m - 3], axis=1)
     assert err.max() < eps, f"{err.max()} >= {eps} in row {err.argmax()}"
     assert not np.any(y[m - 3:])
+
+
+@pytest.mark.parametrize("vid,vname", [v[:2] for v in VARIANTS if v[1].startswith("fr")], ids=[v[1] for v in VARIANTS if v[1].startswith("fr")])
+@pytest.mark.parametrize("k,trans_rhs", [(799, False), (800, True), (800, False), (1025, True), (2111, False), (4096, True)])
+def test_float32_last_round_cut_along_k(vid, vname, k, trans_rhs):
+    """float32 tiles left over from whole rounds are computed in pieces of the contraction from k = 800 on: odd k and n,
+    groups of one row and of a tile's, against the oracle and against the uncut launch; the same bits on a second call."""
+    print(f"float32 k-split, variant {vname} k {k} trans_rhs {trans_rhs}", flush=True)
+    gs = np.array([1, 0, 130, 257, 64, 3], np.int32)
+    g, m, n = len(gs), int(gs.sum()) + 5, 201
+    rng = np.random.default_rng(k)
+    x, A = rng.normal(size=(m, k)).astype(np.float32), (rng.normal(size=(g, k, n)) / np.sqrt(k)).astype(np.float32)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    args = (dev(x), dev(np.swapaxes(A, 1, 2) if trans_rhs else A), dev(gs))
+    run = lambda split: ops._gmm_fwd(*args, trans_rhs=trans_rhs, compute_dtype=None, plan=_capi.Plan(vid, split_k=split), **HP)
+    cut, again, whole = run(0), run(0), run(-1)
+    assert torch.equal(cut, again)
+    assert torch.equal(cut, whole) == (k < 800)
+    ref = oracle.gmm(x, A, gs, out_dtype="float32", acc=np.float64)
+    total = int(gs.sum())
+    for y in (util.to_np(cut), util.to_np(whole)):
+        err = np.linalg.norm(y[:total] - ref[:total], axis=1) / np.linalg.norm(ref[:total], axis=1)
+        assert err.max() < k * 2.0 ** -24, f"{err.max()} in row {err.argmax()}"  # k float32 additions
+        assert not np.any(y[total:])
