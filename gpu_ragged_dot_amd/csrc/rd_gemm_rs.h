@@ -475,6 +475,8 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
 
 // A row tile of a gmm launch with fewer rows than its height: the same routine on the least multiple of 64 that holds them,
 // with as many fewer loads, LDS traffic and matrix-core instructions.  False: the tile is to be computed whole.
+// Not for float32 (FULL): 64 rows inside the 128 x 128 launch gained where its last round was short (8192 x 4096 x 4096 in 8
+// groups 2147 -> 2017 us) and lost elsewhere (8192 x 2048 x 2048 in 8: 607 -> 653), and the cut along K gives the former anyway.
 template <class C, int ROWS = 64>
 __device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict__ Ap, int lda, int rows,
                                               const typename C::Elem* __restrict__ Bp, int ldb, int cols, int klen,
@@ -482,7 +484,7 @@ __device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict
   if constexpr (ROWS >= C::BM || C::FULL) {
     return false;
   } else {
-    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC, C::FULL> S;
+    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC> S;
     static_assert(C::A_KMAJOR && S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "runs in the tall tile's launch");
     if (rows > ROWS) return rs_short_tile<C, ROWS + 64>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, smem, sk);
     gemm_tile_rs<S>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, static_cast<unsigned char*>(smem), sk);
