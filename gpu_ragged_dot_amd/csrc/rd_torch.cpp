@@ -208,11 +208,18 @@ struct TgmmNode : torch::autograd::Function<TgmmNode> {
   }
 };
 
+// Only backward gradients are defined.  An operand that carries a forward-mode tangent is refused, whether or not it asks for
+// a gradient as well: the kernels would run on its value alone, and a result without a tangent reads as one of zero.
+void expect_no_tangent(const Tensor& a, const Tensor& b) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!a._fw_grad(0).defined() && !b._fw_grad(0).defined(), "forward-mode derivatives are not implemented");
+}
+
 bool wants_grad(const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
 }
 
 Tensor gmm(const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int code, int64_t g_first, const py::object& plans) {
+  expect_no_tangent(x, A);
   if (x.scalar_type() != A.scalar_type()) throw py::type_error("x and A have different element types");
   Call c;
   c.code = code; c.trans = trans; c.g_first = g_first; c.plans = plans_from(plans);
@@ -222,6 +229,7 @@ Tensor gmm(const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int c
 }
 
 Tensor tgmm(const Tensor& x, const Tensor& y, const Tensor& gs, int code, int64_t g_first, int64_t g_local, const py::object& plans) {
+  expect_no_tangent(x, y);
   if (x.scalar_type() != y.scalar_type()) throw py::type_error("x and y have different element types");
   Call c;
   // a number of groups without a first one means the first ones (the gradients' A then holds those only)
@@ -336,6 +344,7 @@ struct CombineNode : torch::autograd::Function<CombineNode> {
 
 Tensor moe_dispatch(const Tensor& h, const Tensor& row_of_slot, const Tensor& slot_of_row, int64_t tokens, int64_t top_k) {
   const Routing r{row_of_slot, slot_of_row, tokens, top_k};
+  expect_no_tangent(h, h);
   if (!wants_grad(h, h)) return dispatch_rows(h, r, Tensor());
   return DispatchNode::apply(h, r);
 }
@@ -343,6 +352,7 @@ Tensor moe_dispatch(const Tensor& h, const Tensor& row_of_slot, const Tensor& sl
 Tensor moe_combine(const Tensor& y, const std::optional<Tensor>& weights, const Tensor& row_of_slot, const Tensor& slot_of_row,
                    int64_t tokens, int64_t top_k) {
   const Routing r{row_of_slot, slot_of_row, tokens, top_k};
+  expect_no_tangent(y, weights.value_or(y));
   std::optional<Tensor> w;
   if (weights) {
     Tensor t = weights->reshape({-1});
