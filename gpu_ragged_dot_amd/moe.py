@@ -20,6 +20,7 @@ from typing import NamedTuple, Optional
 
 import torch
 
+from . import _tracing
 from ._native import lib as _native
 
 __all__ = ["Routing", "route", "dispatch", "combine"]
@@ -36,6 +37,9 @@ class Routing(NamedTuple):
 def route(expert_ids: torch.Tensor, num_groups: int) -> Routing:
     """Stable counting sort of the (token, choice) pairs by expert id.  ``expert_ids`` is integer ``[tokens, top_k]``;
     ids outside ``[0, num_groups)`` mark dropped pairs."""
+    if _tracing.active():
+        outs = _tracing.record(lambda ids: _native.moe_route(ids, num_groups), expert_ids)
+        return Routing(*outs, *map(int, expert_ids.shape))
     group_sizes, row_of_slot, slot_of_row = _native.moe_route(expert_ids, num_groups)
     return Routing(group_sizes, row_of_slot, slot_of_row, *expert_ids.shape)
 
@@ -54,10 +58,16 @@ def _combine(y, r: Routing, weights):
 def dispatch(h: torch.Tensor, routing: Routing) -> torch.Tensor:
     """``x[row] = h[token of row]``: ``[tokens, d] -> [tokens * top_k, d]`` sorted by expert; rows past
     ``sum(group_sizes)`` are zero."""
+    if _tracing.active():
+        return _tracing.record(lambda *t: dispatch(t[0], routing._replace(row_of_slot=t[1], slot_of_row=t[2])),
+                               h, routing.row_of_slot, routing.slot_of_row)
     return _native.moe_dispatch(h, routing.row_of_slot, routing.slot_of_row, routing.tokens, routing.top_k)
 
 
 def combine(y: torch.Tensor, routing: Routing, weights: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``out[token] = sum_choice weights[token, choice] * y[row of (token, choice)]`` with fp32 accumulation;
     ``weights`` is ``[tokens, top_k]`` (None = 1)."""
+    if _tracing.active():
+        return _tracing.record(lambda *t: combine(t[0], routing._replace(row_of_slot=t[1], slot_of_row=t[2]), *t[3:]),
+                               y, routing.row_of_slot, routing.slot_of_row, *(() if weights is None else (weights,)))
     return _native.moe_combine(y, weights, routing.row_of_slot, routing.slot_of_row, routing.tokens, routing.top_k)

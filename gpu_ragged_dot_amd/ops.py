@@ -12,7 +12,7 @@ from typing import Optional
 
 import torch
 
-from . import _capi, planner
+from . import _capi, _tracing, planner
 from ._native import lib as _native
 from .planner import CHUNK_M, DEFAULT_BLOCK_K, DEFAULT_BLOCK_M, DEFAULT_BLOCK_N
 
@@ -90,9 +90,11 @@ def _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset
     code = _CODES.get((x.dtype, compute_dtype)) if acc_dtype is torch.float32 else None
     if code is None:
         code = _dtype_code(x, compute_dtype, acc_dtype)
-    if type(group_sizes) is not torch.Tensor:
-        group_sizes = torch.as_tensor(group_sizes)
-    return code, group_sizes, -1 if group_offset is None else _group_offset(group_offset)
+    return code, _sizes(group_sizes), -1 if group_offset is None else _group_offset(group_offset)
+
+
+def _sizes(group_sizes) -> torch.Tensor:
+    return group_sizes if isinstance(group_sizes, torch.Tensor) else torch.as_tensor(group_sizes)
 
 
 def _default_blocks(block_m, block_k, block_n) -> bool:
@@ -129,6 +131,9 @@ def _gmm(x, A, group_sizes, block_m, block_k, block_n, trans_rhs, interpret, com
 
     ``group_offset`` (jax.lax.ragged_dot's parameter; not in the reference): A holds the groups
     [group_offset, group_offset + A.shape[0]) of the ones group_sizes describes; rows of the others come out zero."""
+    if _tracing.active():
+        return _tracing.record(lambda x, A, gs: _gmm(x, A, gs, block_m, block_k, block_n, trans_rhs, interpret, compute_dtype,
+                                                     acc_dtype, chunk_m, plan, group_offset), x, A, _sizes(group_sizes))
     code, gs, g_first = _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset)
     assert A.ndim == 3 and x.ndim == 2, f"but {A.ndim=} {x.ndim=}"  # :188
     assert chunk_m >= 1 and (group_offset is None or g_first >= 0)
@@ -144,6 +149,10 @@ def _tgmm(x, y, group_sizes, block_m, block_k, block_n, interpret, compute_dtype
           plan: Optional[_capi.Plan] = None, group_offset=None, num_actual_groups=None) -> torch.Tensor:
     """gpu_ragged_dot.py:287-342 (_gpu_tgmm_fwd).  With ``group_offset`` / ``num_actual_groups`` only the slices of the
     groups [group_offset, group_offset + num_actual_groups) are computed: out[i] belongs to group group_offset + i."""
+    if _tracing.active():
+        return _tracing.record(lambda x, y, gs: _tgmm(x, y, gs, block_m, block_k, block_n, interpret, compute_dtype, acc_dtype,
+                                                      chunk_m, plan, group_offset, num_actual_groups),
+                               x, y, _sizes(group_sizes))
     del chunk_m  # :303
     code, gs, g_first = _host_args(x, group_sizes, interpret, compute_dtype, acc_dtype, group_offset)
     assert y.ndim == 2 and x.ndim == 2 and x.shape[0] == y.shape[0]  # :304

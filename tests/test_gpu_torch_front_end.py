@@ -1,0 +1,51 @@
+"""The torch front end's host path on real kernels: what a call under a trace, in a gradient or beside other threads does."""
+
+import pytest
+import torch
+
+import gpu_ragged_dot_amd as rd
+from gpu_ragged_dot_amd import moe
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer_inputs(seed):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16).requires_grad_()
+    return rand(40, 64), rand(5, 64, 96), rand(5, 96, 64), torch.rand((40, 2), generator=gen, device="cuda").requires_grad_(), \
+        torch.randint(5, (40, 2), generator=gen, device="cuda", dtype=torch.int32)
+
+
+def _layer(h, w_in, w_out, weights, ids):
+    r = moe.route(ids, 5)
+    hidden = torch.nn.functional.silu(rd.ragged_dot(moe.dispatch(h, r), w_in, r.group_sizes))
+    return moe.combine(rd.ragged_dot(hidden, w_out, r.group_sizes), r, weights)
+
+
+def test_a_traced_layer_runs_its_kernels():
+    """The traced layer gives the eager one's bits and gradients, on other inputs than the recorded ones."""
+    print("traced layer", flush=True)
+    traced = torch.jit.trace(_layer, _layer_inputs(0), check_trace=False)
+    for seed in (1, 2):
+        args = _layer_inputs(seed)
+        want, got = _layer(*args), traced(*args)
+        assert torch.equal(got, want)
+        dout = torch.randn_like(want)
+        for a, b in zip(*(torch.autograd.grad(y, args[:4], dout) for y in (got, want))):
+            assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(traced(*args), want)
+
+
+def test_a_traced_transposed_product_runs_its_kernel():
+    print("traced tgmm", flush=True)
+    gs = torch.tensor([5, 0, 11], dtype=torch.int32, device="cuda")
+    rand = lambda n: torch.randn((16, n), device="cuda").to(torch.bfloat16).requires_grad_()
+    call = lambda x, y: rd.tgmm(x, y, gs)
+    traced = torch.jit.trace(call, (rand(32), rand(24)), check_trace=False)
+    args = rand(32), rand(24)
+    want, got = call(*args), traced(*args)
+    assert torch.equal(got, want)
+    for a, b in zip(*(torch.autograd.grad(y, args, torch.ones_like(want)) for y in (got, want))):
+        assert torch.equal(a, b)

@@ -1,12 +1,14 @@
 """What the torch front end's host path decides before any kernel runs: operands it refuses, plans it picks, how it is
 loaded.  No GPU is needed; tensors are on the CPU, which the calls refuse last."""
 
+import ctypes
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
-from gpu_ragged_dot_amd import moe
+from gpu_ragged_dot_amd import moe, ops
 
 
 def _routing(tokens, top_k):
@@ -32,3 +34,51 @@ def test_forward_mode_tangents_are_refused(call, grad):
         }
         with pytest.raises(NotImplementedError, match="forward-mode"):
             calls[call]()
+
+
+class _HiddenKernels:
+    """Stands in for the native module on CPU tensors: its results are written behind torch's back, as a kernel writes them."""
+
+    @staticmethod
+    def _of(value):
+        out = torch.empty_like(value, requires_grad=False)
+        ctypes.memmove(out.data_ptr(), value.detach().contiguous().data_ptr(), value.numel() * value.element_size())
+        return out.requires_grad_(value.requires_grad)
+
+    def gmm(self, x, A, gs, *_):
+        return self._of(x @ A[0])
+
+    def tgmm(self, x, y, gs, *_):
+        return self._of((x.t() @ y)[None])
+
+    def moe_route(self, ids, groups):
+        return tuple(self._of(ids.flatten() + i) for i in range(3))
+
+    def moe_dispatch(self, h, *_):
+        return self._of(h * 3)
+
+    def moe_combine(self, y, weights, *_):
+        return self._of(y if weights is None else y * weights)
+
+
+@pytest.mark.parametrize("call", ["gmm", "tgmm", "route", "dispatch", "combine", "combine with weights"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_traces_record_the_call_and_not_its_allocation(call, grad, monkeypatch):
+    monkeypatch.setattr(ops, "_native", _HiddenKernels())
+    monkeypatch.setattr(moe, "_native", _HiddenKernels())
+    gs, r = torch.tensor([16], dtype=torch.int32), _routing(16, 1)
+    floats = lambda *shapes: [torch.randn(*s, requires_grad=grad) for s in shapes]
+    fn, inputs = {
+        "gmm": (lambda x, A: rd.gmm(x, A, gs), lambda: floats((16, 24), (1, 24, 8))),
+        "tgmm": (lambda x, y: rd.tgmm(x, y, gs), lambda: floats((16, 24), (16, 8))),
+        "route": (lambda ids: tuple(moe.route(ids, 4)[:3]), lambda: [torch.randint(4, (16, 1), dtype=torch.int32)]),
+        "dispatch": (lambda h: moe.dispatch(h, r), lambda: floats((16, 8))),
+        "combine": (lambda y: moe.combine(y, r), lambda: floats((16, 8))),
+        "combine with weights": (lambda y, w: moe.combine(y, r, w), lambda: floats((16, 8), (16, 1))),
+    }[call]
+    traced = torch.jit.trace(fn, tuple(inputs()), check_trace=False)
+    for _ in range(2):  # on other inputs than the recorded ones
+        args = inputs()
+        got, want = traced(*args), fn(*args)
+        for a, b in zip(*((t,) if isinstance(t, torch.Tensor) else t for t in (got, want))):
+            assert torch.equal(a, b)
