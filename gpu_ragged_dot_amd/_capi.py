@@ -78,6 +78,7 @@ EXPORTS = (
     "rd_last_error",
     "rd_num_variants",
     "rd_get_variant",
+    "rd_variant_takes",
     "rd_default_plan",
     "rd_sched_map",
     "rd_sched_map_len",
@@ -116,6 +117,8 @@ def _load() -> ctypes.CDLL:
     lib.rd_num_variants.restype = i
     lib.rd_get_variant.argtypes = [i, ctypes.POINTER(VariantInfo)]
     lib.rd_get_variant.restype = i
+    lib.rd_variant_takes.argtypes = [i, i, i, i, i, i]
+    lib.rd_variant_takes.restype = i
     lib.rd_default_plan.argtypes = [i, i, i, i, i, i, ctypes.POINTER(Plan)]
     lib.rd_default_plan.restype = i
     lib.rd_sched_map.argtypes = [vp, ip, i, i, i, ip, ip, ip, ip]

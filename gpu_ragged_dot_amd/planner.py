@@ -123,14 +123,14 @@ def select_plan(
         return _tuned_plan(entry)
     plan = _capi.default_plan(op, m, k, n, g)
     if explicit and not plan.decode_nb:
-        # explicit request: nearest compiled shape.  For tgmm the output tile is (block_k, block_n).
+        # explicit request: nearest compiled shape that takes this size.  For tgmm the output tile is (block_k, block_n).
         want_rows = block_k if op == _capi.OP_TGMM else block_m
         best, best_d = None, None
         for v in compiled_variants():
             if bool(v.vec) != vec or v.dtype != _capi.RD_DTYPE_BF16:
                 continue
             d = abs(math.log2(v.tile_m / max(want_rows, 1))) + abs(math.log2(v.tile_n / max(block_n, 1)))
-            if best_d is None or d < best_d:
+            if (best_d is None or d < best_d) and _capi.lib.rd_variant_takes(v.id, op, m, k, n, dtype) == _capi.RD_OK:
                 best, best_d = v.id, d
         if best is not None:
             plan.variant = best

@@ -97,6 +97,10 @@ const char* rd_last_error(void); /* host pointer, valid until the thread's next 
 
 int rd_num_variants(void);
 int rd_get_variant(int id, rd_variant_info* out /* host */);
+/* RD_OK if variant `id` computes product op (0 gmm, 1 gmm trans_rhs, 2 tgmm) of this size and type on 16-byte aligned
+ * buffers, else RD_ERR_UNSUPPORTED (why: rd_last_error()).  rd_variant_info does not say it all: the shapes for odd row
+ * pitches have limits of their own on k and n, and the direct-to-LDS ones on the extent of a tile's operands. */
+int rd_variant_takes(int id, int op, int m, int k, int n, int dtype);
 
 /* The library's own shape-based choice (what variant = -1 resolves to); op: 0 gmm, 1 gmm trans_rhs, 2 tgmm.
  * For op 0 with m <= 4 g (and m <= 1024, n <= 2048, min(g, m) * ceil(n / 256) <= 512) it selects the streaming kernel, which holds 4 rows of a group at a

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import _capi, ops
 from oracle import ragged_dot_oracle as oracle
 from tests import util
@@ -118,3 +119,28 @@ def test_float32_last_round_cut_along_k(vid, vname, k, trans_rhs):
         err = np.linalg.norm(y[:total] - ref[:total], axis=1) / np.linalg.norm(ref[:total], axis=1)
         assert err.max() < k * 2.0 ** -24, f"{err.max()} in row {err.argmax()}"  # k float32 additions
         assert not np.any(y[total:])
+
+
+@pytest.mark.parametrize("k,n", [(5, 16), (16, 3), (7, 100), (1, 1)])
+@pytest.mark.parametrize("blocks", [(128, 64, 128), (256, 256, 256)])
+@pytest.mark.parametrize("trans_rhs", [False, True])
+def test_explicit_blocks_on_rows_of_a_few_elements(k, n, blocks, trans_rhs):
+    """Explicit block sizes ask for a large tile; rows of fewer than 8 elements get the one that takes them, forward and in
+    both gradients."""
+    print(f"explicit blocks {blocks} k {k} n {n} trans_rhs {trans_rhs}", flush=True)
+    gs = np.array([20, 0, 37, 3], np.int32)
+    g, m = len(gs), int(gs.sum()) + 4
+    rng = np.random.default_rng(k * 100 + n)
+    r = lambda a: oracle.round_to(a, "bfloat16")
+    x, A, dy = r(rng.normal(size=(m, k))), r(rng.normal(size=(g, k, n))), r(rng.normal(size=(m, n)))
+    block_m, block_k, block_n = blocks
+    xt = util.bf16_dev(x).requires_grad_()
+    At = util.bf16_dev(np.ascontiguousarray(np.swapaxes(A, 1, 2)) if trans_rhs else A).requires_grad_()
+    y = rd.gmm(xt, At, torch.from_numpy(gs).cuda(), block_m=block_m, block_k=block_k, block_n=block_n, trans_rhs=trans_rhs)
+    dx, dA = torch.autograd.grad(y, (xt, At), util.bf16_dev(dy))
+    f64 = dict(out_dtype="float32", acc=np.float64)
+    dA = dA.transpose(1, 2) if trans_rhs else dA
+    for name, got, ref in (("y", y.detach(), oracle.gmm(x, A, gs, **f64)), ("dx", dx, oracle.gmm(dy, np.swapaxes(A, 1, 2), gs, **f64)),
+                           ("dA", dA, oracle.tgmm(x, dy, gs, **f64))):
+        # one rounding to a significand of 8 bits on top of float32 sums
+        assert np.linalg.norm(util.to_np(got) - ref) <= 2.0 ** -8 * np.linalg.norm(ref), name

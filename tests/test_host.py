@@ -111,6 +111,33 @@ def test_planner_block_rules_match_the_oracle():
         assert planner.normalize_tgmm_blocks(*args) == oracle.tgmm_block_sizes(*args)
 
 
+@pytest.mark.parametrize("op", [_capi.OP_GMM, _capi.OP_GMM_TRANS, _capi.OP_TGMM])
+@pytest.mark.parametrize("block", [16, 64, 128, 256])
+def test_explicit_blocks_pick_a_shape_that_takes_the_call(op, block):
+    """Whatever the block sizes ask for, the product runs: down to rows of one element, and up to rows whose tiles exceed
+    what the large shapes address."""
+    wide = (1 << 22) + 1
+    sizes = [(64, k, n) for k in (*range(1, 10), 100, 1001) for n in (*range(1, 10), 100, 1001)]
+    sizes += [(64, wide, 3), (64, 3, wide), (64, wide, 9), (1 << 20, 4096, 4096), (64, 1 << 22, 64), (64, 64, 1 << 22)]
+    for m, k, n in sizes:
+        for block_m, block_k, block_n in ((block, block, 128), (block, block, block), (128, block, 64)):
+            if (block_m, block_k, block_n) == (64, 64, 64):
+                continue
+            p = planner.select_plan(op, m, k, n, 4, block_m, block_k, block_n)
+            assert _capi.lib.rd_variant_takes(p.variant, op, m, k, n, _capi.RD_DTYPE_BF16) == _capi.RD_OK, (m, k, n, block)
+    # the limits themselves, as the entry points report them (no launch: the workspace is too small for any)
+    one = ctypes.c_void_p(16)
+    for v in _capi.variants():
+        for m, k, n in ((64, 5, 16), (64, 16, 24), (64, 8, 8), (64, 1001, 1515)):
+            plan = ctypes.byref(_capi.Plan(v.id))
+            takes = _capi.lib.rd_variant_takes(v.id, op, m, k, n, v.dtype)
+            if op == _capi.OP_TGMM:
+                rc = _capi.lib.rd_tgmm(None, one, one, one, one, m, k, n, 4, v.dtype, plan, one, 8)
+            else:
+                rc = _capi.lib.rd_gmm(None, one, one, one, one, m, k, n, 4, op, v.dtype, plan, one, 8)
+            assert rc == (_capi.RD_ERR_WORKSPACE if takes == _capi.RD_OK else takes), (v.name, m, k, n)
+
+
 def test_planner_choices():
     vs = {v.id: v for v in _capi.variants()}
     p = planner.select_plan(_capi.OP_GMM, 171, 58, 77, 8)
