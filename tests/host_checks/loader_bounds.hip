@@ -14,12 +14,20 @@
 //     the tile's limit, contraction index below the contraction length and inside the slab being loaded;
 //   * every element of the window that belongs to the slab is read exactly once (nothing missing, nothing twice);
 //   * every offset is 16-byte aligned and non-negative.
+//
+// Second part: the loaders of the any-pitch core (RsLoader in gpu_ragged_dot_amd/csrc/rd_gemm_rs.h), whose loads have no
+// range check of the hardware behind them.  Same invariant - the loads of slab s are issued with the loader advanced s times,
+// here up to kBehind slabs past the last one - on operands that are the whole of their memory: no row in front of the tile's
+// first one or behind its last, except what a cut along K leaves on either side.  Every 16-byte piece must lie inside that
+// memory, and what trim() and the place in LDS make of it must be, for every row or column below the tile's limit, the
+// element of that place, or zero behind the contraction length; every place of a slab is written exactly once.
 // Prints "loader_bounds ok <loads checked>" and returns 0, or the first violation and 1.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
 
 #include "rd_gemm_dlds.h"
+#include "rd_gemm_rs.h"
 
 using namespace rd;
 
@@ -111,6 +119,98 @@ static bool check_loader(const char* what) {
   return true;
 }
 
+constexpr int kBehind = 5;  // rs_kloop asks for slab t + 4 in slab t, and an odd number of slabs is rounded up
+
+// A tile at element (0, c0) of a matrix of pitch ld.  K-major: lim rows, contraction indices c0 .. c0 + klen - 1 of each.
+// MN-major: klen rows, columns c0 .. c0 + lim - 1 of each.  The memory ends with the matrix's last row.
+template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB>
+static bool check_rs_window(int lim, int ld, int c0, int klen) {
+  constexpr int NW = 4;
+  typedef RsLoader<T, BK, NW, KMAJOR, Src, VEC, LB> Ld;
+  constexpr int EPP = Ld::EPP;
+  const int nk = (klen + BK - 1) / BK;
+  const long long memory = (long long)(KMAJOR ? lim : klen) * ld;
+  const uintptr_t origin = (uintptr_t)1 << 40;
+  auto fail = [&](const char* what, int s, int w, int l, int j, long long at) {
+    std::printf("any-pitch core: T=%d BK=%d kmajor=%d elem=%d lds=%d vec=%d lim=%d ld=%d c0=%d klen=%d slab %d wave %d lane %d "
+                "piece %d: %s (%lld)\n", T, BK, (int)KMAJOR, (int)sizeof(Src), LB, (int)VEC, lim, ld, c0, klen, s, w, l, j, what, at);
+    return false;
+  };
+  std::vector<Ld> all((size_t)NW * 64);
+  for (int w = 0; w < NW; ++w)
+    for (int l = 0; l < 64; ++l) all[(size_t)w * 64 + l].init(reinterpret_cast<const Src*>(origin) + c0, ld, lim, klen, w, l);
+  constexpr int PIECE = EPP * LB;  // bytes of a piece in LDS
+  std::vector<unsigned char> placed, written;
+  for (int s = 0; s < nk + kBehind; ++s) {
+    placed.assign((size_t)(KMAJOR ? T : BK) * Ld::PPR, 0);
+    written.assign((size_t)T * BK * LB / PIECE, 0);
+    for (int w = 0; w < NW; ++w)
+      for (int l = 0; l < 64; ++l) {
+        const Ld& L = all[(size_t)w * 64 + l];
+        for (int j = 0; j < Ld::PER; ++j) {
+          ++g_loads;
+          const long long byte = (long long)(reinterpret_cast<uintptr_t>(L.base) - origin) + L.offset(j);
+          if (byte % (int)sizeof(Src) != 0) return fail("address inside an element", s, w, l, j, byte);
+          const long long first = byte / (int)sizeof(Src);  // of EPP elements, from the matrix's origin
+          if (byte < 0 || first + EPP > memory) return fail("load leaves the operand", s, w, l, j, first);
+          const int row = Ld::slab_row(w, l, j), piece = l % Ld::PPR;
+          if (placed[(size_t)row * Ld::PPR + piece]++) return fail("place taken twice", s, w, l, j, row);
+          const int at = L.lds + j * Ld::LDS_STEP;
+          if (at < 0 || at % PIECE != 0 || at / PIECE >= (int)written.size() || written[at / PIECE]++)
+            return fail("place in LDS", s, w, l, j, at);
+          const int down = s >= nk - 1 ? L.surplus(w, l, j, s) : 0;
+          if (down < 0) return fail("negative shift", s, w, l, j, down);
+          for (int e = 0; e < EPP; ++e) {
+            long long got = -1;  // -1: zero
+            if (VEC ? down == 0 : e + down < EPP) got = first + e + down;
+            const int kk = s * BK + (KMAJOR ? piece * EPP + e : row), mn = KMAJOR ? row : piece * EPP + e;
+            if (mn >= lim) continue;
+            const long long want = kk >= klen ? -1 : KMAJOR ? (long long)mn * ld + c0 + kk : (long long)kk * ld + c0 + mn;
+            if (got != want) return fail("wrong element", s, w, l, j, got);
+          }
+        }
+      }
+    for (size_t i = 0; i < placed.size(); ++i)
+      if (!placed[i]) return fail("place never written", s, 0, 0, 0, (long long)i);
+    for (auto& L : all)
+      L.next((int)((&L - all.data()) / 64), (int)((&L - all.data()) % 64));
+  }
+  return true;
+}
+
+template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB = 2>
+static bool check_rs_loader() {
+  std::vector<int> lims, klens;
+  for (int lim : {1, 2, 3, 5, 7, 8, 9, 16, 31, 33, 63, 64, 65, 72, 100, 127, 128, 129, 190, 192, 200, 249, 255, 256})
+    if (lim <= T) lims.push_back(lim);
+  for (int klen : {1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 24, 31, 32, 33, 40, 57, 63, 64, 65, 72, 95, 96, 97, 127, 128, 129, 136, 191, 192, 193, 200, 257, 333})
+    klens.push_back(klen);
+  const int widest = (1 << 30) / (512 * (int)sizeof(Src) / 2) - 8;  // 256 rows stay below 2 GiB
+  for (int lim : lims)
+    for (int klen : klens) {
+      if constexpr (KMAJOR) {
+        if (VEC && klen % 8 != 0) continue;
+        if (klen >= 8 && !check_rs_window<T, BK, true, Src, VEC, LB>(lim, klen, 0, klen)) return false;  // whole rows
+        // pieces of a cut along K: they start at multiples of 64 and end at one, or with the row
+        for (int c0 : {64, 192})
+          for (int behind : {0, 64}) {
+            if (behind && klen % 64 != 0) continue;
+            if (!check_rs_window<T, BK, true, Src, VEC, LB>(lim, c0 + klen + behind, c0, klen)) return false;
+          }
+        if (klen % 64 == 0 && (!check_rs_window<T, BK, true, Src, VEC, LB>(lim, klen + 64, 0, klen) ||
+                               !check_rs_window<T, BK, true, Src, VEC, LB>(lim, widest, 64, klen))) return false;
+      } else {
+        if (VEC && lim % 8 != 0) continue;
+        // the tile that holds the last columns, of one tile's columns and of several, and one with more behind it
+        if (lim >= 8 && !check_rs_window<T, BK, false, Src, VEC, LB>(lim, lim, 0, klen)) return false;
+        if (!check_rs_window<T, BK, false, Src, VEC, LB>(lim, T + lim, T, klen)) return false;
+        if (lim == T && (!check_rs_window<T, BK, false, Src, VEC, LB>(lim, 2 * T + 24, T, klen) ||
+                         !check_rs_window<T, BK, false, Src, VEC, LB>(lim, widest, 0, klen))) return false;
+      }
+    }
+  return true;
+}
+
 int main() {
   bool ok = true;
   // (tile extent, slab depth, waves, K-major): the loader shapes of the compiled cores
@@ -127,6 +227,19 @@ int main() {
   ok = ok && check_loader<64, 32, 4, true>("64-row streaming routine, activations (32-wide slabs)");
   ok = ok && check_loader<64, 64, 4, true>("64-row streaming routine, activations (64-wide slabs)");
   ok = ok && check_loader<128, 64, 4, true>("128-row streaming routine, activations (64-wide slabs)");
+  // the any-pitch core's: 16-bit elements, float32 rounded to bf16 at 16-byte pitches and at any, float32 as it is; the row
+  // tiles' heights, and the column tiles
+  ok = ok && check_rs_loader<64, 64, true, bf16_bits, false>() && check_rs_loader<128, 64, true, bf16_bits, false>() &&
+       check_rs_loader<192, 64, true, bf16_bits, false>() && check_rs_loader<256, 64, true, bf16_bits, false>() &&
+       check_rs_loader<128, 64, false, bf16_bits, false>() && check_rs_loader<256, 64, false, bf16_bits, false>();
+  ok = ok && check_rs_loader<64, 32, true, float, true>() && check_rs_loader<128, 32, true, float, true>() &&
+       check_rs_loader<192, 32, true, float, true>() && check_rs_loader<256, 32, true, float, true>() &&
+       check_rs_loader<128, 32, false, float, true>() && check_rs_loader<256, 32, false, float, true>();
+  ok = ok && check_rs_loader<64, 32, true, float, false>() && check_rs_loader<128, 32, true, float, false>() &&
+       check_rs_loader<192, 32, true, float, false>() && check_rs_loader<256, 32, true, float, false>() &&
+       check_rs_loader<128, 32, false, float, false>() && check_rs_loader<256, 32, false, float, false>();
+  ok = ok && check_rs_loader<64, 32, true, float, false, 4>() && check_rs_loader<128, 32, true, float, false, 4>() &&
+       check_rs_loader<64, 32, false, float, false, 4>() && check_rs_loader<128, 32, false, float, false, 4>();
   if (!ok) return 1;
   std::printf("loader_bounds ok %lld\n", g_loads);
   return 0;

@@ -2,7 +2,9 @@
 (tests/host_checks/loader_bounds.hip, built by the library's Makefile without any GPU code).  Every large-tile core
 addresses its operands through these loaders, the register-staged core with plain buffer loads: every load of every
 slab must stay inside the operand's window, and the window must be covered exactly once, for ragged limits and
-contraction tails at the benchmark shapes' pitches.  Likewise the rule that deals the blocks of long groups among those
+contraction tails at the benchmark shapes' pitches.  The loaders of the any-pitch core, which have no range check of the
+hardware behind them, are walked on operands that are the whole of their memory, slabs behind the last one and pieces of a
+cut along K included.  Likewise the rule that deals the blocks of long groups among those
 of short groups in a gmm launch (tests/host_checks/block_order.hip): every block dealt once, evenly over the XCDs and
 over the launch."""
 
@@ -21,7 +23,7 @@ def test_operand_loaders_stay_inside_their_windows():
     assert r.returncode == 0, r.stdout + r.stderr
     r = subprocess.run([EXE], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
-    assert r.stdout.startswith("loader_bounds ok ") and int(r.stdout.split()[2]) > 10_000_000
+    assert r.stdout.startswith("loader_bounds ok ") and int(r.stdout.split()[2]) > 300_000_000
 
 
 def test_interleaved_block_order_deals_every_block_once_and_evenly():
