@@ -81,6 +81,26 @@ def test_noalloc_float32_arrays():
             assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("with_plan", [False, True])
+def test_noalloc_never_cuts_along_k(with_plan):
+    """float32 contractions that rd_gmm cuts, on every float32 tile with a cut (the smallest one's partial sums are about the
+    size of the scratch buffer): the uncut launch's bits."""
+    k, n, g = 2048, 192, 3
+    gs = np.array([70, 0, 130], np.int32)
+    m = int(gs.sum()) + 5
+    rng = np.random.default_rng(k)
+    x, A = (torch.from_numpy(rng.normal(size=s).astype(np.float32)).cuda() for s in ((m, k), (g, k, n)))
+    gs_d = torch.from_numpy(gs).cuda()
+    default = _capi.default_plan(_capi.OP_GMM, m, k, n, g, _capi.RD_DTYPE_F32).variant
+    for vid in [v.id for v in _capi.variants() if v.name.decode().startswith("fr")] if with_plan else [default]:
+        print(f"noalloc float32 k={k} variant {vid} with_plan={with_plan}", flush=True)
+        whole, cut = _capi.Plan(vid, split_k=-1), _capi.Plan(vid)
+        uncut, got = _run_both(x, A, gs_d, m, k, n, g, False, _capi.RD_DTYPE_F32, whole, torch.float32)
+        pieces, again = _run_both(x, A, gs_d, m, k, n, g, False, _capi.RD_DTYPE_F32, cut if with_plan else None, torch.float32)
+        assert torch.equal(got, uncut) and torch.equal(again, uncut)
+        assert not torch.equal(pieces, uncut)
+
+
 def test_noalloc_float8_operands():
     """float8 e4m3fn operands (bf16 out): the float8 matrix-core tiles in both weight layouts, and the streaming kernel
     for weights stored [g, n, k] (the default plan's choice for one row per group)."""
