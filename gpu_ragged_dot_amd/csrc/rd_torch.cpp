@@ -59,9 +59,10 @@ rd_plan pick_plan(int op, int64_t m, int64_t k, int64_t n, int64_t g, int code, 
   return p;
 }
 
-// The plans of a call that does not leave them to the library: of the product, and of its two gradients.
+// The plans of a call that does not leave them to the library: of the product, and of its two gradients where the caller has
+// chosen those too (a plan for the product says nothing about the others).
 struct Plans {
-  bool given = false;
+  size_t given = 0;
   rd_plan p[3];
 };
 rd_plan plan_from(py::handle h) {
@@ -71,10 +72,8 @@ rd_plan plan_from(py::handle h) {
 Plans plans_from(const py::object& o) {
   Plans r;
   if (o.is_none()) return r;
-  r.given = true;
   const auto t = py::cast<py::tuple>(o);
-  for (size_t i = 0; i < 3 && i < t.size(); ++i) r.p[i] = plan_from(t[i]);
-  for (size_t i = t.size(); i < 3; ++i) r.p[i] = r.p[0];
+  for (; r.given < 3 && r.given < t.size(); ++r.given) r.p[r.given] = plan_from(t[r.given]);
   return r;
 }
 
@@ -115,7 +114,7 @@ struct Call {
 };
 
 // gpu_ragged_dot.py:171-228 (_gpu_gmm_fwd)
-Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const Call& c, int which, bool trans) {
+Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const Call& c, size_t which, bool trans) {
   expect(A_.dim() == 3 && x_.dim() == 2, "x must be [m, k] and A [g, k, n]");  // :188
   same_type(x_, A_);
   expect(gs_.dim() == 1, "group_sizes must have one dimension");
@@ -130,7 +129,7 @@ Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const 
   Tensor y = at::empty({m, n}, x.options().dtype(out_type(x)).requires_grad(false));  // :210
   const bool aligned = aligned16(x) && aligned16(A) && aligned16(y);
   rd_plan p;
-  if (c.plans.given && (which == 0 || aligned || c.code == RD_DTYPE_F32)) p = c.plans.p[which];
+  if (which < c.plans.given && (which == 0 || aligned || c.code == RD_DTYPE_F32)) p = c.plans.p[which];
   else p = pick_plan(trans ? kOpGmmTrans : kOpGmm, m, k, n, g, c.code, aligned);
   if (g_first != 0 || g_local != g) p.decode_nb = 0;  // streaming kernels: all groups only
   const Tensor ws = scratch(rd_gmm_workspace_bytes((int)m, (int)g, &p), dev);
@@ -140,7 +139,7 @@ Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const 
 }
 
 // gpu_ragged_dot.py:287-342 (_gpu_tgmm_fwd)
-Tensor tgmm_forward(const Tensor& x_, const Tensor& y_, const Tensor& gs_, const Call& c, int which, int64_t g_local) {
+Tensor tgmm_forward(const Tensor& x_, const Tensor& y_, const Tensor& gs_, const Call& c, size_t which, int64_t g_local) {
   expect(y_.dim() == 2 && x_.dim() == 2 && x_.size(0) == y_.size(0), "x must be [m, k] and y [m, n]");  // :304
   same_type(x_, y_);
   const int64_t m = x_.size(0), k = x_.size(1), n = y_.size(1), g = gs_.numel(), g_first = c.g_first < 0 ? 0 : c.g_first;
@@ -153,7 +152,7 @@ Tensor tgmm_forward(const Tensor& x_, const Tensor& y_, const Tensor& gs_, const
   Tensor out = at::empty({g_local, k, n}, x.options().dtype(out_type(x)).requires_grad(false));  // :324
   const bool aligned = aligned16(x) && aligned16(y) && aligned16(out);
   rd_plan p;
-  if (c.plans.given && (which == 0 || aligned || c.code == RD_DTYPE_F32)) p = c.plans.p[which];
+  if (which < c.plans.given && (which == 0 || aligned || c.code == RD_DTYPE_F32)) p = c.plans.p[which];
   else p = pick_plan(kOpTgmm, m, k, n, g, c.code, aligned);
   const Tensor ws = scratch(rd_tgmm_workspace_bytes((int)m, (int)g, &p), dev);
   check(rd_tgmm_sharded(stream_of(dev), x.const_data_ptr(), y.const_data_ptr(), gs.const_data_ptr<int32_t>(), out.mutable_data_ptr(),

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import gpu_ragged_dot_amd as rd
-from gpu_ragged_dot_amd import moe
+from gpu_ragged_dot_amd import _capi, moe, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +49,24 @@ def test_a_traced_transposed_product_runs_its_kernel():
     assert torch.equal(got, want)
     for a, b in zip(*(torch.autograd.grad(y, args, torch.ones_like(want)) for y in (got, want))):
         assert torch.equal(a, b)
+
+
+HP = dict(block_m=64, block_k=64, block_n=64, interpret=False, compute_dtype=None, acc_dtype=torch.float32, chunk_m=512)
+
+
+def test_a_plan_for_the_product_leaves_its_gradients_to_the_library():
+    """float32, contractions that are cut along K by default: a plan that forbids the cut holds for the product it is given to."""
+    gs = torch.tensor([70, 0, 130], dtype=torch.int32, device="cuda")
+    vid = [v.id for v in _capi.variants() if v.name.decode().startswith("fr64x64")][0]
+    plan = _capi.Plan(vid, split_k=-1)
+    for call, default, shapes in (
+            (lambda x, A: ops._gmm(x, A, gs, **HP, trans_rhs=False, plan=plan), lambda x, A: rd.gmm(x, A, gs), ((200, 192), (3, 192, 2048))),
+            (lambda x, y: ops._tgmm(x, y, gs, **HP, plan=plan), lambda x, y: rd.tgmm(x, y, gs), ((200, 192), (200, 2048)))):
+        print(f"gradients beside a plan, {shapes}", flush=True)
+        args = [torch.randn(*s, device="cuda", requires_grad=True) for s in shapes]
+        out = call(*args)
+        dout = torch.randn_like(out)
+        got, want = (torch.autograd.grad(y, args, dout) for y in (out, default(*args)))
+        uncut = ops._gmm_fwd(*((dout, args[1]) if out.dim() == 2 else (args[1], dout)), gs, **HP, trans_rhs=True, plan=plan)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        assert not torch.equal(got[0], uncut)
