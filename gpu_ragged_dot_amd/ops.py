@@ -74,8 +74,8 @@ def _group_offset(group_offset) -> int:
 
 def _aligned16(*tensors: torch.Tensor) -> bool:
     """The fast tile shapes move 16 bytes at a time: every buffer must start on a 16-byte boundary (a view at an odd
-    element offset does not, however contiguous it is)."""
-    return all(t.data_ptr() % 16 == 0 for t in tensors)
+    element offset does not, however contiguous it is; what is not contiguous is copied to one that does)."""
+    return all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in tensors)
 
 
 def _fields(plan: _capi.Plan) -> tuple:
@@ -101,17 +101,20 @@ def _default_blocks(block_m, block_k, block_n) -> bool:
     return block_m == DEFAULT_BLOCK_M and block_k == DEFAULT_BLOCK_K and block_n == DEFAULT_BLOCK_N
 
 
+def _select(products, blocks, aligned, operands) -> tuple:
+    """Plans of a product, the first of ``products``, and of its gradients if an operand asks for them."""
+    wanted = products if torch.is_grad_enabled() and any(t.requires_grad for t in operands) else products[:1]
+    return tuple(_fields(planner.select_plan(*p, aligned=aligned or i > 0, **blocks)) for i, p in enumerate(wanted))
+
+
 def _gmm_plans(x, A, trans_rhs, g, code, block_m, block_k, block_n):
-    """Plans of the product and of its two gradients for explicit block sizes (gpu_ragged_dot.py:194-197)."""
+    """Plans for explicit block sizes (gpu_ragged_dot.py:194-197)."""
     (m, k), n = x.shape, A.shape[-2 if trans_rhs else -1]
     planner.normalize_gmm_blocks(block_m, block_k, block_n, m, k, n)  # validates the request
     blocks = dict(block_m=block_m, block_k=block_k, block_n=block_n, dtype=code)
     fwd, bwd = (_capi.OP_GMM_TRANS, _capi.OP_GMM) if trans_rhs else (_capi.OP_GMM, _capi.OP_GMM_TRANS)
     weights = (n, k) if trans_rhs else (k, n)
-    return tuple(_fields(p) for p in (
-        planner.select_plan(fwd, m, k, n, g, aligned=_aligned16(x, A), **blocks),
-        planner.select_plan(bwd, m, n, k, g, **blocks),
-        planner.select_plan(_capi.OP_TGMM, m, *weights, g, **blocks)))
+    return _select(((fwd, m, k, n, g), (bwd, m, n, k, g), (_capi.OP_TGMM, m, *weights, g)), blocks, _aligned16(x, A), (x, A))
 
 
 def _tgmm_plans(x, y, g, code, block_m, block_k, block_n):
@@ -119,10 +122,8 @@ def _tgmm_plans(x, y, g, code, block_m, block_k, block_n):
     (m, k), n = x.shape, y.shape[-1]
     planner.normalize_tgmm_blocks(block_m, block_k, block_n, m, k, n)
     blocks = dict(block_m=block_m, block_k=block_k, block_n=block_n, dtype=code)
-    return tuple(_fields(p) for p in (
-        planner.select_plan(_capi.OP_TGMM, m, k, n, g, aligned=_aligned16(x, y), **blocks),
-        planner.select_plan(_capi.OP_GMM_TRANS, m, n, k, g, **blocks),
-        planner.select_plan(_capi.OP_GMM, m, k, n, g, **blocks)))
+    return _select(((_capi.OP_TGMM, m, k, n, g), (_capi.OP_GMM_TRANS, m, n, k, g), (_capi.OP_GMM, m, k, n, g)), blocks,
+                   _aligned16(x, y), (x, y))
 
 
 def _gmm(x, A, group_sizes, block_m, block_k, block_n, trans_rhs, interpret, compute_dtype, acc_dtype, chunk_m,

@@ -2,13 +2,14 @@
 loaded.  No GPU is needed; tensors are on the CPU, which the calls refuse last."""
 
 import ctypes
+import types
 
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
-from gpu_ragged_dot_amd import moe, ops
+from gpu_ragged_dot_amd import moe, ops, planner
 
 
 def _routing(tokens, top_k):
@@ -82,3 +83,29 @@ def test_traces_record_the_call_and_not_its_allocation(call, grad, monkeypatch):
         got, want = traced(*args), fn(*args)
         for a, b in zip(*((t,) if isinstance(t, torch.Tensor) else t for t in (got, want))):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("op", ["gmm", "gmm trans_rhs", "tgmm"])
+def test_explicit_blocks_plan_what_the_call_computes(op, monkeypatch):
+    """One plan for a product alone, three where an operand asks for a gradient; an operand that is copied because of its
+    strides does not count as one at an odd address."""
+    asked, handed = [], []
+    real = planner.select_plan
+    monkeypatch.setattr(planner, "select_plan", lambda *a, **kw: (asked.append((a, kw)), real(*a, **kw))[1])
+    native = types.SimpleNamespace(gmm=lambda *a: handed.append(a[-1]), tgmm=lambda *a: handed.append(a[-1]))
+    monkeypatch.setattr(ops, "_native", native)
+    gs = torch.tensor([64, 64], dtype=torch.int32)
+    blocks = dict(block_m=128, block_k=128, block_n=128)
+    bf16 = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    call = {"gmm": lambda x, o: rd.gmm(x, o(2, 64, 64), gs, **blocks), "gmm trans_rhs": lambda x, o: rd.gmm(x, o(2, 64, 64), gs, trans_rhs=True, **blocks),
+            "tgmm": lambda x, o: rd.tgmm(x, o(128, 64), gs, **blocks)}[op]
+    call(bf16(128, 64), bf16)
+    call(bf16(128, 64), lambda *s: bf16(*s).requires_grad_())
+    with torch.no_grad():
+        call(bf16(128, 64), lambda *s: bf16(*s).requires_grad_())
+    assert [len(p) for p in handed] == [1, 3, 1] and len(asked) == 5
+    assert all(kw["aligned"] for _, kw in asked) and all(p[0] == handed[0][0] for p in handed)
+    del asked[:], handed[:]
+    call(bf16(128, 72)[:, 1:65], bf16)  # strided, at an odd element: a copy is multiplied
+    call(bf16(128 * 64 + 1)[1:].view(128, 64), bf16)  # contiguous, at an odd element
+    assert [kw["aligned"] for _, kw in asked] == [True, False]
