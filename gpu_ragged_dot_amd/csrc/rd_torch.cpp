@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -22,6 +23,8 @@
 
 namespace py = pybind11;
 using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
 
 namespace {
 
@@ -38,6 +41,39 @@ void check(int status) {
 }
 void expect(bool ok, const char* what) {
   if (!ok) throw CheckError(what);
+}
+
+void set_python_error(const StatusError& e) {
+  const py::object cls = py::module_::import("gpu_ragged_dot_amd._capi").attr("RaggedDotError");
+  PyErr_SetObject(cls.ptr(), cls(e.status, e.what()).ptr());
+}
+void set_python_error(const CheckError& e) { PyErr_SetString(PyExc_AssertionError, e.what()); }
+void set_python_error(const py::builtin_exception& e) { e.set_error(); }
+
+// The body of an autograd node's backward.  Its errors leave through torch's engine, possibly on a thread of its own, which
+// hands on Python errors as they are and makes a RuntimeError of what it does not know: here they become the Python errors
+// that the module's entry points raise.
+template <class E>
+[[noreturn]] void throw_python_error(const E& cause) {
+  python_error e;
+  {
+    const py::gil_scoped_acquire gil;
+    set_python_error(cause);
+    e.persist();
+  }
+  throw e;
+}
+template <class F>
+variable_list in_backward(F&& body) {
+  try {
+    return body();
+  } catch (const StatusError& e) {
+    throw_python_error(e);
+  } catch (const CheckError& e) {
+    throw_python_error(e);
+  } catch (const py::builtin_exception& e) {
+    throw_python_error(e);
+  }
 }
 
 // ---- plans -------------------------------------------------------------------------------------------------------------
@@ -164,8 +200,6 @@ struct CallHolder : torch::CustomClassHolder {
   Call c;
   explicit CallHolder(const Call& call) : c(call) {}
 };
-using torch::autograd::AutogradContext;
-using torch::autograd::variable_list;
 Call call_of(AutogradContext* ctx) { return static_cast<CallHolder*>(ctx->saved_data["call"].toCapsule().get())->c; }
 
 // The custom VJP of gpu_ragged_dot.py:360-405.
@@ -177,14 +211,16 @@ struct GmmNode : torch::autograd::Function<GmmNode> {
     return gmm_forward(x, A, sizes, c, 0, c.trans);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto saved = ctx->get_saved_variables();
-    const Call c = call_of(ctx);
-    const Tensor &x = saved[0], &A = saved[1], &gs = saved[2];
-    const Tensor dy = grads[0].contiguous();
-    Tensor dx, dA;
-    if (ctx->needs_input_grad(0)) dx = gmm_forward(dy, A, gs, c, 1, !c.trans);  // :400
-    if (ctx->needs_input_grad(1)) dA = c.trans ? tgmm_forward(dy, x, gs, c, 2, A.size(0)) : tgmm_forward(x, dy, gs, c, 2, A.size(0));  // :401
-    return {dx, dA, Tensor(), Tensor()};  // group_sizes gets no cotangent, :402
+    return in_backward([&]() -> variable_list {
+      const auto saved = ctx->get_saved_variables();
+      const Call c = call_of(ctx);
+      const Tensor &x = saved[0], &A = saved[1], &gs = saved[2];
+      const Tensor dy = grads[0].contiguous();
+      Tensor dx, dA;
+      if (ctx->needs_input_grad(0)) dx = gmm_forward(dy, A, gs, c, 1, !c.trans);  // :400
+      if (ctx->needs_input_grad(1)) dA = c.trans ? tgmm_forward(dy, x, gs, c, 2, A.size(0)) : tgmm_forward(x, dy, gs, c, 2, A.size(0));  // :401
+      return {dx, dA, Tensor(), Tensor()};  // group_sizes gets no cotangent, :402
+    });
   }
 };
 
@@ -197,13 +233,15 @@ struct TgmmNode : torch::autograd::Function<TgmmNode> {
     return tgmm_forward(x, y, sizes, c, 0, c.g_local);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto saved = ctx->get_saved_variables();
-    const Call c = call_of(ctx);
-    const Tensor dA = grads[0].contiguous();
-    Tensor dx, dy;
-    if (ctx->needs_input_grad(0)) dx = gmm_forward(saved[1], dA, saved[2], c, 1, true);
-    if (ctx->needs_input_grad(1)) dy = gmm_forward(saved[0], dA, saved[2], c, 2, false);
-    return {dx, dy, Tensor(), Tensor()};
+    return in_backward([&]() -> variable_list {
+      const auto saved = ctx->get_saved_variables();
+      const Call c = call_of(ctx);
+      const Tensor dA = grads[0].contiguous();
+      Tensor dx, dy;
+      if (ctx->needs_input_grad(0)) dx = gmm_forward(saved[1], dA, saved[2], c, 1, true);
+      if (ctx->needs_input_grad(1)) dy = gmm_forward(saved[0], dA, saved[2], c, 2, false);
+      return {dx, dy, Tensor(), Tensor()};
+    });
   }
 };
 
@@ -319,7 +357,9 @@ struct DispatchNode : torch::autograd::Function<DispatchNode> {
     return dispatch_rows(h, r, Tensor());
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    return {combine_rows(grads[0], routing_of(ctx), Tensor()), Tensor()};  // each token collects the gradients of its rows
+    return in_backward([&]() -> variable_list {
+      return {combine_rows(grads[0], routing_of(ctx), Tensor()), Tensor()};  // each token collects the gradients of its rows
+    });
   }
 };
 
@@ -331,13 +371,15 @@ struct CombineNode : torch::autograd::Function<CombineNode> {
     return combine_rows(y, r, w);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const auto s = ctx->get_saved_variables();
-    const Routing r = routing_of(ctx);
-    const Tensor &y = s[0], &w = s[1], &dout = grads[0];
-    Tensor dy, dw;
-    if (ctx->needs_input_grad(0)) dy = dispatch_rows(dout, r, w);  // dy[row] = weight of the row's slot * dout[token]
-    if (w.defined() && ctx->needs_input_grad(1)) dw = combine_wgrad(y, dout, r);
-    return {dy, dw, Tensor()};
+    return in_backward([&]() -> variable_list {
+      const auto s = ctx->get_saved_variables();
+      const Routing r = routing_of(ctx);
+      const Tensor &y = s[0], &w = s[1], &dout = grads[0];
+      Tensor dy, dw;
+      if (ctx->needs_input_grad(0)) dy = dispatch_rows(dout, r, w);  // dy[row] = weight of the row's slot * dout[token]
+      if (w.defined() && ctx->needs_input_grad(1)) dw = combine_wgrad(y, dout, r);
+      return {dy, dw, Tensor()};
+    });
   }
 };
 
@@ -370,10 +412,9 @@ PYBIND11_MODULE(_rd_torch, mod) {
     try {
       if (p) std::rethrow_exception(p);
     } catch (const StatusError& e) {
-      const py::object cls = py::module_::import("gpu_ragged_dot_amd._capi").attr("RaggedDotError");
-      PyErr_SetObject(cls.ptr(), cls(e.status, e.what()).ptr());
+      set_python_error(e);
     } catch (const CheckError& e) {
-      PyErr_SetString(PyExc_AssertionError, e.what());
+      set_python_error(e);
     }
   });
   mod.def("set_tuned_plans", [](const py::list& entries) {  // [((op, m, k, n, g), (variant, group_m, group_n, decode_nb, split_k)), ...]

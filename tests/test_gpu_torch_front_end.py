@@ -5,6 +5,7 @@ import torch
 
 import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import _capi, moe, ops
+from gpu_ragged_dot_amd._native import lib as _native
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +71,21 @@ def test_a_plan_for_the_product_leaves_its_gradients_to_the_library():
         uncut = ops._gmm_fwd(*((dout, args[1]) if out.dim() == 2 else (args[1], dout)), gs, **HP, trans_rhs=True, plan=plan)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         assert not torch.equal(got[0], uncut)
+
+
+@pytest.mark.parametrize("op", ["gmm", "tgmm"])
+def test_an_error_in_a_gradient_keeps_its_type(op):
+    """A gradient whose plan names no tile shape: refused on the host, with the error a product of its own raises."""
+    gs = torch.tensor([3, 5], dtype=torch.int32, device="cuda")
+    rand = lambda *s: torch.randn(*s, device="cuda").to(torch.bfloat16).requires_grad_()
+    x, other = rand(8, 64), rand(2, 64, 64) if op == "gmm" else rand(8, 64)
+    good, bad = (-1, 0, 0, 0, 0), (10 ** 6, 0, 0, 0, 0)
+    for plans, wanted in (((good, bad, good), x), ((good, good, bad), other)):
+        print(f"failing gradient of {op}", flush=True)
+        if op == "gmm":
+            out = _native.gmm(x, other, gs, False, _capi.RD_DTYPE_BF16, -1, plans)
+        else:
+            out = _native.tgmm(x, other, gs, _capi.RD_DTYPE_BF16, -1, -1, plans)
+        with pytest.raises(_capi.RaggedDotError, match="out of range") as e:
+            torch.autograd.grad(out, wanted, torch.ones_like(out))
+        assert e.value.status == _capi.RD_ERR_INVALID_ARGUMENT
