@@ -255,22 +255,24 @@ bool wants_grad(const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
 }
 
-Tensor gmm(const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int code, int64_t g_first, const py::object& plans) {
+// Called without the interpreter lock, as everything below that may wait - for memory, for a copy of group_sizes from the
+// host, for the driver - so that other Python threads run meanwhile.
+Tensor gmm(const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int code, int64_t g_first, const Plans& plans) {
   expect_no_tangent(x, A);
   if (x.scalar_type() != A.scalar_type()) throw py::type_error("x and A have different element types");
   Call c;
-  c.code = code; c.trans = trans; c.g_first = g_first; c.plans = plans_from(plans);
+  c.code = code; c.trans = trans; c.g_first = g_first; c.plans = plans;
   if (!wants_grad(x, A)) return gmm_forward(x, A, gs, c, 0, trans);
   check_devices(x, A);
   return GmmNode::apply(x, A, gs, c);
 }
 
-Tensor tgmm(const Tensor& x, const Tensor& y, const Tensor& gs, int code, int64_t g_first, int64_t g_local, const py::object& plans) {
+Tensor tgmm(const Tensor& x, const Tensor& y, const Tensor& gs, int code, int64_t g_first, int64_t g_local, const Plans& plans) {
   expect_no_tangent(x, y);
   if (x.scalar_type() != y.scalar_type()) throw py::type_error("x and y have different element types");
   Call c;
   // a number of groups without a first one means the first ones (the gradients' A then holds those only)
-  c.code = code; c.g_first = g_first < 0 && g_local >= 0 ? 0 : g_first; c.g_local = g_local; c.plans = plans_from(plans);
+  c.code = code; c.g_first = g_first < 0 && g_local >= 0 ? 0 : g_first; c.g_local = g_local; c.plans = plans;
   if (!wants_grad(x, y)) return tgmm_forward(x, y, gs, c, 0, g_local);
   check_devices(x, y);
   return TgmmNode::apply(x, y, gs, c);
@@ -425,13 +427,22 @@ PYBIND11_MODULE(_rd_torch, mod) {
       g_tuned[py::cast<std::tuple<int, int64_t, int64_t, int64_t, int64_t>>(kv[0])] = plan_from(kv[1]);
     }
   });
-  mod.def("gmm", &gmm);
-  mod.def("tgmm", &tgmm);
-  mod.def("moe_route", &moe_route);
-  mod.def("moe_dispatch", &moe_dispatch);
+  typedef py::call_guard<py::gil_scoped_release> unlocked;  // (held again for the result and for errors)
+  mod.def("gmm", [](const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int code, int64_t g_first, const py::object& plans) {
+    const Plans p = plans_from(plans);
+    const py::gil_scoped_release without_lock;
+    return gmm(x, A, gs, trans, code, g_first, p);
+  });
+  mod.def("tgmm", [](const Tensor& x, const Tensor& y, const Tensor& gs, int code, int64_t g_first, int64_t g_local, const py::object& plans) {
+    const Plans p = plans_from(plans);
+    const py::gil_scoped_release without_lock;
+    return tgmm(x, y, gs, code, g_first, g_local, p);
+  });
+  mod.def("moe_route", &moe_route, unlocked());
+  mod.def("moe_dispatch", &moe_dispatch, unlocked());
   mod.def("moe_dispatch_rows", [](const Tensor& h, const std::optional<Tensor>& scale, const Tensor& row_of_slot, const Tensor& slot_of_row,
                                   int64_t tokens, int64_t top_k) {
     return dispatch_rows(h, Routing{row_of_slot, slot_of_row, tokens, top_k}, scale.value_or(Tensor()));
-  });
-  mod.def("moe_combine", &moe_combine);
+  }, unlocked());
+  mod.def("moe_combine", &moe_combine, unlocked());
 }

@@ -1,5 +1,8 @@
 """The torch front end's host path on real kernels: what a call under a trace, in a gradient or beside other threads does."""
 
+import threading
+import time
+
 import pytest
 import torch
 
@@ -89,3 +92,34 @@ def test_an_error_in_a_gradient_keeps_its_type(op):
         with pytest.raises(_capi.RaggedDotError, match="out of range") as e:
             torch.autograd.grad(out, wanted, torch.ones_like(out))
         assert e.value.status == _capi.RD_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("op", ["gmm", "tgmm"])
+def test_other_threads_run_while_a_call_waits_for_the_device(op):
+    """A copy from host memory waits for the stream: other Python threads must not wait with it."""
+    print(f"waiting {op}", flush=True)
+    x, A = torch.randn(16, 64, device="cuda").bfloat16(), torch.randn(2, 64, 64, device="cuda").bfloat16()
+    y, sizes = torch.randn(16, 64, device="cuda").bfloat16(), torch.tensor([9, 7])  # int64 on the host
+    call = {"gmm": lambda: rd.gmm(x, A, sizes), "tgmm": lambda: rd.tgmm(x, y, sizes)}[op]
+    call()
+    big = torch.randn(8192, 8192, device="cuda")
+    big @ big
+    torch.cuda.synchronize()
+    ticks, done = [0], threading.Event()
+
+    def tick():
+        while not done.wait(0.001):
+            ticks[0] += 1
+
+    other = threading.Thread(target=tick)
+    for _ in range(30):
+        big @ big  # 10 ms each and more
+    other.start()
+    before, start = ticks[0], time.perf_counter()
+    call()
+    waited, passed = time.perf_counter() - start, ticks[0] - before
+    done.set()
+    other.join()
+    torch.cuda.synchronize()
+    assert waited > 0.05, "the call was meant to wait"
+    assert passed > 100 * waited, f"{passed} ticks of a millisecond in {waited:.3f} s"
