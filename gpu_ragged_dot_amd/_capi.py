@@ -80,6 +80,7 @@ EXPORTS = (
     "rd_get_variant",
     "rd_variant_takes",
     "rd_default_plan",
+    "rd_default_plan_any_address",
     "rd_sched_map",
     "rd_sched_map_len",
     "rd_gmm_workspace_bytes",
@@ -121,6 +122,8 @@ def _load() -> ctypes.CDLL:
     lib.rd_variant_takes.restype = i
     lib.rd_default_plan.argtypes = [i, i, i, i, i, i, ctypes.POINTER(Plan)]
     lib.rd_default_plan.restype = i
+    lib.rd_default_plan_any_address.argtypes = [i, i, i, i, i, i, ctypes.POINTER(Plan)]
+    lib.rd_default_plan_any_address.restype = i
     lib.rd_sched_map.argtypes = [vp, ip, i, i, i, ip, ip, ip, ip]
     lib.rd_sched_map.restype = i
     lib.rd_sched_map_len.argtypes = [i, i, i]
@@ -173,7 +176,8 @@ def variants() -> list[VariantInfo]:
     return out
 
 
-def default_plan(op: int, m: int, k: int, n: int, g: int, dtype: int = RD_DTYPE_BF16) -> Plan:
+def default_plan(op: int, m: int, k: int, n: int, g: int, dtype: int = RD_DTYPE_BF16, aligned: bool = True) -> Plan:
     plan = Plan()
-    check(lib.rd_default_plan(op, m, k, n, g, dtype, ctypes.byref(plan)))
+    choose = lib.rd_default_plan if aligned else lib.rd_default_plan_any_address
+    check(choose(op, m, k, n, g, dtype, ctypes.byref(plan)))
     return plan

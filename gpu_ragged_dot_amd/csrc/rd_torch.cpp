@@ -85,7 +85,10 @@ bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.const_da
 
 rd_plan pick_plan(int op, int64_t m, int64_t k, int64_t n, int64_t g, int code, bool aligned) {
   rd_plan p{-1, 0, 0, 0, 0};
-  if (!aligned && code != RD_DTYPE_F32) return p;  // the library chooses among the shapes that take any address
+  if (!aligned) {  // the library chooses among the shapes that take any address, whatever the table says
+    check(rd_default_plan_any_address(op, (int)m, (int)k, (int)n, (int)g, code, &p));
+    return p;
+  }
   if (code == RD_DTYPE_BF16 && k % 8 == 0 && n % 8 == 0) {
     std::lock_guard<std::mutex> hold(g_tuned_lock);
     const auto it = g_tuned.find({op, m, k, n, g});

@@ -112,8 +112,8 @@ def select_plan(
 
     ``aligned``: every buffer of the call starts on a 16-byte boundary.  When one does not, the library chooses among the
     tile shapes that take any address, whatever the tuned table or block_* ask for."""
-    if not aligned and dtype != _capi.RD_DTYPE_F32:
-        return _capi.Plan()
+    if not aligned:
+        return _capi.default_plan(op, m, k, n, g, dtype, aligned=False)
     if dtype != _capi.RD_DTYPE_BF16:
         return _capi.default_plan(op, m, k, n, g, dtype)  # the library's own choice: nothing to tune
     vec = k % 8 == 0 and n % 8 == 0

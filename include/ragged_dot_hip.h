@@ -110,6 +110,9 @@ int rd_variant_takes(int id, int op, int m, int k, int n, int dtype);
  * weights stored [g, n, k] 19 us; best tile kernel 35 us; rows spread evenly: 69 us).  Op 1 (weights stored [g, n, k])
  * has a streaming kernel of its own under the same conditions and k <= 8192; it needs no workspace beyond the map's. */
 int rd_default_plan(int op, int m, int k, int n, int g, int dtype, rd_plan* out /* host */);
+/* The same for a call with a buffer that does not start on a 16-byte boundary: among the shapes that take any address.
+ * (variant = -1 resolves to it too, but rd_gmm_workspace_bytes() then has to allow for the largest shape's partial sums.) */
+int rd_default_plan_any_address(int op, int m, int k, int n, int g, int dtype, rd_plan* out /* host */);
 
 /* ---- scheduling map --------------------------------------------------------------------------------------
  * Replaces _make_gmm_group_metadata (gpu_ragged_dot.py:70-90).  Bit-exact int32 outputs:

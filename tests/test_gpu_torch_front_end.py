@@ -123,3 +123,19 @@ def test_other_threads_run_while_a_call_waits_for_the_device(op):
     torch.cuda.synchronize()
     assert waited > 0.05, "the call was meant to wait"
     assert passed > 100 * waited, f"{passed} ticks of a millisecond in {waited:.3f} s"
+
+
+@pytest.mark.parametrize("trans_rhs", [False, True])
+def test_a_small_product_at_an_odd_address_needs_little_memory(trans_rhs):
+    print(f"odd address, trans_rhs {trans_rhs}", flush=True)
+    gs = torch.tensor([20, 0, 30, 14], dtype=torch.int32, device="cuda")
+    A = torch.randn(4, 64, 64, device="cuda").bfloat16()
+    aligned = torch.randn(64, 64, device="cuda").bfloat16()
+    x = torch.empty(64 * 64 + 1, dtype=torch.bfloat16, device="cuda")[1:].view(64, 64).copy_(aligned)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y = rd.gmm(x, A, gs, trans_rhs=trans_rhs)
+    assert torch.cuda.max_memory_allocated() - before < 1 << 20
+    ref = rd.gmm(aligned.float(), A.float(), gs, trans_rhs=trans_rhs)
+    assert torch.linalg.norm(y.float() - ref) <= 2.0 ** -8 * torch.linalg.norm(ref)  # one rounding to bfloat16

@@ -138,6 +138,23 @@ def test_explicit_blocks_pick_a_shape_that_takes_the_call(op, block):
             assert rc == (_capi.RD_ERR_WORKSPACE if takes == _capi.RD_OK else takes), (v.name, m, k, n)
 
 
+@pytest.mark.parametrize("dtype", range(5))
+@pytest.mark.parametrize("op", [_capi.OP_GMM, _capi.OP_GMM_TRANS, _capi.OP_TGMM])
+def test_plans_for_odd_addresses(op, dtype):
+    """A buffer at an odd address: a shape that takes any, no streaming kernel, and no more workspace than that shape uses."""
+    vs = {v.id: v for v in _capi.variants()}
+    for m, k, n, g in ((64, 64, 64, 4), (64, 2048, 768, 128), (1000, 57, 77, 3), (8192, 4096, 4096, 8), (16384, 4096, 14336, 8)):
+        p = planner.select_plan(op, m, k, n, g, dtype=dtype, aligned=False)
+        v = vs[p.variant]
+        assert v.dtype == dtype and not v.vec and p.decode_nb == 0
+        if op != _capi.OP_TGMM:
+            need = _capi.lib.rd_gmm_workspace_bytes(m, g, ctypes.byref(p))
+            assert need <= (1 << 20) + 256 * v.tile_m * v.tile_n * 4
+            assert need <= _capi.lib.rd_gmm_workspace_bytes(m, g, None)
+            if (k, n) == (64, 64) and dtype != _capi.RD_DTYPE_F32:
+                assert need < 1 << 20
+
+
 def test_planner_choices():
     vs = {v.id: v for v in _capi.variants()}
     p = planner.select_plan(_capi.OP_GMM, 171, 58, 77, 8)
