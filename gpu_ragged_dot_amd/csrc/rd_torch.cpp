@@ -77,7 +77,8 @@ variable_list in_backward(F&& body) {
 }
 
 // ---- plans -------------------------------------------------------------------------------------------------------------
-// planner.py owns the tuned table and the choice for explicit block sizes; the table is handed over once, at import.
+// planner.py owns the tuned table and the choice for explicit block sizes; the table is handed over once, at import.  For the
+// default block sizes pick_plan() is planner.select_plan() in native code (a host test compares the two).
 std::map<std::tuple<int, int64_t, int64_t, int64_t, int64_t>, rd_plan> g_tuned;
 std::mutex g_tuned_lock;
 
@@ -429,6 +430,10 @@ PYBIND11_MODULE(_rd_torch, mod) {
       const auto kv = py::cast<py::tuple>(e);
       g_tuned[py::cast<std::tuple<int, int64_t, int64_t, int64_t, int64_t>>(kv[0])] = plan_from(kv[1]);
     }
+  });
+  mod.def("pick_plan", [](int op, int64_t m, int64_t k, int64_t n, int64_t g, int code, bool aligned) {
+    const rd_plan p = pick_plan(op, m, k, n, g, code, aligned);
+    return std::make_tuple(p.variant, p.group_m, p.group_n, p.decode_nb, p.split_k);
   });
   typedef py::call_guard<py::gil_scoped_release> unlocked;  // (held again for the result and for errors)
   mod.def("gmm", [](const Tensor& x, const Tensor& A, const Tensor& gs, bool trans, int code, int64_t g_first, const py::object& plans) {

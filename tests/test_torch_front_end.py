@@ -2,6 +2,7 @@
 loaded.  No GPU is needed; tensors are on the CPU, which the calls refuse last."""
 
 import ctypes
+import random
 import types
 
 import pytest
@@ -10,6 +11,7 @@ import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import moe, ops, planner
+from gpu_ragged_dot_amd._native import lib as _native
 
 
 def _routing(tokens, top_k):
@@ -109,3 +111,18 @@ def test_explicit_blocks_plan_what_the_call_computes(op, monkeypatch):
     call(bf16(128, 72)[:, 1:65], bf16)  # strided, at an odd element: a copy is multiplied
     call(bf16(128 * 64 + 1)[1:].view(128, 64), bf16)  # contiguous, at an odd element
     assert [kw["aligned"] for _, kw in asked] == [True, False]
+
+
+def test_native_and_python_planner_agree():
+    """One rule, written twice: what a torch call gets and what planner.select_plan() - the JAX front end, the benchmark and
+    the tests of the rule itself - says."""
+    assert planner.tuned_plans(), "the tuned table is part of the rule"
+    shapes = [key for key, _ in planner.tuned_plan_fields()]
+    rng = random.Random(0)
+    size = lambda hi: rng.choice([round(2 ** rng.uniform(0, hi)), 8 * round(2 ** rng.uniform(0, hi - 3))])
+    shapes += [(op, size(15), size(13), size(13), round(2 ** rng.uniform(0, 8))) for op in range(3) for _ in range(300)]
+    for op, m, k, n, g in shapes:
+        for code in range(5):
+            for aligned in (True, False):
+                want = ops._fields(planner.select_plan(op, m, k, n, g, dtype=code, aligned=aligned))
+                assert _native.pick_plan(op, m, k, n, g, code, aligned) == want, (op, m, k, n, g, code, aligned)
