@@ -10,6 +10,7 @@ from __future__ import annotations
 import json
 import math
 import os
+import re
 from typing import Optional
 
 from . import _capi
@@ -82,13 +83,21 @@ def _tuned_plan(entry: dict) -> _capi.Plan:
 
 
 def tuned_plan_fields() -> list:
-    """The tuned table as [((op, m, k, n, g), plan fields in the order of rd_plan), ...]."""
+    """The tuned table as [((op, m, k, n, g), plan fields in the order of rd_plan), ...].  Keys of another form name no call
+    and are left out; an entry this build cannot follow (a tile shape it does not have) gets a variant id out of range, so that
+    the one call it is for is refused, as select_plan() refuses it."""
     ops = {"gmm": _capi.OP_GMM, "gmm_t": _capi.OP_GMM_TRANS, "tgmm": _capi.OP_TGMM}
     out = []
     for key, entry in tuned_plans().items():
-        op, *sizes = key.split(":")
-        p = _tuned_plan(entry)
-        out.append(((ops[op], *(int(v[1:]) for v in sizes)), (p.variant, p.group_m, p.group_n, p.decode_nb, p.split_k)))
+        match = re.fullmatch(r"(gmm|gmm_t|tgmm):m(\d+):k(\d+):n(\d+):g(\d+)", key)
+        if match is None or entry is None:
+            continue
+        call = (ops[match[1]], *map(int, match.groups()[1:]))
+        try:
+            p = _tuned_plan(entry)
+        except (KeyError, TypeError, ValueError, AttributeError):
+            p = _capi.Plan(len(compiled_variants()))
+        out.append((call, (p.variant, p.group_m, p.group_n, p.decode_nb, p.split_k)))
     return out
 
 

@@ -2,7 +2,11 @@
 loaded.  No GPU is needed; tensors are on the CPU, which the calls refuse last."""
 
 import ctypes
+import json
+import os
 import random
+import subprocess
+import sys
 import types
 
 import pytest
@@ -12,6 +16,8 @@ import torch.autograd.forward_ad as fwAD
 import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import moe, ops, planner
 from gpu_ragged_dot_amd._native import lib as _native
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _routing(tokens, top_k):
@@ -126,3 +132,19 @@ def test_native_and_python_planner_agree():
             for aligned in (True, False):
                 want = ops._fields(planner.select_plan(op, m, k, n, g, dtype=code, aligned=aligned))
                 assert _native.pick_plan(op, m, k, n, g, code, aligned) == want, (op, m, k, n, g, code, aligned)
+
+
+def test_a_tuned_table_of_another_build_does_not_prevent_the_import(tmp_path):
+    """An entry that names a tile shape this build does not have refuses its own call and no other."""
+    table = {"gmm:m64:k64:n64:g2": {"variant": "no_such_shape"}, "gmm:m64:k64:n128:g2": {"variant": "t64x64x64_w2x2", "group_m": 3},
+             "gmm:m64:k64:n192:g2": {}, "gmm:m64:k64:n256:g2": None, "tgmm:m64": {"variant": "t64x64x64_w2x2"}, "tuned on": "a Tuesday"}
+    path = tmp_path / "plans.json"
+    path.write_text(json.dumps(table))
+    code = ("from gpu_ragged_dot_amd import _capi, planner\nfrom gpu_ragged_dot_amd._native import lib\n"
+            "pick = lambda n: lib.pick_plan(0, 64, 64, n, 2, 0, True)\nids = range(_capi.lib.rd_num_variants())\n"
+            "assert pick(64)[0] not in ids and pick(192)[0] not in ids\n"
+            "assert pick(128)[:2] == (planner.variant_id('t64x64x64_w2x2'), 3)\n"
+            "assert pick(256)[0] in ids and pick(320)[0] in ids\n")
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, RAGGED_DOT_TUNED_PLANS=str(path)), cwd=ROOT,
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
