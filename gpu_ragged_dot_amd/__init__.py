@@ -8,9 +8,10 @@ from .planner import CHUNK_M, DEFAULT_BLOCK_K, DEFAULT_BLOCK_M, DEFAULT_BLOCK_N
 
 try:
     import torch as _torch  # noqa: F401
-except ImportError:  # a JAX-only process: the same names live in gpu_ragged_dot_amd.jax_adapter
+except ImportError:
     _torch = None
-if _torch is not None:
+# without torch, or beside one that has no ROCm, this is a JAX process: the same names live in gpu_ragged_dot_amd.jax_adapter
+if _torch is not None and _torch.version.hip is not None:
     from . import moe  # noqa: F401  (route / dispatch / combine around ragged_dot)
     from .ops import gmm, make_group_metadata, ragged_dot, ragged_dot_vjp, tgmm, trans_ragged_dot
 

@@ -148,3 +148,18 @@ def test_a_tuned_table_of_another_build_does_not_prevent_the_import(tmp_path):
     r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, RAGGED_DOT_TUNED_PLANS=str(path)), cwd=ROOT,
                        capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr
+
+
+def test_a_torch_without_rocm_counts_as_none(tmp_path):
+    """A JAX process often has a CPU build of torch installed: the library builds and the package imports beside it, without
+    the torch front end."""
+    code = ("import sys, torch\ntorch.version.hip = None\nimport gpu_ragged_dot_amd as rd\n"
+            "from gpu_ragged_dot_amd import _capi, planner\n"
+            "assert 'gpu_ragged_dot_amd._native' not in sys.modules and not hasattr(rd, 'ragged_dot')\n"
+            "planner.select_plan(_capi.OP_GMM, 512, 512, 512, 4)\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    csrc = os.path.join(ROOT, "gpu_ragged_dot_amd", "csrc")
+    for variables, built in (([], True), ([f"TORCH_DIR={tmp_path}"], False), (["TORCH_DIR="], False)):
+        r = subprocess.run(["make", "-n", "-W", "rd_torch.cpp", "-C", csrc, *variables], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0 and ("-o _rd_torch.so" in r.stdout) == built, (variables, r.stdout, r.stderr)
