@@ -19,8 +19,12 @@ def _load():
     if not os.path.exists(PATH):
         raise ImportError(f"{PATH} is missing: build it with `make -C {os.path.dirname(PATH)} -j8`")
     spec = importlib.util.spec_from_file_location("_rd_torch", PATH)
-    module = importlib.util.module_from_spec(spec)
-    spec.loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError as e:  # built with another torch or Python
+        raise ImportError(f"{PATH} does not fit torch {torch.__version__} on this Python ({e}): build it again with "
+                          f"`make -C {os.path.dirname(PATH)} -j8`") from e
     module.set_tuned_plans(planner.tuned_plan_fields())
     return module
 

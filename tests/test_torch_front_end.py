@@ -15,6 +15,7 @@ import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import moe, ops, planner
+from gpu_ragged_dot_amd import _native as _native_loader
 from gpu_ragged_dot_amd._native import lib as _native
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -163,3 +164,21 @@ def test_a_torch_without_rocm_counts_as_none(tmp_path):
     for variables, built in (([], True), ([f"TORCH_DIR={tmp_path}"], False), (["TORCH_DIR="], False)):
         r = subprocess.run(["make", "-n", "-W", "rd_torch.cpp", "-C", csrc, *variables], capture_output=True, text=True, timeout=300)
         assert r.returncode == 0 and ("-o _rd_torch.so" in r.stdout) == built, (variables, r.stdout, r.stderr)
+
+
+def test_the_native_module_is_rebuilt_for_another_torch():
+    csrc = os.path.join(ROOT, "gpu_ragged_dot_amd", "csrc")
+    dry = lambda *v: subprocess.run(["make", "-n", "-C", csrc, *v, "_rd_torch.so"], capture_output=True, text=True, timeout=300)
+    other = dry("TORCH_ID=torch-0.0-cpython-00")
+    assert other.returncode == 0 and "-o _rd_torch.so" in other.stdout, other.stderr
+    if os.path.isdir(os.path.join(csrc, "build")):  # (a tree that was shipped built has no record of what it was built with)
+        assert "-o _rd_torch.so" not in dry().stdout
+
+
+def test_a_module_that_does_not_fit_says_what_to_do(tmp_path, monkeypatch):
+    """A module built with another torch misses symbols of this one."""
+    path = tmp_path / "_rd_torch.so"
+    path.write_bytes(b"\x7fELF")
+    monkeypatch.setattr(_native_loader, "PATH", str(path))
+    with pytest.raises(ImportError, match="build it again"):
+        _native_loader._load()
