@@ -13,6 +13,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <limits>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -130,6 +131,12 @@ void same_type(const Tensor& a, const Tensor& b) {
   TORCH_CHECK_TYPE(a.scalar_type() == b.scalar_type(), "the operands are ", a.scalar_type(), " and ", b.scalar_type());
 }
 
+// (the C ABI takes 32-bit sizes)
+void expect_int(std::initializer_list<int64_t> sizes) {
+  for (const int64_t s : sizes)
+    if (s > std::numeric_limits<int>::max()) throw StatusError(RD_ERR_INVALID_ARGUMENT, "a size is beyond 2^31 - 1");
+}
+
 Tensor sizes_on(const Tensor& gs, const at::Device& dev) {
   Tensor t = gs.scalar_type() == at::kInt ? gs : gs.to(at::kInt);
   if (t.device() != dev) t = t.to(dev);
@@ -162,6 +169,7 @@ Tensor gmm_forward(const Tensor& x_, const Tensor& A_, const Tensor& gs_, const 
   expect(c.g_first < 0 ? g_local == g : g_first + g_local <= g, "A does not hold the groups that group_sizes describes");  // :189
   const int64_t m = x_.size(0), k = x_.size(1), n = A_.size(trans ? 1 : 2);  // :190
   expect(A_.size(trans ? 2 : 1) == k, "contraction mismatch between x and A");
+  expect_int({m, k, n, g});
   check_devices(x_, A_);
   const at::Device dev = x_.device();
   const Tensor x = x_.contiguous(), A = A_.contiguous(), gs = sizes_on(gs_, dev);
@@ -185,6 +193,7 @@ Tensor tgmm_forward(const Tensor& x_, const Tensor& y_, const Tensor& gs_, const
   const int64_t m = x_.size(0), k = x_.size(1), n = y_.size(1), g = gs_.numel(), g_first = c.g_first < 0 ? 0 : c.g_first;
   if (g_local < 0) g_local = g - g_first;
   expect(g_local >= 1 && g_first + g_local <= g, "the groups asked for are not within group_sizes");
+  expect_int({m, k, n, g});
   check_devices(x_, y_);
   const at::Device dev = x_.device();
   const Tensor x = x_.contiguous(), y = y_.contiguous(), gs = sizes_on(gs_, dev);
@@ -290,6 +299,7 @@ struct Routing {
 
 std::tuple<Tensor, Tensor, Tensor> moe_route(const Tensor& ids_, int64_t groups) {
   if (ids_.dim() != 2) throw py::value_error("expert_ids must be [tokens, top_k]");
+  expect_int({ids_.size(0), ids_.size(1), groups});
   check_devices(ids_, ids_);
   const at::Device dev = ids_.device();
   const Tensor ids = sizes_on(ids_, dev);
@@ -313,9 +323,10 @@ int rows_code(const Tensor& t) {
 }
 
 Tensor dispatch_rows(const Tensor& h_, const Routing& r, const Tensor& scale) {
+  if (h_.dim() != 2 || h_.size(0) != r.tokens) throw py::value_error("h must be [" + std::to_string(r.tokens) + ", d]");
+  expect_int({r.tokens, r.top_k, h_.size(1)});
   check_devices(h_, r.slot_of_row);
   const Tensor h = h_.contiguous();
-  if (h.dim() != 2 || h.size(0) != r.tokens) throw py::value_error("h must be [" + std::to_string(r.tokens) + ", d]");
   const int code = rows_code(h);
   const c10::DeviceGuard guard(h.device());
   Tensor x = at::empty({r.tokens * r.top_k, h.size(1)}, h.options().requires_grad(false));
@@ -325,9 +336,10 @@ Tensor dispatch_rows(const Tensor& h_, const Routing& r, const Tensor& scale) {
 }
 
 Tensor combine_rows(const Tensor& y_, const Routing& r, const Tensor& weights) {
+  if (y_.dim() != 2 || y_.size(0) != r.tokens * r.top_k) throw py::value_error("y must be [" + std::to_string(r.tokens * r.top_k) + ", d]");
+  expect_int({r.tokens, r.top_k, y_.size(1)});
   check_devices(y_, r.row_of_slot);
   const Tensor y = y_.contiguous();
-  if (y.dim() != 2 || y.size(0) != r.tokens * r.top_k) throw py::value_error("y must be [" + std::to_string(r.tokens * r.top_k) + ", d]");
   const int code = rows_code(y);
   const c10::DeviceGuard guard(y.device());
   Tensor out = at::empty({r.tokens, y.size(1)}, y.options().requires_grad(false));

@@ -14,7 +14,7 @@ import torch
 import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
-from gpu_ragged_dot_amd import moe, ops, planner
+from gpu_ragged_dot_amd import _capi, moe, ops, planner
 from gpu_ragged_dot_amd import _native as _native_loader
 from gpu_ragged_dot_amd._native import lib as _native
 
@@ -182,3 +182,18 @@ def test_a_module_that_does_not_fit_says_what_to_do(tmp_path, monkeypatch):
     monkeypatch.setattr(_native_loader, "PATH", str(path))
     with pytest.raises(ImportError, match="build it again"):
         _native_loader._load()
+
+
+@pytest.mark.parametrize("call", ["gmm", "tgmm", "tgmm columns", "route", "dispatch", "combine"])
+def test_sizes_beyond_32_bits_are_refused(call):
+    """The kernels take 32-bit sizes; one more than 2^32 must not pass as the 9 it is in its low half."""
+    m = 2 ** 32 + 9
+    wide = lambda *s: torch.zeros(1, *s[1:]).expand(*s)  # no memory behind it
+    gs = torch.tensor([9], dtype=torch.int32)
+    r = _routing(9, 1)._replace(tokens=m)
+    calls = {"gmm": lambda: rd.gmm(wide(m, 8), torch.zeros(1, 8, 8), gs), "tgmm": lambda: rd.tgmm(wide(m, 8), wide(m, 8), gs),
+             "tgmm columns": lambda: rd.tgmm(torch.zeros(9, 8), torch.zeros(9, 1).expand(9, m), gs),
+             "route": lambda: moe.route(torch.zeros(1, 1, dtype=torch.int32).expand(m, 1), 4),
+             "dispatch": lambda: moe.dispatch(wide(m, 8), r), "combine": lambda: moe.combine(wide(m, 8), r)}
+    with pytest.raises(_capi.RaggedDotError, match="beyond"):
+        calls[call]()
