@@ -322,10 +322,21 @@ int rows_code(const Tensor& t) {
   }
 }
 
+// Everything a kernel reads through a pointer is on the rows' device and as long as the kernel takes it to be.
+void check_routing(const Tensor& rows, const Routing& r, const Tensor& per_slot) {
+  check_devices(rows, r.row_of_slot);
+  check_devices(rows, r.slot_of_row);
+  if (per_slot.defined()) check_devices(rows, per_slot);
+  const int64_t slots = r.tokens * r.top_k;
+  if (r.row_of_slot.numel() < slots || r.slot_of_row.numel() < slots || !r.row_of_slot.is_contiguous() || !r.slot_of_row.is_contiguous() ||
+      (per_slot.defined() && (per_slot.numel() < slots || !per_slot.is_contiguous())))
+    throw py::value_error("a routing of " + std::to_string(slots) + " slots needs that many contiguous entries in each of its arrays");
+}
+
 Tensor dispatch_rows(const Tensor& h_, const Routing& r, const Tensor& scale) {
   if (h_.dim() != 2 || h_.size(0) != r.tokens) throw py::value_error("h must be [" + std::to_string(r.tokens) + ", d]");
   expect_int({r.tokens, r.top_k, h_.size(1)});
-  check_devices(h_, r.slot_of_row);
+  check_routing(h_, r, scale);
   const Tensor h = h_.contiguous();
   const int code = rows_code(h);
   const c10::DeviceGuard guard(h.device());
@@ -338,7 +349,7 @@ Tensor dispatch_rows(const Tensor& h_, const Routing& r, const Tensor& scale) {
 Tensor combine_rows(const Tensor& y_, const Routing& r, const Tensor& weights) {
   if (y_.dim() != 2 || y_.size(0) != r.tokens * r.top_k) throw py::value_error("y must be [" + std::to_string(r.tokens * r.top_k) + ", d]");
   expect_int({r.tokens, r.top_k, y_.size(1)});
-  check_devices(y_, r.row_of_slot);
+  check_routing(y_, r, weights);
   const Tensor y = y_.contiguous();
   const int code = rows_code(y);
   const c10::DeviceGuard guard(y.device());

@@ -139,3 +139,23 @@ def test_a_small_product_at_an_odd_address_needs_little_memory(trans_rhs):
     assert torch.cuda.max_memory_allocated() - before < 1 << 20
     ref = rd.gmm(aligned.float(), A.float(), gs, trans_rhs=trans_rhs)
     assert torch.linalg.norm(y.float() - ref) <= 2.0 ** -8 * torch.linalg.norm(ref)  # one rounding to bfloat16
+
+
+def test_routing_arrays_that_the_kernels_cannot_read_are_refused():
+    """Host memory and arrays shorter than the routing says are refused on the host: no kernel sees their addresses."""
+    ids = torch.randint(4, (16, 2), device="cuda", dtype=torch.int32)
+    r = moe.route(ids, 4)
+    h, y = torch.randn(16, 8, device="cuda"), torch.randn(32, 8, device="cuda")
+    w = torch.rand(16, 2, device="cuda")
+    for message, call in (
+            ("same device", lambda: moe.combine(y, r, w.cpu())),
+            ("same device", lambda: moe.combine(y, r._replace(row_of_slot=r.row_of_slot.cpu()), w)),
+            ("same device", lambda: moe.dispatch(h, r._replace(row_of_slot=r.row_of_slot.cpu()))),
+            ("same device", lambda: moe.dispatch(h, r._replace(slot_of_row=r.slot_of_row.cpu()))),
+            ("same device", lambda: moe._dispatch(h, r, w.cpu().reshape(-1))),
+            ("32 slots", lambda: moe._dispatch(h, r, w[:8].reshape(-1))),
+            ("32 slots", lambda: moe.dispatch(h, r._replace(slot_of_row=r.slot_of_row[:8]))),
+            ("32 slots", lambda: moe.combine(y, r._replace(row_of_slot=r.row_of_slot.view(16, 2)[:, 0].repeat(1)), w))):
+        with pytest.raises((RuntimeError, ValueError), match=message):
+            call()
+    assert moe.combine(moe.dispatch(h, r), r, w).shape == h.shape
