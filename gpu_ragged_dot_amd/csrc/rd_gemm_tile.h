@@ -80,8 +80,8 @@ struct OperandStager {
                          fp8e4m3x2_to_bf16x2<false>(raw[1]), fp8e4m3x2_to_bf16x2<true>(raw[1])};
       return r;
     } else {
-      const f32x4_t lo = VEC ? *reinterpret_cast<const f32x4_t*>(p) : load_any<f32x4_t>(p);
-      const f32x4_t hi = VEC ? *reinterpret_cast<const f32x4_t*>(p + 4) : load_any<f32x4_t>(p + 4);
+      static_assert(!VEC, "float32 at 16-byte pitches is the any-pitch core's");
+      const f32x4_t lo = load_any<f32x4_t>(p), hi = load_any<f32x4_t>(p + 4);
       return u32x4_t{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3]), pack_bf16x2(hi[0], hi[1]), pack_bf16x2(hi[2], hi[3])};
     }
   }

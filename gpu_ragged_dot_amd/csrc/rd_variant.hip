@@ -33,7 +33,7 @@
 
 namespace rd {
 #if RD_ANY_PITCH
-// 16-byte pieces at any address through registers (rd_gemm_rs.h): bf16, float16, or float32 rounded to bf16
+// 16-byte pieces at any address through registers (rd_gemm_rs.h): bf16, float16, float32 rounded to bf16, or float32 as it is
 #if RD_F32 == 2 || RD_F32 == 1
 typedef float RsElem;
 #elif RD_F32 == 4

@@ -1,5 +1,5 @@
-"""The any-pitch core (register-staged 256 x 256 and 128 x 128 tiles for odd row pitches and for float32 rounded to bf16)
-and the 64 x 64 tiles that share its unaligned loads, against the oracle.
+"""The any-pitch core (register-staged 256 x 256 and 128 x 128 tiles for odd row pitches and for float32 rounded to bf16, 128 x
+128 to 64 x 64 ones for float32 as it is) and the 64 x 64 tiles that share its unaligned loads, against the oracle.
 
 Sizes where it can go wrong: contractions of less than one slab, of one element more and less than a whole number of slabs
 around the point where the pipelined loop takes over, rows of one piece only, tile edges, groups of 0, 1 and one more than
