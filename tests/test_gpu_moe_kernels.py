@@ -1,6 +1,7 @@
 """The routing kernels at the edges of their dispatch, against the oracle: one slot fewer and more than a block ranks, than
 the one-kernel form takes and than the two-kernel form takes; as many experts as their tables hold and one more; dropped
-slots; every element type of the gradient of the combine weights with row lengths on and off 16 bytes."""
+slots; every element type of the gradient of the combine weights with row lengths on and off 16 bytes; matrices larger
+than the last-level cache, which are read past it."""
 
 import numpy as np
 import pytest
@@ -52,6 +53,29 @@ def test_combine_and_weight_gradient(top_k, d, dtype):
     ref, mag = np.einsum("tsd,ts->td", picked, wv), np.einsum("tsd,ts->td", np.abs(picked), wv)
     got = out.detach().double().cpu().numpy()
     assert np.all(np.abs(got - ref) <= half_ulp * np.abs(ref) + (top_k + 1) * 2.0 ** -24 * mag + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 8200), (torch.float16, 8200), (torch.float32, 4100)], ids=["bf16", "f16", "f32"])
+def test_rows_beyond_the_last_level_cache(dtype, d):
+    """More than 256 MiB of rows: the same bits as two calls of half the size, which read through the caches."""
+    print(f"rows beyond the cache {dtype}", flush=True)
+    half, top_k, g = 4099, 2, 5
+    y = torch.randn(2 * half * top_k, d, device="cuda").to(dtype)
+    assert y.numel() * y.element_size() > 256 << 20 > y.numel() * y.element_size() // 2
+    r = moe.route(torch.randint(-1, g, (2 * half, top_k), device="cuda", dtype=torch.int32), g)
+    w = torch.rand(2 * half, top_k, device="cuda").requires_grad_()
+    dout = torch.randn(2 * half, d, device="cuda").to(dtype)
+    out = moe.combine(y, r, w)
+    dw, = torch.autograd.grad(out, w, dout)
+    slots = torch.arange(half * top_k, device="cuda", dtype=torch.int32)
+    for part in (slice(0, half), slice(half, 2 * half)):
+        rows = r.row_of_slot.view(-1, top_k)[part].reshape(-1)
+        own = moe.Routing(r.group_sizes, torch.where(rows < 0, rows, slots), slots, half, top_k)
+        w_part = w.detach()[part].clone().requires_grad_()
+        out_part = moe.combine(y[rows.clamp(min=0).long()], own, w_part)
+        dw_part, = torch.autograd.grad(out_part, w_part, dout[part])
+        assert torch.equal(out[part], out_part) and torch.equal(dw[part], dw_part)
+    assert not dw.view(-1)[r.row_of_slot < 0].any() and dw.any()
 
 
 def test_dispatch_gradient_twice():
