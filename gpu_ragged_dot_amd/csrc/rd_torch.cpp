@@ -52,6 +52,17 @@ void set_python_error(const StatusError& e) {
 void set_python_error(const CheckError& e) { PyErr_SetString(PyExc_AssertionError, e.what()); }
 void set_python_error(const py::builtin_exception& e) { e.set_error(); }
 
+// Only backward gradients are defined.  A tensor that carries a forward-mode tangent is refused, whether or not it asks for
+// a gradient as well, as an operand and as a cotangent: the kernels would run on its value alone, and a result without a
+// tangent reads as one of zero.
+void expect_no_tangent(const Tensor& t) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(0).defined(), "forward-mode derivatives are not implemented");
+}
+void expect_no_tangent(const Tensor& a, const Tensor& b) {
+  expect_no_tangent(a);
+  expect_no_tangent(b);
+}
+
 // The body of an autograd node's backward.  Its errors leave through torch's engine, possibly on a thread of its own, which
 // hands on Python errors as they are and makes a RuntimeError of what it does not know: here they become the Python errors
 // that the module's entry points raise.
@@ -66,7 +77,8 @@ template <class E>
   throw e;
 }
 template <class F>
-variable_list in_backward(F&& body) {
+variable_list in_backward(const variable_list& grads, F&& body) {
+  for (const Tensor& t : grads) expect_no_tangent(t);
   try {
     return body();
   } catch (const StatusError& e) {
@@ -225,7 +237,7 @@ struct GmmNode : torch::autograd::Function<GmmNode> {
     return gmm_forward(x, A, sizes, c, 0, c.trans);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    return in_backward([&]() -> variable_list {
+    return in_backward(grads, [&]() -> variable_list {
       const auto saved = ctx->get_saved_variables();
       const Call c = call_of(ctx);
       const Tensor &x = saved[0], &A = saved[1], &gs = saved[2];
@@ -247,7 +259,7 @@ struct TgmmNode : torch::autograd::Function<TgmmNode> {
     return tgmm_forward(x, y, sizes, c, 0, c.g_local);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    return in_backward([&]() -> variable_list {
+    return in_backward(grads, [&]() -> variable_list {
       const auto saved = ctx->get_saved_variables();
       const Call c = call_of(ctx);
       const Tensor dA = grads[0].contiguous();
@@ -258,12 +270,6 @@ struct TgmmNode : torch::autograd::Function<TgmmNode> {
     });
   }
 };
-
-// Only backward gradients are defined.  An operand that carries a forward-mode tangent is refused, whether or not it asks for
-// a gradient as well: the kernels would run on its value alone, and a result without a tangent reads as one of zero.
-void expect_no_tangent(const Tensor& a, const Tensor& b) {
-  TORCH_CHECK_NOT_IMPLEMENTED(!a._fw_grad(0).defined() && !b._fw_grad(0).defined(), "forward-mode derivatives are not implemented");
-}
 
 bool wants_grad(const Tensor& a, const Tensor& b) {
   return at::GradMode::is_enabled() && (a.requires_grad() || b.requires_grad());
@@ -387,7 +393,7 @@ struct DispatchNode : torch::autograd::Function<DispatchNode> {
     return dispatch_rows(h, r, Tensor());
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    return in_backward([&]() -> variable_list {
+    return in_backward(grads, [&]() -> variable_list {
       return {combine_rows(grads[0], routing_of(ctx), Tensor()), Tensor()};  // each token collects the gradients of its rows
     });
   }
@@ -401,7 +407,7 @@ struct CombineNode : torch::autograd::Function<CombineNode> {
     return combine_rows(y, r, w);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    return in_backward([&]() -> variable_list {
+    return in_backward(grads, [&]() -> variable_list {
       const auto s = ctx->get_saved_variables();
       const Routing r = routing_of(ctx);
       const Tensor &y = s[0], &w = s[1], &dout = grads[0];

@@ -5,6 +5,7 @@ import time
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 import gpu_ragged_dot_amd as rd
 from gpu_ragged_dot_amd import _capi, moe, ops
@@ -92,6 +93,19 @@ def test_an_error_in_a_gradient_keeps_its_type(op):
         with pytest.raises(_capi.RaggedDotError, match="out of range") as e:
             torch.autograd.grad(out, wanted, torch.ones_like(out))
         assert e.value.status == _capi.RD_ERR_INVALID_ARGUMENT
+
+
+def test_a_cotangent_with_a_forward_mode_tangent_is_refused():
+    """The gradient of a gradient along a direction is not implemented: an answer without a tangent would read as zero."""
+    args = _layer_inputs(3)
+    r = moe.route(args[4], 5)
+    y = torch.randn(80, 64, device="cuda").requires_grad_()
+    outs = {"gmm": (rd.gmm(moe.dispatch(args[0].detach(), r), args[1], r.group_sizes), args[1]), "dispatch": (moe.dispatch(args[0], r), args[0]),
+            "tgmm": (rd.tgmm(y, y.detach(), r.group_sizes), y), "combine": (moe.combine(y, r, args[3]), y)}
+    for name, (out, wanted) in outs.items():
+        print(f"dual cotangent of {name}", flush=True)
+        with fwAD.dual_level(), pytest.raises(NotImplementedError, match="forward-mode"):
+            torch.autograd.grad(out, wanted, fwAD.make_dual(torch.ones_like(out), torch.ones_like(out)))
 
 
 @pytest.mark.parametrize("op", ["gmm", "tgmm"])
