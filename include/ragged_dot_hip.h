@@ -133,8 +133,9 @@ int rd_sched_map_len(int m, int g, int chunk_m);
  *   (:155-165) -- also when every group is empty.  Groups that would run past m are clipped to m.
  * Workspace: rd_gmm_workspace_bytes() bytes, 256-byte aligned; holds the scheduling map, 64 KiB for the order in which
  * the tile walk's blocks are dealt (long groups' among short groups') and, unless the plan says split_k = -1, fp32
- * partial sums (64 MiB for the 256 x 256 tiles).  A smaller workspace that has room for the map is accepted: the call
- * then runs without the K-split and, if the order does not fit either, in plain walk order - same results. */
+ * partial sums (64 MiB for the 256 x 256 tiles, 4-16 MiB for the float32 ones).  A smaller workspace that has room for the map is accepted: the call
+ * then runs without the K-split (the same sums, added up in another order where it would have cut) and, if the order does
+ * not fit either, in plain walk order (the same bits). */
 size_t rd_gmm_workspace_bytes(int m, int g, const rd_plan* plan /* host, may be NULL */);
 int rd_gmm(void* stream, const void* x, const void* A, const int32_t* group_sizes, void* y, int m, int k, int n,
            int g, int trans_rhs, int dtype, const rd_plan* plan /* host, may be NULL */, void* workspace,
