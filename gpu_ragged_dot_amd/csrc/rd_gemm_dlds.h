@@ -25,6 +25,7 @@ struct DldsCfg {
   static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, VEC = true, DLDS = true, PINGPONG = PINGPONG_, MIXED = false,
                         SPLITK = true;
   static constexpr int B_AUX = B_AUX_;
+  static constexpr bool ROTATES = B_AUX == 2 /* kCachePolicyStream */ && B_KMAJOR && !PINGPONG;  // gemm_tile_dlds(): tiles may start at any slab
   static constexpr int NW = WAVES_M * WAVES_N;
   static constexpr int NT = 64 * NW;
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
@@ -126,6 +127,12 @@ struct DldsLoader {
     base = reinterpret_cast<const bf16_bits*>(reinterpret_cast<const unsigned char*>(base) + step_bytes);
     records -= step_bytes;  // stays positive for every slab that is issued
   }
+  // the same for several slabs (K-major operands: within a row, so 32 bits hold it), and back to where `first` stands
+  __host__ __device__ __forceinline__ void advance(int slabs) {
+    base = reinterpret_cast<const bf16_bits*>(reinterpret_cast<const unsigned char*>(base) + slabs * step_bytes);
+    records -= slabs * step_bytes;
+  }
+  __host__ __device__ __forceinline__ void rewind(const DldsLoader& first) { base = first.base; records = first.records; }
 };
 
 // Per-lane LDS byte offsets for the matrix-core fragment reads of one operand.
@@ -299,11 +306,16 @@ __device__ __forceinline__ void store_accumulators(const f32x16_t (&acc)[C::TM][
   }
 }
 
+// start: the slab a tile whose configuration ROTATES begins with.  The rows of a K-major operand lie a whole row pitch apart, and
+// where that is a power of two (or close to it) the 128-byte pieces of one slab all fall into the same few memory channels.
+// Tiles that stream weights nobody shares all run in step, so all of them would ask the same channels at the same time; starting
+// at slabs of their own they spread over all.  2048 rows in 128 groups of 16, weights [g, n, k], us before -> after: k 2048, n 768 93
+// -> 73 (k 2112: 74), k 2048, n 1024 121 -> 89, k 4096, n 768 173 -> 138, k 2048, n 7168 689 -> 600; k 768 and 7168 level.
 template <class C>
 __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap, int lda, int a_lim,
                                                const bf16_bits* __restrict__ Bp, int ldb, int b_lim, int klen,
                                                bf16_bits* __restrict__ Op, int ldo, bf16_bits* smem_,
-                                               const SplitK& sk = SplitK()) {
+                                               const SplitK& sk = SplitK(), uint32_t start = 0) {
   unsigned char* smem = reinterpret_cast<unsigned char*>(smem_);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -314,6 +326,20 @@ __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap,
   LdA la; LdB lb;
   la.init(Ap, lda, a_lim, klen, wave, lane);
   lb.init(Bp, ldb, b_lim, klen, wave, lane);
+  const int nk = (klen + C::BK - 1) / C::BK;
+  // The slab the loaders stand at: the slabs are taken in order from `start` on and, past the last one, from the first.
+  int at = 0;
+  const LdA la_first = la;
+  const LdB lb_first = lb;
+  if constexpr (C::ROTATES) {
+    at = (int)(start % (uint32_t)nk);
+    la.advance(at); lb.advance(at);
+  }
+  auto advance = [&]() {
+    ++at;
+    if (C::ROTATES && at == nk) { at = 0; la.rewind(la_first); lb.rewind(lb_first); }
+    else { la.advance(); lb.advance(); }
+  };
   DldsFragReader<C::BM, C::BK, C::TM, C::A_KMAJOR> fra;
   DldsFragReader<C::BN, C::BK, C::TN, C::B_KMAJOR> frb;
   fra.init(wm * C::WM, lane);
@@ -330,13 +356,12 @@ __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap,
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  const int nk = (klen + C::BK - 1) / C::BK;
   constexpr int L = LdA::PER + LdB::PER;  // loads per thread per K-step
 
   // Loads [first, first + count) of slab `step` (the A loads come first in the numbering, then the B loads).
   auto issue_loads = [&](int step, int first, int count) {
     unsigned char* st = smem + (step % C::STAGES) * C::STAGE_BYTES;
-    const int k0 = step * C::BK;
+    const int k0 = at * C::BK;
     const bool tail = k0 + C::BK > klen;
     __amdgpu_buffer_rsrc_t ra_ = la.resource(), rb_ = lb.resource();
 #pragma unroll
@@ -354,7 +379,7 @@ __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap,
   // prologue: STAGES-1 slabs in flight
 #pragma unroll
   for (int s = 0; s < C::STAGES - 1; ++s)
-    if (s < nk) { issue_loads(s, 0, L); la.advance(); lb.advance(); }
+    if (s < nk) { issue_loads(s, 0, L); advance(); }
 
   for (int kt = 0; kt < nk; ++kt) {
     // Slab kt must have landed; the STAGES-2 younger ones may still be in flight.  Near the end fewer loads were
@@ -399,7 +424,7 @@ __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap,
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (more) { la.advance(); lb.advance(); }
+    if (more) advance();
   }
 
   __builtin_amdgcn_s_barrier();  // the ring is no longer read by any wave
