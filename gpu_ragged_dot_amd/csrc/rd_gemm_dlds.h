@@ -184,6 +184,7 @@ struct SplitK {
   float* partials = nullptr;    // [parts][NT * accumulators per thread] of this tile
   int32_t* counter = nullptr;   // arrivals so far; zero when the launch starts
   int parts = 1, part = 0;
+  bool edge_lines = false;      // see store_accumulators()
 };
 
 // Returns true when the caller holds the complete sums and must store them.  All threads of the work-group call it,
@@ -256,10 +257,16 @@ __device__ __forceinline__ bool splitk_combine(f32x16_t (&acc)[C::TM][C::TN], co
 // Only the wave itself touches its area, so no work-group barrier is needed in between.  The stores are nontemporal:
 // nothing in the launch reads the output, and kept out of L2 it leaves the operand slabs there (measured 2-3 % on
 // every product of a memory-bound shape, nothing on a matrix-core-bound one).
+//
+// edge_lines: where the output's row pitch is no multiple of 128 bytes, a row of the tile begins and ends inside a 128-byte
+// line that the neighbouring column tile completes.  Stored nontemporally such a line goes out in two parts and costs more
+// than two whole ones; with edge_lines the parts are stored plainly, so that L2 puts the line together, and only whole lines
+// stay nontemporal.  What L2 holds for it, it does not hold of the operands: it pays while a tile is little more than its
+// stores (kEdgeLineRows in rd_kernels.h).
 template <class C>
 __device__ __forceinline__ void store_accumulators(const f32x16_t (&acc)[C::TM][C::TN], int wm, int wn, int wave,
                                                    int lane, int a_lim, int b_lim, bf16_bits* __restrict__ Op, int ldo,
-                                                   unsigned char* smem) {
+                                                   unsigned char* smem, bool edge_lines = false) {
   unsigned char* st = smem + wave * (C::WM * C::EPI_PITCH);
 #pragma unroll
   for (int i = 0; i < C::TM; ++i)
@@ -300,7 +307,14 @@ __device__ __forceinline__ void store_accumulators(const f32x16_t (&acc)[C::TM][
     for (int b = 0; b < BATCH; ++b) {
       const int grow = wm * C::WM + (t0 + b) * ROWS_PER + r0;
       const int off = (grow < a_lim && col_live) ? (grow * ldo + gcol) * 2 : kOobOffset;
-      __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, off, 0, kCachePolicyStream);
+      if (!edge_lines) {
+        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, off, 0, kCachePolicyStream);
+      } else {
+        const int line = off - (int)(((uint32_t)(uintptr_t)Op + (uint32_t)off) & 127), row_at = grow * ldo * 2;
+        const bool whole = line >= row_at && line + 128 <= row_at + b_lim * 2 && off != kOobOffset;
+        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? off : kOobOffset, 0, kCachePolicyStream);
+        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? kOobOffset : off, 0, 0);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -429,7 +443,7 @@ __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap,
 
   __builtin_amdgcn_s_barrier();  // the ring is no longer read by any wave
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
-  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
+  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem, sk.edge_lines);
 }
 
 // Ping-pong schedule.  The eight waves form two groups of four (one wave of each group per SIMD).  A wave alternates

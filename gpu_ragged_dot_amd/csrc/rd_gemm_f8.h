@@ -221,7 +221,7 @@ __device__ __forceinline__ void gemm_tile_f8(const fp8_bits* __restrict__ Ap, in
 
   __builtin_amdgcn_s_barrier();  // the ring is no longer read by any wave
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
-  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
+  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem, sk.edge_lines);
 }
 
 // The ping-pong schedule of rd_gemm_dlds.h on the float8 fragments: the eight waves form two groups of four (one wave of
@@ -322,7 +322,7 @@ __device__ __forceinline__ void gemm_tile_f8_pingpong(const fp8_bits* __restrict
   }
   if (group == 0) __builtin_amdgcn_s_barrier();
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
-  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
+  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem, sk.edge_lines);
 }
 
 }  // namespace rd

@@ -345,6 +345,12 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   }
 }
 
+// tgmm tiles of at most this many rows store the lines at their edges plainly where the rows of dA are no whole number of
+// 128-byte lines (store_accumulators()).  us, before | now: 364 x 5376 x 9584 in 33 groups 1412 | 955 (128 x 128 tiles) and 1112 |
+// 811 (four-wave 256 x 256; n = 9600, whole lines: 619), 2640 x 2048 x 1000 in 33 60 | 39.  The line: between 80 and 100 rows the
+// two ways meet.  Not for the eight-wave cores, whose tiles are for longer groups: the mere branch cost them 2 %.
+constexpr int kEdgeLineRows = 80;
+
 template <class C>
 __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p) {
   typedef typename C::Elem E;
@@ -386,7 +392,9 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p
   }
   const E* Ap = static_cast<const E*>(p.x) + (size_t)row0 * p.k + kk0;
   const E* Bp = static_cast<const E*>(p.dy) + (size_t)row0 * p.n + col0;
-  run_tile<C>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem);
+  SplitK sk;
+  sk.edge_lines = rows <= kEdgeLineRows && sizeof(O) == 2 && ((p.n % 64) != 0 || (reinterpret_cast<uintptr_t>(p.dA) & 127) != 0);
+  run_tile<C>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem, sk);
 }
 
 // ---- host-side launchers, one set per compiled tile shape -------------------------------------------------------
