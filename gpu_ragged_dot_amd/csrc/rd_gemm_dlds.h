@@ -7,7 +7,7 @@
 // matrix-core fragment reads:
 //   K-major slab  [rows][BK]   : chunk c of row r sits at chunk c ^ ((r >> 1) & 7)        (BK = 64, 128-byte rows)
 //                                                       or c ^ ((r >> 2) & 3)              (BK = 32,  64-byte rows)
-//   MN-major slab [BK][rows]   : chunk c of contraction row kk sits at chunk c ^ ((kk & 3) << 2)
+//   MN-major slab [BK][rows]   : chunk c of contraction row kk sits at chunk c ^ ((kk & 3) << 2)   (64 rows: (kk & 1) << 2)
 // so that the 16 rows of a 128-bit fragment read, and the 4 rows of a transposing 64-bit read, fall into different
 // bank groups.
 #pragma once
@@ -70,6 +70,7 @@ struct DldsLoader {
   static constexpr int RPI = 1024 / ROW_BYTES;   // slab rows per wave-wide load
   static constexpr int CPR = ROW_BYTES / 16;     // 16-byte chunks per slab row
   static constexpr int ROWS = KMAJOR ? T : BK;
+  static constexpr int MN_SWIZZLE = CPR >= 16 ? 3 : CPR / 4 - 1;  // of an MN-major slab row's chunks
   static constexpr int INSTR = ROWS / RPI;       // wave-wide loads per slab
   static constexpr int PER = INSTR / NW;         // of which each wave issues
   static_assert(INSTR % NW == 0 && PER >= 1, "slab does not split evenly over the waves");
@@ -103,7 +104,7 @@ struct DldsLoader {
         voff[j] = r < lim ? (r * ld + c * 8) * 2 : kOobOffset;  // rows past the tile's limit: no memory access, zeros
         kcol = c * 8;  // identical for every j: r advances by a multiple of 16 rows per instruction slot
       } else {
-        const int c = pchunk ^ ((r & 3) << 2);
+        const int c = pchunk ^ ((r & MN_SWIZZLE) << 2);
         voff[j] = c * 8 < lim ? (r * ld + c * 8) * 2 : kOobOffset;
       }
     }
@@ -153,7 +154,7 @@ struct DldsFragReader {
     } else {
       const int q = lane >> 4, i = lane & 15;
       const int row = 8 * (q >> 1) + (i >> 2);
-      const int s = (i >> 2) & 3;
+      const int s = (i >> 2) & (T >= 128 ? 3 : T / 32 - 1);
       const int low = 2 * (q & 1) + ((i & 3) >> 1);
 #pragma unroll
       for (int j = 0; j < TILES; ++j) {

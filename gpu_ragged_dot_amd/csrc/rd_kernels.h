@@ -6,6 +6,7 @@
 #include "rd_gemm_f8.h"
 #include "rd_gemm_w4.h"
 #include "rd_gemm_w4r.h"
+#include "rd_gemm_ws.h"
 #include "rd_gemm_pp.h"
 #include "rd_gemm_rs.h"
 #include "rd_gemm_tile.h"
@@ -92,6 +93,7 @@ __device__ __forceinline__ void run_tile(const typename C::Elem* Ap, int lda, in
     if (klen >= kW4RMinK) gemm_tile_w4r<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
     else gemm_tile_w4<W4Cfg<C::BM, C::BN, true, true, 5, C::HALF>>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
   }
+  else if constexpr (IsWs<C>::value) gemm_tile_ws<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
   else if constexpr (IsW4<C>::value) gemm_tile_w4<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
   else if constexpr (C::MIXED) gemm_tile_pingpong_mixed<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
   else if constexpr (C::DLDS && C::PINGPONG) gemm_tile_pingpong<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
@@ -136,6 +138,11 @@ constexpr int kMaxSplitParts = 8;
 // 4096 x 4096 in 8 groups went from 377 to 429 us: its 256 x 256 pieces cost what a bf16 core's do).
 template <class C, class = void>
 struct SplitCost { static constexpr int QUARTERS = sizeof(typename C::Elem) == 1 ? 2 : 4, MIN_K = 512; };
+// The tiles of rd_gemm_ws.h have an eighth to half the partial sums: cut from k = 3658 on where few tiles are expected, from 5700
+// on always (kWsCutMinK in rd_capi.hip); three pieces already bring most of it.  492 x 4848 x 272 in 19 groups 35 -> 23 us, 720 x
+// 4016 x 352 in 9 31 -> 21, 259 x 10432 x 336 in 3 56 -> 21; 477 x 5920 x 3120 in 4 (128 x 128) 54 -> 40.
+template <class C>
+struct SplitCost<C, typename std::enable_if<IsWs<C>::value>::type> { static constexpr int QUARTERS = 7, MIN_K = 1280; };
 template <class C>
 struct SplitCost<C, typename std::enable_if<IsRs<C>::value>::type> {
   static constexpr int QUARTERS = C::FULL ? 32 : 4, MIN_K = C::FULL ? 256 : 512;
@@ -412,6 +419,7 @@ struct TileVariant {
   int any_pitch_core;  // 1: the register-staged core of rd_gemm_rs.h (k >= 8, n >= 8, 32-bit offsets within 256 rows)
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
   int split_quarters, split_min_k;  // SplitCost of the gmm kernels
+  int ws_core;  // 1: the core of rd_gemm_ws.h
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product
   tgmm_launch_fn tgmm;
 };

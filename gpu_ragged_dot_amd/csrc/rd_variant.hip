@@ -1,5 +1,5 @@
 // One compiled tile shape.  Built once per entry of the variant list in the Makefile, with
-//   -DRD_BM= -DRD_BN= -DRD_BK= -DRD_WAVES_M= -DRD_WAVES_N= -DRD_VEC= -DRD_NAME= [-DRD_DLDS=1|2|3|4 -DRD_STAGES= -DRD_PINGPONG=1
+//   -DRD_BM= -DRD_BN= -DRD_BK= -DRD_WAVES_M= -DRD_WAVES_N= -DRD_VEC= -DRD_NAME= [-DRD_DLDS=1|2|3|4|5 -DRD_STAGES= -DRD_PINGPONG=1
 //   -DRD_F32=1|2|3|4]
 // and exports a getter rd_variant_<name>() for its TileVariant record that the C-ABI file collects.
 #include "rd_kernels.h"
@@ -49,6 +49,11 @@ typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0, RD_F32 == 1> CfgT
 typedef W4Cfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, true> CfgNN;
 typedef W4RCfg<RD_BM, RD_BN, true> CfgNT;
 typedef W4Cfg<RD_BM, RD_BN, false, false, RD_STAGES, true> CfgTN;
+#elif (RD_F32 == 0 || RD_F32 == 4) && RD_DLDS == 5
+// the core of rd_gemm_ws.h, bf16 or float16
+typedef WsCfg<RD_BM, RD_BN, RD_BK, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, RD_F32 == 4> CfgNN;
+typedef WsCfg<RD_BM, RD_BN, RD_BK, true, true, RD_STAGES, RD_F32 == 4> CfgNT;
+typedef WsCfg<RD_BM, RD_BN, RD_BK, false, false, RD_STAGES, RD_F32 == 4> CfgTN;
 #elif RD_F32 == 3 && RD_DLDS
 // float8 e4m3fn arrays on the float8 matrix-core instruction, direct-to-LDS (rd_gemm_f8.h).  tgmm reads x^T as an
 // MN-major operand, whose slab rows span the tile's rows: only for tile heights that are multiples of 256.
@@ -105,7 +110,7 @@ extern "C" const rd::TileVariant* RD_CAT(rd_variant_, RD_NAME)() {
   static const rd::TileVariant v = {
       RD_STR(RD_NAME), RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, RD_VEC, /*dtype: RD_DTYPE_* */ RD_F32, RD_DLDS != 0, RD_STAGES,
       RD_ANY_PITCH, /*splitk*/ RD_ANY_PITCH || (RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4)),
-      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K,
+      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::IsWs<rd::CfgNN>::value,
 #ifdef RD_NO_TGMM
       &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr};
 #else

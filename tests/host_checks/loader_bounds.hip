@@ -224,6 +224,9 @@ int main() {
   ok = ok && check_loader<128, 32, 8, false>("128 x 256 ping-pong core, MN-major rows (tgmm)");
   ok = ok && check_loader<128, 32, 4, true>("128 x 128 core, K-major");
   ok = ok && check_loader<128, 32, 4, false>("128 x 128 core, MN-major");
+  ok = ok && check_loader<128, 64, 4, false>("128-column tiles, 64-wide MN-major slabs");
+  ok = ok && check_loader<256, 64, 4, false>("128 x 256 tiles, 64-wide MN-major slabs");
+  ok = ok && check_loader<64, 32, 4, false>("64-column tiles, MN-major") && check_loader<64, 64, 4, false>("64-column tiles, 64-wide MN-major slabs");
   ok = ok && check_loader<64, 32, 4, true>("64-row streaming routine, activations (32-wide slabs)");
   ok = ok && check_loader<64, 64, 4, true>("64-row streaming routine, activations (64-wide slabs)");
   ok = ok && check_loader<128, 64, 4, true>("128-row streaming routine, activations (64-wide slabs)");
