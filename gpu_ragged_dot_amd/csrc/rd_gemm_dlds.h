@@ -322,10 +322,9 @@ __device__ __forceinline__ void store_accumulators(const f32x16_t (&acc)[C::TM][
 }
 
 // start: the slab a tile whose configuration ROTATES begins with.  The rows of a K-major operand lie a whole row pitch apart, and
-// where that is a power of two (or close to it) the 128-byte pieces of one slab all fall into the same few memory channels.
-// Tiles that stream weights nobody shares all run in step, so all of them would ask the same channels at the same time; starting
-// at slabs of their own they spread over all.  2048 rows in 128 groups of 16, weights [g, n, k], us before -> after: k 2048, n 768 93
-// -> 73 (k 2112: 74), k 2048, n 1024 121 -> 89, k 4096, n 768 173 -> 138, k 2048, n 7168 689 -> 600; k 768 and 7168 level.
+// where that is a multiple of 4 KiB the 128-byte pieces of one slab all fall into the same few memory channels.  Tiles that stream
+// weights nobody shares all run in step, so all of them would ask the same channels at the same time; starting at slabs of their
+// own they spread over all (kRotatePitch in rd_kernels.h has the line and the times).
 template <class C>
 __device__ __forceinline__ void gemm_tile_dlds(const bf16_bits* __restrict__ Ap, int lda, int a_lim,
                                                const bf16_bits* __restrict__ Bp, int ldb, int b_lim, int klen,

@@ -184,6 +184,12 @@ __device__ __forceinline__ void band_walk(int id, int rows, int cols, int group_
   ri = band * group_m + (within - cj * gm);
 }
 
+// trans_rhs: the tiles that stream their weights begin at different slabs (gemm_tile_dlds()) where the weights' row pitch in
+// elements is a multiple of this.  us, all from slab 0 | spread: 2048 rows in 128 groups of 16: k 2048, n 768 93 | 73, n 1024 121 |
+// 89, n 7168 675 | 584, k 4096, n 768 172 | 137; 1024 rows in 64, n 1024: k 6144 152 | 126.  At other pitches, same rows: k 1536,
+// 1792, 2176, 2304, 2560, 5120, 7168 level, 3584 76 | 77, 3072 67 | 74.
+constexpr int kRotatePitch = 2048;
+
 template <class C, bool TRANS_RHS>
 __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) {
   typedef typename C::Elem E;
@@ -312,7 +318,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
         static_assert(S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT && S::BN == C::BN, "the short routine runs in the tall one's launch");
         static_assert(M::LDS_BYTES <= C::LDS_BYTES && M::NT == C::NT && M::BN == C::BN, "the 128-row routine runs in the tall one's launch");
         const int ldb = TRANS_RHS ? p.k : p.n;
-        const uint32_t start = (uint32_t)(mi * p.n_tiles + nj) * 13u;  // (odd: neighbouring tiles start far apart)
+        const uint32_t start = p.k % kRotatePitch == 0 ? (uint32_t)(mi * p.n_tiles + nj) * 13u : 0u;  // (odd: neighbouring tiles start far apart)
         if (rows <= kShortRows) gemm_tile_dlds<S>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk, start);
         else gemm_tile_dlds<M>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk, start);
         return;
