@@ -69,6 +69,11 @@ struct IsW4R { static constexpr bool value = false; };
 template <class C>
 struct IsW4R<C, decltype((void)C::W4R)> { static constexpr bool value = true; };
 
+template <class C, class = void>
+struct IsMixed { static constexpr bool value = false; };
+template <class C>
+struct IsMixed<C, typename std::enable_if<C::MIXED>::type> { static constexpr bool value = true; };
+
 // Element type of a configuration's output: its Out when it names one (float8 operands give bf16), else that of its operands.
 template <class C, class = void>
 struct OutOf { typedef typename C::Elem type; };
@@ -324,6 +329,27 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
         return;
       }
     }
+    if constexpr (IsMixed<C>::value) {
+      // The eight-wave core with a ring per operand: every row tile of at most 128 rows, a group's only one or its last, on
+      // eight-wave routines of 64 or 128 rows with 64-wide slabs of both operands, four or three of them in LDS.  On the tall
+      // routine such a tile takes about as long as a whole one: its waves skip their matrix-core work, but the launch pays the
+      // slab for slab hand-over of 256 rows.  Unlike on the four-wave core it pays for last tiles too: these routines keep the
+      // weights in L2 for the neighbouring tiles (no streaming policy).  Over 75 calls (4282 - 32768 rows, k and n of 448 - 8064, 4
+      // - 131 groups) 0.987 (gmm) and 0.983 times (trans_rhs) what the core took without them; with the 64-row routine
+      // alone 0.992 and 0.989, with the tall core's own schedule on 128 rows 0.991 and 0.986.  us, before | now: 11122 x 1088 x
+      // 768 in 64 skewed groups 52 | 46, trans_rhs 56 | 49; trans_rhs 26452 x 704 x 3712 in 46 199 | 177; 23628 x 2528 x
+      // 2112 in 218 skewed groups 548 | 505.
+      typedef DldsCfg<kShortRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 4> S;
+      typedef DldsCfg<kMidRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 3> M;
+      static_assert(S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "the short routine runs in the tall one's launch");
+      static_assert(M::LDS_BYTES <= C::LDS_BYTES && M::NT == C::NT, "the 128-row routine runs in the tall one's launch");
+      if (rows <= kMidRows) {
+        const int ldb = TRANS_RHS ? p.k : p.n;
+        if (rows <= kShortRows) gemm_tile_dlds<S>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk);
+        else gemm_tile_dlds<M>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk);
+        return;
+      }
+    }
     if constexpr (IsF8Direct<C>::value) {
       if constexpr (C::NW == 8 && C::WAVES_M == 2 && C::A_KMAJOR && C::BM > kShortRows) {
         // a group's single row tile of at most kShortRows rows, as above: a 64-row routine on 128-deep slabs (every load
@@ -426,6 +452,7 @@ struct TileVariant {
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
   int split_quarters, split_min_k;  // SplitCost of the gmm kernels
   int ws_core;  // 1: the core of rd_gemm_ws.h
+  int split_rings;  // 1: the core of rd_gemm_pp.h with a ring per operand
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product
   tgmm_launch_fn tgmm;
 };

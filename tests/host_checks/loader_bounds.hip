@@ -230,6 +230,8 @@ int main() {
   ok = ok && check_loader<64, 32, 4, true>("64-row streaming routine, activations (32-wide slabs)");
   ok = ok && check_loader<64, 64, 4, true>("64-row streaming routine, activations (64-wide slabs)");
   ok = ok && check_loader<128, 64, 4, true>("128-row streaming routine, activations (64-wide slabs)");
+  ok = ok && check_loader<64, 64, 8, true>("eight-wave 64-row routine, activations") && check_loader<128, 64, 8, true>("eight-wave 128-row routine, activations") &&
+       check_loader<256, 64, 8, false>("eight-wave short routines, MN-major weights");
   // the any-pitch core's: 16-bit elements, float32 rounded to bf16 at 16-byte pitches and at any, float32 as it is; the row
   // tiles' heights, and the column tiles
   ok = ok && check_rs_loader<64, 64, true, bf16_bits, false>() && check_rs_loader<128, 64, true, bf16_bits, false>() &&
