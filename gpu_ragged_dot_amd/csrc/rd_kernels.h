@@ -323,7 +323,9 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
         static_assert(S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT && S::BN == C::BN, "the short routine runs in the tall one's launch");
         static_assert(M::LDS_BYTES <= C::LDS_BYTES && M::NT == C::NT && M::BN == C::BN, "the 128-row routine runs in the tall one's launch");
         const int ldb = TRANS_RHS ? p.k : p.n;
-        const uint32_t start = p.k % kRotatePitch == 0 ? (uint32_t)(mi * p.n_tiles + nj) * 13u : 0u;  // (odd: neighbouring tiles start far apart)
+        // from the group, not the tile's place in the launch: a row's sums are added up in an order that the other groups'
+        // sizes do not change (odd factor: neighbouring tiles start far apart)
+        const uint32_t start = p.k % kRotatePitch == 0 ? (uint32_t)(gi * p.n_tiles + nj) * 13u : 0u;
         if (rows <= kShortRows) gemm_tile_dlds<S>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk, start);
         else gemm_tile_dlds<M>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk, start);
         return;

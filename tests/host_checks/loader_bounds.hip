@@ -2,8 +2,10 @@
 // every large-tile core shares - with direct-to-LDS loads and, in the register-staged core, with plain buffer loads.
 // No GPU is used: DldsLoader::init / advance are integer arithmetic and run here as they do on the device.
 //
-// Every K loop in the tree keeps one invariant: the loads of slab s are issued when the loader has been advanced s
-// times (resource() then describes the bytes from slab s to the end of the operand window), with the per-lane offsets
+// Every K loop in the tree keeps one invariant: the loads of slab s are issued when the loader stands at slab s - advanced
+// s times, or, in the streaming routines that begin at a slab of their own, advanced by the first slab's number, then once a
+// slab, and back to where it started behind the last one (resource() describes the bytes from slab s to the end of the
+// operand window) - with the per-lane offsets
 // voff[], and - for a K-major operand whose slab runs past the contraction length - the chunks at or past it replaced
 // by an offset beyond the buffer.  Under that invariant this program walks every load of every slab of every wave and
 // lane for the loader shapes compiled into the library, on operand windows with ragged edges (row / column limits,
@@ -33,8 +35,9 @@ using namespace rd;
 
 static long long g_loads = 0;
 
+// start: the slab the walk begins with; past the last slab it goes on with the first.
 template <int T, int BK, int NW, bool KMAJOR>
-static bool check_window(int lim, int ld, int klen, const char* what) {
+static bool check_window(int lim, int ld, int klen, const char* what, int start = 0) {
   typedef DldsLoader<T, BK, NW, KMAJOR> Ld;
   const int nk = (klen + BK - 1) / BK;
   // all (wave, lane) loaders, advanced in lock step
@@ -42,8 +45,12 @@ static bool check_window(int lim, int ld, int klen, const char* what) {
   for (int w = 0; w < NW; ++w)
     for (int l = 0; l < 64; ++l) ld_all[(size_t)w * 64 + l].init(nullptr, ld, lim, klen, w, l);
   const long long window = KMAJOR ? ((long long)(lim - 1) * ld + klen) * 2 : ((long long)(klen - 1) * ld + lim) * 2;
+  const std::vector<Ld> first = ld_all;
+  if (start > 0)
+    for (auto& L : ld_all) L.advance(start);
   std::vector<unsigned char> seen;
-  for (int s = 0; s < nk; ++s) {
+  for (int i = 0; i < nk; ++i) {
+    const int s = (start + i) % nk;
     const int k0 = s * BK, kend = k0 + BK < klen ? k0 + BK : klen;
     const int rows = KMAJOR ? lim : kend - k0, cols = KMAJOR ? kend - k0 : lim;  // the slab's valid elements, [rows][cols]
     seen.assign((size_t)rows * cols, 0);
@@ -94,8 +101,27 @@ static bool check_window(int lim, int ld, int klen, const char* what) {
                     (int)KMAJOR, lim, ld, klen, s, i / cols, i % cols);
         return false;
       }
-    for (auto& L : ld_all) L.advance();
+    for (size_t l = 0; l < ld_all.size(); ++l) {
+      if (s + 1 == nk) ld_all[l].rewind(first[l]);
+      else ld_all[l].advance();
+    }
   }
+  return true;
+}
+
+// The streaming routines' walks: from every slab of short contractions - fewer slabs than the ring is deep among them - and from
+// the first, second, middle and last of long ones; whole ranges, last slabs that are not full, and pieces of a cut along K.
+template <int T, int BK, int NW>
+static bool check_rotated(const char* what) {
+  for (int ld : {2048, 6144})
+    for (int lim : {1, 7, 33, 64, 128, 255, 256})
+      for (int klen : {8, 64, 72, 128, 136, 192, 320, 328, 640, 1344, 2048}) {
+        if (lim > T) continue;
+        const int nk = (klen + BK - 1) / BK;
+        for (int start = 0; start < nk; ++start)
+          if (nk <= 10 || start < 2 || start == nk / 2 || start == nk - 1)
+            if (!check_window<T, BK, NW, true>(lim, ld, klen, what, start)) return false;
+      }
   return true;
 }
 
@@ -230,6 +256,9 @@ int main() {
   ok = ok && check_loader<64, 32, 4, true>("64-row streaming routine, activations (32-wide slabs)");
   ok = ok && check_loader<64, 64, 4, true>("64-row streaming routine, activations (64-wide slabs)");
   ok = ok && check_loader<128, 64, 4, true>("128-row streaming routine, activations (64-wide slabs)");
+  ok = ok && check_rotated<64, 64, 4>("64-row streaming routine from any slab, activations") &&
+       check_rotated<128, 64, 4>("128-row streaming routine from any slab, activations") &&
+       check_rotated<256, 64, 4>("streaming routines from any slab, weights");
   ok = ok && check_loader<64, 64, 8, true>("eight-wave 64-row routine, activations") && check_loader<128, 64, 8, true>("eight-wave 128-row routine, activations") &&
        check_loader<256, 64, 8, false>("eight-wave short routines, MN-major weights");
   // the any-pitch core's: 16-bit elements, float32 rounded to bf16 at 16-byte pitches and at any, float32 as it is; the row
