@@ -272,7 +272,7 @@ def test_interleaved_block_order_is_transparent(vname, walk, trans_rhs):
     must equal, bit for bit, that of a call whose workspace holds the scheduling map and nothing else (blocks in walk
     order), and the oracle's within the usual bounds.  Long and short groups in every order, empty ones, a zero tail."""
     print(f"interleaved block order {vname} walk={walk} trans_rhs={trans_rhs}", flush=True)
-    k, n = 72, 4096
+    k, n = 72, 8192
     rng = np.random.default_rng(5)
     lens = list(rng.integers(1, 120, size=58)) + [0, 0, 0, 700, 1300, 257, 129, 128, 530]
     rng.shuffle(lens)
@@ -282,16 +282,17 @@ def test_interleaved_block_order_is_transparent(vname, walk, trans_rhs):
     lhs = oracle.round_to(rng.standard_normal((m, k)).astype(np.float32), "bfloat16")
     rhs = oracle.round_to((rng.standard_normal((g, k, n)) / k ** 0.5).astype(np.float32), "bfloat16")
     vid = [v.id for v in _capi.variants() if v.name.decode() == vname][0]
-    bm = [v.tile_m for v in _capi.variants() if v.id == vid][0]
+    bm, bn = [(v.tile_m, v.tile_n) for v in _capi.variants() if v.id == vid][0]
     plan = _capi.Plan(vid, walk[0], 0, walk[1], split_k=-1)
     x, A, gsd = util.bf16_dev(lhs), util.bf16_dev(rhs), torch.from_numpy(gs).cuda()
     Ad = A.mT.contiguous() if trans_rhs else A
     U = -(-m // bm) + g
-    assert U * (n // 256) >= 1024 and (-(-gs // bm)).sum() * (n // 256) >= 1024   # several rounds of live tiles
     map_only = -(-((g + 3 * U + 1) * 4) // 256) * 256
+    per_block = walk[0] * walk[1]
+    n_blocks, live_blocks = -(-U * (n // bn) // per_block), -(-int((-(-gs // bm)).sum()) * (n // bn) // per_block)
     outs = []
     for ws_bytes in (_capi.lib.rd_gmm_workspace_bytes(m, g, ctypes.byref(plan)), map_only):
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+        ws = torch.full((ws_bytes,), 0xA5, dtype=torch.uint8, device="cuda")
         y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
         rc = _capi.lib.rd_gmm(torch.cuda.current_stream().cuda_stream, x.data_ptr(), Ad.data_ptr(), gsd.data_ptr(),
                               y.data_ptr(), m, k, n, g, int(trans_rhs), _capi.RD_DTYPE_BF16, ctypes.byref(plan),
@@ -299,6 +300,12 @@ def test_interleaved_block_order_is_transparent(vname, walk, trans_rhs):
         assert rc == _capi.RD_OK, _capi.lib.rd_last_error()
         torch.cuda.synchronize()
         outs.append(y)
+        if ws_bytes > map_only:  # the order was built: behind the map, its two lists hold every live block once
+            order = ws[map_only:map_only + 4 * (2 + n_blocks)].view(torch.int32).tolist()
+            n_long = order[0]
+            assert 0 < n_long < live_blocks and order[1] == live_blocks
+            dealt = order[2:2 + n_long] + order[2 + n_blocks - (live_blocks - n_long):2 + n_blocks]
+            assert sorted(dealt) == list(range(live_blocks))
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     got = util.to_np(outs[0])
     util.assert_close_rows(got, oracle.gmm(lhs, rhs, gs), int(gs.sum()), util.BF16_EPS, "interleaved")
