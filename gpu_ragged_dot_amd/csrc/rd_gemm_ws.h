@@ -16,15 +16,16 @@
 // round of 256 x 256 tiles it moves more bytes through LDS per product than those and is behind (small_tile_variant() in
 // rd_capi.hip has the lines).
 //
+// STREAMS: a kernel whose tiles read the weights of groups of one row tile past the caches (gmm_kernel).
 #pragma once
 #include "rd_gemm_dlds.h"
 
 namespace rd {
 
-template <int BM_, int BN_, int BK_, bool A_KMAJOR_, bool B_KMAJOR_, int STAGES_, bool HALF_ = false>
+template <int BM_, int BN_, int BK_, bool A_KMAJOR_, bool B_KMAJOR_, int STAGES_, bool HALF_ = false, bool STREAMS_ = false>
 struct WsCfg {
   typedef bf16_bits Elem;  // 16 bits per element: bf16, or float16 with HALF
-  static constexpr bool F32 = false, WS = true, HALF = HALF_;
+  static constexpr bool F32 = false, WS = true, HALF = HALF_, STREAMS = STREAMS_;
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WAVES_M = 2, WAVES_N = 2, STAGES = STAGES_;
   static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, VEC = true, DLDS = true, PINGPONG = false, MIXED = false,
                         SPLITK = true;
@@ -54,14 +55,14 @@ template <int V>
 struct Int { static constexpr int value = V; };
 }  // namespace ws_detail
 
-template <class C, bool LIVE>
+template <class C, bool LIVE, int B_AUX>
 __device__ __forceinline__ void ws_kloop(const bf16_bits* __restrict__ Ap, int lda, int a_lim,
                                          const bf16_bits* __restrict__ Bp, int ldb, int b_lim, int klen,
                                          unsigned char* smem, int wave, int lane, f32x16_t (&acc)[C::TM][C::TN]) {
   const int wm = wave >> 1, wn = wave & 1;
   constexpr int S = C::STAGES;
   typedef DldsLoader<C::BM, C::BK, C::NW, C::A_KMAJOR> LdA;
-  typedef DldsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR> LdB;
+  typedef DldsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR, B_AUX> LdB;
   LdA la; LdB lb;
   la.init(Ap, lda, a_lim, klen, wave, lane);
   lb.init(Bp, ldb, b_lim, klen, wave, lane);
@@ -159,7 +160,8 @@ __device__ __forceinline__ void ws_kloop(const bf16_bits* __restrict__ Ap, int l
   }
 }
 
-template <class C>
+// B_AUX: cache policy of the B operand's loads, as in rd_gemm_dlds.h
+template <class C, int B_AUX = 0>
 __device__ __forceinline__ void gemm_tile_ws(const bf16_bits* __restrict__ Ap, int lda, int a_lim,
                                              const bf16_bits* __restrict__ Bp, int ldb, int b_lim, int klen,
                                              bf16_bits* __restrict__ Op, int ldo, bf16_bits* smem_,
@@ -176,8 +178,8 @@ __device__ __forceinline__ void gemm_tile_ws(const bf16_bits* __restrict__ Ap, i
     for (int j = 0; j < C::TN; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  if (patch_live) ws_kloop<C, true>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
-  else ws_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
+  if (patch_live) ws_kloop<C, true, B_AUX>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
+  else ws_kloop<C, false, B_AUX>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
   store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem, sk.edge_lines);
 }

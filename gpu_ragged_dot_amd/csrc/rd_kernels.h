@@ -331,6 +331,16 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
         return;
       }
     }
+    if constexpr (IsWs<C>::value) {
+      if constexpr (C::STREAMS) {
+        // a group's only row tile: nothing else reads its weights (streams_weights() in rd_capi.hip says when).  A kernel of
+        // its own: the loops of the tile of 128 x 256 fill the register file, and launches that do not stream stay as they are
+        if (it == 0 && group_rows <= C::BM) {
+          gemm_tile_ws<C, kCachePolicyStream>(Ap, p.k, rows, Bp, TRANS_RHS ? p.k : p.n, cols, klen, Op, p.n, smem, sk);
+          return;
+        }
+      }
+    }
     if constexpr (IsMixed<C>::value) {
       // The eight-wave core with a ring per operand: every row tile of at most 128 rows, a group's only one or its last, on
       // eight-wave routines of 64 or 128 rows with 64-wide slabs of both operands, four or three of them in LDS.  On the tall
@@ -457,6 +467,7 @@ struct TileVariant {
   int split_rings;  // 1: the core of rd_gemm_pp.h with a ring per operand
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product
   tgmm_launch_fn tgmm;
+  gmm_launch_fn gmm_nn_stream, gmm_nt_stream;  // the same products, the weights of groups of one row tile streamed past the caches; null: no such kernel
 };
 
 // Kernels that use more than 64 KB of LDS must opt in, once per device.

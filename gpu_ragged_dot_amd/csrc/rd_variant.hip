@@ -54,6 +54,15 @@ typedef W4Cfg<RD_BM, RD_BN, false, false, RD_STAGES, true> CfgTN;
 typedef WsCfg<RD_BM, RD_BN, RD_BK, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, RD_F32 == 4> CfgNN;
 typedef WsCfg<RD_BM, RD_BN, RD_BK, true, true, RD_STAGES, RD_F32 == 4> CfgNT;
 typedef WsCfg<RD_BM, RD_BN, RD_BK, false, false, RD_STAGES, RD_F32 == 4> CfgTN;
+// ... and with the weights of short groups streamed past the caches: the tiles that the default rules name for such launches
+#if RD_BN == 2 * RD_BM
+typedef WsCfg<RD_BM, RD_BN, RD_BK, true, false, RD_STAGES, RD_F32 == 4, /*streams*/ true> CfgNNStream;
+#define RD_NN_STREAM &rd::launch_gmm<rd::CfgNNStream, false>
+#endif
+#if RD_BK == 64
+typedef WsCfg<RD_BM, RD_BN, RD_BK, true, true, RD_STAGES, RD_F32 == 4, true> CfgNTStream;
+#define RD_NT_STREAM &rd::launch_gmm<rd::CfgNTStream, true>
+#endif
 #elif RD_F32 == 3 && RD_DLDS
 // float8 e4m3fn arrays on the float8 matrix-core instruction, direct-to-LDS (rd_gemm_f8.h).  tgmm reads x^T as an
 // MN-major operand, whose slab rows span the tile's rows: only for tile heights that are multiples of 256.
@@ -106,15 +115,23 @@ typedef TileCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, false, false, RD_VE
 #endif
 }  // namespace rd
 
+#ifndef RD_NN_STREAM
+#define RD_NN_STREAM nullptr
+#endif
+#ifndef RD_NT_STREAM
+#define RD_NT_STREAM nullptr
+#endif
+
 extern "C" const rd::TileVariant* RD_CAT(rd_variant_, RD_NAME)() {
   static const rd::TileVariant v = {
       RD_STR(RD_NAME), RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, RD_VEC, /*dtype: RD_DTYPE_* */ RD_F32, RD_DLDS != 0, RD_STAGES,
       RD_ANY_PITCH, /*splitk*/ RD_ANY_PITCH || (RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4)),
       rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::IsWs<rd::CfgNN>::value, rd::IsMixed<rd::CfgNN>::value,
 #ifdef RD_NO_TGMM
-      &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr};
+      &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr,
 #else
-      &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, &rd::launch_tgmm<rd::CfgTN>};
+      &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, &rd::launch_tgmm<rd::CfgTN>,
 #endif
+      RD_NN_STREAM, RD_NT_STREAM};
   return &v;
 }
