@@ -11,6 +11,8 @@
 // so that the 16 rows of a 128-bit fragment read, and the 4 rows of a transposing 64-bit read, fall into different
 // bank groups.
 #pragma once
+#include <type_traits>
+
 #include "rd_common.h"
 
 namespace rd {
@@ -259,9 +261,9 @@ __device__ __forceinline__ bool splitk_combine(f32x16_t (&acc)[C::TM][C::TN], co
 // nothing in the launch reads the output, and kept out of L2 it leaves the operand slabs there (measured 2-3 % on
 // every product of a memory-bound shape, nothing on a matrix-core-bound one).
 //
-// edge_lines: where the output's row pitch is no multiple of 128 bytes, a row of the tile begins and ends inside a 128-byte
-// line that the neighbouring column tile completes.  Stored nontemporally such a line goes out in two parts and costs more
-// than two whole ones; with edge_lines the parts are stored plainly, so that L2 puts the line together, and only whole lines
+// edge_lines: where the output's row pitch is no multiple of 64 bytes, a row of the tile begins and ends inside one half of a
+// 128-byte line that the neighbouring column tile completes.  Stored nontemporally such a line goes out in two parts and costs
+// more than two whole ones (whole halves cost nothing more); with edge_lines the parts are stored plainly, so that L2 puts the line together, and only whole lines
 // stay nontemporal.  What L2 holds for it, it does not hold of the operands: it pays while a tile is little more than its
 // stores (kEdgeLineRows in rd_kernels.h).
 template <class C>
@@ -297,28 +299,33 @@ __device__ __forceinline__ void store_accumulators(const f32x16_t (&acc)[C::TM][
   constexpr int NIT = C::WM / ROWS_PER;       // wave-wide stores per patch
   constexpr int BATCH = NIT < 8 ? NIT : 8;    // LDS reads in flight ahead of their stores
   static_assert(NIT % BATCH == 0, "whole batches");
+  auto store = [&](auto edge_tag) {
+    constexpr bool EDGE = decltype(edge_tag)::value;
 #pragma unroll
-  for (int t0 = 0; t0 < NIT; t0 += BATCH) {
-    u32x4_t v[BATCH];
+    for (int t0 = 0; t0 < NIT; t0 += BATCH) {
+      u32x4_t v[BATCH];
 #pragma unroll
-    for (int b = 0; b < BATCH; ++b)
-      v[b] = *reinterpret_cast<const u32x4_t*>(st + ((t0 + b) * ROWS_PER + r0) * C::EPI_PITCH + chunk * 16);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int b = 0; b < BATCH; ++b)
+        v[b] = *reinterpret_cast<const u32x4_t*>(st + ((t0 + b) * ROWS_PER + r0) * C::EPI_PITCH + chunk * 16);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int b = 0; b < BATCH; ++b) {
-      const int grow = wm * C::WM + (t0 + b) * ROWS_PER + r0;
-      const int off = (grow < a_lim && col_live) ? (grow * ldo + gcol) * 2 : kOobOffset;
-      if (!edge_lines) {
-        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, off, 0, kCachePolicyStream);
-      } else {
-        const int line = off - (int)(((uint32_t)(uintptr_t)Op + (uint32_t)off) & 127), row_at = grow * ldo * 2;
-        const bool whole = line >= row_at && line + 128 <= row_at + b_lim * 2 && off != kOobOffset;
-        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? off : kOobOffset, 0, kCachePolicyStream);
-        __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? kOobOffset : off, 0, 0);
+      for (int b = 0; b < BATCH; ++b) {
+        const int grow = wm * C::WM + (t0 + b) * ROWS_PER + r0;
+        const int off = (grow < a_lim && col_live) ? (grow * ldo + gcol) * 2 : kOobOffset;
+        if constexpr (!EDGE) {
+          __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, off, 0, kCachePolicyStream);
+        } else {
+          const int line = off - (int)(((uint32_t)(uintptr_t)Op + (uint32_t)off) & 127), row_at = grow * ldo * 2;
+          const bool whole = line >= row_at && line + 128 <= row_at + b_lim * 2 && off != kOobOffset;
+          __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? off : kOobOffset, 0, kCachePolicyStream);
+          __builtin_amdgcn_raw_buffer_store_b128(v[b], orsrc, whole ? kOobOffset : off, 0, 0);
+        }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  };
+  if (edge_lines) store(std::true_type());
+  else store(std::false_type());
 }
 
 // start: the slab a tile whose configuration ROTATES begins with.  The rows of a K-major operand lie a whole row pitch apart, and

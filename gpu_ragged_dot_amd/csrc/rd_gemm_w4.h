@@ -192,7 +192,7 @@ __device__ __forceinline__ void gemm_tile_w4(const bf16_bits* __restrict__ Ap, i
   else w4_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
 
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
-  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem, sk.edge_lines);
+  store_accumulators<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
 }
 
 }  // namespace rd

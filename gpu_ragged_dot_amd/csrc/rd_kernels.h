@@ -54,6 +54,7 @@ struct TgmmArgs {
   int g_first;     // dA[i] belongs to group g_first + i of group_sizes / group_offsets
   int k_tiles, n_tiles;  // ceil(k / BM), ceil(n / BN)
   int group_m;
+  bool edge_lines;  // the launch takes the kernel that stores the lines at its tiles' edges apart, where it has one (kEdgeLineRows)
   const int32_t* group_order;  // null, or the records of the order in which the launch visits the groups (launch_sched_map)
 };
 
@@ -397,12 +398,26 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
 }
 
 // tgmm tiles of at most this many rows store the lines at their edges plainly where the rows of dA are no whole number of
-// 128-byte lines (store_accumulators()).  us, before | now: 364 x 5376 x 9584 in 33 groups 1412 | 955 (128 x 128 tiles) and 1112 |
-// 811 (four-wave 256 x 256; n = 9600, whole lines: 619), 2640 x 2048 x 1000 in 33 60 | 39.  The line: between 80 and 100 rows the
-// two ways meet.  Not for the eight-wave cores, whose tiles are for longer groups: the mere branch cost them 2 %.
+// 64-byte halves of a line (store_accumulators()) and the groups average no more (tgmm_impl()).  A kernel of its own: in one
+// kernel for both the mere branch cost launches with whole lines 1 to 3 %, those of the four-wave 256 x 256 core 5 %.  Times with over
+// without, geometric means over 1640 random calls with such rows, groups averaging under 20 | 20 to 40 | 40 to 60 | 60 to 80 | 80 to
+// 120 | 120 to 400 rows:
+//   128 x 128, three work-groups to a unit    0.66 | 0.70 | 0.81 | 0.81 | 0.90 | 0.97
+//   128 x 256 of rd_gemm_ws.h, bf16           0.78 | 0.85 | 0.86 | 0.93 | 0.97 | 1.00
+//                              float16        0.78 | 0.79 | 0.88 | 0.92 | 0.95 | 1.00
+//   128 x 128 of rd_gemm_ws.h                 0.81 | 0.87 | 0.93 | 0.93 | 0.99 | 1.00
+//   256 x 256, float8                         0.87 | 0.89 | 0.90 | 0.92 | 0.99 | 1.03
+// 364 x 5376 x 9584 in 33 groups (128 x 128) 1412 -> 955 us, 2640 x 2048 x 1000 in 33 60 -> 39.  Rows of whole halves: 1.04, up to 1.3
+// (7459 x 14112 x 544 in 199 groups 933 | 996).  Not for the bf16 and float16 256 x 256 cores, whose tiles are for longer groups.
 constexpr int kEdgeLineRows = 80;
-
+template <class C, class = void>
+struct StoresEdgeLines { static constexpr bool value = IsF8Direct<C>::value || IsWs<C>::value; };
 template <class C>
+struct StoresEdgeLines<C, typename std::enable_if<C::DLDS && !C::PINGPONG && !IsF8Direct<C>::value && !IsWs<C>::value>::type> {
+  static constexpr bool value = !IsW4<C>::value && !IsW4R<C>::value;
+};
+
+template <class C, bool EDGE_LINES = false>
 __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p) {
   typedef typename C::Elem E;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -444,7 +459,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p
   const E* Ap = static_cast<const E*>(p.x) + (size_t)row0 * p.k + kk0;
   const E* Bp = static_cast<const E*>(p.dy) + (size_t)row0 * p.n + col0;
   SplitK sk;
-  sk.edge_lines = rows <= kEdgeLineRows && sizeof(O) == 2 && ((p.n % 64) != 0 || (reinterpret_cast<uintptr_t>(p.dA) & 127) != 0);
+  sk.edge_lines = EDGE_LINES && rows <= kEdgeLineRows;
   run_tile<C>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem, sk);
 }
 
@@ -495,6 +510,8 @@ int launch_gmm(hipStream_t s, const GmmArgs& a) {
 template <class C>
 int launch_tgmm(hipStream_t s, const TgmmArgs& a) {
   auto kern = tgmm_kernel<C>;
+  if constexpr (StoresEdgeLines<C>::value)
+    if (a.edge_lines) kern = tgmm_kernel<C, true>;
   const int attr_rc = allow_big_lds(reinterpret_cast<const void*>(kern), C::LDS_BYTES);
   if (attr_rc != hipSuccess) return attr_rc;
   const int grid = 8 * a.g * ((a.k_tiles * a.n_tiles + 7) / 8);
