@@ -84,3 +84,16 @@ def test_default_plans_name_a_tile_that_takes_the_product():
             seen.add(_capi.variants()[plan.variant].name.decode())
     missing = {v[1] for v in VARIANTS} - seen
     assert not missing, missing
+
+
+def test_default_tiles_by_rounds():
+    """Which core the rules name where a launch is two thirds to one round of 256 x 256 tiles, a round and a bit, or several rounds; and
+    for groups of a quarter to half a tile's height whose weights the last-level cache holds."""
+    name = lambda op, m, k, n, g: _capi.variants()[_capi.default_plan(op, m, k, n, g, _capi.RD_DTYPE_BF16).variant].name.decode()
+    assert name(1, 4096, 4096, 2048, 16) == "w256x256x32_w2x2_s5"      # 192 expected tiles
+    assert name(1, 5120, 4096, 2560, 20) == "v128x256x64_w2x2_s3"      # 300
+    assert name(1, 5476, 10296, 3256, 39) == "w256x256x32_w2x2_s5"     # 540
+    assert name(1, 2560, 1024, 2048, 32) == "q256x256x32_w2x4"         # 80 rows a group, 134 MB of weights
+    assert name(0, 2560, 1024, 2048, 32) == "q256x256x32_w2x4"
+    assert name(1, 2560, 4096, 4096, 32) == "w256x256x32_w2x2_s5"      # 80 rows, 1.1 GB
+    assert name(1, 2560, 1024, 4096, 64) == name(0, 2560, 1024, 4096, 64) == "w256x256x32_w2x2_s5"  # 40 rows
