@@ -144,7 +144,7 @@ constexpr int kMaxSplitParts = 8;
 // 4096 x 4096 in 8 groups went from 377 to 429 us: its 256 x 256 pieces cost what a bf16 core's do).
 template <class C, class = void>
 struct SplitCost { static constexpr int QUARTERS = sizeof(typename C::Elem) == 1 ? 2 : 4, MIN_K = 512; };
-// The tiles of rd_gemm_ws.h have an eighth to half the partial sums: cut from k = 3658 on where few tiles are expected, from 5700
+// The tiles of rd_gemm_ws.h have a sixteenth to half the partial sums: cut from k = 3658 on where few tiles are expected, from 5700
 // on always (kWsCutMinK in rd_capi.hip); three pieces already bring most of it.  492 x 4848 x 272 in 19 groups 35 -> 23 us, 720 x
 // 4016 x 352 in 9 31 -> 21, 259 x 10432 x 336 in 3 56 -> 21; 477 x 5920 x 3120 in 4 (128 x 128) 54 -> 40.
 template <class C>
