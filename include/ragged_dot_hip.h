@@ -87,9 +87,11 @@ typedef struct rd_plan {
                     this many columns (32, 64 or 128) of one expert; RD_DECODE_ROWS the one that gives it whole rows
                     for a slice of the contraction range (fp32 partial sums in the workspace, n <= 2048) or, with
                     trans_rhs, whole weight rows of a slice of the columns (no partial sums, k <= 8192) */
-  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round and k >= 6400 (float8: 12800, float32: 800), cut
-                  those tiles' contraction range over up to sqrt(k)/20 work-groups (float32: sqrt(k)/7; fp32 partial sums in the workspace); n > 0 =
-                  cut them over up to n (at most 8) whatever k is; -1 = never */
+  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round and k >= 6400 (float8: 12800, float32: 800,
+                  the variants v* and hv*: 3658 where about half a round of tiles or less is expected, 5700 otherwise), cut
+                  those tiles' contraction range over up to sqrt(k)/20 work-groups (float32: sqrt(k)/7, v* and hv*: sqrt(k)/15; fp32 partial
+                  sums in the workspace); n > 0 = cut them over up to n (at most 8) whatever k is; -1 = never.  A default plan may name
+                  one of v* / hv* for any bfloat16 or float16 call: who relies on uncut sums asks for -1 */
 } rd_plan;
 
 int rd_abi_version(void);
