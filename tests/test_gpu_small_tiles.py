@@ -97,3 +97,5 @@ def test_default_tiles_by_rounds():
     assert name(0, 2560, 1024, 2048, 32) == "q256x256x32_w2x4"
     assert name(1, 2560, 4096, 4096, 32) == "w256x256x32_w2x2_s5"      # 80 rows, 1.1 GB
     assert name(1, 2560, 1024, 4096, 64) == name(0, 2560, 1024, 4096, 64) == "w256x256x32_w2x2_s5"  # 40 rows
+    assert name(2, 32768, 768, 2048, 128) == "v128x256x32_w2x2_s3"     # tgmm, x of 50 MB
+    assert name(2, 32768, 2048, 768, 128) == "p256x256x32_w2x4_s4"     # 134 MB
