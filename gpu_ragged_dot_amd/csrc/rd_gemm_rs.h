@@ -1,8 +1,8 @@
-// Four-wave GEMM core for operands that cannot be loaded straight into LDS: row pitches that are no multiple of 16 bytes
+// GEMM core for operands that cannot be loaded straight into LDS: row pitches that are no multiple of 16 bytes
 // (bf16 and float16), float32 arrays that are rounded to bf16 on the way (compute_dtype = bfloat16), and float32 arrays of
-// any pitch multiplied as they are.  A 256 x 256 tile held by a 2 x 2 grid of waves, 128 x 128 per wave, as in
-// rd_gemm_w4.h (or a smaller tile, several work-groups to a compute unit); HBM -> registers -> LDS as in rd_gemm_w4r.h, for
-// any of the four operand layouts.
+// any pitch multiplied to float32's accuracy.  A 256 x 256 tile held by a 2 x 2 grid of waves, 128 x 128 per wave, as in
+// rd_gemm_w4.h, or a smaller tile, several work-groups to a compute unit (float32 to its accuracy: 2 x 4 waves); HBM -> registers
+// -> LDS as in rd_gemm_w4r.h, for any of the four operand layouts.
 //
 // What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
 // element per instruction where the pitch is odd, one slab in flight where the source is float32 - at 40-85 and 300-430
@@ -17,9 +17,21 @@
 //    operands, and two slabs are in flight in registers beside the two in LDS (bf16: 2 x 64 KB, float32 rounded: 2 x 32 KB);
 //  * the pieces are converted and written to LDS, and their registers refilled, spread evenly over the gaps between the
 //    matrix-core instructions of a slab.
-// float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most: the plain tile of
-// rd_gemm_f32.h, one slab of 16 ahead with element-wise LDS traffic, kept it busy 72-78 % of the time (4096 x 4096 x 3072:
-// 946 / 870 / 883 us), this core 86-92 % (766 / 733 / 713 us).
+// float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most, of which this core reaches 86-92 %
+// (4096 x 4096 x 3072: 766 / 733 / 713 us).  So float32 goes through the bf16 matrix cores, 16 times as fast, as three bf16 terms a number
+// (THREE): x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1) holds all 24 bits, and of the nine products
+// of two numbers' terms the three left out (x1 y2, x2 y1, x2 y2: |x1| <= 2^-8 |x|, |x2| <= 2^-17 |x|) come to at most 2^-24 of the whole one,
+// what one rounding of float32 may cost, and to a fifth of that as a root mean square.
+//  * The terms are made on the way into LDS, which holds three planes of a slab in the bf16 layout, and all three of a
+//    fragment are read per substep: 24 matrix-core instructions per 12 fragments (128 x 256 tile, eight waves of 64 x 64), half the
+//    fragment reads of a bf16 product.  A piece's way takes 28 vector instructions, in seven steps spread over the gaps between matrix-core
+//    instructions; eight waves, two on a SIMD, keep the matrix cores busy 74 % of the time, four of 64 x 128 69 %.
+//  * 16384 x 4096 x 2048 in one group, tgmm: 1274 us (216 TFLOP/s, i.e. 1294 on the bf16 matrix cores; 881 us on zeros), FULL on
+//    128 x 128 tiles 1879; 8192 x 2048 x 2048 in 16 softmax-sized groups, fwd / dlhs / drhs: 377 / 378 / 380, FULL 574 / 594 / 595.
+//    Power bounds it, as it does the bf16 products.
+//  * The error against sums in float64 is 0.83-0.87 of FULL's (16 products are added up per rounding, two there): relative 2-norm on N(0, 1) data
+//    2.4e-7 (FULL 2.9e-7) for 256 products, 6.8e-7 (8.0e-7) for 2048; over 90 random sizes never above FULL's.
+//  * Where the terms do not hold a number, the tile is computed again by FULL (kThreeLeast).
 // One loop serves all slabs.  Where a load goes is a clamped offset from a base; on the slab that holds the last contraction
 // index the base, the offset and its limit change (enter_last), so that no load touches memory outside the operand's rows,
 // and from there on what is not the operand's is cut off on the way into LDS (trim).  A second loop for those slabs, with
@@ -32,31 +44,34 @@
 namespace rd {
 
 // Src: bf16_bits, f16_t, or float (float32 out).  FULL: float32 stays float32 on its way through LDS and is multiplied by
-// v_mfma_f32_32x32x2_f32; otherwise it is rounded to bf16.  VEC: k and n are multiples of 8 (FULL: of 4), so that no piece
+// v_mfma_f32_32x32x2_f32; THREE: it becomes three bf16 terms; otherwise it is rounded to bf16.  VEC: k and n are multiples of 8 (float32: of 4), so that no piece
 // crosses the end of a row and the last slab needs no shifting.
-template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, typename Src, bool VEC_, bool FULL_ = false>
+template <int BM_, int BN_, bool A_KMAJOR_, bool B_KMAJOR_, typename Src, bool VEC_, bool FULL_ = false, bool THREE_ = false, int WAVES_N_ = 2>
 struct RsCfg {
   typedef Src Elem;
   static constexpr bool F32 = false, RS = true, HALF = std::is_same<Src, f16_t>::value;
-  static constexpr int BM = BM_, BN = BN_, BK = 128 / (int)sizeof(Src), WAVES_M = 2, WAVES_N = 2, STAGES = 2;
+  static constexpr int BM = BM_, BN = BN_, BK = 128 / (int)sizeof(Src), WAVES_M = 2, WAVES_N = WAVES_N_, STAGES = 2;
   static constexpr bool A_KMAJOR = A_KMAJOR_, B_KMAJOR = B_KMAJOR_, VEC = VEC_, DLDS = false, PINGPONG = false, MIXED = false,
                         SPLITK = true;
-  static constexpr int NW = 4, NT = 256;
-  static constexpr int WM = BM / 2, WN = BN / 2;
+  static constexpr int NW = WAVES_M * WAVES_N, NT = 64 * NW;
+  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
   static constexpr int TM = WM / 32, TN = WN / 32;
-  static constexpr bool FULL = FULL_;
-  static constexpr int LB = FULL ? 4 : 2;                  // bytes of an element in LDS
-  static constexpr int KMF = FULL ? 4 : 1;                 // matrix-core instructions per block and substep
+  static constexpr bool FULL = FULL_, THREE = THREE_;
+  static constexpr int LB = FULL ? 4 : 2;                  // bytes of an element (THREE: of each of its terms) in LDS
+  static constexpr int TERMS = THREE ? 3 : 1;
+  static constexpr int KMF = FULL ? 4 : THREE ? 6 : 1;     // matrix-core instructions per block and substep
   static constexpr int KSTEPS = FULL ? BK / 8 : BK / 16;   // substeps per slab
-  static constexpr int WAVES_PER_EU = BM * BN > 128 * 128 ? 1 : BM * BN < 128 * 128 ? 3 : 2;  // work-groups per compute unit
-  static constexpr int A_BYTES = BM * BK * LB, B_BYTES = BN * BK * LB;  // one slab in LDS
+  // work-groups per compute unit
+  static constexpr int WAVES_PER_EU = THREE ? (NW == 8 || BM * BN < 128 * 128 ? 2 : 1) : BM * BN > 128 * 128 ? 1 : BM * BN < 128 * 128 ? 3 : 2;
+  static constexpr int A_TERM = BM * BK * LB, B_TERM = BN * BK * LB;         // one term of a slab in LDS
+  static constexpr int A_BYTES = TERMS * A_TERM, B_BYTES = TERMS * B_TERM;  // one slab in LDS
   static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;
   static constexpr int EPI_PITCH = WN * 2 + 16;
   static constexpr int EPI_BYTES = sizeof(Src) == 2 ? NW * WM * EPI_PITCH : 0;
   static constexpr int RING_BYTES = 2 * SLOT_BYTES;
   static constexpr int LDS_BYTES = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
-  static_assert(FULL ? BM % 64 == 0 && BN % 64 == 0 : BM % (A_KMAJOR ? 64 : 128) == 0 && BN % 128 == 0, "tile shape");
-  static_assert(!FULL || std::is_same<Src, float>::value, "float32 only");
+  static_assert(FULL || THREE ? BM % 64 == 0 && BN % 64 == 0 : BM % (A_KMAJOR ? 64 : 128) == 0 && BN % 128 == 0, "tile shape");
+  static_assert(!(FULL && THREE) && (!(FULL || THREE) || std::is_same<Src, float>::value), "float32 only");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
@@ -114,7 +129,7 @@ struct RsLoader {
     row_step = (uint32_t)(NW * RPI * sizeof(Src)) * (uint32_t)ld;
     const int chunk = sizeof(Src) == LB ? piece : piece >> 1;  // 16-byte chunk of the LDS row; a rounded float32 piece fills half of one
     const int c = KMAJOR ? (LDS_ROW == 128 ? chunk ^ ((row0 >> 1) & 7) : chunk ^ ((row0 >> 2) & 3))
-                : LB == 4 ? chunk ^ (((row0 >> 2) & 1) << 3) : chunk ^ ((row0 & 3) << 2);
+                : LB == 4 ? chunk ^ (((row0 >> 2) & 1) << 3) : chunk ^ ((row0 & (T >= 128 ? 3 : T / 32 - 1)) << 2);
     lds = row0 * LDS_ROW + (c << 4) + (sizeof(Src) == LB ? 0 : (piece & 1) * 8);
     if (last == 0) enter_last(wave, lane);
   }
@@ -164,6 +179,9 @@ struct RsLoader {
       *reinterpret_cast<u32x2_t*>(d) = u32x2_t{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
     }
   }
+  __device__ __forceinline__ void put(unsigned char* region, int j, u32x2_t v) const {
+    *reinterpret_cast<u32x2_t*>(region + lds + j * LDS_STEP) = v;
+  }
   // The new base and the lane's offset are opaque to the compiler: it would otherwise carry an address per piece through
   // the loop, and there are no registers for those.
   __device__ __forceinline__ void advance(int wave, int lane) {
@@ -211,6 +229,13 @@ struct RsFrag {
   typedef typename std::conditional<C::FULL, RsFullFrag<T, TILES, KMAJOR>, DldsFragReader<T, C::BK, TILES, KMAJOR>>::type type;
 };
 
+// THREE multiplies exactly what FULL multiplies only where the terms hold the whole number, 24 bits: not below 2^-110, where the third
+// one's last bit leaves bf16 (2^-133), and not for infinities, NaN and what rounds to infinity.  The least magnitude seen on
+// the way into LDS (as bits << 1, less one: zeros come out on top) tells the former, a sum that is no finite number the
+// latter; a tile that has either is computed again by FULL.
+constexpr uint32_t kThreeLeast = ((127u - 110u) << 24) - 1u;
+__device__ __forceinline__ uint32_t umin(uint32_t a, uint32_t b) { return a < b ? a : b; }
+
 namespace rs_detail {
 template <int V>
 struct Int { static constexpr int value = V; };
@@ -224,9 +249,9 @@ struct Int { static constexpr int value = V; };
 template <class C, bool LIVE>
 __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap, int lda, int a_lim,
                                          const typename C::Elem* __restrict__ Bp, int ldb, int b_lim, int klen,
-                                         unsigned char* smem, int wave, int lane, f32x16_t (&acc)[C::TM][C::TN]) {
+                                         unsigned char* smem, int wave, int lane, f32x16_t (&acc)[C::TM][C::TN], uint32_t& least) {
   typedef typename C::Elem E;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   typedef RsLoader<C::BM, C::BK, C::NW, C::A_KMAJOR, E, C::VEC, C::LB> LdA;
   typedef RsLoader<C::BN, C::BK, C::NW, C::B_KMAJOR, E, C::VEC, C::LB> LdB;
   LdA la; LdB lb;
@@ -234,12 +259,15 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
   lb.init(Bp, ldb, b_lim, klen, wave, lane);
   typename RsFrag<C, C::BM, C::TM, C::A_KMAJOR>::type fra;
   typename RsFrag<C, C::BN, C::TN, C::B_KMAJOR>::type frb;
+  auto read_a = [&](const unsigned char* region, int r, int ks) { return fra.read(region + r / C::TM * C::A_TERM, r % C::TM, ks); };
+  auto read_b = [&](const unsigned char* region, int r, int ks) { return frb.read(region + r / C::TN * C::B_TERM, r % C::TN, ks); };
   fra.init(wm * C::WM, lane);
   frb.init(wn * C::WN, lane);
 
   const int nk = (klen + C::BK - 1) / C::BK;  // the last slab, nk - 1, holds the last contraction index
   constexpr int PA = LdA::PER, PB = LdB::PER, P = PA + PB;
-  constexpr int MF = C::TM * C::TN * C::KMF, R0 = C::TM + C::TN;
+  constexpr int RA = C::TM * C::TERMS, RB = C::TN * C::TERMS;  // fragments per substep
+  constexpr int MF = C::TM * C::TN * C::KMF, R0 = RA + RB;
   // pieces moved per substep: the last one, which follows the slab's barrier, takes pieces 0 .. HEAD - 1 (of the slab after
   // next), substep u of the others pieces part(u + 1) .. part(u + 2) - 1
   constexpr auto part = [](int u) constexpr { return u * P / C::KSTEPS; };
@@ -247,18 +275,43 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
   // What the gaps between a substep's matrix-core instructions carry.  Large patches: one fragment read each in the first
   // ones, then the pieces, spread out (a write and the load that refills its registers in one gap or in two).  Small
   // patches have fewer gaps than reads and pieces: every gap carries its share of both.
-  constexpr bool ROOMY = MF - R0 >= MOST;
+  constexpr bool ROOMY = !C::THREE && MF - R0 >= MOST;
   constexpr int GAP = MF - R0 >= 2 * MOST ? 2 : 1;
-  static_assert(HEAD >= 1, "every substep moves a piece");
 
   u32x4_t regs[2][P];
   auto fetch_one = [&](auto set_tag, int q) {
     constexpr int SET = decltype(set_tag)::value;
     regs[SET][q] = q < PA ? la.fetch(q) : lb.fetch(q - PA);
   };
+  // THREE: step st of a piece's way into LDS - its first term, what that leaves, the second term, what that leaves, the third -
+  // a few vector instructions each, for one gap between two matrix-core instructions.
+  constexpr int kThreeSteps = 7;
+  u32x2_t term;
+  auto three_step = [&](auto set_tag, int slot_off, int q, int st) {
+    constexpr int SET = decltype(set_tag)::value;
+    u32x4_t& r = regs[SET][q];
+    auto f = [&](int e) { const uint32_t w = r[e]; return __builtin_bit_cast(float, w); };
+    auto leave = [&](int h) {  // elements 2 h and 2 h + 1 minus their term: exact
+      r[2 * h] = __builtin_bit_cast(uint32_t, f(2 * h) - __builtin_bit_cast(float, term[h] << 16));
+      r[2 * h + 1] = __builtin_bit_cast(uint32_t, f(2 * h + 1) - __builtin_bit_cast(float, term[h] & 0xffff0000u));
+    };
+    auto note = [&](int h) { least = umin(least, umin((r[2 * h] << 1) - 1u, (r[2 * h + 1] << 1) - 1u)); };
+    if (st % 3 == 0) {
+      term = u32x2_t{pack_bf16x2(f(0), f(1)), pack_bf16x2(f(2), f(3))};
+      if (q < PA) la.put(smem + slot_off + st / 3 * C::A_TERM, q, term);
+      else lb.put(smem + slot_off + C::A_BYTES + st / 3 * C::B_TERM, q - PA, term);
+      if (st == 0) note(0);
+    } else {
+      if (st == 1) note(1);
+      leave(st % 3 - 1);
+    }
+  };
   auto commit_one = [&](auto set_tag, int slot_off, int q) {
     constexpr int SET = decltype(set_tag)::value;
-    if (q < PA) la.commit(smem + slot_off, q, regs[SET][q]);
+    if constexpr (C::THREE) {
+#pragma unroll
+      for (int st = 0; st < kThreeSteps; ++st) three_step(set_tag, slot_off, q, st);
+    } else if (q < PA) la.commit(smem + slot_off, q, regs[SET][q]);
     else lb.commit(smem + slot_off + C::A_BYTES, q - PA, regs[SET][q]);
   };
   // Before pieces first .. first + count - 1 of slab `step` are written: where that slab holds the last contraction index or
@@ -297,13 +350,13 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
   };
 
   typedef typename std::conditional<C::FULL, f32x4_t, bf16x8_t>::type frag_t;
-  frag_t fa[2][C::TM], fb[2][C::TN];
+  frag_t fa[2][RA], fb[2][RB];
   auto first_fragments = [&]() {
     if (LIVE) {
 #pragma unroll
-      for (int i = 0; i < C::TM; ++i) fa[0][i] = fra.read(smem, i, 0);
+      for (int i = 0; i < RA; ++i) fa[0][i] = read_a(smem, i, 0);
 #pragma unroll
-      for (int j = 0; j < C::TN; ++j) fb[0][j] = frb.read(smem + C::A_BYTES, j, 0);
+      for (int j = 0; j < RB; ++j) fb[0][j] = read_b(smem + C::A_BYTES, j, 0);
     }
   };
 
@@ -330,13 +383,13 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
       for (int m = 0; m < MF; ++m) {
         const int i = m % (C::TM * C::TN) / C::TN, j = m % C::TN, ke = m / (C::TM * C::TN);
         if (LIVE && ROOMY) {
-          if (m < C::TM) fa[(u + 1) & 1][m] = fra.read(ra, m, us);
-          else if (m < R0) fb[(u + 1) & 1][m - C::TM] = frb.read(rb, m - C::TM, us);
+          if (m < RA) fa[(u + 1) & 1][m] = read_a(ra, m, us);
+          else if (m < R0) fb[(u + 1) & 1][m - RA] = read_b(rb, m - RA, us);
         } else if (LIVE) {
 #pragma unroll
           for (int r = m * R0 / MF; r < (m + 1) * R0 / MF; ++r) {
-            if (r < C::TM) fa[(u + 1) & 1][r] = fra.read(ra, r, us);
-            else fb[(u + 1) & 1][r - C::TM] = frb.read(rb, r - C::TM, us);
+            if (r < RA) fa[(u + 1) & 1][r] = read_a(ra, r, us);
+            else fb[(u + 1) & 1][r - RA] = read_b(rb, r - RA, us);
           }
         }
         auto write = [&](int p) {
@@ -353,6 +406,14 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
             if ((m - R0) % GAP == 0) write(p);
             if ((m - R0) % GAP == GAP - 1) load(p);
           }
+        } else if constexpr (C::THREE) {
+          constexpr int ST = kThreeSteps + 1;  // the last one is the load
+#pragma unroll
+          for (int s = m * count * ST / MF; s < (m + 1) * count * ST / MF; ++s) {
+            if (s % ST == kThreeSteps) load(s / ST);
+            else if (last) three_step(rs_detail::Int<1 - NEXT>{}, cur_off, s / ST, s % ST);
+            else three_step(next_tag, next_off, first + s / ST, s % ST);
+          }
         } else {
 #pragma unroll
           for (int p = m * count / MF; p < (m + 1) * count / MF; ++p) { write(p); load(p); }
@@ -361,7 +422,11 @@ __device__ __forceinline__ void rs_kloop(const typename C::Elem* __restrict__ Ap
           // float32 results leave straight from the accumulators, a register holding 32 consecutive columns of a row;
           // 16-bit results go through LDS and want four consecutive columns per lane (operands swapped)
           if constexpr (C::FULL) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u & 1][i][ke], fb[u & 1][j][ke], acc[i][j], 0, 0, 0);
-          else if constexpr (sizeof(E) == 2) acc[i][j] = mfma_32x32x16<C::HALF>(fb[u & 1][j], fa[u & 1][i], acc[i][j]);
+          else if constexpr (C::THREE) {
+            // the six products of two terms that are not below the last bit of the whole one, the small ones first
+            constexpr int TA[6] = {0, 2, 1, 0, 1, 0}, TB[6] = {2, 0, 1, 1, 0, 0};
+            acc[i][j] = mfma_32x32x16<false>(fa[u & 1][TA[ke] * C::TM + i], fb[u & 1][TB[ke] * C::TN + j], acc[i][j]);
+          } else if constexpr (sizeof(E) == 2) acc[i][j] = mfma_32x32x16<C::HALF>(fb[u & 1][j], fa[u & 1][i], acc[i][j]);
           else acc[i][j] = mfma_32x32x16<false>(fa[u & 1][i], fb[u & 1][j], acc[i][j]);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -454,7 +519,7 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
                                              const SplitK& sk = SplitK()) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   const bool patch_live = wm * C::WM < a_lim && wn * C::WN < b_lim;
 
   f32x16_t acc[C::TM][C::TN];
@@ -465,8 +530,39 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  if (patch_live) rs_kloop<C, true>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
-  else rs_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc);
+  uint32_t least = ~0u;
+  if (patch_live) rs_kloop<C, true>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc, least);
+  else rs_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc, least);
+
+  if constexpr (C::THREE) {
+    // Values that the three terms do not hold: see kThreeLeast.  All four waves must agree, they share the slabs.
+    float probe = 0.f;  // NaN once a sum is no finite number
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) probe = fmaf(acc[i][j][v], 0.f, probe);
+    uint32_t* flags = reinterpret_cast<uint32_t*>(smem);
+    if (tid == 0) flags[0] = 0;
+    __syncthreads();
+    if (least < kThreeLeast || probe != probe) flags[0] = 1;
+    __syncthreads();
+    const uint32_t any = flags[0];
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane((int)any)) {
+      typedef RsCfg<C::BM, C::BN, C::A_KMAJOR, C::B_KMAJOR, typename C::Elem, C::VEC, true, false, C::WAVES_N> Full;
+      static_assert(Full::LDS_BYTES <= C::LDS_BYTES && Full::NT == C::NT, "runs in this launch");
+#pragma unroll
+      for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+      if (patch_live) rs_kloop<Full, true>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc, least);
+      else rs_kloop<Full, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc, least);
+    }
+  }
 
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
   if constexpr (sizeof(typename C::Elem) == 2) rs_store16<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
@@ -475,8 +571,7 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
 
 // A row tile of a gmm launch with fewer rows than its height: the same routine on the least multiple of 64 that holds them,
 // with as many fewer loads, LDS traffic and matrix-core instructions.  False: the tile is to be computed whole.
-// Not for float32 (FULL): 64 rows inside the 128 x 128 launch gained where its last round was short (8192 x 4096 x 4096 in 8
-// groups 2147 -> 2017 us) and lost elsewhere (8192 x 2048 x 2048 in 8: 607 -> 653), and the cut along K gives the former anyway.
+// (FULL is compiled with tiles of 64 rows only, and as what THREE falls back to.)
 template <class C, int ROWS = 64>
 __device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict__ Ap, int lda, int rows,
                                               const typename C::Elem* __restrict__ Bp, int ldb, int cols, int klen,
@@ -484,7 +579,7 @@ __device__ __forceinline__ bool rs_short_tile(const typename C::Elem* __restrict
   if constexpr (ROWS >= C::BM || C::FULL) {
     return false;
   } else {
-    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC> S;
+    typedef RsCfg<ROWS, C::BN, true, C::B_KMAJOR, typename C::Elem, C::VEC, false, C::THREE, C::WAVES_N> S;
     static_assert(C::A_KMAJOR && S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "runs in the tall tile's launch");
     if (rows > ROWS) return rs_short_tile<C, ROWS + 64>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, smem, sk);
     gemm_tile_rs<S>(Ap, lda, rows, Bp, ldb, cols, klen, Op, ldo, static_cast<unsigned char*>(smem), sk);

@@ -131,16 +131,14 @@ struct ShortTileCfg {
 struct SplitPlan {
   int first_tile;  // walk positions >= first_tile (and < live) are split; == live when nothing is
   int parts;
-  int tiles;       // live - first_tile
+  int tiles;       // live - first_tile, or twice that where each is computed in two halves
 };
 constexpr int kMaxSplitParts = 8;
 
 // What a cut is worth depends on the core: its K loop per contraction index and how much a piece's partial sums are.
 // QUARTERS: the former over the latter, in quarters of the 256 x 256 bf16 cores' (float8: twice the rate; float32
-// multiplied as it is: 16 times the time per multiplication, so twice per tile of a quarter of the size).  MIN_K: contraction indices a piece must keep.  float32 without
-// and with the cut, forward product: 256 x 16384 x 256 in 2 groups 291 -> 52 us, 2048 x 8192 x 1024 in 4 372 -> 283,
-// 512 x 4096 x 4096 in 3 202 -> 166, 8192 x 2048 x 2048 in 8 549 -> 506, 4096 x 4096 x 4096 in 4 1073 -> 992; level where the
-// last round is full or more than half full.  float32 rounded to bf16 stays at the bf16 cores' limit (cut from k = 3700 on, 8192 x
+// as three bf16 terms: 6 times the time per multiplication, partial sums of half a tile or a quarter; on the float32 instruction 16 times).
+// MIN_K: contraction indices a piece must keep.  float32 rounded to bf16 stays at the bf16 cores' limit (cut from k = 3700 on, 8192 x
 // 4096 x 4096 in 8 groups went from 377 to 429 us: its 256 x 256 pieces cost what a bf16 core's do).
 template <class C, class = void>
 struct SplitCost { static constexpr int QUARTERS = sizeof(typename C::Elem) == 1 ? 2 : 4, MIN_K = 512; };
@@ -151,16 +149,24 @@ template <class C>
 struct SplitCost<C, typename std::enable_if<IsWs<C>::value>::type> { static constexpr int QUARTERS = 7, MIN_K = 1280; };
 template <class C>
 struct SplitCost<C, typename std::enable_if<IsRs<C>::value>::type> {
-  static constexpr int QUARTERS = C::FULL ? 32 : 4, MIN_K = C::FULL ? 256 : 512;
+  static constexpr int QUARTERS = C::FULL ? 32 : C::THREE ? 24 : 4, MIN_K = C::FULL || C::THREE ? 256 : 512;
 };
 
+// Whether a launch computes the tiles of its last, partly filled round in halves of the columns, on the same core's tile of half the width.
+template <class C, class = void>
+struct HalvesLastRound { static constexpr bool value = false; };
+template <class C>
+struct HalvesLastRound<C, typename std::enable_if<IsRs<C>::value>::type> { static constexpr bool value = C::THREE && C::BN == 256 && C::A_KMAJOR; };
+
 // k_cost: k in units of what a bf16 K loop spends per element.
-__device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int min_k, int slots, int num_cus, int max_parts) {
+// halves: 2 where the pieces are pieces of half a tile's columns (HalvesLastRound): then the last round's tiles are halved whenever
+// all halves run at a time, and each half cut along K where the above says so.
+__device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int min_k, int slots, int num_cus, int max_parts, int halves = 1) {
   SplitPlan sp{live, 1, 0};
   if (slots <= 0 || live <= 0) return sp;
   const int first = (live / num_cus) * num_cus;
-  const int tiles = live - first;
-  if (tiles <= 0) return sp;
+  const int tiles = (live - first) * halves;
+  if (tiles <= 0 || tiles > imin(slots, num_cus)) return sp;
   // The piece that arrives last reads every piece's 256 KB of partial sums at what one compute unit can pull (about
   // 25 GB/s: ~10 us per piece), so the gain of a finer cut, T/parts for a K loop of T us, is soon eaten: parts ~
   // sqrt(T / 10 us), with T ~ k / 32 x 0.77 us, i.e. sqrt(k) / 20 - and below k = 6400 (4 pieces) cutting was measured
@@ -171,10 +177,12 @@ __device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int
   } else {
     int by_k = 1;
     while ((by_k + 1) * (by_k + 1) * 400 <= k_cost) ++by_k;
-    if (by_k < 4) return sp;
-    parts = imin(parts, by_k);
+    parts = by_k < 4 ? 1 : imin(parts, by_k);
   }
-  if (parts < 2) return sp;
+  if (parts < 2) {
+    if (halves == 1) return sp;
+    parts = 1;
+  }
   sp.first_tile = first; sp.parts = parts; sp.tiles = tiles;
   return sp;
 }
@@ -218,9 +226,10 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   const int total = imin(mapped ? uniform(*p.total_tiles) : scan.total_tiles, p.U);
   const int live = total * p.n_tiles;
   SplitPlan sp{live, 1, 0};
-  if constexpr (C::SPLITK) sp = split_plan(live, p.k, (int)((long long)p.k * SplitCost<C>::QUARTERS / 4), SplitCost<C>::MIN_K, p.split_slots, p.num_cus, p.max_parts);
+  if constexpr (C::SPLITK) sp = split_plan(live, p.k, (int)((long long)p.k * SplitCost<C>::QUARTERS / 4), SplitCost<C>::MIN_K, p.split_slots, p.num_cus, p.max_parts,
+                                               HalvesLastRound<C>::value ? 2 : 1);
 
-  int t;
+  int t, half = 0;
   SplitK sk;
   int k0 = 0, klen = p.k;
   if ((int)blockIdx.x < p.main_grid) {
@@ -262,10 +271,11 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
     if (id >= pieces) return;
     const int part = id / sp.tiles, tt = id - part * sp.tiles;
     t = sp.first_tile + tt;
+    if constexpr (HalvesLastRound<C>::value) { t = sp.first_tile + (tt >> 1); half = tt & 1; }
     const int k64 = (p.k + 63) >> 6;
     k0 = (int)((long long)k64 * part / sp.parts) << 6;
     klen = imin(p.k, (int)((long long)k64 * (part + 1) / sp.parts) << 6) - k0;
-    sk.partials = p.partials + (size_t)tt * sp.parts * (C::BM * C::BN);
+    sk.partials = p.partials + (size_t)tt * sp.parts * (C::BM * C::BN / (HalvesLastRound<C>::value ? 2 : 1));
     sk.counter = p.counters + tt;
     sk.parts = sp.parts;
     sk.part = part;
@@ -288,8 +298,9 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   const int w = t - band_row0 * p.n_tiles;
   const int nj = w / band_rows;
   const int mi = band_row0 + (w - nj * band_rows);
-  const int col0 = nj * C::BN;
-  const int cols = imin(C::BN, p.n - col0);
+  const int col0 = nj * C::BN + half * (C::BN / 2);
+  const int cols = imin(HalvesLastRound<C>::value && t >= sp.first_tile && t < live ? C::BN / 2 : C::BN, p.n - col0);
+  if (cols <= 0) return;  // the second half of a tile of few columns
 
   if (mi < total) {
     int it = mi - first_tile;
@@ -375,6 +386,15 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
             return;
           }
         }
+      }
+    }
+    if constexpr (HalvesLastRound<C>::value) {
+      if (t >= sp.first_tile) {
+        typedef RsCfg<C::BM, C::BN / 2, true, C::B_KMAJOR, E, C::VEC, C::FULL, C::THREE, C::WAVES_N> H;
+        static_assert(H::LDS_BYTES <= C::LDS_BYTES && H::NT == C::NT, "runs in the whole tile's launch");
+        const int ldb = TRANS_RHS ? p.k : p.n;
+        if (!rs_short_tile<H>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk)) run_tile<H>(Ap, p.k, rows, Bp, ldb, cols, klen, Op, p.n, smem, sk);
+        return;
       }
     }
     if constexpr (IsRs<C>::value) {
@@ -478,6 +498,7 @@ struct TileVariant {
   int any_pitch_core;  // 1: the register-staged core of rd_gemm_rs.h (k >= 8, n >= 8, 32-bit offsets within 256 rows)
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
   int split_quarters, split_min_k;  // SplitCost of the gmm kernels
+  int split_bn;  // columns of a piece of the K-split
   int ws_core;  // 1: the core of rd_gemm_ws.h
   int split_rings;  // 1: the core of rd_gemm_pp.h with a ring per operand
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product

@@ -23,8 +23,13 @@
 #define RD_F32 0
 #endif
 
-#if RD_DLDS == 4
+#if RD_DLDS == 4 || RD_DLDS == 6
 #define RD_ANY_PITCH 1
+#if RD_DLDS == 6
+#define RD_IS_THREE 1
+#else
+#define RD_IS_THREE 0
+#endif
 #undef RD_DLDS
 #define RD_DLDS 0
 #else
@@ -41,9 +46,9 @@ typedef f16_t RsElem;
 #else
 typedef bf16_bits RsElem;
 #endif
-typedef RsCfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RsElem, RD_VEC != 0, RD_F32 == 1> CfgNN;
-typedef RsCfg<RD_BM, RD_BN, true, true, RsElem, RD_VEC != 0, RD_F32 == 1> CfgNT;
-typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0, RD_F32 == 1> CfgTN;
+typedef RsCfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RsElem, RD_VEC != 0, RD_F32 == 1 && !RD_IS_THREE, RD_IS_THREE, RD_WAVES_N> CfgNN;
+typedef RsCfg<RD_BM, RD_BN, true, true, RsElem, RD_VEC != 0, RD_F32 == 1 && !RD_IS_THREE, RD_IS_THREE, RD_WAVES_N> CfgNT;
+typedef RsCfg<RD_BM, RD_BN, false, false, RsElem, RD_VEC != 0, RD_F32 == 1 && !RD_IS_THREE, RD_IS_THREE, RD_WAVES_N> CfgTN;
 #elif RD_F32 == 4 && RD_DLDS == 3
 // float16 arrays on the four-wave direct-to-LDS core: the bf16 core's data movement with the float16 instruction
 typedef W4Cfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, true> CfgNN;
@@ -126,7 +131,7 @@ extern "C" const rd::TileVariant* RD_CAT(rd_variant_, RD_NAME)() {
   static const rd::TileVariant v = {
       RD_STR(RD_NAME), RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, RD_VEC, /*dtype: RD_DTYPE_* */ RD_F32, RD_DLDS != 0, RD_STAGES,
       RD_ANY_PITCH, /*splitk*/ RD_ANY_PITCH || (RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4)),
-      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::IsWs<rd::CfgNN>::value, rd::IsMixed<rd::CfgNN>::value,
+      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::HalvesLastRound<rd::CfgNN>::value ? RD_BN / 2 : RD_BN, rd::IsWs<rd::CfgNN>::value, rd::IsMixed<rd::CfgNN>::value,
 #ifdef RD_NO_TGMM
       &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr,
 #else

@@ -87,9 +87,9 @@ typedef struct rd_plan {
                     this many columns (32, 64 or 128) of one expert; RD_DECODE_ROWS the one that gives it whole rows
                     for a slice of the contraction range (fp32 partial sums in the workspace, n <= 2048) or, with
                     trans_rhs, whole weight rows of a slice of the columns (no partial sums, k <= 8192) */
-  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round and k >= 6400 (float8: 12800, float32: 800,
+  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round and k >= 6400 (float8: 12800, float32: 1067,
                   the variants v* and hv*: 3658 where about half a round of tiles or less is expected, 5700 otherwise), cut
-                  those tiles' contraction range over up to sqrt(k)/20 work-groups (float32: sqrt(k)/7, v* and hv*: sqrt(k)/15; fp32 partial
+                  those tiles' contraction range over up to sqrt(k)/20 work-groups (float32: sqrt(k)/8, v* and hv*: sqrt(k)/15; fp32 partial
                   sums in the workspace); n > 0 = cut them over up to n (at most 8) whatever k is; -1 = never.  A default plan may name
                   one of v* / hv* for any bfloat16 or float16 call: who relies on uncut sums asks for -1 */
 } rd_plan;
@@ -135,7 +135,7 @@ int rd_sched_map_len(int m, int g, int chunk_m);
  *   (:155-165) -- also when every group is empty.  Groups that would run past m are clipped to m.
  * Workspace: rd_gmm_workspace_bytes() bytes, 256-byte aligned; holds the scheduling map, 64 KiB for the order in which
  * the tile walk's blocks are dealt (long groups' among short groups') and, unless the plan says split_k = -1, fp32
- * partial sums (64 MiB for the 256 x 256 tiles, 4-16 MiB for the float32 ones).  A smaller workspace that has room for the map is accepted: the call
+ * partial sums (64 MiB for the 256 x 256 tiles, 4-16 MiB for the float32 ones a default plan names).  A smaller workspace that has room for the map is accepted: the call
  * then runs without the K-split (the same sums, added up in another order where it would have cut) and, if the order does
  * not fit either, in plain walk order (the same bits). */
 size_t rd_gmm_workspace_bytes(int m, int g, const rd_plan* plan /* host, may be NULL */);

@@ -149,9 +149,8 @@ constexpr int kBehind = 5;  // rs_kloop asks for slab t + 4 in slab t, and an od
 
 // A tile at element (0, c0) of a matrix of pitch ld.  K-major: lim rows, contraction indices c0 .. c0 + klen - 1 of each.
 // MN-major: klen rows, columns c0 .. c0 + lim - 1 of each.  The memory ends with the matrix's last row.
-template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB>
+template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB, int NW>
 static bool check_rs_window(int lim, int ld, int c0, int klen) {
-  constexpr int NW = 4;
   typedef RsLoader<T, BK, NW, KMAJOR, Src, VEC, LB> Ld;
   constexpr int EPP = Ld::EPP;
   const int nk = (klen + BK - 1) / BK;
@@ -204,7 +203,7 @@ static bool check_rs_window(int lim, int ld, int c0, int klen) {
   return true;
 }
 
-template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB = 2>
+template <int T, int BK, bool KMAJOR, typename Src, bool VEC, int LB = 2, int NW = 4>
 static bool check_rs_loader() {
   std::vector<int> lims, klens;
   for (int lim : {1, 2, 3, 5, 7, 8, 9, 16, 31, 33, 63, 64, 65, 72, 100, 127, 128, 129, 190, 192, 200, 249, 255, 256})
@@ -216,22 +215,22 @@ static bool check_rs_loader() {
     for (int klen : klens) {
       if constexpr (KMAJOR) {
         if (VEC && klen % 8 != 0) continue;
-        if (klen >= 8 && !check_rs_window<T, BK, true, Src, VEC, LB>(lim, klen, 0, klen)) return false;  // whole rows
+        if (klen >= 8 && !check_rs_window<T, BK, true, Src, VEC, LB, NW>(lim, klen, 0, klen)) return false;  // whole rows
         // pieces of a cut along K: they start at multiples of 64 and end at one, or with the row
         for (int c0 : {64, 192})
           for (int behind : {0, 64}) {
             if (behind && klen % 64 != 0) continue;
-            if (!check_rs_window<T, BK, true, Src, VEC, LB>(lim, c0 + klen + behind, c0, klen)) return false;
+            if (!check_rs_window<T, BK, true, Src, VEC, LB, NW>(lim, c0 + klen + behind, c0, klen)) return false;
           }
-        if (klen % 64 == 0 && (!check_rs_window<T, BK, true, Src, VEC, LB>(lim, klen + 64, 0, klen) ||
-                               !check_rs_window<T, BK, true, Src, VEC, LB>(lim, widest, 64, klen))) return false;
+        if (klen % 64 == 0 && (!check_rs_window<T, BK, true, Src, VEC, LB, NW>(lim, klen + 64, 0, klen) ||
+                               !check_rs_window<T, BK, true, Src, VEC, LB, NW>(lim, widest, 64, klen))) return false;
       } else {
         if (VEC && lim % 8 != 0) continue;
         // the tile that holds the last columns, of one tile's columns and of several, and one with more behind it
-        if (lim >= 8 && !check_rs_window<T, BK, false, Src, VEC, LB>(lim, lim, 0, klen)) return false;
-        if (!check_rs_window<T, BK, false, Src, VEC, LB>(lim, T + lim, T, klen)) return false;
-        if (lim == T && (!check_rs_window<T, BK, false, Src, VEC, LB>(lim, 2 * T + 24, T, klen) ||
-                         !check_rs_window<T, BK, false, Src, VEC, LB>(lim, widest, 0, klen))) return false;
+        if (lim >= 8 && !check_rs_window<T, BK, false, Src, VEC, LB, NW>(lim, lim, 0, klen)) return false;
+        if (!check_rs_window<T, BK, false, Src, VEC, LB, NW>(lim, T + lim, T, klen)) return false;
+        if (lim == T && (!check_rs_window<T, BK, false, Src, VEC, LB, NW>(lim, 2 * T + 24, T, klen) ||
+                         !check_rs_window<T, BK, false, Src, VEC, LB, NW>(lim, widest, 0, klen))) return false;
       }
     }
   return true;
@@ -274,6 +273,13 @@ int main() {
        check_rs_loader<128, 32, false, float, false>() && check_rs_loader<256, 32, false, float, false>();
   ok = ok && check_rs_loader<64, 32, true, float, false, 4>() && check_rs_loader<128, 32, true, float, false, 4>() &&
        check_rs_loader<64, 32, false, float, false, 4>() && check_rs_loader<128, 32, false, float, false, 4>();
+  // float32 as three bf16 terms on eight waves, and float32 as it is where a tile falls back to it
+  ok = ok && check_rs_loader<64, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, true, float, false, 2, 8>() &&
+       check_rs_loader<256, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, false, float, false, 2, 8>() &&
+       check_rs_loader<256, 32, false, float, false, 2, 8>() && check_rs_loader<64, 32, false, float, false, 2>();
+  ok = ok && check_rs_loader<64, 32, true, float, false, 4, 8>() && check_rs_loader<128, 32, true, float, false, 4, 8>() &&
+       check_rs_loader<256, 32, true, float, false, 4, 8>() && check_rs_loader<128, 32, false, float, false, 4, 8>() &&
+       check_rs_loader<256, 32, false, float, false, 4, 8>();
   if (!ok) return 1;
   std::printf("loader_bounds ok %lld\n", g_loads);
   return 0;

@@ -1,0 +1,123 @@
+"""float32 products as six products of bf16 terms (RsCfg with THREE in csrc/rd_gemm_rs.h): as accurate as products on the float32
+instruction at every magnitude, and on that instruction where the terms do not hold the numbers."""
+
+import functools
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_ragged_dot_amd import _capi, ops
+
+pytestmark = pytest.mark.gpu
+
+HP = dict(block_m=64, block_k=64, block_n=64, interpret=False, compute_dtype=None, acc_dtype=torch.float32, chunk_m=512)
+TERMS = ["ft128x256x32_w2x4", "ft128x128x32_w2x4", "ft64x128x32_w2x2"]
+WHOLE = "fr64x64x32_w2x2"
+CASES = [(name, op) for name in TERMS for op in (0, 1, 2)]
+
+
+@functools.lru_cache(None)
+def variant(name):
+    return next(v.id for v in _capi.variants() if v.name.decode() == name)
+
+
+def product(op, a, b, sizes, name, split_k=0):
+    plan = _capi.Plan(variant(name), split_k=split_k)
+    a, b, gs = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), torch.tensor(sizes, dtype=torch.int32).cuda()
+    if op == 2:
+        return ops._tgmm_fwd(a, b, gs, **HP, plan=plan).cpu().numpy()
+    return ops._gmm_fwd(a, b, gs, **HP, trans_rhs=op == 1, plan=plan).cpu().numpy()
+
+
+def operands(op, k, n, sizes, draw):
+    m, g = sum(sizes), len(sizes)
+    return draw((m, k)), draw((m, n) if op == 2 else (g, n, k) if op == 1 else (g, k, n))
+
+
+def reference(op, a, b, sizes):
+    """The sums and the sums of magnitudes, in float64."""
+    out, at = [], 0
+    for i, s in enumerate(sizes):
+        x, y = a[at:at + s].astype(np.float64), (b[at:at + s] if op == 2 else b[i]).astype(np.float64)
+        x, y = (x.T, y) if op == 2 else (x, y.T if op == 1 else y)
+        out.append((x @ y, np.abs(x) @ np.abs(y)))
+        at += s
+    join = np.stack if op == 2 else np.concatenate
+    return join([o[0] for o in out]), join([o[1] for o in out])
+
+
+# edges of tiles and of slabs, odd pitches, a group of one row, an empty one, groups of up to 64 rows behind whole tiles
+SHAPES = [(8, 8, [3]), (33, 257, [1, 0, 64, 65]), (64, 128, [127, 129]), (100, 300, [130, 256, 17]), (1027, 385, [321])]
+
+
+@pytest.mark.parametrize("k,n,sizes", SHAPES)
+@pytest.mark.parametrize("name,op", CASES)
+def test_every_magnitude(name, op, k, n, sizes):
+    rng = np.random.default_rng(k + n)
+    # 2^-30 .. 2^30, with zeros: what a term loses of a small number would show beside a large one's zero partner
+    def draw(shape):
+        v = rng.standard_normal(shape) * np.exp2(rng.integers(-30, 31, shape))
+        return np.where(rng.random(shape) < 0.3, 0, v).astype(np.float32)
+    a, b = operands(op, k, n, sizes, draw)
+    want, magnitudes = reference(op, a, b, sizes)
+    got = product(op, a, b, sizes, name)
+    length = max(sizes) if op == 2 else k
+    # one rounding for every contraction index at most, and the products of terms left out: two of at most 2^-25 of the whole one
+    assert (np.abs(got - want) <= (length + 1) * 2.0 ** -24 * magnitudes).all()
+
+
+@pytest.mark.parametrize("name,op", CASES)
+@pytest.mark.parametrize("low,high", [(0, 0), (-108, 100), (100, -70)])
+def test_no_less_accurate_than_the_float32_instruction(name, op, low, high):
+    rng = np.random.default_rng(5)
+    k, n, sizes = 512, 256, [400, 112]
+    a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    a, b = np.ldexp(np.where(np.abs(a) < 0.25, 0.25, a), low), np.ldexp(b, high)  # all above 2^-110
+    want, _ = reference(op, a, b, sizes)
+    error = [np.linalg.norm(product(op, a, b, sizes, v) - want) for v in (name, WHOLE)]
+    assert error[0] <= error[1]
+
+
+ODD_ONES = [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 1e-40, 2.0 ** -111, 1e30]
+
+
+@pytest.mark.parametrize("split_k", [-1, 3])
+@pytest.mark.parametrize("odd", ODD_ONES)
+@pytest.mark.parametrize("name,op", CASES)
+def test_numbers_that_the_terms_do_not_hold(name, op, odd, split_k):
+    rng = np.random.default_rng(7)
+    k, n, sizes = 1024, 256, [64, 64, 64]
+    a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    plain = product(op, a, b, sizes, name, split_k)
+    a[70, 1000] = odd  # group 1; in the last piece of a cut
+    if odd == 1e30:    # a sum beyond the type's range
+        b[70 if op == 2 else 1] *= 1e30
+    if op == 2:
+        split_k = 0
+    got = product(op, a, b, sizes, name, split_k)
+    whole = product(op, a, b, sizes, WHOLE, split_k)
+    touched, others = (slice(1, 2), [0, 2]) if op == 2 else (slice(64, 128), list(range(64)) + list(range(128, 192)))
+    assert np.array_equal(np.isfinite(got), np.isfinite(whole)) and np.array_equal(got[others], plain[others])
+    if split_k <= 0 and op != 2:
+        assert np.array_equal(got[touched], whole[touched], equal_nan=True)
+    else:
+        want, magnitudes = reference(op, np.where(np.isfinite(a), a, 0), b, sizes)
+        ok = np.isfinite(whole)
+        assert (np.abs(got - want) <= 1024 * 2.0 ** -24 * magnitudes)[ok].all()
+        assert np.array_equal(got[~ok], whole[~ok], equal_nan=True)
+
+
+@pytest.mark.parametrize("m,k,n,g", [(3000, 2048, 1111, 5), (1640, 4100, 900, 3), (5000, 300, 2000, 40)])
+def test_default_plan(m, k, n, g):
+    rng = np.random.default_rng(m)
+    p = np.exp(rng.standard_normal(g))
+    sizes = rng.multinomial(m - 7, p / p.sum()).tolist()
+    for op in (0, 1, 2):
+        plan = _capi.default_plan(op, m, k, n, g, _capi.RD_DTYPE_F32)
+        name = _capi.variants()[plan.variant].name.decode()
+        assert name.startswith("ft")
+        a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+        want, magnitudes = reference(op, a, b, sizes)
+        got = product(op, a, b, sizes, name)
+        assert (np.abs(got - want) <= (max(sizes) if op == 2 else k) * 2.0 ** -24 * magnitudes).all()
