@@ -1,7 +1,7 @@
 // GEMM core for operands that cannot be loaded straight into LDS: row pitches that are no multiple of 16 bytes
 // (bf16 and float16), float32 arrays that are rounded to bf16 on the way (compute_dtype = bfloat16), and float32 arrays of
 // any pitch multiplied to float32's accuracy.  A 256 x 256 tile held by a 2 x 2 grid of waves, 128 x 128 per wave, as in
-// rd_gemm_w4.h, or a smaller tile, several work-groups to a compute unit (float32 to its accuracy: 2 x 4 waves); HBM -> registers
+// rd_gemm_w4.h, or a smaller tile, several work-groups to a compute unit, or 2 x 4 waves on a 128 x 256 tile; HBM -> registers
 // -> LDS as in rd_gemm_w4r.h, for any of the four operand layouts.
 //
 // What bounds it: with the 64 x 64 and 128 x 128 tiles of rd_gemm_tile.h these products were bound by their loads - one
@@ -15,6 +15,7 @@
 //    accesses at any alignment.  Every 8 lanes (K-major) or every 32 / 64 (MN-major) read consecutive memory;
 //  * a slab is 128 bytes of every K-major row (64 bf16 or 32 float32 contraction indices), 16 pieces per lane for both
 //    operands, and two slabs are in flight in registers beside the two in LDS (bf16: 2 x 64 KB, float32 rounded: 2 x 32 KB);
+//  * 128 x 256 on eight waves: three quarters of the 128 x 128 tile's loads, and two waves on a SIMD (fills_rounds_128x256() in rd_capi.hip);
 //  * the pieces are converted and written to LDS, and their registers refilled, spread evenly over the gaps between the
 //    matrix-core instructions of a slab.
 // float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most, of which this core reaches 86-92 %
@@ -62,7 +63,7 @@ struct RsCfg {
   static constexpr int KMF = FULL ? 4 : THREE ? 6 : 1;     // matrix-core instructions per block and substep
   static constexpr int KSTEPS = FULL ? BK / 8 : BK / 16;   // substeps per slab
   // work-groups per compute unit
-  static constexpr int WAVES_PER_EU = THREE ? (NW == 8 || BM * BN < 128 * 128 ? 2 : 1) : BM * BN > 128 * 128 ? 1 : BM * BN < 128 * 128 ? 3 : 2;
+  static constexpr int WAVES_PER_EU = NW == 8 ? 2 : THREE ? (BM * BN < 128 * 128 ? 2 : 1) : BM * BN > 128 * 128 ? 1 : BM * BN < 128 * 128 ? 3 : 2;
   static constexpr int A_TERM = BM * BK * LB, B_TERM = BN * BK * LB;         // one term of a slab in LDS
   static constexpr int A_BYTES = TERMS * A_TERM, B_BYTES = TERMS * B_TERM;  // one slab in LDS
   static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;
@@ -463,7 +464,7 @@ __device__ __forceinline__ void rs_store16(const f32x16_t (&acc)[C::TM][C::TN], 
         w[1] = pack_out_x2<C::HALF>(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
         *reinterpret_cast<u32x2_t*>(st + row * C::EPI_PITCH + col * 2) = w;
       }
-  constexpr int CPR = C::WN / 8, ROWS_PER = 64 / CPR, NIT = C::WM / ROWS_PER, BATCH = NIT < 8 ? NIT : 8;
+  constexpr int CPR = C::WN / 8, ROWS_PER = 64 / CPR, NIT = C::WM / ROWS_PER, BATCH = NIT < 8 ? NIT : NIT % 8 == 0 ? 8 : 6;
   static_assert(NIT % BATCH == 0, "whole batches");
   const int chunk = lane % CPR, r0 = lane / CPR;
   const int gcol = wn * C::WN + chunk * 8, live = b_lim - gcol;  // live: the lane's columns inside the tile

@@ -273,6 +273,10 @@ int main() {
        check_rs_loader<128, 32, false, float, false>() && check_rs_loader<256, 32, false, float, false>();
   ok = ok && check_rs_loader<64, 32, true, float, false, 4>() && check_rs_loader<128, 32, true, float, false, 4>() &&
        check_rs_loader<64, 32, false, float, false, 4>() && check_rs_loader<128, 32, false, float, false, 4>();
+  // the 128 x 256 tile of 16-bit elements, eight waves
+  ok = ok && check_rs_loader<64, 64, true, bf16_bits, false, 2, 8>() && check_rs_loader<128, 64, true, bf16_bits, false, 2, 8>() &&
+       check_rs_loader<256, 64, true, bf16_bits, false, 2, 8>() && check_rs_loader<128, 64, false, bf16_bits, false, 2, 8>() &&
+       check_rs_loader<256, 64, false, bf16_bits, false, 2, 8>();
   // float32 as three bf16 terms on eight waves, and float32 as it is where a tile falls back to it
   ok = ok && check_rs_loader<64, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, true, float, false, 2, 8>() &&
        check_rs_loader<256, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, false, float, false, 2, 8>() &&

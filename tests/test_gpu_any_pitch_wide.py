@@ -1,0 +1,42 @@
+"""The 128 x 256 tile of the any-pitch core: sizes that the default rules give to it, and their neighbours on either side of the rule's lines."""
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_ragged_dot_amd as rd
+from gpu_ragged_dot_amd import _capi
+from oracle import ragged_dot_oracle as oracle
+from tests import util
+
+pytestmark = pytest.mark.gpu
+
+# m, k, n, g, taken: a round of tiles, two rounds; contractions and tile counts below the lines; short groups
+SIZES = [(2178, 831, 2203, 3, True), (3000, 701, 1601, 4, True), (3900, 1501, 1030, 5, True), (6700, 303, 1799, 3, True),
+         (2178, 699, 2203, 3, False), (1100, 831, 2203, 3, False), (2178, 831, 2203, 30, False)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("m,k,n,g,taken", SIZES)
+def test_default_rule(m, k, n, g, taken, dtype):
+    rng = np.random.default_rng(m + k)
+    p = np.exp(rng.standard_normal(g))
+    gs = rng.multinomial(m - 9, p / p.sum()).astype(np.int32)
+    code = _capi.RD_DTYPE_BF16 if dtype == torch.bfloat16 else _capi.RD_DTYPE_F16
+    names = [v.name.decode() for v in _capi.variants()]
+    for op in (_capi.OP_GMM, _capi.OP_GMM_TRANS):
+        name = names[_capi.default_plan(op, m, k, n, g, code).variant]
+        assert name.endswith("r128x256x64_w2x4") == taken, name
+    rounding = "bfloat16" if dtype == torch.bfloat16 else "float16"
+    x = oracle.round_to(rng.standard_normal((m, k)).astype(np.float32), rounding)
+    A = oracle.round_to((rng.standard_normal((g, k, n)) / np.sqrt(k)).astype(np.float32), rounding)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda().to(dtype)
+    xd, Ad, gsd = dev(x), dev(A), torch.from_numpy(gs).cuda()
+    ref = oracle.gmm(x, A, gs, out_dtype="float32", acc=np.float64)
+    live = int(gs.sum())
+    # one rounding to 8 or 11 bits, and float32 sums of k products
+    eps = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + k * 2.0 ** -24
+    for y in (rd.ragged_dot(xd, Ad, gsd), rd.ragged_dot(xd, Ad.mT.contiguous(), gsd, trans_rhs=True)):
+        y = util.to_np(y)
+        err = np.linalg.norm(y[:live] - ref[:live], axis=1) / np.linalg.norm(ref[:live], axis=1)
+        assert err.max() < eps and not np.any(y[live:])

@@ -121,3 +121,23 @@ def test_default_plan(m, k, n, g):
         want, magnitudes = reference(op, a, b, sizes)
         got = product(op, a, b, sizes, name)
         assert (np.abs(got - want) <= (max(sizes) if op == 2 else k) * 2.0 ** -24 * magnitudes).all()
+
+
+@pytest.mark.parametrize("k,n", [(8, 8), (57, 77), (65, 257), (225, 131), (321, 72)])
+@pytest.mark.parametrize("name,op", CASES)
+def test_another_groups_numbers_do_not_reach_a_group(name, op, k, n):
+    """Loads that run past a row or a group read NaN there: the other groups' bits stay (a tile that saw one would be computed another way)."""
+    rng = np.random.default_rng(k)
+    sizes = [257, 0, 1, 63, 40, 129, 7]
+    a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    clean = product(op, a, b, sizes, name)
+    first, rows = sum(sizes[:4]), sizes[4]
+    a[first:first + rows] = np.nan
+    if op == 2:
+        b[first:first + rows] = np.nan
+    else:
+        b[4] = np.nan
+    got = product(op, a, b, sizes, name)
+    hit = np.zeros(len(got), bool)
+    hit[4 if op == 2 else slice(first, first + rows)] = True
+    assert np.isnan(got[hit]).all() and np.array_equal(got[~hit], clean[~hit])
