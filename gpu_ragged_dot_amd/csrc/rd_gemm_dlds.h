@@ -198,6 +198,7 @@ struct SplitK {
 // every piece - so the partial sums go around the problem instead: they are stored and loaded with the sc1 cache policy
 // (coherent at device scope: written through, re-fetched), and the only ordering needed is that a piece's stores have
 // completed before its arrival is counted.
+constexpr int imin_const(int a, int b) { return a < b ? a : b; }
 constexpr int kCachePolicyDevice = 16;  // sc1 in the aux operand of the buffer intrinsics
 
 template <class C>
@@ -230,25 +231,39 @@ __device__ __forceinline__ bool splitk_combine(f32x16_t (&acc)[C::TM][C::TN], co
   __syncthreads();  // everyone has read the slot before the epilogue reuses LDS
   if (arrived != sk.parts - 1) return false;
   // Sum the pieces in index order, this work-group's own included, so that the result does not depend on which piece
-  // happened to arrive last.
+  // happened to arrive last.  Some of the accumulators over all pieces, then the next ones: what is in flight, two pieces'
+  // vectors, and the sums then fit beside the accumulators that are done.  (All accumulators piece by piece, the four-wave
+  // 256 x 256 cores' 64 loads of a piece went out one by one, each behind the wait for the one before.)
+  constexpr int BATCH = imin_const(QUADS, C::NT == 256 && QUADS >= 64 && C::DLDS ? 16 : 8);
+  static_assert(QUADS % BATCH == 0, "whole batches");
 #pragma unroll
-  for (int i = 0; i < C::TM; ++i)
+  for (int first = 0; first < QUADS; first += BATCH) {
+    f32x4_t sum[BATCH];
 #pragma unroll
-    for (int j = 0; j < C::TN; ++j)
+    for (int q = 0; q < BATCH; ++q) sum[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < sk.parts; s += 2) {
+      u32x4_t in[2][BATCH];
+      const bool both = s + 1 < sk.parts;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  for (int s = 0; s < sk.parts; ++s) {
+      for (int h = 0; h < 2; ++h)
+        if (h == 0 || both)
 #pragma unroll
-    for (int i = 0; i < C::TM; ++i)
+          for (int q = 0; q < BATCH; ++q)
+            in[h][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + (first + q) * (C::NT * 16), (s + h) * PIECE_BYTES, kCachePolicyDevice);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < C::TN; ++j)
+      for (int q = 0; q < BATCH; ++q) sum[q] += __builtin_bit_cast(f32x4_t, in[0][q]);
+      if (both) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const u32x4_t raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + ((i * C::TN + j) * 4 + g) * (C::NT * 16),
-                                                                        s * PIECE_BYTES, kCachePolicyDevice);
-          const f32x4_t v = __builtin_bit_cast(f32x4_t, raw);
-          acc[i][j][4 * g + 0] += v[0]; acc[i][j][4 * g + 1] += v[1]; acc[i][j][4 * g + 2] += v[2]; acc[i][j][4 * g + 3] += v[3];
-        }
+        for (int q = 0; q < BATCH; ++q) sum[q] += __builtin_bit_cast(f32x4_t, in[1][q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < BATCH; ++q) {
+      const int i = (first + q) / 4 / C::TN, j = (first + q) / 4 % C::TN, g = (first + q) % 4;
+      acc[i][j][4 * g + 0] = sum[q][0]; acc[i][j][4 * g + 1] = sum[q][1]; acc[i][j][4 * g + 2] = sum[q][2]; acc[i][j][4 * g + 3] = sum[q][3];
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   return true;
 }

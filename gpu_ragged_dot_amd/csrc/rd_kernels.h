@@ -124,17 +124,6 @@ struct ShortTileCfg {
   typedef DldsCfg<ROWS, C::BN, BK, 1, 4, true, C::B_KMAJOR, STAGES, false, kCachePolicyStream, C::HALF> type;
 };
 
-// How the last round of a gmm launch is cut along K.  The device runs num_cus tiles at a time; when the live tiles do
-// not fill the last round, the tiles from position `first_tile` of the walk on (the ones that round would hold) are each
-// computed by `parts` work-groups over a `parts`-th of the contraction range instead, so the round takes about
-// 1 / parts as long.
-struct SplitPlan {
-  int first_tile;  // walk positions >= first_tile (and < live) are split; == live when nothing is
-  int parts;
-  int tiles;       // live - first_tile, or twice that where each is computed in two halves
-};
-constexpr int kMaxSplitParts = 8;
-
 // What a cut is worth depends on the core: its K loop per contraction index and how much a piece's partial sums are.
 // QUARTERS: the former over the latter, in quarters of the 256 x 256 bf16 cores' (float8: twice the rate; float32
 // as three bf16 terms: 6 times the time per multiplication, partial sums of half a tile or a quarter; on the float32 instruction 16 times).
@@ -158,34 +147,9 @@ struct HalvesLastRound { static constexpr bool value = false; };
 template <class C>
 struct HalvesLastRound<C, typename std::enable_if<IsRs<C>::value>::type> { static constexpr bool value = C::THREE && C::BN == 256 && C::A_KMAJOR; };
 
-// k_cost: k in units of what a bf16 K loop spends per element.
-// halves: 2 where the pieces are pieces of half a tile's columns (HalvesLastRound): then the last round's tiles are halved whenever
-// all halves run at a time, and each half cut along K where the above says so.
-__device__ __forceinline__ SplitPlan split_plan(int live, int k, int k_cost, int min_k, int slots, int num_cus, int max_parts, int halves = 1) {
-  SplitPlan sp{live, 1, 0};
-  if (slots <= 0 || live <= 0) return sp;
-  const int first = (live / num_cus) * num_cus;
-  const int tiles = (live - first) * halves;
-  if (tiles <= 0 || tiles > imin(slots, num_cus)) return sp;
-  // The piece that arrives last reads every piece's 256 KB of partial sums at what one compute unit can pull (about
-  // 25 GB/s: ~10 us per piece), so the gain of a finer cut, T/parts for a K loop of T us, is soon eaten: parts ~
-  // sqrt(T / 10 us), with T ~ k / 32 x 0.77 us, i.e. sqrt(k) / 20 - and below k = 6400 (4 pieces) cutting was measured
-  // to gain nothing.  max_parts > 0 is the caller's own choice and is taken as it is.
-  int parts = imin(imin(slots / tiles, kMaxSplitParts), k / min_k);
-  if (max_parts > 0) {
-    parts = imin(parts, max_parts);
-  } else {
-    int by_k = 1;
-    while ((by_k + 1) * (by_k + 1) * 400 <= k_cost) ++by_k;
-    parts = by_k < 4 ? 1 : imin(parts, by_k);
-  }
-  if (parts < 2) {
-    if (halves == 1) return sp;
-    parts = 1;
-  }
-  sp.first_tile = first; sp.parts = parts; sp.tiles = tiles;
-  return sp;
-}
+// Which launches are cut by split_parts_by_gain(); the others by the square root of the K loop over what a piece costs.
+template <class C>
+struct SplitsByGain { static constexpr bool value = C::SPLITK && C::DLDS && C::BM * C::BN == 256 * 256; };
 
 // Walk tiles in bands of `group_m` rows: consecutive ids share B columns / A rows so that the ~32 tiles one XCD
 // has in flight re-use each other's operands out of its L2.
@@ -226,8 +190,10 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   const int total = imin(mapped ? uniform(*p.total_tiles) : scan.total_tiles, p.U);
   const int live = total * p.n_tiles;
   SplitPlan sp{live, 1, 0};
-  if constexpr (C::SPLITK) sp = split_plan(live, p.k, (int)((long long)p.k * SplitCost<C>::QUARTERS / 4), SplitCost<C>::MIN_K, p.split_slots, p.num_cus, p.max_parts,
-                                               HalvesLastRound<C>::value ? 2 : 1);
+  if constexpr (C::SPLITK) {
+    const SplitRule rule{p.k, (int)((long long)p.k * SplitCost<C>::QUARTERS / 4), SplitCost<C>::MIN_K, p.split_slots, p.num_cus, p.max_parts, SplitsByGain<C>::value};
+    sp = split_plan(live, rule, HalvesLastRound<C>::value ? 2 : 1);
+  }
 
   int t, half = 0;
   SplitK sk;
@@ -499,6 +465,7 @@ struct TileVariant {
   int splitk;  // 1: the gmm kernels can cut the last round of tiles along K (needs partials in the workspace)
   int split_quarters, split_min_k;  // SplitCost of the gmm kernels
   int split_bn;  // columns of a piece of the K-split
+  int split_by_gain;  // SplitsByGain of the gmm kernels
   int ws_core;  // 1: the core of rd_gemm_ws.h
   int split_rings;  // 1: the core of rd_gemm_pp.h with a ring per operand
   gmm_launch_fn gmm_nn, gmm_nt;  // null: the shape has no kernel for that product

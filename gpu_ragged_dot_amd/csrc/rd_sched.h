@@ -11,6 +11,69 @@ constexpr int kBandShift = 7;
 constexpr int kBandMaxRows = (1 << kBandShift) - 1;
 constexpr int kBandDeferred = 1 << 30;  // mark of a short last row tile listed behind all other tiles (see launch_sched_map)
 
+// What split_plan() cuts by.  k_cost: k in units of what a bf16 K loop spends per element (SplitCost in rd_kernels.h); slots: pieces
+// the workspace has room for, 0: none are cut; max_parts > 0: most pieces, as the caller asked.
+struct SplitRule {
+  int k, k_cost, min_k, slots, num_cus, max_parts;
+  bool by_gain;  // see split_parts_by_gain()
+};
+
+// How the last round of a gmm launch is cut along K.  The device runs num_cus tiles at a time; when the live tiles do
+// not fill the last round, the tiles from position `first_tile` of the walk on (the ones that round would hold) are each
+// computed by `parts` work-groups over a `parts`-th of the contraction range instead, so the round takes about
+// 1 / parts as long.
+struct SplitPlan {
+  int first_tile;  // walk positions >= first_tile (and < live) are split; == live when nothing is
+  int parts;
+  int tiles;       // live - first_tile, or twice that where each is computed in two halves
+};
+constexpr int kMaxSplitParts = 8;
+
+// The cut of a round of 256 x 256 tiles, in units of what their K loop takes per contraction index (0.0135 us in bf16, of a tile that
+// has its share of memory): p pieces save all but a p-th of the loop and cost p times 100 (1.4 us: the piece that arrives last reads every
+// piece's 256 KB), 7 for every piece of the round (0.09 us: all pieces' partial sums through memory and back) and 400 for the scheduling
+// map, which an uncut launch mostly goes without, and a margin; 600 less where the round is the launch's only one and its pieces fill
+// a device that is mostly idle.  Fitted to 110 random calls of 0.3 to 4 rounds (4-8 % off).  Time over uncut: k 2800 to 4000, 10 tiles in
+// the last round 0.86-0.91, 50 0.92, 110 1.0-1.2 (not cut); 4000 to 5600 0.80-0.97; 5600 to 9000 0.77-0.87; 2000 to 2800, 90 tiles
+// 1.03-1.17 (not cut).  5000 x 3000 x 3000 in 8 groups 138 -> 122 us.
+__host__ __device__ __forceinline__ int split_parts_by_gain(int tiles, int k_cost, int most, bool only_round) {
+  int parts = 1, best = 0;
+  for (int p = 2; p <= most; ++p) {
+    const int gain = k_cost - k_cost / p - p * (100 + 7 * tiles) - (only_round ? -200 : 400);
+    if (gain > best) { best = gain; parts = p; }
+  }
+  return parts;
+}
+
+// halves: 2 where the pieces are pieces of half a tile's columns (HalvesLastRound in rd_kernels.h): then the last round's tiles are
+// halved whenever all halves run at a time, and each half cut along K where that pays.
+__host__ __device__ __forceinline__ SplitPlan split_plan(int live, const SplitRule& r, int halves = 1) {
+  SplitPlan sp{live, 1, 0};
+  if (r.slots <= 0 || live <= 0) return sp;
+  const int first = (live / r.num_cus) * r.num_cus;
+  const int tiles = (live - first) * halves;
+  if (tiles <= 0 || tiles > r.slots || tiles > r.num_cus) return sp;
+  int most = r.slots / tiles < kMaxSplitParts ? r.slots / tiles : kMaxSplitParts;
+  if (r.k / r.min_k < most) most = r.k / r.min_k;
+  int parts = 1;
+  if (r.max_parts > 0) {
+    parts = most < r.max_parts ? most : r.max_parts;
+  } else if (r.by_gain) {
+    parts = split_parts_by_gain(tiles, r.k_cost, most, first == 0);
+  } else {
+    // parts ~ sqrt(K loop / what a piece costs), and no fewer than four are worth it
+    int by_k = 1;
+    while ((by_k + 1) * (by_k + 1) * 400 <= r.k_cost) ++by_k;
+    if (by_k >= 4) parts = most < by_k ? most : by_k;
+  }
+  if (parts < 2) {
+    if (halves == 1) return sp;
+    parts = 1;
+  }
+  sp.first_tile = first; sp.parts = parts; sp.tiles = tiles;
+  return sp;
+}
+
 // Arrays as in the reference's GMMGroupLookupMetadata (gpu_ragged_dot.py:60-90); tile2group / tile2it hold
 // ceil(m / chunk) + g entries.  `counters` (may be null) are n_counters int32 cleared by the same launch.
 // `tile2band` (may be null; same length) receives, for every row tile, the band of at most band_rows consecutive row
@@ -31,13 +94,13 @@ constexpr int kBandDeferred = 1 << 30;  // mark of a short last row tile listed 
 // `defer_rows` > 0 (internal maps of gmm launches only, needs tile2band): the last row tile of a group of two or more
 // row tiles, when it holds at most defer_rows rows, is listed behind all other tiles instead of behind its group's - as a
 // band of its own, marked kBandDeferred - provided all such tiles then lie in the launch's partly filled last round
-// (defer_cus tiles run at a time) and that round holds at most defer_slots / 2 tiles, i.e. is cut along K.
+// and that round is cut along K (split_plan() by `cut`).
 int launch_sched_map(hipStream_t s, const int32_t* group_sizes, int g, int m, int chunk, int32_t* group_offsets,
                      int32_t* tile2group, int32_t* tile2it, int32_t* total_tiles, int32_t* counters = nullptr,
                      int n_counters = 0, int32_t* tile2band = nullptr, int band_rows = 1, int32_t* block_order = nullptr,
                      int n_blocks = 0, int per_block = 1, int n_tiles = 1, int long_rows = 0,
                      int32_t* group_order = nullptr, int order_first = 0, int order_count = 0, int defer_rows = 0,
-                     int defer_cus = 0, int defer_slots = 0);
+                     const SplitRule& cut = SplitRule());
 
 // Which block the i-th block position of a gmm launch takes from the two lists of block_order.  Positions are dealt to
 // the 8 XCDs round-robin (position i runs on XCD i mod 8), so the launch is a sequence of rounds of 8.  The long groups'

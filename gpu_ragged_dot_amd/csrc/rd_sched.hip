@@ -55,8 +55,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_map_kernel(const int32_t*
                                                                   int32_t* __restrict__ block_order, int n_blocks,
                                                                   int per_block, int n_tiles, int long_rows,
                                                                   int32_t* __restrict__ group_order, int order_first,
-                                                                  int order_count, int defer_rows, int defer_cus,
-                                                                  int defer_slots) {
+                                                                  int order_count, int defer_rows, SplitRule cut) {
   // arrival counters of the K-split tiles of the launch that follows start at zero
   for (int i = threadIdx.x; i < n_counters; i += kSchedThreads) counters[i] = 0;
   __shared__ uint32_t wave_a[kSchedWaves], wave_b[kSchedWaves];
@@ -69,7 +68,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_map_kernel(const int32_t*
   // K; never the map rd_sched_map returns): the last row tile of a group of several row tiles, when it holds at most
   // defer_rows rows, may be taken out of its group's run of tiles and listed behind all other tiles, as a band of its
   // own with the kBandDeferred mark.  That is done when all such tiles then fall into the partly filled last round of
-  // the launch (defer_cus tiles run at a time) and that round is cut along K (at most defer_slots / 2 tiles in it): the
+  // the launch and that round is cut along K: the
   // rounds before it then hold whole tiles of full height only - the layout of a dense product - and the pieces of the
   // last round, which run alone at the end of the launch either way, go through the streaming routines instead of the
   // tall one.  Anywhere else a tile moved out of its group's run would cost a pass of its own over the group's weights.
@@ -78,7 +77,7 @@ __global__ __launch_bounds__(kSchedThreads) void sched_map_kernel(const int32_t*
     return defer_on && bpg >= 2 && sz - (bpg - 1) * chunk <= defer_rows ? 1 : 0;
   };
   uint32_t total_regular = 0;
-  if (defer_rows > 0 && defer_cus > 0) {  // count the candidates and all tiles, then decide
+  if (defer_rows > 0 && cut.num_cus > 0) {  // count the candidates and all tiles, then decide
     uint32_t all = 0, cand = 0;
     defer_on = true;
     for (int base = 0; base < g; base += kSchedThreads) {
@@ -90,8 +89,8 @@ __global__ __launch_bounds__(kSchedThreads) void sched_map_kernel(const int32_t*
       all += ta; cand += tb;
     }
     const long long live = (long long)imin((int32_t)all, U) * n_tiles;
-    const long long first = live / defer_cus * defer_cus;  // where the last round starts
-    defer_on = cand > 0 && (long long)(all - cand) * n_tiles >= first && (live - first) * 2 <= defer_slots && all <= (uint32_t)U;
+    const SplitPlan sp = split_plan((int)live, cut);
+    defer_on = cand > 0 && sp.parts >= 2 && (long long)(all - cand) * n_tiles >= sp.first_tile && all <= (uint32_t)U;
     total_regular = all - cand;
   }
 
@@ -274,15 +273,14 @@ int launch_sched_map(hipStream_t s, const int32_t* gs, int g, int m, int chunk, 
                      int32_t* tile2group, int32_t* tile2it, int32_t* total_tiles, int32_t* counters, int n_counters,
                      int32_t* tile2band, int band_rows, int32_t* block_order, int n_blocks, int per_block, int n_tiles,
                      int long_rows, int32_t* group_order, int order_first, int order_count, int defer_rows,
-                     int defer_cus, int defer_slots) {
+                     const SplitRule& cut) {
   const int U = (m + chunk - 1) / chunk + g;  // gpu_ragged_dot.py:77
   if (band_rows < 1) band_rows = 1;
   if (band_rows > kBandMaxRows) band_rows = kBandMaxRows;
   hipLaunchKernelGGL(sched_map_kernel, dim3(1), dim3(kSchedThreads), 0, s, gs, g, U, chunk, group_offsets,
                      tile2group, tile2it, total_tiles, counters, counters ? n_counters : 0, tile2band, band_rows,
                      n_blocks > 0 ? block_order : nullptr, n_blocks, per_block > 0 ? per_block : 1, n_tiles > 0 ? n_tiles : 1,
-                     long_rows, order_count > 0 ? group_order : nullptr, order_first, order_count, tile2band ? defer_rows : 0, defer_cus,
-                     defer_slots);
+                     long_rows, order_count > 0 ? group_order : nullptr, order_first, order_count, tile2band ? defer_rows : 0, cut);
   return (int)hipGetLastError();
 }
 

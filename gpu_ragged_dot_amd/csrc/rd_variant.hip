@@ -131,7 +131,7 @@ extern "C" const rd::TileVariant* RD_CAT(rd_variant_, RD_NAME)() {
   static const rd::TileVariant v = {
       RD_STR(RD_NAME), RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, RD_VEC, /*dtype: RD_DTYPE_* */ RD_F32, RD_DLDS != 0, RD_STAGES,
       RD_ANY_PITCH, /*splitk*/ RD_ANY_PITCH || (RD_DLDS != 0 && (!RD_F32 || RD_F32 == 3 || RD_F32 == 4)),
-      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::HalvesLastRound<rd::CfgNN>::value ? RD_BN / 2 : RD_BN, rd::IsWs<rd::CfgNN>::value, rd::IsMixed<rd::CfgNN>::value,
+      rd::SplitCost<rd::CfgNN>::QUARTERS, rd::SplitCost<rd::CfgNN>::MIN_K, rd::HalvesLastRound<rd::CfgNN>::value ? RD_BN / 2 : RD_BN, rd::SplitsByGain<rd::CfgNN>::value, rd::IsWs<rd::CfgNN>::value, rd::IsMixed<rd::CfgNN>::value,
 #ifdef RD_NO_TGMM
       &rd::launch_gmm<rd::CfgNN, false>, &rd::launch_gmm<rd::CfgNT, true>, nullptr,
 #else
