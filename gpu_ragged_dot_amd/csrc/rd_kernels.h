@@ -329,8 +329,8 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
       // alone 0.992 and 0.989, with the tall core's own schedule on 128 rows 0.991 and 0.986.  us, before | now: 11122 x 1088 x
       // 768 in 64 skewed groups 52 | 46, trans_rhs 56 | 49; trans_rhs 26452 x 704 x 3712 in 46 199 | 177; 23628 x 2528 x
       // 2112 in 218 skewed groups 548 | 505.
-      typedef DldsCfg<kShortRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 4> S;
-      typedef DldsCfg<kMidRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 3> M;
+      typedef DldsCfg<kShortRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 4, false, 0, C::HALF> S;
+      typedef DldsCfg<kMidRows, C::BN, 64, 2, 4, true, C::B_KMAJOR, 3, false, 0, C::HALF> M;
       static_assert(S::LDS_BYTES <= C::LDS_BYTES && S::NT == C::NT, "the short routine runs in the tall one's launch");
       static_assert(M::LDS_BYTES <= C::LDS_BYTES && M::NT == C::NT, "the 128-row routine runs in the tall one's launch");
       if (rows <= kMidRows) {

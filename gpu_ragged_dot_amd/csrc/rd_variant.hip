@@ -68,6 +68,17 @@ typedef WsCfg<RD_BM, RD_BN, RD_BK, true, false, RD_STAGES, RD_F32 == 4, /*stream
 typedef WsCfg<RD_BM, RD_BN, RD_BK, true, true, RD_STAGES, RD_F32 == 4, true> CfgNTStream;
 #define RD_NT_STREAM &rd::launch_gmm<rd::CfgNTStream, true>
 #endif
+#elif (RD_F32 == 0 || RD_F32 == 4) && RD_DLDS == 2
+// one LDS ring per operand: one K-major operand in 64-wide slabs (3 slots) - the activations in the forward product,
+// the weights A[g,n,k] with trans_rhs (measured 1-3 % ahead of giving them to dout) - everything else in 32-wide
+// slabs (4 slots); bf16 or float16
+typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, /*A K-major*/ true, /*B K-major*/ false, 64, 3, 32, 4, RD_F32 == 4> CfgNN;
+typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, true, true, 32, 4, 64, 3, RD_F32 == 4> CfgNT;
+typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, false, false, 32, 4, 32, 4, RD_F32 == 4> CfgTN;
+#elif (RD_F32 == 0 || RD_F32 == 4) && RD_DLDS == 1
+typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, RD_PINGPONG != 0, 0, RD_F32 == 4> CfgNN;
+typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, true, true, RD_STAGES, RD_PINGPONG != 0, 0, RD_F32 == 4> CfgNT;
+typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, false, false, RD_STAGES, RD_PINGPONG != 0, 0, RD_F32 == 4> CfgTN;
 #elif RD_F32 == 3 && RD_DLDS
 // float8 e4m3fn arrays on the float8 matrix-core instruction, direct-to-LDS (rd_gemm_f8.h).  tgmm reads x^T as an
 // MN-major operand, whose slab rows span the tile's rows: only for tile heights that are multiples of 256.
@@ -102,17 +113,6 @@ typedef W4Cfg<RD_BM, RD_BN, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES> 
 // both operands K-major: the 64-wide, register-staged form of the core (rd_gemm_w4r.h)
 typedef W4RCfg<RD_BM, RD_BN> CfgNT;
 typedef W4Cfg<RD_BM, RD_BN, false, false, RD_STAGES> CfgTN;
-#elif RD_DLDS == 2
-// one LDS ring per operand: one K-major operand in 64-wide slabs (3 slots) - the activations in the forward product,
-// the weights A[g,n,k] with trans_rhs (measured 1-3 % ahead of giving them to dout) - everything else in 32-wide
-// slabs (4 slots)
-typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, /*A K-major*/ true, /*B K-major*/ false, 64, 3, 32, 4> CfgNN;
-typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, true, true, 32, 4, 64, 3> CfgNT;
-typedef PpCfg<RD_BM, RD_BN, RD_WAVES_M, RD_WAVES_N, false, false, 32, 4, 32, 4> CfgTN;
-#elif RD_DLDS
-typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, /*A K-major*/ true, /*B K-major*/ false, RD_STAGES, RD_PINGPONG != 0> CfgNN;
-typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, true, true, RD_STAGES, RD_PINGPONG != 0> CfgNT;
-typedef DldsCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, false, false, RD_STAGES, RD_PINGPONG != 0> CfgTN;
 #else
 typedef TileCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, /*A K-major*/ true, /*B K-major*/ false, RD_VEC != 0> CfgNN;
 typedef TileCfg<RD_BM, RD_BN, RD_BK, RD_WAVES_M, RD_WAVES_N, true, true, RD_VEC != 0> CfgNT;
