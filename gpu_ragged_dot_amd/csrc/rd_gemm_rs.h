@@ -16,6 +16,8 @@
 //  * a slab is 128 bytes of every K-major row (64 bf16 or 32 float32 contraction indices), 16 pieces per lane for both
 //    operands, and two slabs are in flight in registers beside the two in LDS (bf16: 2 x 64 KB, float32 rounded: 2 x 32 KB);
 //  * 128 x 256 on eight waves: three quarters of the 128 x 128 tile's loads, and two waves on a SIMD (fills_rounds_128x256() in rd_capi.hip);
+//  * float32 rounded to bf16: 256 x 256 on eight waves of 128 x 64, whose second wave on a SIMD multiplies while the first converts and
+//    writes: 0.98 times the four waves' time in gmm (1144 random calls at 16-byte pitches; 803 at others 0.99), 0.94 in tgmm (163);
 //  * the pieces are converted and written to LDS, and their registers refilled, spread evenly over the gaps between the
 //    matrix-core instructions of a slab.
 // float32 multiplied as float32 (FULL) is bound by its matrix-core instruction, 157 TFLOP/s at most, of which this core reaches 86-92 %

@@ -281,6 +281,9 @@ int main() {
   ok = ok && check_rs_loader<64, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, true, float, false, 2, 8>() &&
        check_rs_loader<256, 32, true, float, false, 2, 8>() && check_rs_loader<128, 32, false, float, false, 2, 8>() &&
        check_rs_loader<256, 32, false, float, false, 2, 8>() && check_rs_loader<64, 32, false, float, false, 2>();
+  ok = ok && check_rs_loader<192, 32, true, float, false, 2, 8>() && check_rs_loader<64, 32, true, float, true, 2, 8>() &&
+       check_rs_loader<128, 32, true, float, true, 2, 8>() && check_rs_loader<192, 32, true, float, true, 2, 8>() &&
+       check_rs_loader<256, 32, true, float, true, 2, 8>() && check_rs_loader<256, 32, false, float, true, 2, 8>();
   ok = ok && check_rs_loader<64, 32, true, float, false, 4, 8>() && check_rs_loader<128, 32, true, float, false, 4, 8>() &&
        check_rs_loader<256, 32, true, float, false, 4, 8>() && check_rs_loader<128, 32, false, float, false, 4, 8>() &&
        check_rs_loader<256, 32, false, float, false, 4, 8>();
