@@ -16,9 +16,25 @@ SIZES = [(2178, 831, 2203, 3, True), (3000, 701, 1601, 4, True), (3900, 1501, 10
          (2178, 699, 2203, 3, False), (1100, 831, 2203, 3, False), (2178, 831, 2203, 30, False)]
 
 
+# m, k, n, g, tile: few tiles and contractions on either side of the 64 x 64 tile's lines; up to four rounds of 128 x 256 tiles, and more
+FEW = [(300, 2049, 301, 3, "r128x128x64_w2x2"), (300, 1025, 301, 3, "64x64x32_w2x2"), (1000, 1025, 501, 3, "r128x128x64_w2x2"),
+       (1000, 513, 501, 3, "64x64x32_w2x2"), (2100, 513, 501, 3, "r128x128x64_w2x2"), (9001, 777, 1999, 12, "r128x256x64_w2x4"),
+       (9001, 777, 3999, 12, "r256x256x64_w2x2")]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("m,k,n,g,taken", SIZES)
 def test_default_rule(m, k, n, g, taken, dtype):
+    _check(m, k, n, g, dtype, lambda name: name.endswith("r128x256x64_w2x4") == taken)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("m,k,n,g,tile", FEW)
+def test_few_tiles(m, k, n, g, tile, dtype):
+    _check(m, k, n, g, dtype, lambda name: name.endswith(tile))
+
+
+def _check(m, k, n, g, dtype, expected):
     rng = np.random.default_rng(m + k)
     p = np.exp(rng.standard_normal(g))
     gs = rng.multinomial(m - 9, p / p.sum()).astype(np.int32)
@@ -26,7 +42,7 @@ def test_default_rule(m, k, n, g, taken, dtype):
     names = [v.name.decode() for v in _capi.variants()]
     for op in (_capi.OP_GMM, _capi.OP_GMM_TRANS):
         name = names[_capi.default_plan(op, m, k, n, g, code).variant]
-        assert name.endswith("r128x256x64_w2x4") == taken, name
+        assert expected(name), name
     rounding = "bfloat16" if dtype == torch.bfloat16 else "float16"
     x = oracle.round_to(rng.standard_normal((m, k)).astype(np.float32), rounding)
     A = oracle.round_to((rng.standard_normal((g, k, n)) / np.sqrt(k)).astype(np.float32), rounding)
