@@ -56,3 +56,19 @@ def _check(m, k, n, g, dtype, expected):
         y = util.to_np(y)
         err = np.linalg.norm(y[:live] - ref[:live], axis=1) / np.linalg.norm(ref[:live], axis=1)
         assert err.max() < eps and not np.any(y[live:])
+
+
+# m, k, n, g, whether tgmm takes the 128 x 128 tile: rows of a group times tiles, rows alone, few columns
+@pytest.mark.parametrize("m,k,n,g,taken", [(9000, 65, 99, 3, False), (9000, 165, 199, 3, True), (9000, 301, 77, 3, True), (4000, 301, 77, 16, False),
+                                           (9000, 301, 55, 8, False)])
+def test_tgmm_few_tiles(m, k, n, g, taken):
+    name = _capi.variants()[_capi.default_plan(_capi.OP_TGMM, m, k, n, g, _capi.RD_DTYPE_BF16).variant].name.decode()
+    assert name == ("r128x128x64_w2x2" if taken else "s64x64x32_w2x2")
+    rng = np.random.default_rng(m + k)
+    gs = rng.multinomial(m - 9, np.ones(g) / g).astype(np.int32)
+    x, dy = (oracle.round_to(rng.standard_normal(s).astype(np.float32), "bfloat16") for s in ((m, k), (m, n)))
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda().to(torch.bfloat16)
+    dA = util.to_np(rd.tgmm(dev(x), dev(dy), torch.from_numpy(gs).cuda()))
+    ref = oracle.tgmm(x, dy, gs, out_dtype="float32", acc=np.float64)
+    err = np.linalg.norm(dA - ref, axis=(1, 2)) / np.linalg.norm(ref, axis=(1, 2))
+    assert err.max() < 2.0 ** -8 + gs.max() * 2.0 ** -24  # one rounding to 8 bits, and float32 sums
