@@ -33,7 +33,8 @@
 //    128 x 128 tiles 1879; 8192 x 2048 x 2048 in 16 softmax-sized groups, fwd / dlhs / drhs: 377 / 378 / 380, FULL 574 / 594 / 595.
 //    Power bounds it, as it does the bf16 products.
 //  * The error against sums in float64 is 0.83-0.87 of FULL's (16 products are added up per rounding, two there): relative 2-norm on N(0, 1) data
-//    2.4e-7 (FULL 2.9e-7) for 256 products, 6.8e-7 (8.0e-7) for 2048; over 90 random sizes never above FULL's.
+//    2.4e-7 (FULL 2.9e-7) for 256 products, 6.8e-7 (8.0e-7) for 2048; over 90 random sizes never above FULL's, nor where products are
+//    subnormal.  Of one and two products it would be: see kFewProducts.
 //  * Where the terms do not hold a number, the tile is computed again by FULL (kThreeLeast).
 // One loop serves all slabs.  Where a load goes is a clamped offset from a base; on the slab that holds the last contraction
 // index the base, the offset and its limit change (enter_last), so that no load touches memory outside the operand's rows,
@@ -237,6 +238,10 @@ struct RsFrag {
 // the way into LDS (as bits << 1, less one: zeros come out on top) tells the former, a sum that is no finite number the
 // latter; a tile that has either is computed again by FULL.
 constexpr uint32_t kThreeLeast = ((127u - 110u) << 24) - 1u;
+// A product alone is rounded once there, and the products of terms left out come on top of that here (up to half of the last bit: rows of a
+// group 1, 2, 3, 4, 16: 2-norm error in units of 2^-24 0.58 | 0.42, 0.56 | 0.52, 0.55 | 0.60, 0.54 | 0.67, 0.56 | 1.24, THREE | FULL).  So
+// contractions of at most this many indices, tgmm over groups of one and two rows, are multiplied as float32 (rs_few_products()).
+constexpr int kFewProducts = 2;
 __device__ __forceinline__ uint32_t umin(uint32_t a, uint32_t b) { return a < b ? a : b; }
 
 namespace rs_detail {
@@ -513,6 +518,35 @@ __device__ __forceinline__ void rs_store32(const f32x16_t (&acc)[C::TM][C::TN], 
     }
 }
 
+// A tgmm tile of one or two rows: a product, and another one added with one rounding, the bits of the float32 matrix-core instruction.
+// Bound by its stores.  230 groups of one row among 256 of 16384 rows, k 2048, n 768: 502 us, as slabs of 32 indices on FULL 814, on terms 719.
+template <class C>
+__device__ __forceinline__ void rs_few_products(const float* __restrict__ Ap, int lda, int a_lim, const float* __restrict__ Bp, int ldb,
+                                                int b_lim, int klen, int wm, int wn, int lane, float* __restrict__ Op, int ldo) {
+  const float* __restrict__ A1 = Ap + (size_t)(klen - 1) * lda;  // the second row, or the first one again
+  const float* __restrict__ B1 = Bp + (size_t)(klen - 1) * ldb;
+  float b0[C::TN], b1[C::TN];
+#pragma unroll
+  for (int j = 0; j < C::TN; ++j) {
+    const int col = wn * C::WN + j * 32 + (lane & 31), c = col < b_lim ? col : b_lim - 1;  // (what lies outside is not stored)
+    b0[j] = Bp[c]; b1[j] = B1[c];
+  }
+  f32x16_t acc[C::TM][C::TN];
+#pragma unroll
+  for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = wm * C::WM + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), r = row < a_lim ? row : a_lim - 1;
+      const float a0 = Ap[r], a1 = A1[r];
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j) {
+        const float f = fmaf(a0, b0[j], 0.f);  // (no zero leaves with a sign, as from the matrix cores)
+        acc[i][j][v] = klen > 1 ? fmaf(a1, b1[j], f) : f;
+      }
+    }
+  rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
+}
+
 // Same contract as gemm_tile(), and: the rows the operands are read along hold at least 8 elements (16-bit) or 4
 // (float32) up to and including the tile's last one - k >= 8 and n >= 8.
 template <class C>
@@ -524,6 +558,13 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   const bool patch_live = wm * C::WM < a_lim && wn * C::WN < b_lim;
+
+  if constexpr (C::THREE && !C::A_KMAJOR) {
+    if (klen <= kFewProducts) {
+      rs_few_products<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, wm, wn, lane, Op, ldo);
+      return;
+    }
+  }
 
   f32x16_t acc[C::TM][C::TN];
 #pragma unroll
@@ -538,7 +579,7 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
   else rs_kloop<C, false>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, smem, wave, lane, acc, least);
 
   if constexpr (C::THREE) {
-    // Values that the three terms do not hold: see kThreeLeast.  All four waves must agree, they share the slabs.
+    // Values that the three terms do not hold: see kThreeLeast.  All waves of the work-group must agree, they share the slabs.
     float probe = 0.f;  // NaN once a sum is no finite number
 #pragma unroll
     for (int i = 0; i < C::TM; ++i)

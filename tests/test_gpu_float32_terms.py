@@ -79,6 +79,46 @@ def test_no_less_accurate_than_the_float32_instruction(name, op, low, high):
     assert error[0] <= error[1]
 
 
+@pytest.mark.parametrize("name", TERMS)
+def test_groups_of_few_rows_are_no_less_accurate(name):
+    """A product alone is rounded once on the float32 instruction; with few of them what the terms leave out shows."""
+    rng = np.random.default_rng(9)
+    k, n, few = 256, 512, [1, 2, 3, 4, 5, 6, 8, 12, 16, 24]
+    sizes = few + few[::-1]
+    a, b = operands(2, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    want, _ = reference(2, a, b, sizes)
+    got, whole = (product(2, a, b, sizes, v) for v in (name, WHOLE))
+    for i, rows in enumerate(sizes):
+        assert np.linalg.norm(got[i] - want[i]) <= np.linalg.norm(whole[i] - want[i]), rows
+
+
+@pytest.mark.parametrize("k,n", [(8, 8), (57, 77), (129, 257), (256, 512)])
+@pytest.mark.parametrize("name", TERMS)
+def test_groups_of_one_and_two_rows_have_the_float32_instructions_bits(name, k, n):
+    rng = np.random.default_rng(k)
+    sizes = [1, 2, 0, 2, 1, 40, 1, 2]
+    a, b = operands(2, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    a[0, ::3], b[1, ::2], a[3, 1], b[4, 2], a[5, 3], a[46, ::4] = 0, 0, np.inf, np.nan, 1e-40, 2.0 ** -70
+    b[46] *= 2.0 ** -60
+    got, whole = (product(2, a, b, sizes, v) for v in (name, WHOLE))
+    some = [i for i, rows in enumerate(sizes) if rows <= 2]
+    assert np.array_equal(got[some].view(np.int32)[~np.isnan(got[some])], whole[some].view(np.int32)[~np.isnan(whole[some])])
+    assert np.array_equal(np.isnan(got[some]), np.isnan(whole[some])) and np.isnan(got[some]).any()
+
+
+@pytest.mark.parametrize("name,op", CASES)
+@pytest.mark.parametrize("low,high", [(-50, -50), (-60, -60), (-62, -62), (-63, -63), (-64, -64), (-66, -66), (-70, -50), (-100, -20)])
+def test_products_near_the_bottom_of_the_range(name, op, low, high):
+    """Products of terms, and from 2^-126 down sums too, below the normal numbers: no less accurate than the float32 instruction."""
+    rng = np.random.default_rng(11)
+    k, n, sizes = 512, 256, [400, 112]
+    a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    a, b = (np.ldexp(np.where(np.abs(v) < 0.25, 0.25, v), by).astype(np.float32) for v, by in ((a, low), (b, high)))
+    want, _ = reference(op, a, b, sizes)
+    error = [np.linalg.norm((product(op, a, b, sizes, v) - want) * 2.0 ** 100) for v in (name, WHOLE)]  # (norms of squares above 2^-1022)
+    assert error[0] <= error[1]
+
+
 ODD_ONES = [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38, 1e-40, 2.0 ** -111, 1e30]
 
 
