@@ -383,7 +383,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
   }
 }
 
-// tgmm tiles of at most this many rows store the lines at their edges plainly where the rows of dA are no whole number of
+// tgmm tiles of at most this many rows (16-bit results) store the lines at their edges plainly where the rows of dA are no whole number of
 // 64-byte halves of a line (store_accumulators()) and the groups average no more (tgmm_impl()).  A kernel of its own: in one
 // kernel for both the mere branch cost launches with whole lines 1 to 3 %, those of the four-wave 256 x 256 core 5 %.  Times with over
 // without, geometric means over 1640 random calls with such rows, groups averaging under 20 | 20 to 40 | 40 to 60 | 60 to 80 | 80 to
@@ -395,12 +395,29 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void gmm_kernel(GmmArgs p) 
 //   256 x 256, float8                         0.87 | 0.89 | 0.90 | 0.92 | 0.99 | 1.03
 // 364 x 5376 x 9584 in 33 groups (128 x 128) 1412 -> 955 us, 2640 x 2048 x 1000 in 33 60 -> 39.  Rows of whole halves: 1.04, up to 1.3
 // (7459 x 14112 x 544 in 199 groups 933 | 996).  Not for the bf16 and float16 256 x 256 cores, whose tiles are for longer groups.
-constexpr int kEdgeLineRows = 80;
+//
+// float32 results of the any-pitch core: a half wave stores 32 columns of a row at a time, so that inside a tile too every line goes out in two
+// parts where rows are no whole number of halves.  Those tiles are stored plainly altogether.  Times with over without, 1100 to 1700 random
+// calls with such rows, by rows of a group 4 to 20 | 20 to 40 | 40 to 60 | 60 to 80 | 80 to 100 | 100 to 120 | 120 to 160 | 240 to 400:
+//   rounded to bf16, 128 x 128, multiples of 8    0.70 | 0.69 | 0.73 | 0.79 | 0.82 | 0.84 | 0.89 | 0.95
+//                    256 x 256                    0.64 | 0.61 | 0.65 | 0.69 | 0.72 | 0.73 | 0.76 | 0.84
+//                    128 x 128, other pitches     0.61 | 0.63 | 0.62 | 0.69 | 0.74 | 0.73 | 0.76 | 0.89
+//                    256 x 256                    0.57 | 0.57 | 0.56 | 0.61 | 0.68 | 0.62 | 0.66 | 0.80
+//   as terms, 128 x 256                           0.76 | 0.84 | 0.84 | 0.89 | 0.93 | 0.92 | 0.95 | 0.99
+//   as terms, 128 x 128                           0.98 | 1.05 | 1.04 | 1.05 | 1.04 | 1.03 | 1.02 | 1.01   (not for this one, nor for
+//   float32 instruction, 64 x 64                  1.03 | 1.05 | 1.05 | 1.05 | 1.04 | 1.02 | 1.01 | 0.99    this one)
+// Rounded to bf16, us: 50 x 5112 x 13016 in 6 groups 779 -> 345 (64 x 64 tile 392), 606 x 3928 x 2472 in 72 1253 -> 662 (717), 270 x 1050 x 14931
+// in 3 139 -> 64 (83).
+constexpr int kEdgeLineRows = 80, kEdgeLineRowsF32 = 120;
 template <class C, class = void>
 struct StoresEdgeLines { static constexpr bool value = IsF8Direct<C>::value || IsWs<C>::value; };
 template <class C>
 struct StoresEdgeLines<C, typename std::enable_if<C::DLDS && !C::PINGPONG && !IsF8Direct<C>::value && !IsWs<C>::value>::type> {
   static constexpr bool value = !IsW4<C>::value && !IsW4R<C>::value;
+};
+template <class C>
+struct StoresEdgeLines<C, typename std::enable_if<IsRs<C>::value>::type> {
+  static constexpr bool value = sizeof(typename C::Elem) == 4 && !C::FULL && !(C::THREE && C::BN < 256);
 };
 
 template <class C, bool EDGE_LINES = false>
@@ -445,7 +462,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p
   const E* Ap = static_cast<const E*>(p.x) + (size_t)row0 * p.k + kk0;
   const E* Bp = static_cast<const E*>(p.dy) + (size_t)row0 * p.n + col0;
   SplitK sk;
-  sk.edge_lines = EDGE_LINES && rows <= kEdgeLineRows;
+  sk.edge_lines = EDGE_LINES && rows <= (sizeof(O) == 4 ? kEdgeLineRowsF32 : kEdgeLineRows);
   run_tile<C>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem, sk);
 }
 
