@@ -14,8 +14,17 @@ SIZES = [(9000, 1000, 1504, 6, "cr256x256x32_w2x4", "cr128x128x32_w2x2"), (6000,
          (1270, 1000, 1504, 40, "cr128x128x32_w2x2", "cr128x128x32_w2x2"), (255, 520, 496, 32, "cr128x128x32_w2x2", "c64x64x32_w2x2"),
          (1500, 512, 48, 4, "c64x64x32_w2x2", "cr128x128x32_w2x2"), (240, 512, 64, 4, "cr128x128x32_w2x2", "c64x64x32_w2x2"),
          (9000, 1001, 1515, 6, "cs256x256x32_w2x4", "cs128x128x32_w2x2"), (2800, 265, 703, 45, "cs128x128x32_w2x2", "c64x64x32_w2x2"),
-         (300, 31, 99, 2, "c64x64x32_w2x2", "cs128x128x32_w2x2"), (300, 33, 99, 2, "cs128x128x32_w2x2", "cs128x128x32_w2x2"),
-         (300, 7, 99, 2, "c64x64x32_w2x2", "c64x64x32_w2x2")]
+         (300, 31, 99, 2, "c64x64x32_w2x2", "c64x64x32_w2x2"), (300, 33, 99, 2, "c64x64x32_w2x2", "c64x64x32_w2x2"),
+         (300, 7, 99, 2, "c64x64x32_w2x2", "c64x64x32_w2x2"),
+         # brief launches, and their neighbours with a few more tiles, a longer contraction or longer groups
+         (1000, 120, 960, 4, "cr128x128x32_w2x2", "cr128x128x32_w2x2"), (1000, 120, 896, 4, "c64x64x32_w2x2", "cr128x128x32_w2x2"),
+         (1000, 136, 896, 4, "cr128x128x32_w2x2", "cr128x128x32_w2x2"), (768, 512, 512, 6, "cr128x128x32_w2x2", "c64x64x32_w2x2"),
+         (768, 576, 512, 7, "cr128x128x32_w2x2", "c64x64x32_w2x2"), (768, 576, 576, 7, "cr128x128x32_w2x2", "cr128x128x32_w2x2"),
+         (900, 250, 900, 2, "c64x64x32_w2x2", "cs128x128x32_w2x2"), (900, 250, 1100, 2, "cs128x128x32_w2x2", "cs128x128x32_w2x2"),
+         (900, 270, 900, 2, "cs128x128x32_w2x2", "cs128x128x32_w2x2"), (900, 509, 900, 8, "cs128x128x32_w2x2", "c64x64x32_w2x2"),
+         (900, 509, 1100, 8, "cs128x128x32_w2x2", "cs128x128x32_w2x2"), (9000, 45, 1900, 5, "c64x64x32_w2x2", "cs128x128x32_w2x2"),
+         (9000, 45, 1700, 5, "cs128x128x32_w2x2", "cs128x128x32_w2x2"), (760, 509, 900, 5, "cs128x128x32_w2x2", "cs128x128x32_w2x2"),
+         (760, 450, 700, 5, "cs128x128x32_w2x2", "c64x64x32_w2x2"), (760, 125, 700, 3, "c64x64x32_w2x2", "c64x64x32_w2x2")]
 OPS = (_capi.OP_GMM, _capi.OP_TGMM)
 
 
