@@ -12,8 +12,9 @@ from tests import util
 
 TILES = {256: "x256x256x64_w2x4_s4", 128: "x128x256x64_w2x4_s3", 64: "x64x256x64_w1x4_s8"}
 # m, k, n, g, tile of gmm, tile of gmm on weights [g, n, k]
-SIZES = [(2283, 240, 3152, 7, 128, 128), (9000, 208, 4096, 5, 128, 128), (300, 256, 528, 2, 64, 128), (16384, 4096, 14336, 8, 256, 256),
-         (2283, 1680, 3152, 7, 256, 256), (596, 6400, 288, 213, 128, 128)]
+SIZES = [(2283, 240, 3152, 7, 128, 128), (9000, 208, 4096, 5, 128, 128), (300, 256, 528, 2, 64, 64), (16384, 4096, 14336, 8, 256, 256),
+         (2283, 1680, 3152, 7, 256, 256), (596, 6400, 288, 213, 128, 128),
+         (1000, 208, 3840, 2, 64, 64), (1000, 208, 4096, 2, 128, 128), (64, 16, 64, 3, 64, 64)]  # up to a round of 64 x 256 tiles
 
 
 @pytest.mark.parametrize("m,k,n,g,gmm,gmm_t", SIZES)
