@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 # m, k, n, g, taken: a round of tiles, two rounds; contractions and tile counts below the lines; short groups
 SIZES = [(2178, 831, 2203, 3, True), (3000, 701, 1601, 4, True), (3900, 1501, 1030, 5, True), (6700, 303, 1799, 3, True),
-         (2178, 699, 2203, 3, False), (1100, 831, 2203, 3, False), (2178, 831, 2203, 30, False)]
+         (2178, 699, 2203, 3, False), (1100, 831, 2203, 3, False), (2178, 831, 2203, 30, False),
+         (3000, 701, 1301, 4, True), (2800, 1001, 1301, 4, False)]  # 156 and 144 tiles
 
 
 # m, k, n, g, tile: few tiles and contractions on either side of the 64 x 64 tile's lines; up to four rounds of 128 x 256 tiles, and more
@@ -60,7 +61,8 @@ def _check(m, k, n, g, dtype, expected):
 
 # m, k, n, g, whether tgmm takes the 128 x 128 tile: rows of a group times tiles, rows alone, few columns
 @pytest.mark.parametrize("m,k,n,g,taken", [(9000, 65, 99, 3, False), (9000, 165, 199, 3, True), (9000, 301, 77, 3, True), (4000, 301, 77, 16, False),
-                                           (9000, 301, 55, 8, False)])
+                                           (9000, 301, 55, 8, False), (1304, 137, 1358, 4, False), (3000, 301, 301, 5, False),
+                                           (3000, 601, 601, 5, True), (3000, 401, 501, 3, False), (3000, 701, 901, 3, True)])
 def test_tgmm_few_tiles(m, k, n, g, taken):
     name = _capi.variants()[_capi.default_plan(_capi.OP_TGMM, m, k, n, g, _capi.RD_DTYPE_BF16).variant].name.decode()
     assert name == ("r128x128x64_w2x2" if taken else "s64x64x32_w2x2")
