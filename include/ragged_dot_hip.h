@@ -78,7 +78,9 @@ typedef struct rd_variant_info {
 
 /* Launch plan for one call; the host planner (or the caller) fills it.  variant = -1 with every other field 0 = library defaults. */
 typedef struct rd_plan {
-  int variant; /* index into the variant table, or -1: let the library choose by shape */
+  int variant; /* index into the variant table, or -1: let the library choose by shape.  rd_gmm on float32: with split_k = 0 a plan that
+                  names ft128x128x32_w2x4 leaves to the library whether a work-group takes two columns of its tiles at a time
+                  (ft128x256x32_w2x4, whose last round is computed in 128 x 128 halves; the same workspace); split_k = -1 or more than 0 runs it as named */
   int group_m; /* tile walk.  rd_gmm: a group's row tiles are cut into bands of at most group_m (1..127) row tiles and the
                   walk goes band by band, column by column inside a band.  rd_tgmm: row tiles per band.  0 = default */
   int group_n; /* rd_gmm: the walk is dealt to the 8 XCDs in blocks of group_m x group_n (<= 4096) consecutive tiles;

@@ -181,3 +181,25 @@ def test_another_groups_numbers_do_not_reach_a_group(name, op, k, n):
     hit = np.zeros(len(got), bool)
     hit[4 if op == 2 else slice(first, first + rows)] = True
     assert np.isnan(got[hit]).all() and np.array_equal(got[~hit], clean[~hit])
+
+
+def test_a_named_tile_is_the_one_that_runs():
+    """356 tiles of 128 x 128, the last 100 of them in two pieces, or 178 of 128 x 256, too many to be halved: other sums, whichever the
+    library would choose itself."""
+    rng = np.random.default_rng(13)
+    k, n, sizes = 4096, 512, [89 * 128]
+    a, b = operands(0, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    cut, whole, wide = (product(0, a, b, sizes, name, split_k) for name, split_k in (("ft128x128x32_w2x4", 2), ("ft128x128x32_w2x4", -1), ("ft128x256x32_w2x4", 2)))
+    assert not np.array_equal(cut, whole) and np.array_equal(wide, whole)
+
+
+@pytest.mark.parametrize("m,k,n,g", [(3000, 2048, 1111, 5), (4096, 2048, 2048, 4), (777, 333, 421, 5)])
+def test_default_tile_without_pieces(m, k, n, g):
+    """split_k = -1 with the library's own tile: the choice counts no halves and no pieces."""
+    rng = np.random.default_rng(k)
+    sizes = rng.multinomial(m, np.ones(g) / g).tolist()
+    a, b = operands(0, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+    want, magnitudes = reference(0, a, b, sizes)
+    x, w, gs = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), torch.tensor(sizes, dtype=torch.int32).cuda()
+    got = ops._gmm_fwd(x, w, gs, **HP, trans_rhs=False, plan=_capi.Plan(-1, split_k=-1)).cpu().numpy()
+    assert (np.abs(got - want) <= k * 2.0 ** -24 * magnitudes).all()
