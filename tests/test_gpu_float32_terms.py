@@ -183,6 +183,18 @@ def test_another_groups_numbers_do_not_reach_a_group(name, op, k, n):
     assert np.isnan(got[hit]).all() and np.array_equal(got[~hit], clean[~hit])
 
 
+@pytest.mark.parametrize("k,n,names", [(2048, 56, [WHOLE]), (2048, 128, TERMS), (63, 4000, ["ft64x128x32_w2x2", WHOLE]), (64, 4000, TERMS)])
+def test_narrow_and_short_products(k, n, names):
+    rng = np.random.default_rng(k)
+    sizes = [300, 0, 1700, 1, 999]
+    for op in (0, 1):
+        name = _capi.variants()[_capi.default_plan(op, sum(sizes), k, n, len(sizes), _capi.RD_DTYPE_F32).variant].name.decode()
+        assert name in names
+        a, b = operands(op, k, n, sizes, lambda shape: rng.standard_normal(shape).astype(np.float32))
+        want, magnitudes = reference(op, a, b, sizes)
+        assert (np.abs(product(op, a, b, sizes, name) - want) <= k * 2.0 ** -24 * magnitudes).all()
+
+
 def test_a_named_tile_is_the_one_that_runs():
     """356 tiles of 128 x 128, the last 100 of them in two pieces, or 178 of 128 x 256, too many to be halved: other sums, whichever the
     library would choose itself."""
