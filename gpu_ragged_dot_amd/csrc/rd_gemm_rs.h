@@ -497,9 +497,9 @@ __device__ __forceinline__ void rs_store16(const f32x16_t (&acc)[C::TM][C::TN], 
 
 // float32 results: register v of a 32 x 32 block is 32 consecutive columns of row 8 (v >> 2) + 4 (lane >> 5) + (v & 3) - a
 // whole 128-byte line per half wave.  Rows and columns past the tile's limits get an offset outside the output's window,
-// which the hardware drops.  Nontemporal, as in store_accumulators(); edge_lines: plainly, where rows are no whole number of 64-byte halves of
+// which the hardware drops.  Nontemporal, as in store_accumulators(); with SplitK::edge_lines plainly, where rows are no whole number of 64-byte halves of
 // a line, so that what a half wave stores ends inside two lines and L2 has to put them together (kEdgeLineRows in rd_kernels.h).
-template <class C, int POLICY>
+template <class C, int POLICY = kCachePolicyStream>
 __device__ __forceinline__ void rs_store32(const f32x16_t (&acc)[C::TM][C::TN], int wm, int wn, int lane, int a_lim, int b_lim,
                                            float* __restrict__ Op, int ldo) {
   const int bytes = ((a_lim - 1) * ldo + b_lim) * 4;  // below 2 GiB: checked on the host
@@ -518,18 +518,12 @@ __device__ __forceinline__ void rs_store32(const f32x16_t (&acc)[C::TM][C::TN], 
       }
     }
 }
-template <class C>
-__device__ __forceinline__ void rs_store32(const f32x16_t (&acc)[C::TM][C::TN], int wm, int wn, int lane, int a_lim, int b_lim,
-                                           float* __restrict__ Op, int ldo, bool edge_lines) {
-  if (edge_lines) rs_store32<C, 0>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
-  else rs_store32<C, kCachePolicyStream>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
-}
 
 // A tgmm tile of one or two rows: a product, and another one added with one rounding, the bits of the float32 matrix-core instruction.
 // Bound by its stores.  230 groups of one row among 256 of 16384 rows, k 2048, n 768: 502 us, as slabs of 32 indices on FULL 814, on terms 719.
-template <class C>
+template <class C, int POLICY>
 __device__ __forceinline__ void rs_few_products(const float* __restrict__ Ap, int lda, int a_lim, const float* __restrict__ Bp, int ldb,
-                                                int b_lim, int klen, int wm, int wn, int lane, float* __restrict__ Op, int ldo, bool edge_lines) {
+                                                int b_lim, int klen, int wm, int wn, int lane, float* __restrict__ Op, int ldo) {
   const float* __restrict__ A1 = Ap + (size_t)(klen - 1) * lda;  // the second row, or the first one again
   const float* __restrict__ B1 = Bp + (size_t)(klen - 1) * ldb;
   float b0[C::TN], b1[C::TN];
@@ -551,12 +545,12 @@ __device__ __forceinline__ void rs_few_products(const float* __restrict__ Ap, in
         acc[i][j][v] = klen > 1 ? fmaf(a1, b1[j], f) : f;
       }
     }
-  rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo, edge_lines);
+  rs_store32<C, POLICY>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
 }
 
 // Same contract as gemm_tile(), and: the rows the operands are read along hold at least 8 elements (16-bit) or 4
 // (float32) up to and including the tile's last one - k >= 8 and n >= 8.
-template <class C>
+template <class C, bool EDGE_LINES = false>
 __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict__ Ap, int lda, int a_lim,
                                              const typename C::Elem* __restrict__ Bp, int ldb, int b_lim, int klen,
                                              typename C::Elem* __restrict__ Op, int ldo, unsigned char* smem,
@@ -568,7 +562,8 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
 
   if constexpr (C::THREE && !C::A_KMAJOR) {
     if (klen <= kFewProducts) {
-      rs_few_products<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, wm, wn, lane, Op, ldo, sk.edge_lines);
+      if (EDGE_LINES && sk.edge_lines) rs_few_products<C, 0>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, wm, wn, lane, Op, ldo);
+      else rs_few_products<C, kCachePolicyStream>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, wm, wn, lane, Op, ldo);
       return;
     }
   }
@@ -617,7 +612,8 @@ __device__ __forceinline__ void gemm_tile_rs(const typename C::Elem* __restrict_
 
   if (!splitk_combine<C>(acc, sk, tid, smem)) return;
   if constexpr (sizeof(typename C::Elem) == 2) rs_store16<C>(acc, wm, wn, wave, lane, a_lim, b_lim, Op, ldo, smem);
-  else rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo, sk.edge_lines);
+  else if (EDGE_LINES && sk.edge_lines) rs_store32<C, 0>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
+  else rs_store32<C>(acc, wm, wn, lane, a_lim, b_lim, Op, ldo);
 }
 
 // A row tile of a gmm launch with fewer rows than its height: the same routine on the least multiple of 64 that holds them,

@@ -83,12 +83,12 @@ struct OutOf<C, decltype((void)sizeof(typename C::Out))> { typedef typename C::O
 
 constexpr int kW4RMinK = 1792;  // measured: level at 1536, 7 % ahead at 2048, 13 % at 8192 (eight groups of 2048 rows)
 
-template <class C>
+template <class C, bool EDGE_LINES = false>
 __device__ __forceinline__ void run_tile(const typename C::Elem* Ap, int lda, int a_lim, const typename C::Elem* Bp,
                                          int ldb, int b_lim, int klen, typename OutOf<C>::type* Op, int ldo,
                                          typename C::Elem* smem, const SplitK& sk = SplitK()) {
   if constexpr (C::F32) gemm_tile_f32<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem);
-  else if constexpr (IsRs<C>::value) gemm_tile_rs<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, reinterpret_cast<unsigned char*>(smem), sk);
+  else if constexpr (IsRs<C>::value) gemm_tile_rs<C, EDGE_LINES>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, reinterpret_cast<unsigned char*>(smem), sk);
   else if constexpr (IsF8Direct<C>::value) {
     if constexpr (C::PINGPONG) gemm_tile_f8_pingpong<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
     else gemm_tile_f8<C>(Ap, lda, a_lim, Bp, ldb, b_lim, klen, Op, ldo, smem, sk);
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES_PER_EU) void tgmm_kernel(TgmmArgs p
   const E* Bp = static_cast<const E*>(p.dy) + (size_t)row0 * p.n + col0;
   SplitK sk;
   sk.edge_lines = EDGE_LINES && rows <= (sizeof(O) == 4 ? kEdgeLineRowsF32 : kEdgeLineRows);
-  run_tile<C>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem, sk);
+  run_tile<C, EDGE_LINES>(Ap, p.k, krows, Bp, p.n, cols, rows, Op, p.n, smem, sk);
 }
 
 // ---- host-side launchers, one set per compiled tile shape -------------------------------------------------------
