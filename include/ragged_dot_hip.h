@@ -92,11 +92,14 @@ typedef struct rd_plan {
                     this many columns (32, 64 or 128) of one expert; RD_DECODE_ROWS the one that gives it whole rows
                     for a slice of the contraction range (fp32 partial sums in the workspace, n <= 2048) or, with
                     trans_rhs, whole weight rows of a slice of the columns (no partial sums, k <= 8192) */
-  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round and k >= 6400 (float8: 12800, float32: 1067,
-                  the variants v* and hv*: 3658 where about half a round of tiles or less is expected, 5700 otherwise), cut
-                  those tiles' contraction range over up to sqrt(k)/20 work-groups (float32: sqrt(k)/8, v* and hv*: sqrt(k)/15; fp32 partial
-                  sums in the workspace); n > 0 = cut them over up to n (at most 8) whatever k is; -1 = never.  A default plan may name
-                  one of v* / hv* for any bfloat16 or float16 call: who relies on uncut sums asks for -1 */
+  int split_k; /* rd_gmm only: 0 = when the tiles do not fill the device's last round, cut those tiles' contraction range over several
+                  work-groups where that pays (fp32 partial sums in the workspace, at most 8 pieces).  The direct-to-LDS 256 x 256 tiles (w*, p*, q*, x*, h*): by
+                  what a cut saves and costs, from k = 1024 on - with 10 tiles in an only round 2 pieces at 1024, 3 at 2048, 4 at 3000, 6 at 6000;
+                  with 90 tiles in a last round behind others 2 pieces from about 3700 on (float8: of half the contraction; p128x256x32 and d128x128x32:
+                  the next rule).  The others from k >= 6400 on (x64x256 and x128x256: 12800, ft*: 1067, fr*: 800, the variants v* and hv*: 3658 where about half a round of tiles or less
+                  is expected, 5700 otherwise), into up to sqrt(k)/20 pieces (x*: sqrt(k)/28, ft*: sqrt(k)/8, fr*: sqrt(k)/7, v* and hv*: sqrt(k)/15).
+                  So the last bits of a row may follow from the other groups' sizes.  n > 0 = cut them over up to n (at most 8) whatever k is;
+                  -1 = never.  A default plan may name a tile that is cut for any call: who relies on uncut sums asks for -1 */
 } rd_plan;
 
 int rd_abi_version(void);

@@ -67,6 +67,23 @@ def test_every_magnitude(name, op, k, n, sizes):
     assert (np.abs(got - want) <= (length + 1) * 2.0 ** -24 * magnitudes).all()
 
 
+@pytest.mark.parametrize("k,n,sizes", SHAPES + [(65, 513, [300, 1, 0, 129]), (200, 250, [128, 127, 200])])
+@pytest.mark.parametrize("op", [0, 1])
+def test_whole_tiles_of_256_columns(op, k, n, sizes):
+    """With the cut off every tile of 128 x 256 is computed whole; otherwise launches of under a round are all halves."""
+    rng = np.random.default_rng(k + n + 1)
+    a, b = operands(op, k, n, sizes, lambda shape: (rng.standard_normal(shape) * np.exp2(rng.integers(-30, 31, shape))).astype(np.float32))
+    want, magnitudes = reference(op, a, b, sizes)
+    got = product(op, a, b, sizes, TERMS[0], -1)
+    assert (np.abs(got - want) <= (k + 1) * 2.0 ** -24 * magnitudes).all()
+    # another group's numbers stay out: loads past a row or a group would bring NaN
+    last = len(sizes) - 1
+    a[sum(sizes[:last]):], b[last] = np.nan, np.nan
+    again = product(op, a, b, sizes, TERMS[0], -1)
+    rows = sum(sizes[:last])
+    assert np.array_equal(again[:rows], got[:rows]) and np.isnan(again[rows:]).all()
+
+
 @pytest.mark.parametrize("name,op", CASES)
 @pytest.mark.parametrize("low,high", [(0, 0), (-108, 100), (100, -70)])
 def test_no_less_accurate_than_the_float32_instruction(name, op, low, high):
