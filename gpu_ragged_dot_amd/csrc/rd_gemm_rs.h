@@ -28,7 +28,7 @@
 //  * The terms are made on the way into LDS, which holds three planes of a slab in the bf16 layout, and all three of a
 //    fragment are read per substep: 24 matrix-core instructions per 12 fragments (128 x 256 tile, eight waves of 64 x 64), half the
 //    fragment reads of a bf16 product.  A piece's way takes 28 vector instructions, in seven steps spread over the gaps between matrix-core
-//    instructions; eight waves, two on a SIMD, keep the matrix cores busy 74 % of the time, four of 64 x 128 69 %.
+//    instructions; eight waves, two on a SIMD, keep the matrix cores busy 77 % of a work-group's time (profiles/any_pitch_core.md).
 //  * 16384 x 4096 x 2048 in one group, tgmm: 1274 us (216 TFLOP/s, i.e. 1294 on the bf16 matrix cores; 881 us on zeros), FULL on
 //    128 x 128 tiles 1879; 8192 x 2048 x 2048 in 16 softmax-sized groups, fwd / dlhs / drhs: 377 / 378 / 380, FULL 574 / 594 / 595.
 //    Power bounds it, as it does the bf16 products.
