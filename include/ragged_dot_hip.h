@@ -34,7 +34,7 @@ extern "C" {
  * cores multiply.  RD_DTYPE_F32: every number as three bf16 terms (all 24 bits), six products of terms on the bf16 matrix cores, fp32 sums;
  * numbers that terms do not hold (infinities, NaN, below 2^-110), and groups of one and two rows in rd_tgmm, are multiplied as float32.  The error
  * against exact sums is no larger than that of float32 products, but for a product that stands alone among zeros: 1.5 units
- * of 2^-24 at most instead of 1.  RD_DTYPE_F32_BF16 is compute_dtype = bfloat16 on float32 arrays (gpu_ragged_dot.py:116-119, 145, 149): the
+ * of 2^-24 at most instead of 1 (a plan that names fr64x64x32_w2x2 or f64x64x16_w2x2 multiplies as float32 throughout).  RD_DTYPE_F32_BF16 is compute_dtype = bfloat16 on float32 arrays (gpu_ragged_dot.py:116-119, 145, 149): the
  * float32 elements are rounded to bfloat16 (nearest even) as they are loaded, multiplied on the bf16 matrix cores with
  * fp32 accumulation, and stored as float32.  (compute_dtype = float32 on bfloat16 arrays is RD_DTYPE_BF16 itself: a
  * product of two bfloat16 values is exact in fp32, and the accumulation is fp32 either way.)
